@@ -293,9 +293,60 @@ def test_delta_rule_whole_portions_and_single_tokens(H, G, d, dv, per_channel):
     a_log, dt_bias = torch.randn(H, generator=g) * 0.5 - 1, torch.randn(decay.shape[1], generator=g) * 0.5
     ref = _delta_ref(qkv, beta, decay, a_log, dt_bias, H, G, d, dv, per_channel)
     for cuts in ([T], [1] * T, [2, 3, 1, 17, 2, 16]):
-        for long_chunks in (False, True):             # one column per lane; rows split over lanes (single tokens: always the former)
+        for long_chunks in (False, True):             # one column per lane; tiles of 16 rows (single tokens: always the former)
             got = _delta_in_cuts(qkv, beta, decay, a_log, dt_bias, cuts, H, G, d, dv, per_channel, long_chunks=long_chunks)
             assert (got - ref).abs().max() <= 3e-5 * ref.abs().max(), (cuts, long_chunks)
+
+
+@pytest.mark.parametrize("H,G,d,dv,per_channel,dtype", [(2, 1, 64, 64, False, torch.bfloat16), (2, 2, 128, 120, True, torch.bfloat16),
+                                                        (4, 2, 128, 128, False, torch.float16), (1, 1, 20, 17, False, torch.bfloat16),
+                                                        (1, 1, 192, 16, True, torch.float32), (2, 1, 136, 200, False, torch.float32),
+                                                        (1, 1, 256, 40, True, torch.bfloat16), (1, 1, 256, 300, False, torch.float16)])
+def test_delta_rule_tiles_of_a_mixed_batch(H, G, d, dv, per_channel, dtype):
+    """Chunks of 1, 15, 16, 17, 0, 64 and 33 rows side by side, some from a state, some at position 0 (whose slot holds
+    anything); some decays are far below what a float holds.  Against the recurrence in float64.  Bound: every number is a
+    float32 sum of up to d + 16 products of size <= 1 times the largest result, (256 + 16) 2^-24 = 1.6e-5."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(d)
+    lens = [1, 15, 16, 17, 0, 64, 33]
+    cu = torch.tensor([0] + lens).cumsum(0)
+    T, S, qk = int(cu[-1]), len(lens), G * d
+    first = [0, 3, 0, 100, 0, 0, 7]
+    qkv, beta = torch.randn(T, 2 * qk + H * dv, generator=g).to(dtype), torch.randn(T, H, generator=g).to(dtype)
+    decay = torch.randn(T, H * d if per_channel else H, generator=g)
+    decay[torch.rand(decay.shape, generator=g) < 0.05] = 60.0
+    decay = decay.to(dtype)
+    a_log, dt_bias = torch.randn(H, generator=g) * 0.5, torch.randn(decay.shape[1], generator=g) * 0.5
+    slots = torch.tensor([5, 0, 3, 1, 2, 6, 4], dtype=torch.int32)
+    state = torch.randn(S + 1, H, d, dv, generator=g)
+    start = state.double()
+    for s in range(S):
+        if first[s] == 0:
+            state[slots[s]] = float("nan")
+            start[slots[s]] = 0.0
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)])
+    dev = state.cuda()
+    out = ops.gated_delta_rule(qkv.cuda(), 0, qk, 2 * qk, beta.cuda(), decay.cuda(), a_log.cuda(), dt_bias.cuda(), dev,
+                               cu.to(torch.int32).cuda(), pos.cuda(), slots.cuda(), H, G, d, dv, per_channel=per_channel, long_chunks=True)
+    f = qkv.double()
+    q = (R.unit(f[:, :qk].view(T, G, d)) * d ** -0.5).repeat_interleave(H // G, dim=1)
+    k = R.unit(f[:, qk:2 * qk].view(T, G, d)).repeat_interleave(H // G, dim=1)
+    v, b = f[:, 2 * qk:].view(T, H, dv), torch.sigmoid(beta.double())
+    z = torch.nn.functional.softplus(decay.double() + dt_bias.double()).view(T, H, -1)
+    a = torch.exp(-torch.exp(a_log.double())[None, :, None] * z)
+    want = torch.zeros(T, H, dv, dtype=torch.float64)
+    for s in range(S):
+        St = start[slots[s]]
+        for t in range(int(cu[s]), int(cu[s + 1])):
+            St = a[t][:, :, None] * St
+            u = b[t][:, None] * (v[t] - torch.einsum("hdv,hd->hv", St, k[t]))
+            St = St + k[t][:, :, None] * u[:, None, :]
+            want[t] = torch.einsum("hdv,hd->hv", St, q[t])
+        if lens[s]:
+            assert (dev[slots[s]].cpu() - St).abs().max() <= 1.6e-5 * St.abs().max(), (s, "state")
+            rows = slice(int(cu[s]), int(cu[s + 1]))
+            assert (out[rows].cpu() - want[rows]).abs().max() <= 1.6e-5 * want[rows].abs().max(), s
+    assert torch.equal(dev[S].cpu(), state[S]) and torch.isnan(dev[slots[4]]).all()     # no chunk of theirs: untouched
 
 
 def test_delta_rule_keeps_a_far_write_and_loses_it_with_decay():

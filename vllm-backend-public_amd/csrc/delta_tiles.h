@@ -1,0 +1,26 @@
+// The gated delta rule over tiles of 16 rows (delta_tiles.hip), called by mi355_gated_delta_rule.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace mi355 {
+
+struct DeltaTiles {
+  float* o;                     // [rows][H][dv]
+  const void *qkv, *beta, *decay;
+  int64_t stride, beta_stride, decay_stride;
+  const float *a_log, *dt_bias;
+  float* state;                 // [slots][H][d][dv]
+  const int32_t *cu_seqlens, *state_slots;
+  const int64_t* positions;
+  float* ws;
+  int64_t rows;
+  int q_off, k_off, v_off, per_channel, S, H, G, d, dv;
+};
+
+// floats of workspace
+int64_t delta_tiles_workspace(int64_t rows, int H, int d);
+// dtype: an mi355_dtype code; d at most 256
+void launch_delta_tiles(const DeltaTiles& a, int dtype, hipStream_t stream);
+
+}  // namespace mi355

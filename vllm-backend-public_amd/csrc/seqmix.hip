@@ -19,6 +19,7 @@
 //   mingru_scan             S <- (1 - z) S + z c per channel, z = sigmoid(zp + bz), c = u + 1/2 (u >= 0) or sigmoid(u),
 //                           u = xp + bx; out = S * silu(gp)
 #include "common.h"
+#include "delta_tiles.h"
 
 namespace mi355 {
 
@@ -460,15 +461,6 @@ __global__ __launch_bounds__(64) void gated_delta_rule_kernel(
   }
 }
 
-// ---- the gated delta rule for chunks of many tokens -------------------------------------------------
-// With one state column per lane a token costs 4 * d dependent vector operations per wave and a
-// prompt keeps only heads * dv / 64 waves busy.  Here the d rows of a column are split over R = 16
-// (or 8) adjacent lanes (a wave holds 64 / R columns, DR = ceil(d / R) rows each), the two dot products
-// of a token are finished with four (three) cross-lane steps each, and everything that does not depend on the
-// state -- unit-length key and query, decay, beta -- is computed for all tokens at once by
-// delta_prep_kernel, in fp32, into rows padded to R * DR (key / query 0, decay 1 in the padding).
-// The loop then reads the next token's rows while it works on the current one.
-
 // sum over the 8 adjacent lanes of a group, in every lane of it, by data-parallel-primitive moves
 // (no trip through the LDS crossbar): swap within pairs, swap pairs within quads, mirror the half row
 template <int CTRL>
@@ -482,138 +474,6 @@ __device__ __forceinline__ float sum_lanes(float v) {
   v += dpp_move<0x141>(v);      // row_half_mirror: lane i of 8 takes lane 7 - i
   if (R == 16) v += dpp_move<0x128>(v);   // row_ror 8: the other half of the 16-lane row
   return v;
-}
-
-template <typename T>
-__global__ __launch_bounds__(64) void delta_prep_kernel(
-    float* __restrict__ kq, float* __restrict__ dec, float* __restrict__ bet, const typename Elem<T>::S* __restrict__ qkv,
-    int64_t stride, int q_off, int k_off, const typename Elem<T>::S* __restrict__ beta, int64_t beta_stride,
-    const typename Elem<T>::S* __restrict__ decay, int64_t decay_stride, const float* __restrict__ a_log,
-    const float* __restrict__ dt_bias, int per_channel, int H, int G, int d, int dp) {
-  const int64_t t = blockIdx.x;
-  const int y = blockIdx.y, lane = threadIdx.x;
-  if (y < G) {                                          // unit-length key and scaled unit-length query of kv head y
-    const typename Elem<T>::S* row = qkv + t * stride;
-    float kk = 0.f, qq = 0.f;
-    for (int c = lane; c < d; c += 64) {
-      const float kv = MI355_LDF(T, qkv, row + k_off + y * d + c), qv = MI355_LDF(T, qkv, row + q_off + y * d + c);
-      kk += kv * kv;
-      qq += qv * qv;
-    }
-    kk = 1.0f / sqrtf(wave_sum(kk) + 1e-6f);
-    qq = (1.0f / sqrtf(static_cast<float>(d))) / sqrtf(wave_sum(qq) + 1e-6f);
-    float* o = kq + (t * G + y) * 2 * dp;
-    for (int c = lane; c < dp; c += 64) {
-      MI355_ST(float, kq, o + c, c < d ? MI355_LDF(T, qkv, row + k_off + y * d + c) * kk : 0.f);
-      MI355_ST(float, kq, o + dp + c, c < d ? MI355_LDF(T, qkv, row + q_off + y * d + c) * qq : 0.f);
-    }
-    return;
-  }
-  const int h = y - G;
-  const float na = -expf(MI355_LD(float, a_log, a_log + h));
-  float* o = dec + (t * H + h) * dp;
-  for (int c = lane; c < dp; c += 64) {
-    float a = 1.0f;
-    if (c < d) {
-      const float z = per_channel
-                          ? MI355_LDF(T, decay, decay + t * decay_stride + h * d + c) + MI355_LD(float, dt_bias, dt_bias + h * d + c)
-                          : MI355_LDF(T, decay, decay + t * decay_stride + h) + MI355_LD(float, dt_bias, dt_bias + h);
-      a = expf(na * (z > 20.0f ? z : log1pf(expf(z))));
-    }
-    MI355_ST(float, dec, o + c, a);
-  }
-  if (lane == 0)
-    MI355_ST(float, bet, bet + t * H + h, 1.0f / (1.0f + expf(-MI355_LDF(T, beta, beta + t * beta_stride + h))));
-}
-
-template <typename T, int R, int DR, int PF>
-__global__ __launch_bounds__(64) void gated_delta_rule_split_kernel(
-    float* __restrict__ o, const typename Elem<T>::S* __restrict__ qkv, int64_t stride, int v_off,
-    const float* __restrict__ kq, const float* __restrict__ dec, const float* __restrict__ bet, float* __restrict__ state,
-    const int32_t* __restrict__ cu_seqlens, const int64_t* __restrict__ positions,
-    const int32_t* __restrict__ state_slots, int H, int G, int d, int dv) {
-  constexpr int dp = R * DR;
-  const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int r = lane & (R - 1), col = blockIdx.z * (64 / R) + lane / R;
-  const int g = h / (H / G);
-  const int64_t cs = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s);
-  const int64_t n = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s + 1) - cs;
-  if (n <= 0) return;
-  const int64_t slot = MI355_LD(int32_t, state_slots, state_slots + s);
-  float* sp = state + ((slot * H + h) * d) * dv;
-  const bool live = col < dv;
-  const bool fresh = MI355_LD(int64_t, positions, positions + cs) == 0;
-  float S[DR];
-#pragma unroll
-  for (int j = 0; j < DR; ++j) {
-    const int i = r * DR + j;
-    S[j] = (live && !fresh && i < d) ? MI355_LD(float, state, sp + static_cast<int64_t>(i) * dv + col) : 0.f;
-  }
-  // Two register sets of PF tokens each: while one is worked on, the rows of the PF tokens after
-  // it travel into the other (a token's arithmetic is far shorter than a trip to memory).
-  struct Rows {
-    float k[PF][DR], q[PF][DR], a[PF][DR], b[PF], v[PF];
-  };
-  Rows A, B;
-  auto fetch = [&](Rows& w, int64_t first) {
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      int64_t t = first + u;
-      if (t > cs + n - 1) t = cs + n - 1;               // past the chunk: a row that is loaded and not used
-      const float* kp = kq + (t * G + g) * 2 * dp + r * DR;
-      const float* ap = dec + (t * H + h) * dp + r * DR;
-#pragma unroll
-      for (int j = 0; j < DR; j += 4) {
-        const float4 a4 = MI355_LD(float4, kq, kp + j), b4 = MI355_LD(float4, kq, kp + dp + j), c4 = MI355_LD(float4, dec, ap + j);
-        w.k[u][j] = a4.x, w.k[u][j + 1] = a4.y, w.k[u][j + 2] = a4.z, w.k[u][j + 3] = a4.w;
-        w.q[u][j] = b4.x, w.q[u][j + 1] = b4.y, w.q[u][j + 2] = b4.z, w.q[u][j + 3] = b4.w;
-        w.a[u][j] = c4.x, w.a[u][j + 1] = c4.y, w.a[u][j + 2] = c4.z, w.a[u][j + 3] = c4.w;
-      }
-      w.b[u] = MI355_LD(float, bet, bet + t * H + h);
-      w.v[u] = live ? MI355_LDF(T, qkv, qkv + t * stride + v_off + h * dv + col) : 0.f;
-    }
-  };
-  auto work = [&](const Rows& w, int64_t i0) {
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      if (i0 + u >= n) break;
-      float d0 = 0.f, d1 = 0.f;
-#pragma unroll
-      for (int j = 0; j < DR; j += 2) {
-        S[j] *= w.a[u][j];
-        S[j + 1] *= w.a[u][j + 1];
-        d0 += S[j] * w.k[u][j];
-        d1 += S[j + 1] * w.k[u][j + 1];
-      }
-      const float dot = sum_lanes<R>(d0 + d1);
-      const float uu = w.b[u] * (w.v[u] - dot);
-      float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-      for (int j = 0; j < DR; j += 2) {
-        S[j] += w.k[u][j] * uu;
-        S[j + 1] += w.k[u][j + 1] * uu;
-        o0 += S[j] * w.q[u][j];
-        o1 += S[j + 1] * w.q[u][j + 1];
-      }
-      const float out = sum_lanes<R>(o0 + o1);
-      if (live && r == 0) MI355_ST(float, o, o + ((cs + i0 + u) * H + h) * dv + col, out);
-    }
-  };
-  fetch(A, cs);
-  for (int64_t i0 = 0; i0 < n; i0 += 2 * PF) {
-    if (i0 + PF < n) fetch(B, cs + i0 + PF);
-    work(A, i0);
-    if (i0 + PF >= n) break;
-    if (i0 + 2 * PF < n) fetch(A, cs + i0 + 2 * PF);
-    work(B, i0 + PF);
-  }
-  if (live) {
-#pragma unroll
-    for (int j = 0; j < DR; ++j) {
-      const int i = r * DR + j;
-      if (i < d) MI355_ST(float, state, sp + static_cast<int64_t>(i) * dv + col, S[j]);
-    }
-  }
 }
 
 // ---- the general delta rule ------------------------------------------------------------------------
@@ -1116,8 +976,8 @@ static void launch_delta(hipStream_t s, float* o, const void* qkv, int64_t strid
 
 extern "C" int64_t mi355_gated_delta_rule_workspace(int64_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
                                                     int32_t head_dim) {
-  const int64_t dp = 8 * (head_dim <= 32 ? 4 : head_dim <= 64 ? 8 : head_dim <= 128 ? 16 : 32);
-  return num_tokens * (static_cast<int64_t>(num_kv_heads) * 2 * dp + static_cast<int64_t>(num_heads) * dp + num_heads + 4) / 4 * 4;
+  (void)num_kv_heads;
+  return delta_tiles_workspace(num_tokens, num_heads, head_dim);
 }
 
 extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t stride, int32_t q_off, int32_t k_off,
@@ -1139,36 +999,21 @@ extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t str
   if (num_seqs == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (workspace != nullptr && num_tokens > 0) {
-    // the form for chunks of many tokens: rows split over 8 lanes, per-token vectors prepared up front
-    // state rows of a column over 16 adjacent lanes (8 for heads of up to 32 rows); rows padded to dp
-    const int64_t dp = head_dim <= 32 ? 32 : head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : 256;
-    const int lanes = head_dim <= 32 ? 8 : 16;
+    // the form for chunks of many tokens: tiles of 16 rows on the matrix cores
     const int64_t need = mi355_gated_delta_rule_workspace(num_tokens, num_heads, num_kv_heads, head_dim);
     MI355_REQUIRE(workspace_floats >= need && aligned16(workspace), MI355_ERR_INVALID,
                   "gated_delta_rule: workspace of %lld floats, %lld needed, 16-byte aligned",
                   static_cast<long long>(workspace_floats), static_cast<long long>(need));
-    float* kq = workspace;
-    float* dec = kq + num_tokens * num_kv_heads * 2 * dp;
-    float* bet = dec + num_tokens * num_heads * dp;
-    const dim3 pgrid(static_cast<unsigned>(num_tokens), static_cast<unsigned>(num_kv_heads + num_heads));
-    const int cols = 64 / lanes;
-    const dim3 grid(static_cast<unsigned>(num_seqs), static_cast<unsigned>(num_heads), static_cast<unsigned>((v_dim + cols - 1) / cols));
-#define MI355_DSPLIT(TT, R, DR, PF)                                                                                   \
-  hipLaunchKernelGGL((gated_delta_rule_split_kernel<TT, R, DR, PF>), grid, dim3(64), 0, s, o,                         \
-                     static_cast<const Elem<TT>::S*>(qkv), stride, v_off, kq, dec, bet, state, cu_seqlens, positions, \
-                     state_slots, num_heads, num_kv_heads, head_dim, v_dim)
-    MI355_DISPATCH_DTYPE3(dtype, {
-      hipLaunchKernelGGL((delta_prep_kernel<TT>), pgrid, dim3(64), 0, s, kq, dec, bet, static_cast<const Elem<TT>::S*>(qkv),
-                         stride, q_off, k_off, static_cast<const Elem<TT>::S*>(beta), beta_stride,
-                         static_cast<const Elem<TT>::S*>(decay), decay_stride, a_log, dt_bias, per_channel, num_heads,
-                         num_kv_heads, head_dim, static_cast<int>(dp));
-      if (dp == 32) MI355_DSPLIT(TT, 8, 4, 4);
-      else if (dp == 64) MI355_DSPLIT(TT, 16, 4, 4);
-      else if (dp == 128) MI355_DSPLIT(TT, 16, 8, 4);
-      else MI355_DSPLIT(TT, 16, 16, 2);
-    });
-#undef MI355_DSPLIT
-    return check_launch("gated_delta_rule (split rows)");
+    DeltaTiles a = {};
+    a.o = o, a.qkv = qkv, a.beta = beta, a.decay = decay;
+    a.stride = stride, a.beta_stride = beta_stride, a.decay_stride = decay_stride;
+    a.a_log = a_log, a.dt_bias = dt_bias, a.state = state;
+    a.cu_seqlens = cu_seqlens, a.state_slots = state_slots, a.positions = positions;
+    a.ws = workspace, a.rows = num_tokens;
+    a.q_off = q_off, a.k_off = k_off, a.v_off = v_off, a.per_channel = per_channel;
+    a.S = num_seqs, a.H = num_heads, a.G = num_kv_heads, a.d = head_dim, a.dv = v_dim;
+    launch_delta_tiles(a, dtype, s);
+    return check_launch("gated_delta_rule (tiles)");
   }
   MI355_DISPATCH_DTYPE3(dtype, launch_delta<TT>(s, o, qkv, stride, q_off, k_off, v_off, beta, beta_stride, decay,
                                                decay_stride, a_log, dt_bias, per_channel, state, cu_seqlens, positions,

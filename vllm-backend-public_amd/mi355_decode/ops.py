@@ -1295,7 +1295,7 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
     [tokens, heads * head_dim] are raw projection outputs (column slices are fine); a_log [heads] and
     dt_bias (decay's width) float32; state float32 [slots, heads, head_dim, v_dim].
     Returns o float32 [tokens, heads, v_dim].  long_chunks: the batch holds chunks of many tokens -- take
-    the form that splits the state rows over lanes (it allocates a float32 workspace; not for graphs)."""
+    the form that goes by tiles of 16 rows (it allocates a float32 workspace; not for graphs)."""
     dt = _dt3(qkv, "qkv")
     T = qkv.shape[0]
     S = cu_seqlens.numel() - 1
