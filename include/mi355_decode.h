@@ -447,6 +447,18 @@ int32_t mi355_sample_topk_topp_hinted(int64_t* out_ids, const void* logits,
                                       const int64_t* steps, int32_t cut_rows, void* stream);
 
 /*
+ * The same with a workspace of mi355_sample_workspace(num_rows, logits_dtype) bytes (16-byte aligned, need not be
+ * cleared): every row, with a cut or without, is spread over many workgroups, and nothing is shared
+ * with other calls.  The same tokens.
+ */
+int64_t mi355_sample_workspace(int32_t num_rows, int32_t logits_dtype);
+int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logits, int64_t logits_stride,
+                                  int32_t num_rows, int32_t vocab, int32_t logits_dtype,
+                                  const float* temperature, const int32_t* top_k, const float* top_p,
+                                  const int64_t* seeds, const int64_t* steps, void* workspace,
+                                  int64_t workspace_bytes, void* stream);
+
+/*
  * Log-probabilities for the `logprobs` field of POST /v1/completions
  * (benchmark-deployer/docs/deployment/post_run.md:46):
  *   out_lse[b]     = log(sum_v exp(logits[b, v]))            (fp32, fixed-order sum)

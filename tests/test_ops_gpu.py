@@ -622,6 +622,38 @@ def test_linear_decode_strided_out_and_in(ops):
     assert float(yb[:, :128].abs().max()) == 0.0 and float(yb[:, 384:].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("ldt,B,V", [("bfloat16", 1, 16384), ("bfloat16", 64, 16391), ("bfloat16", 65, 16384), ("float16", 42, 18433),
+                                     ("float16", 43, 16390), ("float32", 32, 16387), ("float32", 33, 16384), ("bfloat16", 3, 131077)])
+def test_sample_spread_over_workgroups(ops, ldt, B, V):
+    """Either side of the line between a row spread over many workgroups and one workgroup a row, and rows whose cut
+    falls on the borders of the column ranges: the same tokens as the restatement and as without the hint, exactly."""
+    rng = np.random.default_rng(V + B)
+    tdt = {"float32": torch.float32, **DT}[ldt]
+    lg = torch.from_numpy(rng.normal(0, 3, (B, V)).astype(np.float32)).to(tdt)
+    temperature, top_k = np.full(B, 0.9, np.float32), rng.choice([-1, 1, 50, 2047, V - 1], B).astype(np.int32)
+    top_p = rng.choice([1.0, 0.95, 0.5, 1e-6], B).astype(np.float32)
+    for r in range(B):
+        if r % 7 == 1:
+            lg[r, 2040:2060] = 20.0                      # a tie over the border of two ranges, cut inside
+            top_k[r], top_p[r] = 5, 0.5
+        elif r % 7 == 2:
+            lg[r, rng.integers(0, V)] = float("nan")
+        elif r % 7 == 3:
+            lg[r, V - 1] = float("inf")
+        elif r % 7 == 4:
+            lg[r] = -float("inf")
+            lg[r, V - 3:] = 1.0
+        elif r % 7 == 5:
+            temperature[r], top_k[r], top_p[r] = (0.0, 3, 0.5) if r % 2 else (1.0, 0, 1.0)
+    seeds, steps = rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B, dtype=np.int64)
+    wide = torch.zeros(B, (V + 7) // 8 * 8, dtype=tdt, device="cuda")
+    wide[:, :V] = lg.cuda()
+    args = [torch.from_numpy(a).cuda() for a in (temperature, top_k, top_p, seeds, steps)]
+    ref = R.sample_topk_topp(lg.float().numpy(), temperature, top_k, top_p, seeds, steps)
+    np.testing.assert_array_equal(ops.sample(wide[:, :V], *args).cpu().numpy(), ref)
+    np.testing.assert_array_equal(ops.sample(wide[:, :V], *args, cut_rows=False).cpu().numpy(), ref)
+
+
 # --------------------------------------------------------------------------- #
 # random sampling: bit-exact token ids (fixed-order fp32 algorithm on both sides)
 # --------------------------------------------------------------------------- #

@@ -29,6 +29,37 @@ __device__ __forceinline__ unsigned long long umax64(unsigned long long a, unsig
   return a > b ? a : b;
 }
 
+// Inclusive scan of 64-bit values over the wave's lanes, 0 the neutral element, by data-parallel moves: shifts inside
+// the rows of 16 lanes, then a row's last lane to the next row, then lane 31 to the upper half.  (Six moves of two
+// registers; the same through the LDS crossbar took ten times as long, and a radix pick is little else.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp64(unsigned long long v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(v & 0xFFFFFFFFull), CTRL, ROWS, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(v >> 32), CTRL, ROWS, 0xF, false);
+  return (static_cast<unsigned long long>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo);
+}
+template <typename F>
+__device__ __forceinline__ unsigned long long wave_scan64(unsigned long long v, F&& op) {
+  v = op(v, dpp64<0x111, 0xF>(v));              // row_shr 1, 2, 4, 8 (lanes shifted in from outside a row: 0)
+  v = op(v, dpp64<0x112, 0xF>(v));
+  v = op(v, dpp64<0x114, 0xF>(v));
+  v = op(v, dpp64<0x118, 0xF>(v));
+  v = op(v, dpp64<0x142, 0xA>(v));              // row_bcast 15 into rows 1 and 3
+  v = op(v, dpp64<0x143, 0xC>(v));              // row_bcast 31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ unsigned long long lane64(unsigned long long v, int lane) {      // a lane's value, for all (lane uniform)
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(v & 0xFFFFFFFFull), lane);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(v >> 32), lane);
+  return (static_cast<unsigned long long>(hi) << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long wave_max64(unsigned long long v) {
+  return lane64(wave_scan64(v, [](unsigned long long a, unsigned long long b) { return umax64(a, b); }), 63);
+}
+__device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
+  return lane64(wave_scan64(v, [](unsigned long long a, unsigned long long b) { return a + b; }), 63);
+}
+
 // KEYED: out[row] is the row's best key itself, with the index moved by index_offset (the
 // position of this slice of the vocabulary in the whole one) and the top bit flipped so that
 // SIGNED 64-bit max over the slices' keys orders them as the unsigned keys do.
@@ -299,7 +330,7 @@ __device__ __forceinline__ void for_each_logit_in(const void* base, int vocab, i
   constexpr int PER = LDT == MI355_F32 ? 4 : 8;
   const int nvec = min(v1, vocab / PER);
 #pragma unroll UNROLL
-  for (int v = v0 + threadIdx.x; v < nvec; v += kSampleThreads) {
+  for (int v = v0 + threadIdx.x; v < nvec; v += static_cast<int>(blockDim.x)) {
     float f[8];
     if (LDT == MI355_F32) {
       const float4 q = MI355_LD(float4, base, static_cast<const float*>(base) + 4 * v);
@@ -312,7 +343,7 @@ __device__ __forceinline__ void for_each_logit_in(const void* base, int vocab, i
     for (int j = 0; j < PER; ++j) fn(f[j], v * PER + j);
   }
   if (tail)
-    for (int i = vocab / PER * PER + threadIdx.x; i < vocab; i += kSampleThreads) fn(load_logit<LDT>(base, i), i);
+    for (int i = vocab / PER * PER + threadIdx.x; i < vocab; i += static_cast<int>(blockDim.x)) fn(load_logit<LDT>(base, i), i);
 }
 
 // fn(f, n, i0) for every 16-byte vector of the row (n = 4 or 8 logits f[0, n) starting at index
@@ -331,7 +362,7 @@ __device__ __forceinline__ void for_each_vector_in(const void* base, int vocab, 
   constexpr int PER = LDT == MI355_F32 ? 4 : 8;
   const int nvec = min(v1, vocab / PER);
 #pragma unroll UNROLL
-  for (int v = v0 + threadIdx.x; v < nvec; v += kSampleThreads) {
+  for (int v = v0 + threadIdx.x; v < nvec; v += static_cast<int>(blockDim.x)) {
     float f[8];
     if (LDT == MI355_F32) {
       const float4 q = MI355_LD(float4, base, static_cast<const float*>(base) + 4 * v);
@@ -344,7 +375,7 @@ __device__ __forceinline__ void for_each_vector_in(const void* base, int vocab, 
     fn(f, PER, v * PER);
   }
   if (tail)
-    for (int i = vocab / PER * PER + threadIdx.x; i < vocab; i += kSampleThreads) {
+    for (int i = vocab / PER * PER + threadIdx.x; i < vocab; i += static_cast<int>(blockDim.x)) {
       float f[8] = {load_logit<LDT>(base, i), 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       fn(f, 1, i);
     }
@@ -352,13 +383,11 @@ __device__ __forceinline__ void for_each_vector_in(const void* base, int vocab, 
 
 // Workgroup-wide max of the 64-bit keys; thread 0 gets the result.
 __device__ __forceinline__ unsigned long long sample_reduce_max(unsigned long long best, unsigned long long* part) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) best = umax64(best, __shfl_xor(best, off, 64));
+  best = wave_max64(best);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
   __syncthreads();
   if (threadIdx.x == 0)
-#pragma unroll
-    for (int i = 1; i < kSampleThreads / 64; ++i) best = umax64(best, part[i]);
+    for (unsigned i = 1; i < blockDim.x >> 6; ++i) best = umax64(best, part[i]);
   return best;
 }
 
@@ -545,12 +574,6 @@ __device__ __forceinline__ void radix_pick64(const unsigned long long* hist, uns
   }
 }
 
-__device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 // for_each_vector that stops early: `go()` is asked before every vector of a thread (the tail elements are
 // visited only if it still says yes).
 template <int LDT, typename G, typename F>
@@ -600,7 +623,7 @@ __device__ __forceinline__ void ordered_kept_pass(const void* base, int vocab, i
                                                   uint32_t Tp, unsigned long long take,
                                                   unsigned long long ties_before, int* eq_base, F&& fn) {
   constexpr int PER = LDT == MI355_F32 ? 4 : 8;
-  constexpr int kWaves = kSampleThreads / 64;
+  const int kWaves = blockDim.x >> 6;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   v_end = min(v_end, vocab / PER);
   v_begin = min(v_begin, v_end);
@@ -836,40 +859,55 @@ struct ExactState {
   unsigned long long need;
 };
 
-// radix_pick64 on bins already in registers (lane l holds bins 4l .. 4l+3), result in every lane.
+// radix_pick64 on bins already in registers, result in every lane.  Lane l holds bins 255 - 4l .. 252 - 4l in this order
+// (the scan then runs from the highest bin down).
 __device__ __forceinline__ void radix_pick_regs(const unsigned long long (&h4)[4], unsigned long long need, int& digit,
                                                 unsigned long long& rem) {
   const int lane = threadIdx.x & 63;
   const unsigned long long s = h4[0] + h4[1] + h4[2] + h4[3];
-  unsigned long long suf = s;                   // weight in the bins of lanes >= this one
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const unsigned long long t = __shfl_down(suf, off, 64);
-    if (lane + off < 64) suf += t;
-  }
-  unsigned long long run = suf - s, left = 0ull;
+  unsigned long long run = wave_scan64(s, [](unsigned long long a, unsigned long long b) { return a + b; }) - s, left = 0ull;
   int best = -1;
 #pragma unroll
-  for (int j = 3; j >= 0; --j) {
+  for (int j = 0; j < 4; ++j) {
     if (best < 0 && run + h4[j] >= need) {
-      best = 4 * lane + j;
+      best = 255 - 4 * lane - j;
       left = need - run;
     }
     run += h4[j];
   }
   const unsigned long long any = __ballot(best >= 0);
-  const int win = any != 0ull ? 63 - __builtin_clzll(any) : 0;      // the highest lane with a hit wins
-  digit = any != 0ull ? __shfl(best, win, 64) : 0;
-  rem = any != 0ull ? __shfl(left, win, 64) : need;
+  const int win = any != 0ull ? __builtin_ctzll(any) : 0;          // the lowest lane with a hit holds the highest bin
+  digit = any != 0ull ? __builtin_amdgcn_readlane(best, win) : 0;
+  rem = any != 0ull ? lane64(left, win) : need;
 }
 
-// Replays the picks of stages [0, upto) for `row` from the finished histograms.  Wave 0 does it alone: it asks
+// Where a row's histograms and its best key lie.  In a caller's workspace (all 64-bit; all but `last` zeroed ahead of
+// the launches):
+//   [rows] x 32 words: best at 0, the draw's key at 16 | histograms [rows][2 NL][256] | last [rows][chunks][256]
+// (each on a line of its own: a line's atomics are served one after the other, and 60 workgroups of every row meet here)
+// last: the masses of the last stage, for every column range by itself (how many tokens of the key at which the
+// top-p prefix ends lie in the ranges ahead follows from them: such tokens weigh the same).
+// best: the order-preserving key of the row's largest logit and its inverted index (a NaN on top); without a
+// workspace, in the library's own scratch, for the rows whose flag is up.
+constexpr int kSampleWsHead = 32;
+__host__ __device__ __forceinline__ int64_t sample_ws_words(int64_t rows, int stages) { return rows * (kSampleWsHead + stages * 256); }
+constexpr int kSampleWsThreads = 256;                       // of a workgroup of this way
+constexpr int kSampleWsGroups = 2048;                       // rows x chunks is below this plus the rows
+
+struct ExactRow {
+  unsigned long long* hists;     // null: the row takes no part
+  float l0;                      // its largest logit
+};
+template <int LDT>
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp);
+
+// Replays the picks of stages [0, upto) of a row from its finished histograms [stage][256].  Wave 0 does it alone: it asks
 // for every histogram it will need at once (one memory round trip instead of one per level, each followed by two
 // workgroup barriers -- a third of the follow-up launches' time), picks level after level with shuffles only and
-// hands the state to the workgroup through LDS (shi / shl scratch).  upto = 2 * NL: the full state.
+// hands the state to the workgroup through LDS (shl scratch).  upto = 2 * NL: the full state.
 template <int LDT>
-__device__ __forceinline__ ExactState exact_replay(int row, int upto, int K1, float tp, float temp, float l0, int* shi,
-                                                   unsigned long long* shl) {
+__device__ __forceinline__ ExactState exact_replay(const unsigned long long* hists, int upto, int K1, float tp, float temp,
+                                                   float l0, unsigned long long* shl) {
   using L = ExactLevels<LDT>;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   ExactState st;
@@ -880,7 +918,7 @@ __device__ __forceinline__ ExactState exact_replay(int row, int upto, int K1, fl
     for (int s_ = 0; s_ < 2 * L::NL; ++s_) {
       const bool on = s_ < upto && (s_ < L::NL ? K1 > 0 : tp < 1.0f);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) h[s_][j] = on ? g_exact_hist[row][s_][4 * lane + j] : 0ull;
+      for (int j = 0; j < 4; ++j) h[s_][j] = on ? MI355_LD(unsigned long long, hists, hists + s_ * 256 + 255 - 4 * lane - j) : 0ull;
     }
     // top-k: stages 0 .. NL-1
     if (K1 > 0) {
@@ -934,85 +972,148 @@ __device__ __forceinline__ ExactState exact_replay(int row, int upto, int K1, fl
   st.Tk = static_cast<uint32_t>(shl[2] >> 32), st.Tp = static_cast<uint32_t>(shl[2] & 0xFFFFFFFFull);
   st.prefix = static_cast<uint32_t>(shl[3] >> 32), st.mask = static_cast<uint32_t>(shl[3] & 0xFFFFFFFFull);
   __syncthreads();
-  (void)shi;
   return st;
+}
+
+// Rows that need one key only: greedy ones and draws with neither top-k nor top-p.
+__device__ __forceinline__ bool sample_one_key(float temp, int top_k, float top_p) {
+  return !(temp > 0.0f) || (top_k <= 0 && !(top_p < 1.0f));
+}
+
+template <int LDT>
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp) {
+  if (ws == nullptr) return ExactRow{row < kExactRows && g_exact_flag[row] != 0u ? &g_exact_hist[row][0][0] : nullptr,
+                                     row < kExactRows ? g_exact_l0[row] : 0.f};
+  const uint32_t key = static_cast<uint32_t>(MI355_LD(unsigned long long, ws, ws + static_cast<int64_t>(row) * kSampleWsHead) >> 32);
+  if (sample_one_key(temp, k, tp) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
+  return ExactRow{ws + static_cast<int64_t>(rows) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256, key_to_logit(key)};
+}
+
+// Adds val(logit) of the logits [f, f + nf) with key >= from and the masked bits at prefix to their digits' bins: one
+// LDS add per run of equal digits inside the vector (a row's neighbours mostly share their leading bits).
+template <typename V>
+__device__ __forceinline__ void hist_add(unsigned long long* hist, const float (&f)[8], int nf, uint32_t from, uint32_t mask,
+                                         uint32_t prefix, int shift, V&& val) {
+  unsigned long long acc = 0ull;
+  uint32_t cur = 0xFFFFFFFFu;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (j < nf) {
+      const uint32_t key = sample_key(f[j]);
+      if (key >= from && (key & mask) == prefix) {
+        const uint32_t d = (key >> shift) & 255u;
+        if (d != cur) {
+          if (cur != 0xFFFFFFFFu && acc != 0ull) atomicAdd(&hist[cur], acc);
+          cur = d;
+          acc = 0ull;
+        }
+        acc += val(f[j]);
+      }
+    }
+  }
+  if (cur != 0xFFFFFFFFu && acc != 0ull) atomicAdd(&hist[cur], acc);
 }
 
 template <int LDT>
 __global__ __launch_bounds__(kSampleThreads) void exact_hist_kernel(
-    const void* __restrict__ logits, int64_t stride, int vocab, const float* __restrict__ temperature,
-    const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int chunk_vecs, int stage) {
+    unsigned long long* __restrict__ ws, const void* __restrict__ logits, int64_t stride, int vocab,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int chunk_vecs,
+    int stage) {
   using L = ExactLevels<LDT>;
-  const int row = blockIdx.x;
-  if (row >= kExactRows || g_exact_flag[row] == 0u) return;
+  const int row = ws != nullptr ? blockIdx.y : blockIdx.x, range = ws != nullptr ? blockIdx.x : blockIdx.y;
+  const int rows = ws != nullptr ? gridDim.y : gridDim.x, ranges = ws != nullptr ? gridDim.x : gridDim.y;
   const int k = MI355_LD(int32_t, top_k, top_k + row);
   const int K1 = (k > 0 && k < vocab) ? k : 0;
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp);
+  if (er.hists == nullptr) return;
   const bool counting = stage < L::NL;
   if (counting ? K1 == 0 : !(tp < 1.0f)) return;       // this selection is off for the row
-  const float l0 = g_exact_l0[row];
+  const float l0 = er.l0;
+  constexpr int kListed = 2048;
   __shared__ unsigned long long hist[256];
-  __shared__ int shi[2];
   __shared__ unsigned long long shl[4];
+  __shared__ float list[kListed];
+  __shared__ int listed;
   const int tid = threadIdx.x;
-  const ExactState st = exact_replay<LDT>(row, stage, K1, tp, temp, l0, shi, shl);
+  const ExactState st = exact_replay<LDT>(er.hists, stage, K1, tp, temp, l0, shl);
   const int shift = 24 - 8 * (counting ? stage : stage - L::NL);
   if (tid < 256) hist[tid] = 0ull;
   __syncthreads();
   const void* base = LDT == MI355_F32 ? static_cast<const void*>(static_cast<const float*>(logits) + row * stride)
                                       : static_cast<const void*>(static_cast<const uint16_t*>(logits) + row * stride);
-  const int v0 = blockIdx.y * chunk_vecs, v1 = v0 + chunk_vecs;
-  const bool tail = blockIdx.y == gridDim.y - 1;
-  for_each_vector_in<LDT, 2>(base, vocab, v0, v1, tail, [&](const float (&f)[8], int nf, int) {
-    unsigned long long acc = 0ull;
-    uint32_t cur = 0xFFFFFFFFu;
+  const int v0 = range * chunk_vecs, v1 = v0 + chunk_vecs;
+  const bool tail = range == ranges - 1;
+  if (counting || (st.Tk == 0u && st.mask == 0u)) {
+    for_each_vector_in<LDT, 2>(base, vocab, v0, v1, tail, [&](const float (&f)[8], int nf, int) {
+      hist_add(hist, f, nf, st.Tk, st.mask, st.prefix, shift,
+               [&](float l) -> unsigned long long { return counting ? 1ull : sample_mass(l, l0, temp); });
+    });
+  } else {
+    // few logits weigh here, but some of nearly every wave: collected first, so that full waves compute the masses
+    if (tid == 0) listed = 0;
+    __syncthreads();
+    for_each_vector_in<LDT, 2>(base, vocab, v0, v1, tail, [&](const float (&f)[8], int nf, int) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j < nf) {
-        const uint32_t key = sample_key(f[j]);
-        if (key >= st.Tk && (key & st.mask) == st.prefix) {
-          const uint32_t d = (key >> shift) & 255u;
-          if (d != cur) {
-            if (cur != 0xFFFFFFFFu && acc != 0ull) atomicAdd(&hist[cur], acc);
-            cur = d;
-            acc = 0ull;
+      for (int j = 0; j < 8; ++j) {
+        if (j < nf) {
+          const uint32_t key = sample_key(f[j]);
+          if (key >= st.Tk && (key & st.mask) == st.prefix) {
+            const int at = atomicAdd(&listed, 1);
+            if (at < kListed) list[at] = f[j];
+            else atomicAdd(&hist[(key >> shift) & 255u], sample_mass(f[j], l0, temp));
           }
-          acc += counting ? 1ull : sample_mass(f[j], l0, temp);
         }
       }
-    }
-    if (cur != 0xFFFFFFFFu && acc != 0ull) atomicAdd(&hist[cur], acc);
-  });
+    });
+    __syncthreads();
+    const int n = min(listed, kListed);
+    for (int i = tid; i < n; i += static_cast<int>(blockDim.x)) atomicAdd(&hist[(sample_key(list[i]) >> shift) & 255u], sample_mass(list[i], l0, temp));
+  }
   __syncthreads();
-  if (tid < 256 && hist[tid] != 0ull) atomicAdd(&g_exact_hist[row][stage][tid], hist[tid]);
+  if (tid < 256) {
+    if (hist[tid] != 0ull) atomicAdd(er.hists + stage * 256 + tid, hist[tid]);
+    if (ws != nullptr && stage == 2 * L::NL - 1)
+      MI355_ST(unsigned long long, ws,
+               ws + sample_ws_words(rows, 2 * L::NL) + (static_cast<int64_t>(row) * ranges + range) * 256 + tid, hist[tid]);
+  }
 }
 
 template <int LDT>
 __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
-    int64_t* __restrict__ out, const void* __restrict__ logits, int64_t stride, int vocab,
+    int64_t* __restrict__ out, unsigned long long* __restrict__ ws, const void* __restrict__ logits, int64_t stride, int vocab,
     const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
     const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps, int chunk_vecs) {
   using L = ExactLevels<LDT>;
-  const int row = blockIdx.x;
-  if (row >= kExactRows || g_exact_flag[row] == 0u) return;
+  const int row = ws != nullptr ? blockIdx.y : blockIdx.x, range = ws != nullptr ? blockIdx.x : blockIdx.y;
+  const int rows = ws != nullptr ? gridDim.y : gridDim.x, ranges = ws != nullptr ? gridDim.x : gridDim.y, tid = threadIdx.x;
   const int k = MI355_LD(int32_t, top_k, top_k + row);
   const int K1 = (k > 0 && k < vocab) ? k : 0;
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
-  const float l0 = g_exact_l0[row];
-  __shared__ int shi[2];
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp);
+  if (er.hists == nullptr) return;
+  const float l0 = er.l0;
   __shared__ unsigned long long shl[4];
   __shared__ int eq_base[kSampleThreads / 64 + 1];
   __shared__ unsigned long long part[kSampleThreads / 64];
-  const int tid = threadIdx.x;
-  const ExactState st = exact_replay<LDT>(row, 2 * L::NL, K1, tp, temp, l0, shi, shl);
+  const ExactState st = exact_replay<LDT>(er.hists, 2 * L::NL, K1, tp, temp, l0, shl);
   const void* base = LDT == MI355_F32 ? static_cast<const void*>(static_cast<const float*>(logits) + row * stride)
                                       : static_cast<const void*>(static_cast<const uint16_t*>(logits) + row * stride);
   // tokens at the cut key in the column ranges before this one (only when top-p cuts inside that tie): counted
   // here, from the row itself -- a compare per logit, cheaper than a launch of its own that would leave the counts
   unsigned long long before = 0ull;
-  if (st.take != ~0ull && blockIdx.y != 0) {
+  if (st.take != ~0ull && range != 0 && ws != nullptr) {
+    const unsigned long long* last = ws + sample_ws_words(rows, 2 * L::NL) + static_cast<int64_t>(row) * ranges * 256 +
+                                     ((st.Tp >> L::kLastShift) & 255u);
+    unsigned long long m = tid < range ? MI355_LD(unsigned long long, ws, last + tid * 256) : 0ull;
+    m = wave_sum64(m);                                   // (at most 64 ranges: the first wave has them all)
+    if (tid == 0) part[0] = m / sample_mass(key_to_logit(st.Tp), l0, temp);
+    __syncthreads();
+    before = part[0];
+    __syncthreads();
+  } else if (st.take != ~0ull && range != 0) {
     unsigned int mine = 0u;
-    for_each_vector_in<LDT, 2>(base, vocab, 0, static_cast<int>(blockIdx.y) * chunk_vecs, false,
+    for_each_vector_in<LDT, 2>(base, vocab, 0, range * chunk_vecs, false,
                                [&](const float (&f)[8], int nf, int) {
 #pragma unroll
                                  for (int j = 0; j < 8; ++j) mine += (j < nf && sample_key(f[j]) == st.Tp) ? 1u : 0u;
@@ -1020,20 +1121,20 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
     unsigned long long w = wave_sum64(static_cast<unsigned long long>(mine));
     if ((tid & 63) == 0) part[tid >> 6] = w;
     __syncthreads();
-    for (int q = 0; q < kSampleThreads / 64; ++q) before += part[q];
+    for (unsigned q = 0; q < blockDim.x >> 6; ++q) before += part[q];
     __syncthreads();
   }
   const uint32_t row_hash = sample_hash(static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)),
                                         static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row)));
   unsigned long long best = 0ull;
-  ordered_kept_pass<LDT>(base, vocab, static_cast<int>(blockIdx.y) * chunk_vecs, (static_cast<int>(blockIdx.y) + 1) * chunk_vecs,
-                         blockIdx.y == gridDim.y - 1, st.Tp, st.take, before, eq_base, [&](float f, int i) {
+  ordered_kept_pass<LDT>(base, vocab, range * chunk_vecs, (range + 1) * chunk_vecs,
+                         range == ranges - 1, st.Tp, st.take, before, eq_base, [&](float f, int i) {
                            best = umax64(best, gumbel_key(f, static_cast<uint32_t>(i), temp, row_hash));
                          });
   __syncthreads();
   best = sample_reduce_max(best, part);
-  if (tid == 0 && best != 0ull && MI355_OK_AT(out, out + row, 8))
-    atomicMax(reinterpret_cast<unsigned long long*>(out) + row, best);
+  unsigned long long* key = ws != nullptr ? ws + static_cast<int64_t>(row) * kSampleWsHead + 16 : reinterpret_cast<unsigned long long*>(out) + row;
+  if (tid == 0 && best != 0ull && MI355_OK_AT((ws != nullptr ? static_cast<void*>(ws) : out), key, 8)) atomicMax(key, best);
 }
 
 // ---- the k most likely tokens of a row (the `logprobs` / `top_logprobs` lists of the completion routes): an
@@ -1120,11 +1221,6 @@ __global__ __launch_bounds__(kSampleThreads) void topk_logits_kernel(
   }
 }
 
-// Rows that need one key only: greedy ones and draws with neither top-k nor top-p.
-__device__ __forceinline__ bool sample_one_key(float temp, int top_k, float top_p) {
-  return !(temp > 0.0f) || (top_k <= 0 && !(top_p < 1.0f));
-}
-
 __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __restrict__ temperature,
                                      const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1136,6 +1232,91 @@ __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __r
     return;
   const unsigned long long b = static_cast<unsigned long long>(MI355_LD(int64_t, out, out + i));
   MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
+}
+
+// One pass, one key: the row is cut into column ranges, every workgroup merges the best key of its
+// range into *key (cleared ahead) with a 64-bit atomic max -- order-free, so the same on every launch --
+// and a later launch turns it into the index.
+template <int LDT>
+__device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, const void* base, int vocab, bool greedy, float temp,
+                                                    uint64_t seed, uint64_t step, int range, int ranges, int chunk_vecs,
+                                                    unsigned long long* part) {
+  const int v0 = range * chunk_vecs, v1 = v0 + chunk_vecs;
+  const bool tail = range == ranges - 1;
+  unsigned long long best = 0ull;
+  if (greedy)
+    for_each_logit_in<LDT, 2>(base, vocab, v0, v1, tail,
+                              [&](float f, int i) { best = umax64(best, argmax_key(f, static_cast<uint32_t>(i))); });
+  else
+    best = sample_full_vocab<LDT>(base, vocab, v0, v1, tail, temp, seed, step);
+  best = sample_reduce_max(best, part);
+  if (threadIdx.x == 0 && best != 0ull && MI355_OK_AT(key, key, 8)) atomicMax(key, best);
+}
+
+// ---- sampling with a caller's workspace: every row spread over all of its workgroups.  The list way above keeps a row
+// with a cut in one workgroup, at the pace of one CU (32 rows of 128256 bf16 logits: 83 us, most of it the masses);
+// here the exact search, whose passes split over the launch, serves all of them, and nothing is shared between calls:
+//   sample_clear    keys and histograms <- 0
+//   sample_first    one-key rows: their pass.  Rows with a cut: the largest logit, and with top-k the first counts
+//   exact_hist      the other stages; exact_final: the draw; sample_ws_finish: the keys turned into indices
+// 32 rows of 128256 bf16 logits with a mix of cuts: 94 us a call, here 40 (the draws of uncut rows and the launches' gaps).
+__global__ __launch_bounds__(256) void sample_clear_kernel(unsigned long long* __restrict__ ws, int64_t words) {
+  const int64_t i = 2 * (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x);
+  if (i + 1 < words) MI355_ST(uint4, ws, ws + i, make_uint4(0u, 0u, 0u, 0u));
+}
+
+__global__ void sample_ws_finish_kernel(int64_t* __restrict__ out, const unsigned long long* __restrict__ ws,
+                                        const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+                                        const float* __restrict__ top_p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const unsigned long long* head = ws + static_cast<int64_t>(i) * kSampleWsHead;
+  unsigned long long b = MI355_LD(unsigned long long, ws, head + 16);
+  const unsigned long long top = MI355_LD(unsigned long long, ws, head);
+  if (!sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i), MI355_LD(float, top_p, top_p + i)) &&
+      static_cast<uint32_t>(top >> 32) == 0xFFFFFFFFu)
+    b = top;                                               // a NaN: its first index
+  MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
+}
+
+template <int LDT>
+__global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
+    unsigned long long* __restrict__ ws, const void* __restrict__ logits, int64_t stride, int vocab,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
+    const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps, int chunk_vecs) {
+  const int row = blockIdx.y, tid = threadIdx.x;          // (a row's ranges one after the other: they land on different CUs)
+  const void* base = LDT == MI355_F32 ? static_cast<const void*>(static_cast<const float*>(logits) + row * stride)
+                                      : static_cast<const void*>(static_cast<const uint16_t*>(logits) + row * stride);
+  __shared__ unsigned long long part[kSampleThreads / 64];
+  __shared__ unsigned long long hist[256];
+  const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
+  const int k = MI355_LD(int32_t, top_k, top_k + row);
+  if (sample_one_key(temp, k, tp)) {
+    sample_one_key_pass<LDT>(ws + static_cast<int64_t>(row) * kSampleWsHead + 16, base, vocab, !(temp > 0.0f), temp, static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)),
+                             static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row)), blockIdx.x,
+                             gridDim.x, chunk_vecs, part);
+    return;
+  }
+  const bool counts = k > 0 && k < vocab;
+  if (counts) {
+    if (tid < 256) hist[tid] = 0ull;
+    __syncthreads();
+  }
+  const int v0 = blockIdx.x * chunk_vecs, v1 = v0 + chunk_vecs;
+  unsigned long long best = 0ull;
+  for_each_vector_in<LDT, 2>(base, vocab, v0, v1, blockIdx.x == gridDim.x - 1, [&](const float (&f)[8], int nf, int i0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j < nf) best = umax64(best, argmax_key(f[j], static_cast<uint32_t>(i0 + j)));
+    if (counts) hist_add(hist, f, nf, 0u, 0u, 0u, 24, [](float) -> unsigned long long { return 1ull; });
+  });
+  best = sample_reduce_max(best, part);                  // (its barrier also ends the counting)
+  unsigned long long* top = ws + static_cast<int64_t>(row) * kSampleWsHead;
+  if (tid == 0 && best != 0ull && MI355_OK_AT(ws, top, 8)) atomicMax(top, best);
+  if (counts && tid < 256 && hist[tid] != 0ull) {
+    unsigned long long* h = ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256 + tid;
+    if (MI355_OK_AT(ws, h, 8)) atomicAdd(h, hist[tid]);
+  }
 }
 
 template <int LDT>
@@ -1168,20 +1349,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const uint64_t step = static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row));
   const bool greedy = !(temp > 0.0f);
   if (sample_one_key(temp, k, tp)) {
-    // one pass, one key: the row is cut into gridDim.y column ranges, every workgroup merges the
-    // best key of its range into out[row] (cleared by the launcher) with a 64-bit atomic max --
-    // order-free, so the same on every launch -- and sample_finish_kernel turns it into the index
-    const int v0 = blockIdx.y * chunk_vecs, v1 = v0 + chunk_vecs;
-    const bool tail = blockIdx.y == gridDim.y - 1;
-    unsigned long long best = 0ull;
-    if (greedy)
-      for_each_logit_in<LDT, 2>(base, vocab, v0, v1, tail,
-                                [&](float f, int i) { best = umax64(best, argmax_key(f, static_cast<uint32_t>(i))); });
-    else
-      best = sample_full_vocab<LDT>(base, vocab, v0, v1, tail, temp, seed, step);
-    best = sample_reduce_max(best, part);
-    if (tid == 0 && best != 0ull && MI355_OK_AT(out, out + row, 8))
-      atomicMax(reinterpret_cast<unsigned long long*>(out) + row, best);
+    sample_one_key_pass<LDT>(reinterpret_cast<unsigned long long*>(out) + row, base, vocab, greedy, temp, seed, step, blockIdx.y,
+                             gridDim.y, chunk_vecs, part);
     return;
   }
   if (blockIdx.y != 0) return;
@@ -1503,9 +1672,9 @@ static int32_t sample_entry(const char* name, int64_t* out_ids, const void* logi
     if (spread_exact) {                                                                                               \
       dim3 xgrid(num_rows < kExactRows ? num_rows : kExactRows, chunks);                                              \
       for (int stage = 0; stage < 2 * ExactLevels<LDT>::NL; ++stage)                                                   \
-        hipLaunchKernelGGL((exact_hist_kernel<LDT>), xgrid, block, 0, s, logits, logits_stride, vocab, temperature,    \
+        hipLaunchKernelGGL((exact_hist_kernel<LDT>), xgrid, block, 0, s, nullptr, logits, logits_stride, vocab, temperature, \
                            top_k, top_p, chunk_vecs, stage);                                                          \
-      hipLaunchKernelGGL((exact_final_kernel<LDT>), xgrid, block, 0, s, out_ids, logits, logits_stride, vocab,         \
+      hipLaunchKernelGGL((exact_final_kernel<LDT>), xgrid, block, 0, s, out_ids, nullptr, logits, logits_stride, vocab,  \
                          temperature, top_k, top_p, seeds, steps, chunk_vecs);                                         \
     }                                                                                                                 \
   } while (0)
@@ -1536,6 +1705,57 @@ extern "C" int32_t mi355_sample_topk_topp_hinted(int64_t* out_ids, const void* l
                                                  void* stream) {
   return mi355::sample_entry("mi355_sample_topk_topp_hinted", out_ids, logits, logits_stride, num_rows, vocab,
                              logits_dtype, temperature, top_k, top_p, seeds, steps, cut_rows, stream);
+}
+
+extern "C" int64_t mi355_sample_workspace(int32_t num_rows, int32_t logits_dtype) {
+  using namespace mi355;
+  const int stages = 2 * (logits_dtype == MI355_F32 ? ExactLevels<MI355_F32>::NL : logits_dtype == MI355_BF16 ? ExactLevels<MI355_BF16>::NL
+                                                                                                             : ExactLevels<MI355_F16>::NL);
+  return num_rows > 0 ? 8 * (sample_ws_words(num_rows, stages) + (static_cast<int64_t>(kSampleWsGroups) + num_rows) * 256) : 0;
+}
+
+extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logits, int64_t logits_stride, int32_t num_rows,
+                                             int32_t vocab, int32_t logits_dtype, const float* temperature,
+                                             const int32_t* top_k, const float* top_p, const int64_t* seeds,
+                                             const int64_t* steps, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace mi355;
+  const char* name = "mi355_sample_topk_topp_ws";
+  MI355_REQUIRE(temperature && top_k && top_p && seeds && steps, MI355_ERR_INVALID, "%s: null pointer", name);
+  const int32_t rc = check_logits(name, out_ids, logits, logits_stride, num_rows, vocab, logits_dtype, 0);
+  if (rc != MI355_OK || num_rows == 0) return rc;
+  const int64_t need = mi355_sample_workspace(num_rows, logits_dtype);
+  MI355_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), MI355_ERR_INVALID,
+                "%s: workspace of %lld bytes, %lld needed, 16-byte aligned", name, static_cast<long long>(workspace_bytes),
+                static_cast<long long>(need));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  unsigned long long* ws = static_cast<unsigned long long*>(workspace);
+  // whole turns of a workgroup's threads (a vector each), few enough that 2048 workgroups or 64 a row do
+  const int nvec = vocab / (logits_dtype == MI355_F32 ? 4 : 8);
+  int chunks = (kSampleWsGroups + num_rows - 1) / num_rows;
+  chunks = chunks > 64 ? 64 : chunks;
+  const int chunk_vecs = ((nvec + chunks * kSampleWsThreads - 1) / (chunks * kSampleWsThreads) + (nvec == 0)) * kSampleWsThreads;
+  chunks = nvec > chunk_vecs ? (nvec + chunk_vecs - 1) / chunk_vecs : 1;
+  const int64_t words = sample_ws_words(num_rows, 2 * (logits_dtype == MI355_F32 ? 4 : logits_dtype == MI355_BF16 ? 2 : 3));
+  const int64_t threads = words / 2;                     // (two words each)
+  hipLaunchKernelGGL(sample_clear_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s, ws, words);
+  const dim3 grid(chunks, num_rows), block(kSampleWsThreads);
+#define MI355_SAMPLE_LAUNCH(LDT)                                                                                      \
+  do {                                                                                                                \
+    hipLaunchKernelGGL((sample_first_kernel<LDT>), grid, block, 0, s, ws, logits, logits_stride, vocab,       \
+                       temperature, top_k, top_p, seeds, steps, chunk_vecs);                                           \
+    for (int stage = 1; stage < 2 * ExactLevels<LDT>::NL; ++stage)                                                     \
+      hipLaunchKernelGGL((exact_hist_kernel<LDT>), grid, block, 0, s, ws, logits, logits_stride, vocab, temperature,   \
+                         top_k, top_p, chunk_vecs, stage);                                                            \
+    hipLaunchKernelGGL((exact_final_kernel<LDT>), grid, block, 0, s, out_ids, ws, logits, logits_stride, vocab,        \
+                       temperature, top_k, top_p, seeds, steps, chunk_vecs);                                           \
+  } while (0)
+  if (logits_dtype == MI355_F32) MI355_SAMPLE_LAUNCH(MI355_F32);
+  else if (logits_dtype == MI355_BF16) MI355_SAMPLE_LAUNCH(MI355_BF16);
+  else MI355_SAMPLE_LAUNCH(MI355_F16);
+#undef MI355_SAMPLE_LAUNCH
+  hipLaunchKernelGGL(sample_ws_finish_kernel, dim3((num_rows + 255) / 256), dim3(256), 0, s, out_ids, ws, temperature, top_k, top_p,
+                     num_rows);
+  return check_launch(name);
 }
 
 extern "C" int32_t mi355_topk_logits(int64_t* out_ids, float* out_vals, const void* logits, int64_t logits_stride,

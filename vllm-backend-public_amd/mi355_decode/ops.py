@@ -594,6 +594,14 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
     return out
 
 
+# Rows with a cut are spread over many workgroups (a pass per 8 key bits and cut: 2 x 2 for bfloat16, 2 x 3 for float16,
+# 2 x 4 for float32) up to this many rows times passes, from this vocabulary on; more rows fill the chip with a workgroup
+# each.  Measured, us a call (spread / a workgroup each), 128256 bfloat16 logits: 32 rows top-p 41 / 95, 64 rows top-p 54 / 95, top-k
+# 38 / 41; 128 rows top-p 82 / 99, top-k 53 / 45; float32, 64 rows top-k 75 / 55, 16 rows 40 / 49; a vocabulary of 1000: 28 / 20.
+SAMPLE_SPREAD_PASSES, SAMPLE_SPREAD_VOCAB = 128, 16384
+_KEY_PASSES = {torch.bfloat16: 2, torch.float16: 3, torch.float32: 4}
+
+
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
            seeds: torch.Tensor, steps: torch.Tensor, out: torch.Tensor | None = None, cut_rows: bool = True):
     """Per-row sampling (greedy where temperature <= 0).  temperature/top_p float32 [B], top_k int32 [B],
@@ -610,10 +618,13 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
             raise ValueError(f"{n} must be contiguous {dt} [num_rows]")
     if out is None:
         out = torch.empty(B, dtype=torch.int64, device=logits.device)
-    check(lib.mi355_sample_topk_topp_hinted(out.data_ptr(), logits.data_ptr(), _rows(logits, "logits"), B, V,
-                                            _DT[logits.dtype], temperature.data_ptr(), top_k.data_ptr(),
-                                            top_p.data_ptr(), seeds.data_ptr(), steps.data_ptr(),
-                                            1 if cut_rows else 0, _stream()))
+    args = (out.data_ptr(), logits.data_ptr(), _rows(logits, "logits"), B, V, _DT[logits.dtype], temperature.data_ptr(),
+            top_k.data_ptr(), top_p.data_ptr(), seeds.data_ptr(), steps.data_ptr())
+    if cut_rows and B * _KEY_PASSES[logits.dtype] <= SAMPLE_SPREAD_PASSES and V >= SAMPLE_SPREAD_VOCAB:
+        ws = torch.empty(lib.mi355_sample_workspace(B, _DT[logits.dtype]), dtype=torch.uint8, device=logits.device)
+        check(lib.mi355_sample_topk_topp_ws(*args, ws.data_ptr(), ws.numel(), _stream()))
+    else:
+        check(lib.mi355_sample_topk_topp_hinted(*args, 1 if cut_rows else 0, _stream()))
     return out
 
 
