@@ -370,6 +370,82 @@ def test_delta_rule_keeps_a_far_write_and_loses_it_with_decay():
         assert abs(float(got[-1, 0, 7]) * d ** 0.5 - want) < 1e-3
 
 
+@pytest.mark.parametrize("W", [8, 72, 2040, 2048, 2056, 4096, 4104, 8192, 8200])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_row_kernels_at_the_edges_of_their_vectors(W, dtype):
+    """Widths either side of a thread's turns (2048 columns a turn, up to 8192 in registers; beyond, the element-wise form),
+    against float64.  Float32 arithmetic on values of size 1 and a sum of W squares: 1e-5; 16-bit rows: half a unit in
+    the last place, 2^-9 of bfloat16, 2^-12 of float16, and that again for a value next to a tie."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(W)
+    T, eps, half = 3, 1e-6, 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    rnd = lambda *n: torch.randn(*n, generator=g)                                   # noqa: E731
+    resid, other = rnd(T, W), rnd(T, W)
+    add, xb, wa, wb, vec = (rnd(T, W).to(dtype), rnd(T, W).to(dtype), rnd(W).to(dtype), rnd(W).to(dtype), rnd(W).to(dtype))
+    rms = lambda x: x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)            # noqa: E731
+    close = lambda got, want, tol: ((got.cpu().double() - want).abs() <= tol * (1 + want.abs())).all()      # noqa: E731
+    for weight in (wa, wa[:1].clone()):
+        for extra in (add, None):
+            r = resid.cuda()
+            out = ops.add_rms_norm_f32(r, weight.cuda(), eps, add=None if extra is None else extra.cuda())
+            want = resid.double() + (0 if extra is None else extra.double())
+            assert close(r, want, 1e-6) and close(out, rms(want) * weight.double(), half + 1e-5)
+    for two in (True, False):
+        r = resid.cuda()
+        ops.rms_norm_mix_f32(r, add.cuda(), wa.cuda(), xb.cuda() if two else None, wb.cuda() if two else None, eps, 0.5)
+        mix = rms(add.double()) * wa.double() + (rms(xb.double()) * wb.double() if two else 0)
+        assert close(r, resid.double() + 0.5 * mix, 1e-5)
+    r = resid.cuda()
+    ops.resid_add_f32(r, other=other.cuda(), rows=add.cuda(), vec=vec.cuda())
+    assert close(r, resid.double() + other.double() + add.double() + vec.double(), 1e-6)
+    ids = torch.tensor([2, 0, 1])
+    assert close(ops.embed_scale_f32(add.cuda(), ids.cuda(), 1.5), add.double()[ids] * 1.5, 1e-6)
+
+
+@pytest.mark.parametrize("H,dv", [(3, 64), (5, 128), (1, 256), (2, 72), (7, 256)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_head_norm_and_gate_rows(H, dv, act):
+    """Head sizes with several rows a wave (64, 128, 256) and another; a last workgroup of few rows; gates that are a column
+    slice.  Tolerance: the 16-bit store, 2^-8, on float32 arithmetic."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(dv + H)
+    T = 37
+    o, w = torch.randn(T, H, dv, generator=g), torch.randn(dv, generator=g)
+    wide = torch.randn(T, 8 + H * dv, generator=g).to(torch.bfloat16)
+    gate = wide[:, 8:]
+    got = ops.gated_head_rms_norm(o.cuda(), wide.cuda()[:, 8:], w.cuda(), 1e-6, act).cpu().double()
+    z = gate.double().view(T, H, dv)
+    want = o.double() / torch.sqrt((o.double() ** 2).mean(-1, keepdim=True) + 1e-6) * w.double() * torch.sigmoid(z) * (z if act == 0 else 1.0)
+    assert ((got - want.reshape(T, -1)).abs() <= 2.0 ** -8 * want.reshape(T, -1).abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_convolution_of_long_batches_by_groups_of_rows(taps):
+    """1024 rows and more go four rows a thread: groups that start a chunk, cross into the next or end the batch, chunks that
+    continue from their state.  Tolerance: the 16-bit store, 2^-8 of the result, on float32 sums of `taps` products."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(taps)
+    lens, first, C = [1, 2, 3, 5, 600, 4, 417, 2], [0, 9, 0, 1, 0, 50, 2, 0], 24
+    cu = torch.tensor([0] + lens).cumsum(0)
+    T, S = int(cu[-1]), len(lens)
+    x, w = torch.randn(T, C, generator=g).to(torch.bfloat16), torch.randn(C, taps, generator=g).to(torch.bfloat16)
+    state = torch.randn(S, taps - 1, C, generator=g)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)])
+    seq = torch.repeat_interleave(torch.arange(S), torch.tensor(lens)).to(torch.int32)
+    dev = state.cuda()
+    got = ops.causal_conv_silu(x.cuda(), w.cuda(), dev, seq.cuda(), pos.cuda(), cu.to(torch.int32).cuda(),
+                               torch.arange(S, dtype=torch.int32, device="cuda")).cpu().double()
+    for s in range(S):
+        seen = min(first[s], taps - 1)
+        before = state[s].double().clone()
+        before[:taps - 1 - seen] = 0.0
+        rows = torch.cat([before, x[cu[s]:cu[s + 1]].double()])
+        want = torch.nn.functional.silu(sum(rows[j:j + lens[s]] * w[:, j].double() for j in range(taps)))
+        assert ((got[cu[s]:cu[s + 1]] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all(), s
+        now, old = dev[s].cpu().double(), torch.cat([state[s].double(), x[cu[s]:cu[s + 1]].double()])[-(taps - 1):]
+        assert torch.equal(now, old), s
+
+
 @pytest.mark.parametrize("taps,dtype,C", [(1, torch.float32, 70), (2, torch.float32, 70), (3, torch.float32, 70),
                                           (5, torch.float32, 70), (2, torch.bfloat16, 72), (4, torch.bfloat16, 136),
                                           (3, torch.bfloat16, 70), (5, torch.bfloat16, 72)])

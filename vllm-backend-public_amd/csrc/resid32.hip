@@ -40,6 +40,36 @@ __global__ __launch_bounds__(256) void embed_scale_f32_kernel(float* __restrict_
   }
 }
 
+// ---- the forms for 16-bit storage, rows of a multiple of 8 columns on 16-byte boundaries: 8 columns a thread and turn, and
+// where a kernel needs a row twice it stays in registers (rows of up to 2048 * NV columns).  HBM-bound for prompts,
+// bound by one trip to memory for decoded rows: the element-wise forms above make two, of 2 and 4 bytes a lane.
+// Measured, 8192 rows of 2048 / 32 rows: embed_scale 33 -> 20 us, resid_add 46 -> 32, add_rms_norm 45 -> 26 / 5.7 -> 3.9,
+// rms_norm_mix 84 -> 34 / 11.7 -> 4.6, gated_head_rms_norm (16 heads of 128) 60 -> 25.
+__device__ __forceinline__ void load8f(const float* base, const float* p, float (&f)[8]) {
+  const float4 a = MI355_LD(float4, base, p), b = MI355_LD(float4, base, p + 4);
+  f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w, f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
+}
+__device__ __forceinline__ void store8f(float* base, float* p, const float (&f)[8]) {
+  MI355_ST(float4, base, p, make_float4(f[0], f[1], f[2], f[3]));
+  MI355_ST(float4, base, p + 4, make_float4(f[4], f[5], f[6], f[7]));
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void embed_scale_f32_vec_kernel(float* __restrict__ out, const uint16_t* __restrict__ embed,
+                                                                  const int64_t* __restrict__ ids, int W, float scale,
+                                                                  uint16_t* __restrict__ act) {
+  const int64_t t = blockIdx.x;
+  const int64_t id = MI355_LD(int64_t, ids, ids + t);
+  for (int c = threadIdx.x * 8; c < W; c += blockDim.x * 8) {
+    float f[8];
+    unpack8<T>(MI355_LD(uint4, embed, embed + id * W + c), f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] *= scale;
+    store8f(out, out + t * W + c, f);
+    if (act != nullptr) MI355_ST(uint4, act, act + t * W + c, pack8<T>(f));
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void embed_scale_pos_f32_kernel(float* __restrict__ out,
                                                                   const typename Elem<T>::S* __restrict__ embed,
@@ -71,6 +101,27 @@ __global__ __launch_bounds__(256) void resid_add_f32_kernel(float* __restrict__ 
 }
 
 template <typename T>
+__global__ __launch_bounds__(256) void resid_add_f32_vec_kernel(float* __restrict__ resid, const float* __restrict__ other,
+                                                                const uint16_t* __restrict__ rows,
+                                                                const uint16_t* __restrict__ vec, int W) {
+  const int64_t t = blockIdx.x;
+  for (int c = threadIdx.x * 8; c < W; c += blockDim.x * 8) {
+    float v[8], a[8] = {}, b[8] = {}, d[8] = {};
+    load8f(resid, resid + t * W + c, v);
+    if (other != nullptr) load8f(other, other + t * W + c, a);
+    if (rows != nullptr) unpack8<T>(MI355_LD(uint4, rows, rows + t * W + c), b);
+    if (vec != nullptr) unpack8<T>(MI355_LD(uint4, vec, vec + c), d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (other != nullptr) v[j] += a[j];
+      if (rows != nullptr) v[j] += b[j];
+      if (vec != nullptr) v[j] += d[j];
+    }
+    store8f(resid, resid + t * W + c, v);
+  }
+}
+
+template <typename T>
 __global__ __launch_bounds__(256) void add_rms_norm_f32_kernel(typename Elem<T>::S* __restrict__ out,
                                                                float* __restrict__ resid,
                                                                const typename Elem<T>::S* __restrict__ add,
@@ -94,6 +145,50 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32_kernel(typename Elem<T>:
     const float v = MI355_LD(float, resid, resid + t * W + c);      // own writes of this thread: same c
     const float g = weight_numel == 1 ? g1 : MI355_LDF(T, weight, weight + c);
     MI355_STF(T, out, out + t * W + c, v * r * g);
+  }
+}
+
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void add_rms_norm_f32_vec_kernel(uint16_t* __restrict__ out, float* __restrict__ resid,
+                                                                   const uint16_t* __restrict__ add,
+                                                                   const uint16_t* __restrict__ weight, int weight_numel, int W,
+                                                                   float eps) {
+  __shared__ float scratch[32];
+  const int64_t t = blockIdx.x;
+  float v[NV][8];
+  uint4 wv[NV];
+  const float g1 = weight_numel == 1 ? T::to_f(MI355_LD(uint16_t, weight, weight)) : 0.f;
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (threadIdx.x + 256 * i) * 8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
+    wv[i] = make_uint4(0, 0, 0, 0);
+    if (c < W) {
+      load8f(resid, resid + t * W + c, v[i]);
+      if (weight_numel != 1) wv[i] = MI355_LD(uint4, weight, weight + c);
+      if (add != nullptr) {
+        float y[8];
+        unpack8<T>(MI355_LD(uint4, add, add + t * W + c), y);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] += y[j];
+        store8f(resid, resid + t * W + c, v[i]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
+  }
+  const float r = 1.0f / sqrtf(block_sum32(ss, scratch) / static_cast<float>(W) + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (threadIdx.x + 256 * i) * 8;
+    if (c >= W) continue;
+    float f[8];
+    unpack8<T>(wv[i], f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = v[i][j] * r * (weight_numel == 1 ? g1 : f[j]);
+    MI355_ST(uint4, out, out + t * W + c, pack8<T>(f));
   }
 }
 
@@ -238,6 +333,60 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_kernel(float* __restrict
   }
 }
 
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __restrict__ resid, const uint16_t* __restrict__ xa,
+                                                                   const uint16_t* __restrict__ wa,
+                                                                   const uint16_t* __restrict__ xb,
+                                                                   const uint16_t* __restrict__ wb, int W, float eps,
+                                                                   float alpha) {
+  __shared__ float scratch[2][4];
+  const int64_t t = blockIdx.x;
+  uint4 a[NV], b[NV], ga[NV], gb[NV];
+  float v[NV][8], sa = 0.f, sb = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (threadIdx.x + 256 * i) * 8;
+    a[i] = b[i] = ga[i] = gb[i] = make_uint4(0, 0, 0, 0);
+    if (c < W) {
+      a[i] = MI355_LD(uint4, xa, xa + t * W + c);
+      ga[i] = MI355_LD(uint4, wa, wa + c);
+      if (xb != nullptr) {
+        b[i] = MI355_LD(uint4, xb, xb + t * W + c);
+        gb[i] = MI355_LD(uint4, wb, wb + c);
+      }
+      load8f(resid, resid + t * W + c, v[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[8], g[8];
+    unpack8<T>(a[i], f), unpack8<T>(b[i], g);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sa += f[j] * f[j], sb += g[j] * g[j];
+  }
+  sa = wave_sum(sa), sb = wave_sum(sb);                 // both sums over one barrier
+  if ((threadIdx.x & 63) == 0) scratch[0][threadIdx.x >> 6] = sa, scratch[1][threadIdx.x >> 6] = sb;
+  __syncthreads();
+  sa = scratch[0][0] + scratch[0][1] + scratch[0][2] + scratch[0][3];
+  sb = scratch[1][0] + scratch[1][1] + scratch[1][2] + scratch[1][3];
+  const float ra = 1.0f / sqrtf(sa / static_cast<float>(W) + eps);
+  const float rb = 1.0f / sqrtf(sb / static_cast<float>(W) + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (threadIdx.x + 256 * i) * 8;
+    if (c >= W) continue;
+    float f[8], g[8], x[8], y[8];
+    unpack8<T>(a[i], f), unpack8<T>(ga[i], x), unpack8<T>(b[i], g), unpack8<T>(gb[i], y);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float m = f[j] * ra * x[j];
+      if (xb != nullptr) m += g[j] * rb * y[j];
+      v[i][j] += alpha * m;
+    }
+    store8f(resid, resid + t * W + c, v[i]);
+  }
+}
+
 // 0.5 z (1 + tanh(w)) = z / (1 + exp(-2 w)), w = sqrt(2 / pi) (z + 0.044715 z^3)
 __device__ __forceinline__ float gelu_tanh_f(float z) {
   return z / (1.0f + expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
@@ -307,6 +456,36 @@ __global__ __launch_bounds__(256) void gated_head_rms_norm_kernel(typename Elem<
     MI355_STF(T, out, out + t * out_stride + static_cast<int64_t>(h) * dv + c,
               v * r * MI355_LD(float, w, w + (w_heads > 1 ? h * dv : 0) + c) * a);
   }
+}
+
+// L = dv / 8 lanes (a power of two, at most 64) a row
+template <typename T, int L>
+__global__ __launch_bounds__(256) void gated_head_rms_norm_vec_kernel(uint16_t* __restrict__ out, const float* __restrict__ o,
+                                                                      const uint16_t* __restrict__ gate, int64_t gate_stride,
+                                                                      const float* __restrict__ w, int w_heads, int64_t rows,
+                                                                      int H, float eps, int act, int64_t out_stride) {
+  constexpr int dv = 8 * L;
+  const int64_t row = blockIdx.x * static_cast<int64_t>(256 / L) + threadIdx.x / L;
+  if (row >= rows) return;                              // (all lanes of a row together)
+  const int c = (threadIdx.x & (L - 1)) * 8;
+  const int64_t t = row / H;
+  const int h = static_cast<int>(row - t * H);
+  float v[8], wv[8], g[8], ss = 0.f;
+  load8f(o, o + row * dv + c, v);
+  const uint4 graw = MI355_LD(uint4, gate, gate + t * gate_stride + static_cast<int64_t>(h) * dv + c);
+  load8f(w, w + (w_heads > 1 ? h * dv : 0) + c, wv);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
+#pragma unroll
+  for (int off = 1; off < L; off <<= 1) ss += __shfl_xor(ss, off, 64);
+  const float r = 1.0f / sqrtf(ss / static_cast<float>(dv) + eps);
+  unpack8<T>(graw, g);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float sg = 1.0f / (1.0f + expf(-g[j]));
+    v[j] = v[j] * r * wv[j] * (act == 0 ? g[j] * sg : sg);
+  }
+  MI355_ST(uint4, out, out + t * out_stride + static_cast<int64_t>(h) * dv + c, pack8<T>(v));
 }
 
 // one workgroup per row, for rows of many columns (a norm over all heads at once)
@@ -721,6 +900,14 @@ extern "C" int32_t mi355_embed_scale_f32(float* out, void* act_out, const void* 
   REQ_DTYPE(dtype);
   if (num_tokens == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype != MI355_F32 && width % 8 == 0 && aligned16(out) && aligned16(embed) && aligned16(act_out)) {
+#define MI355_EMBED(TT)                                                                                                     \
+  hipLaunchKernelGGL((embed_scale_f32_vec_kernel<TT>), dim3(num_tokens), dim3(256), 0, s, out,                              \
+                     static_cast<const uint16_t*>(embed), ids, width, scale, static_cast<uint16_t*>(act_out))
+    if (dtype == MI355_BF16) MI355_EMBED(BF16); else MI355_EMBED(F16);
+#undef MI355_EMBED
+    return check_launch("embed_scale_f32");
+  }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((embed_scale_f32_kernel<TT>), dim3(num_tokens), dim3(256), 0, s, out,
                                                   static_cast<const Elem<TT>::S*>(embed), ids, width, scale,
                                                   static_cast<Elem<TT>::S*>(act_out)));
@@ -800,6 +987,14 @@ extern "C" int32_t mi355_resid_add_f32(float* resid, const float* other, const v
   REQ_DTYPE(dtype);
   if (num_tokens == 0 || (!other && !rows && !vec)) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype != MI355_F32 && width % 8 == 0 && aligned16(resid) && aligned16(other) && aligned16(rows) && aligned16(vec)) {
+#define MI355_RADD(TT)                                                                                                     \
+  hipLaunchKernelGGL((resid_add_f32_vec_kernel<TT>), dim3(num_tokens), dim3(256), 0, s, resid, other,                      \
+                     static_cast<const uint16_t*>(rows), static_cast<const uint16_t*>(vec), width)
+    if (dtype == MI355_BF16) MI355_RADD(BF16); else MI355_RADD(F16);
+#undef MI355_RADD
+    return check_launch("resid_add_f32");
+  }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((resid_add_f32_kernel<TT>), dim3(num_tokens), dim3(256), 0, s, resid,
                                                   other, static_cast<const Elem<TT>::S*>(rows),
                                                   static_cast<const Elem<TT>::S*>(vec), width));
@@ -816,6 +1011,22 @@ extern "C" int32_t mi355_add_rms_norm_f32(void* out, float* resid, const void* a
   REQ_DTYPE(dtype);
   if (num_tokens == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) && aligned16(add) &&
+      (weight_numel == 1 || aligned16(weight))) {
+#define MI355_RN(TT, NV)                                                                                                     \
+  hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, static_cast<const uint16_t*>(add), static_cast<const uint16_t*>(weight), weight_numel, width, eps)
+#define MI355_RN_NV(TT)                      \
+  do {                                       \
+    if (width <= 2048) MI355_RN(TT, 1);      \
+    else if (width <= 4096) MI355_RN(TT, 2); \
+    else MI355_RN(TT, 4);                    \
+  } while (0)
+    if (dtype == MI355_BF16) MI355_RN_NV(BF16); else MI355_RN_NV(F16);
+#undef MI355_RN_NV
+#undef MI355_RN
+    return check_launch("add_rms_norm_f32");
+  }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((add_rms_norm_f32_kernel<TT>), dim3(num_tokens), dim3(256), 0, s,
                                                   static_cast<Elem<TT>::S*>(out), resid,
                                                   static_cast<const Elem<TT>::S*>(add),
@@ -866,6 +1077,23 @@ extern "C" int32_t mi355_rms_norm_mix_f32(float* resid, const void* xa, const vo
   REQ_DTYPE(dtype);
   if (num_tokens == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(resid) && aligned16(xa) && aligned16(wa) &&
+      aligned16(xb) && aligned16(wb)) {
+#define MI355_MIX(TT, NV)                                                                                                \
+  hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV>), dim3(num_tokens), dim3(256), 0, s, resid,                    \
+                     static_cast<const uint16_t*>(xa), static_cast<const uint16_t*>(wa), static_cast<const uint16_t*>(xb), \
+                     static_cast<const uint16_t*>(wb), width, eps, alpha)
+#define MI355_MIX_NV(TT)                      \
+  do {                                       \
+    if (width <= 2048) MI355_MIX(TT, 1);      \
+    else if (width <= 4096) MI355_MIX(TT, 2); \
+    else MI355_MIX(TT, 4);                    \
+  } while (0)
+    if (dtype == MI355_BF16) MI355_MIX_NV(BF16); else MI355_MIX_NV(F16);
+#undef MI355_MIX_NV
+#undef MI355_MIX
+    return check_launch("rms_norm_mix_f32");
+  }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((rms_norm_mix_f32_kernel<TT>), dim3(num_tokens), dim3(256), 0, s, resid,
                                                   static_cast<const Elem<TT>::S*>(xa), static_cast<const Elem<TT>::S*>(wa),
                                                   static_cast<const Elem<TT>::S*>(xb), static_cast<const Elem<TT>::S*>(wb),
@@ -934,6 +1162,23 @@ extern "C" int32_t mi355_gated_head_rms_norm(void* out, int64_t out_stride, cons
                                                     static_cast<Elem<TT>::S*>(out), o,
                                                     static_cast<const Elem<TT>::S*>(gate), gate_stride, weight, head_dim, eps,
                                                     activation, out_stride));
+    return check_launch("gated_head_rms_norm");
+  }
+  if (dtype != MI355_F32 && (head_dim == 64 || head_dim == 128 || head_dim == 256) && gate_stride % 8 == 0 && out_stride % 8 == 0 &&
+      aligned16(out) && aligned16(o) && aligned16(gate) && aligned16(weight)) {
+#define MI355_HEAD(TT, L)                                                                                                   \
+  hipLaunchKernelGGL((gated_head_rms_norm_vec_kernel<TT, L>), dim3((rows + 256 / L - 1) / (256 / L)), dim3(256), 0, s,       \
+                     static_cast<uint16_t*>(out), o, static_cast<const uint16_t*>(gate), gate_stride, weight, weight_heads, rows, \
+                     num_heads, eps, activation, out_stride)
+#define MI355_HEAD_L(TT)                        \
+  do {                                          \
+    if (head_dim == 64) MI355_HEAD(TT, 8);      \
+    else if (head_dim == 128) MI355_HEAD(TT, 16); \
+    else MI355_HEAD(TT, 32);                    \
+  } while (0)
+    if (dtype == MI355_BF16) MI355_HEAD_L(BF16); else MI355_HEAD_L(F16);
+#undef MI355_HEAD_L
+#undef MI355_HEAD
     return check_launch("gated_head_rms_norm");
   }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((gated_head_rms_norm_kernel<TT>), dim3((rows + 3) / 4), dim3(256), 0, s,
