@@ -324,6 +324,19 @@ int32_t mi355_paged_attn_prefill_ext(void* out, int64_t out_stride, const void* 
                                      int32_t chunk, int32_t window, int32_t keep, const float* sink,
                                      const void* gate, int64_t gate_stride, float out_scale, float softcap,
                                      int32_t dtype, void* stream);
+/*
+ * The same launch with sigmoid weights in place of the softmax (what mi355_sigmoid_window_attn computes): out[t, h] =
+ * sigmoid(gate[t, h]) * sum over the keys j with 0 <= p - j < window of sigmoid(q.k_j scale temp[h] + bias[h]) v_j.
+ * head_dim 64 or 128, v_dim 64 or 128, 16-bit dtypes, at most 16 query heads per kv head.
+ */
+int32_t mi355_sigmoid_window_attn_prefill(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                          const void* k_cache, const void* v_cache, int32_t num_blocks,
+                                          const int32_t* block_tables, int32_t max_blocks_per_seq,
+                                          const int32_t* cu_seqlens, const int32_t* context_lens,
+                                          int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
+                                          int32_t num_kv_heads, int32_t head_dim, int32_t v_dim, float scale,
+                                          int32_t window, const float* temp, const float* bias, const void* gate,
+                                          int64_t gate_stride, int32_t dtype, void* stream);
 
 /*
  * SwiGLU gate:  out[t, :] = round(round(silu(x[t, :F])) * x[t, F:2F]).

@@ -231,6 +231,64 @@ def test_window_attention_on_the_matrix_cores(H, G, d, dv, window, rot):
         assert (got - ref).abs().max() <= 1.5e-2 * ref.abs().max(), cuts
 
 
+@pytest.mark.parametrize("H,G,d,dv,window,dt", [(4, 1, 128, 128, 33, torch.bfloat16), (16, 1, 64, 128, 100, torch.float16),
+                                                (3, 3, 128, 64, 1, torch.bfloat16), (8, 2, 64, 64, 2000, torch.bfloat16),
+                                                (6, 2, 128, 128, 64, torch.float16)])
+def test_window_attention_of_staged_prompts_and_of_single_rows(H, G, d, dv, window, dt):
+    """The forms for prompts (K and V through LDS) and for single rows against the 16-row tile form in float32's restatement:
+    new rows behind 0, 15, 16, 63, 130 and 300 keys, column slices as inputs, unwritten slots NaN, a head of temperature 0
+    (whose masked weights must be 0, not sigmoid of 0 * infinity).  Bound: weights and results in 16 bits."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(H * 7 + d)
+    rn = lambda *s: torch.randn(*s, generator=g)                             # noqa: E731
+    new, before = [70, 1, 33, 128, 5, 200], [0, 15, 16, 63, 130, 300]
+    ctx = [a + b for a, b in zip(new, before)]
+    pages = [-(-c // 16) for c in ctx]
+    order, at, bt = torch.randperm(sum(pages) + 3, generator=g), 0, torch.zeros(len(new), max(pages) + 2, dtype=torch.int32)
+    kc, vc = torch.full((sum(pages) + 3, G, 16, d), float("nan")), torch.full((sum(pages) + 3, G, dv, 16), float("nan"))
+    temp, bias = torch.rand(H, generator=g) + 0.5, rn(H) - 1.0
+    temp[0] = 0.0
+    T, W = sum(new), H * d + 24
+    wide, gate = rn(T, W).to(dt), rn(T, H + 3).to(dt)
+    refs, r0 = [], 0
+    for i, c in enumerate(ctx):
+        k, v = rn(c, G, d).to(dt), rn(c, G, dv).to(dt)
+        for b in range(pages[i]):
+            n, pg = min(16, c - 16 * b), int(order[at])
+            bt[i, b] = pg
+            kc[pg, :, :n], vc[pg, :, :, :n] = k[16 * b: 16 * b + n].transpose(0, 1).float(), v[16 * b: 16 * b + n].permute(1, 2, 0).float()
+            at += 1
+        q = wide[r0: r0 + new[i], 16: 16 + H * d].float().view(new[i], H, d)
+        full = torch.cat([torch.zeros(before[i], H, d), q])
+        refs.append(R.sigmoid_window_attention(full, k.float(), v.float(), window, 0.3, temp, bias)[before[i]:])
+        r0 += new[i]
+    ref = torch.cat(refs) * torch.sigmoid(gate[:, 3:].float())[:, :, None]
+    kc, vc, bt, wide, gate, temp, bias = (t.cuda() for t in (kc.to(dt), vc.to(dt), bt, wide, gate, temp, bias))
+    cu = np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
+    pos = torch.cat([torch.arange(b, b + n) for n, b in zip(new, before)]).cuda()
+    seq = torch.repeat_interleave(torch.arange(len(new), dtype=torch.int32), torch.tensor(new)).cuda()
+    lens = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    u = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    # |error| <= u * (sum of |w v| for the weights' rounding, and again for the result's); both bounded by the same sum
+    # over the absolute values, plus fp32 noise of scores of up to 40 through the sigmoid's slope
+    bound = 2.5 * u * ref.abs().max() + 2e-4
+    def near(o, rows=slice(None)):
+        assert torch.isfinite(o).all()
+        assert (o.float().cpu().view(-1, H, dv) - ref[rows]).abs().max() <= bound
+    qs, gs = wide[:, 16: 16 + H * d], gate[:, 3:]
+    near(ops.sigmoid_window_attn_prefill(qs, kc, vc, bt, torch.from_numpy(cu).cuda(), lens, max(new), temp, bias, gs, H, window, 0.3))
+    tiles = torch.from_numpy(ops.query_tiles(cu)).cuda()
+    near(ops.sigmoid_window_attn(qs, kc, vc, bt, seq, pos, temp, bias, gs, H, window, 0.3, tiles=tiles))
+    # single rows: the last of every chunk (an odd number of key ranges, and none)
+    last = torch.from_numpy(cu[1:].astype(np.int64) - 1).cuda()
+    one = torch.arange(len(new), dtype=torch.int32, device="cuda")
+    tiles = torch.stack([one, one, torch.ones_like(one)], 1).contiguous()
+    for n in (1, 3, 16):
+        near(ops.sigmoid_window_attn(wide[last][:, 16: 16 + H * d], kc, vc, bt, one, pos[last].contiguous(), temp, bias,
+                                     gate[last][:, 3:], H, window, 0.3, tiles=tiles, num_splits=n,
+                                     partial=torch.full((n * len(new) * H * dv,), float("nan"), device="cuda")), cu[1:] - 1)
+
+
 @pytest.mark.parametrize("window", [16, 17, 31, 48])
 def test_window_edge_shows_with_one_loud_key(window):
     """One key far louder than the rest: the token window - 1 after it still hears it, the next one

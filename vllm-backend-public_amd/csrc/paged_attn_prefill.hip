@@ -39,6 +39,10 @@
 // MODE 2: all earlier keys as in MODE 0, with the term, gate and constant of MODE 1, keys of 192 too, and a soft
 // cap on the scores (cap_x > 0), cap * tanh(q.k scale / cap).  Two modes because masks and cap together do not fit
 // the registers of two workgroups per CU.
+// MODE 3: sigmoid weights in place of the softmax, sigmoid(q.k scale temp[head] + bias[head]) over the last `window`
+// keys: MODE 1's walk and masks, no reference, no sum, a masked weight is 0 (not a score of -inf: temp may be 0).  Bound by
+// the vector ALU (exp2 and rcp of every weight): 4 prompts of 2048 rows, 16 heads of 128 on 4 kv heads, window 1024
+// 88 us (the form of a wave per 16 queries, K and V from memory for each: 249).
 #include "common.h"
 
 #include <math.h>
@@ -66,8 +70,8 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ cu_seqlens,
     const int32_t* __restrict__ context_lens, int num_heads, int num_kv_heads, float scale_log2e, int qt,
     int chunk, int window, int keep, const float* __restrict__ sink, const uint16_t* __restrict__ gate, int64_t gate_stride,
-    float out_scale, float cap_x) {
-  constexpr bool EXT = MODE >= 1, MASK = MODE == 1, CAP = MODE == 2;
+    float out_scale, float cap_x, const float* __restrict__ temp, const float* __restrict__ bias) {
+  constexpr bool EXT = MODE >= 1, SIG = MODE == 3, MASK = MODE == 1 || SIG, CAP = MODE == 2;
   constexpr int KS = D / 32;
   constexpr int NT = DV / 16;
   constexpr int BS = MI355_BLOCK_SIZE;
@@ -138,6 +142,14 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     for (int ks = 0; ks < KS; ++ks) {
       const uint4 v = MI355_LD(uint4, q, qp + 32 * ks);     // always a valid row; dropped if not ours
       qf[t][ks] = col_ok[t] ? v : make_uint4(0, 0, 0, 0);
+    }
+  }
+  float w_mul[NQ], w_add[NQ];                    // SIG: weight = 1 / (1 + 2^(score w_mul + w_add))
+  if (SIG) {
+#pragma unroll
+    for (int t = 0; t < NQ; ++t) {
+      w_mul[t] = -scale_log2e * MI355_LD(float, temp, temp + (col_ok[t] ? col_head[t] : 0));
+      w_add[t] = -1.4426950408889634f * MI355_LD(float, bias, bias + (col_ok[t] ? col_head[t] : 0));
     }
   }
   int kmin = 0x7FFFFFFF;                                         // smallest position among the wave's valid columns
@@ -265,14 +277,25 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
         }
       }
     }
+    if (SIG) {
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          sa[t][j] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sa[t][j] * w_mul[t] + w_add[t]));
+          sb[t][j] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sb[t][j] * w_mul[t] + w_add[t]));
+        }
+      }
+    }
+    constexpr float kMasked = SIG ? 0.f : -INFINITY;
     const int tok0 = s * 32 + tok_h;
     if (s * 32 + 32 > t_min + 1) {         // wave-uniform: on or beyond the diagonal for some column
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          sa[t][j] = (tok0 + j <= col_pos[t]) ? sa[t][j] : -INFINITY;
-          sb[t][j] = (tok0 + 4 + j <= col_pos[t]) ? sb[t][j] : -INFINITY;
+          sa[t][j] = (tok0 + j <= col_pos[t]) ? sa[t][j] : kMasked;
+          sb[t][j] = (tok0 + 4 + j <= col_pos[t]) ? sb[t][j] : kMasked;
         }
       }
     }
@@ -281,8 +304,8 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
       for (int t = 0; t < NQ; ++t) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          sa[t][j] = (tok0 + j >= col_lo[t] || tok0 + j < keep) ? sa[t][j] : -INFINITY;
-          sb[t][j] = (tok0 + 4 + j >= col_lo[t] || tok0 + 4 + j < keep) ? sb[t][j] : -INFINITY;
+          sa[t][j] = (tok0 + j >= col_lo[t] || tok0 + j < keep) ? sa[t][j] : kMasked;
+          sb[t][j] = (tok0 + 4 + j >= col_lo[t] || tok0 + 4 + j < keep) ? sb[t][j] : kMasked;
         }
       }
     }
@@ -305,55 +328,63 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
   auto half_step = [&](int s, int image) {
     f32x4 sa[NQ], sb[NQ];
     scores(s, image, sa, sb);
-    // does any score of this lane leave the slack above its column's reference?  (scale > 0: the
-    // maximum commutes with the scaling; a masked score is -inf and never does)
-    float lm[NQ];
-    bool grow = false;
-#pragma unroll
-    for (int t = 0; t < NQ; ++t) {
-      lm[t] = scale_log2e * max3(max3(max3(sa[t][0], sa[t][1], sa[t][2]), sa[t][3], sb[t][0]),
-                                 max3(sb[t][1], sb[t][2], sb[t][3]), -INFINITY);
-      grow |= lm[t] > m_thr[t];
-    }
-    if (__any(grow)) {                                           // wave-uniform; rare after a tile's first step
+    uint4 pf[NQ];
+    if constexpr (SIG) {
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
-        float v = lm[t];
-        v = fmaxf(v, __shfl_xor(v, 16, 64));                     // the column's keys of this step sit on 4 lanes
-        v = fmaxf(v, __shfl_xor(v, 32, 64));
-        const float m_new = fmaxf(m_ref[t], v);
-        // -inf -> finite: alpha = 0 (O and l are still zero); no key seen yet: nothing to rescale
-        const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
-        l[t] *= alpha;                                           // both halves
+        const float p[8] = {sa[t][0], sa[t][1], sa[t][2], sa[t][3], sb[t][0], sb[t][1], sb[t][2], sb[t][3]};
+        pf[t] = pack8<T>(p);
+      }
+    } else {
+      // does any score of this lane leave the slack above its column's reference?  (scale > 0: the
+      // maximum commutes with the scaling; a masked score is -inf and never does)
+      float lm[NQ];
+      bool grow = false;
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          o[t][n][0] *= alpha;
-          o[t][n][1] *= alpha;
-          o[t][n][2] *= alpha;
-          o[t][n][3] *= alpha;
+      for (int t = 0; t < NQ; ++t) {
+        lm[t] = scale_log2e * max3(max3(max3(sa[t][0], sa[t][1], sa[t][2]), sa[t][3], sb[t][0]),
+                                   max3(sb[t][1], sb[t][2], sb[t][3]), -INFINITY);
+        grow |= lm[t] > m_thr[t];
+      }
+      if (__any(grow)) {                                           // wave-uniform; rare after a tile's first step
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) {
+          float v = lm[t];
+          v = fmaxf(v, __shfl_xor(v, 16, 64));                     // the column's keys of this step sit on 4 lanes
+          v = fmaxf(v, __shfl_xor(v, 32, 64));
+          const float m_new = fmaxf(m_ref[t], v);
+          // -inf -> finite: alpha = 0 (O and l are still zero); no key seen yet: nothing to rescale
+          const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
+          l[t] *= alpha;                                           // both halves
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            o[t][n][0] *= alpha;
+            o[t][n][1] *= alpha;
+            o[t][n][2] *= alpha;
+            o[t][n][3] *= alpha;
+          }
+          m_ref[t] = m_new;
+          m_thr[t] = m_new + kSlack;                               // -inf stays -inf
+          neg_m[t] = (m_new == -INFINITY) ? 0.f : -m_new;
         }
-        m_ref[t] = m_new;
-        m_thr[t] = m_new + kSlack;                               // -inf stays -inf
-        neg_m[t] = (m_new == -INFINITY) ? 0.f : -m_new;
       }
-    }
-    // p = exp2(s * scale - m_ref): the softmax scale is folded into the exponent, one fma per score
-    uint4 pf[NQ];
+      // p = exp2(s * scale - m_ref): the softmax scale is folded into the exponent, one fma per score
 #pragma unroll
-    for (int t = 0; t < NQ; ++t) {
-      const f32x2 sc = {scale_log2e, scale_log2e}, nm = {neg_m[t], neg_m[t]};
-      const f32x2 e[4] = {__builtin_elementwise_fma(f32x2{sa[t][0], sa[t][1]}, sc, nm),   // v_pk_fma_f32
-                          __builtin_elementwise_fma(f32x2{sa[t][2], sa[t][3]}, sc, nm),
-                          __builtin_elementwise_fma(f32x2{sb[t][0], sb[t][1]}, sc, nm),
-                          __builtin_elementwise_fma(f32x2{sb[t][2], sb[t][3]}, sc, nm)};
-      float p[8];
+      for (int t = 0; t < NQ; ++t) {
+        const f32x2 sc = {scale_log2e, scale_log2e}, nm = {neg_m[t], neg_m[t]};
+        const f32x2 e[4] = {__builtin_elementwise_fma(f32x2{sa[t][0], sa[t][1]}, sc, nm),   // v_pk_fma_f32
+                            __builtin_elementwise_fma(f32x2{sa[t][2], sa[t][3]}, sc, nm),
+                            __builtin_elementwise_fma(f32x2{sb[t][0], sb[t][1]}, sc, nm),
+                            __builtin_elementwise_fma(f32x2{sb[t][2], sb[t][3]}, sc, nm)};
+        float p[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        p[2 * j] = __builtin_amdgcn_exp2f(e[j][0]);
-        p[2 * j + 1] = __builtin_amdgcn_exp2f(e[j][1]);
+        for (int j = 0; j < 4; ++j) {
+          p[2 * j] = __builtin_amdgcn_exp2f(e[j][0]);
+          p[2 * j + 1] = __builtin_amdgcn_exp2f(e[j][1]);
+        }
+        l[t] += (f32x2{p[0], p[1]} + f32x2{p[2], p[3]}) + (f32x2{p[4], p[5]} + f32x2{p[6], p[7]});   // v_pk_add_f32
+        pf[t] = pack8<T>(p);
       }
-      l[t] += (f32x2{p[0], p[1]} + f32x2{p[2], p[3]}) + (f32x2{p[4], p[5]} + f32x2{p[6], p[7]});   // v_pk_add_f32
-      pf[t] = pack8<T>(p);
     }
     // O^T += V^T . P^T: a V fragment is read once and used NQ times (the V columns of tokens beyond
     // the tile's last query were cleared when the image was staged)
@@ -403,7 +434,7 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     if (!col_ok[t]) continue;
     if (EXT && sink != nullptr)          // the value-less term, against the column's reference (a valid column has seen a key)
       lt += __builtin_amdgcn_exp2f(MI355_LD(float, sink, sink + col_head[t]) * 1.4426950408889634f - m_ref[t]);
-    float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    float inv = SIG ? 1.0f : lt > 0.f ? 1.0f / lt : 0.f;
     if (EXT) inv *= out_scale;
     if (EXT && gate != nullptr)
       inv /= 1.0f + expf(-T::to_f(MI355_LD(uint16_t, gate, gate + (q_begin + col_q[t]) * gate_stride + col_head[t])));
@@ -423,7 +454,7 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
 }  // namespace mi355
 
 static int32_t launch_paged_attn_prefill(const char* name, bool ext, int32_t chunk, int32_t window, int32_t keep, const float* sink,
-                                          const void* gate, int64_t gate_stride, float out_scale, float softcap, int32_t v_dim, void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                          const void* gate, int64_t gate_stride, float out_scale, float softcap, const float* temp, const float* bias, int32_t v_dim, void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                             const void* k_cache, const void* v_cache, int32_t num_blocks,
                                             const int32_t* block_tables, int32_t max_blocks_per_seq,
                                             const int32_t* cu_seqlens, const int32_t* context_lens,
@@ -475,10 +506,12 @@ static int32_t launch_paged_attn_prefill(const char* name, bool ext, int32_t chu
                      num_blocks, block_tables, max_blocks_per_seq, cu_seqlens, context_lens, num_heads, \
                      num_kv_heads, (softcap > 0.f ? softcap : scale) * 1.4426950408889634f, qt, chunk, window,  \
                      keep, sink, static_cast<const uint16_t*>(gate), gate_stride, out_scale,            \
-                     softcap > 0.f ? 2.0f * 1.4426950408889634f * scale / softcap : 0.f)
+                     softcap > 0.f ? 2.0f * 1.4426950408889634f * scale / softcap : 0.f, temp, bias)
 #define MI355_PRE(TT, DD, NN)                                                                           \
   do {                                                                                                  \
-    if (ext && masked && v_dim == 64) MI355_PRE_E(TT, DD, 64, NN, 1);                                   \
+    if (temp != nullptr && v_dim == 64) MI355_PRE_E(TT, DD, 64, NN, 3);                                 \
+    else if (temp != nullptr) MI355_PRE_E(TT, DD, 128, NN, 3);                                          \
+    else if (ext && masked && v_dim == 64) MI355_PRE_E(TT, DD, 64, NN, 1);                              \
     else if (ext && masked) MI355_PRE_E(TT, DD, 128, NN, 1);                                            \
     else if (ext && v_dim == 64) MI355_PRE_E(TT, DD, 64, NN, 2);                                        \
     else if (ext) MI355_PRE_E(TT, DD, 128, NN, 2);                                                      \
@@ -517,7 +550,7 @@ extern "C" int32_t mi355_paged_attn_prefill(void* out, int64_t out_stride, const
                                             int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
                                             int32_t num_kv_heads, int32_t head_dim, float scale,
                                             int32_t dtype, void* stream) {
-  return launch_paged_attn_prefill("mi355_paged_attn_prefill", false, 0, 0, 0, nullptr, nullptr, 0, 1.0f, 0.f, head_dim, out, out_stride, q, q_stride, k_cache,
+  return launch_paged_attn_prefill("mi355_paged_attn_prefill", false, 0, 0, 0, nullptr, nullptr, 0, 1.0f, 0.f, nullptr, nullptr, head_dim, out, out_stride, q, q_stride, k_cache,
                                    v_cache, num_blocks, block_tables, max_blocks_per_seq, cu_seqlens, context_lens, num_seqs,
                                    max_q_len, num_heads, num_kv_heads, head_dim, scale, dtype, stream);
 }
@@ -536,7 +569,24 @@ extern "C" int32_t mi355_paged_attn_prefill_ext(void* out, int64_t out_stride, c
                 "mi355_paged_attn_prefill_ext: window %d, keep %d (not with chunks)", window, keep);
   MI355_REQUIRE(chunk >= 0 && (gate == nullptr || gate_stride >= num_heads), MI355_ERR_INVALID,
                 "mi355_paged_attn_prefill_ext: chunk %d, gate rows shorter than the heads", chunk);
-  return launch_paged_attn_prefill("mi355_paged_attn_prefill_ext", true, chunk, window, keep, sink, gate, gate_stride, out_scale, softcap, v_dim, out, out_stride, q,
+  return launch_paged_attn_prefill("mi355_paged_attn_prefill_ext", true, chunk, window, keep, sink, gate, gate_stride, out_scale, softcap, nullptr, nullptr, v_dim, out, out_stride, q,
                                    q_stride, k_cache, v_cache, num_blocks, block_tables, max_blocks_per_seq, cu_seqlens,
                                    context_lens, num_seqs, max_q_len, num_heads, num_kv_heads, head_dim, scale, dtype, stream);
+}
+
+extern "C" int32_t mi355_sigmoid_window_attn_prefill(void* out, int64_t out_stride, const void* q, int64_t q_stride,
+                                                     const void* k_cache, const void* v_cache, int32_t num_blocks,
+                                                     const int32_t* block_tables, int32_t max_blocks_per_seq,
+                                                     const int32_t* cu_seqlens, const int32_t* context_lens,
+                                                     int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
+                                                     int32_t num_kv_heads, int32_t head_dim, int32_t v_dim, float scale,
+                                                     int32_t window, const float* temp, const float* bias, const void* gate,
+                                                     int64_t gate_stride, int32_t dtype, void* stream) {
+  MI355_REQUIRE(temp && bias, MI355_ERR_INVALID, "mi355_sigmoid_window_attn_prefill: null pointer");
+  MI355_REQUIRE(window > 0 && head_dim <= 128 && (gate == nullptr || gate_stride >= num_heads), MI355_ERR_INVALID,
+                "mi355_sigmoid_window_attn_prefill: window %d, head_dim %d, gate rows shorter than the heads", window, head_dim);
+  return launch_paged_attn_prefill("mi355_sigmoid_window_attn_prefill", true, 0, window, 0, nullptr, gate, gate_stride, 1.0f, 0.f,
+                                   temp, bias, v_dim, out, out_stride, q, q_stride, k_cache, v_cache, num_blocks, block_tables,
+                                   max_blocks_per_seq, cu_seqlens, context_lens, num_seqs, max_q_len, num_heads, num_kv_heads,
+                                   head_dim, scale, dtype, stream);
 }

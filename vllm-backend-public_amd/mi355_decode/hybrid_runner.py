@@ -117,6 +117,16 @@ class WindowAttention:
         kc, vc = r.k_cache[self.ci], r.v_cache[self.ci]
         ops.rope_partial_kv_write(q, k, v, r.rotary(s.rot_dims, s.rot_base), b.positions, b.slot_mapping, kc, vc,
                                   s.heads, s.kv_heads, s.dim, s.vdim)
+        # prompts and portions: K/V steps staged through LDS once for a workgroup's tile of queries.  A workgroup walks
+        # 1024 keys in 22 us however few they are (and starts in 14), so fewer than 32 of them leave it to the form that
+        # spreads a tile's keys: 4 x 2048 rows 88 us against 249, 32 x 33 rows 14 against 34, 256 new rows 14.7 against
+        # 30, 128 new rows behind 1900 keys 37 against 27.
+        groups = max(b.num_tokens * s.heads // 128, b.num_seqs * s.kv_heads)
+        if b.long_chunks and b.context_lens is not None and groups >= 32 and s.dim <= 128 and proj.stride(0) % 8 == 0 \
+                and q.data_ptr() % 16 == 0 and ops.chunk_attn_prefill_ok(q.dtype, s.heads, s.kv_heads, s.dim, s.vdim):
+            o = ops.sigmoid_window_attn_prefill(q, kc, vc, b.block_tables, b.cu_seqlens, b.context_lens, b.max_q_len,
+                                                self.lw.attn_temp, self.lw.attn_bias, g, s.heads, s.window, s.scale)
+            return r.linear(o, self.lw.attn_o_w)
         o = ops.sigmoid_window_attn(q, kc, vc, b.block_tables, b.tok_seq, b.positions, self.lw.attn_temp,
                                     self.lw.attn_bias, g, s.heads, s.window, s.scale, tiles=b.tiles,
                                     **r.key_splits(b, s))
@@ -803,8 +813,16 @@ class HybridRunner(ModelRunner):
         of heads) would leave most of the chip idle -- decoded tokens, and short or single prompts."""
         if b.tiles is None or self.dtype == torch.float32:
             return {}
-        waves = int(b.tiles.shape[0]) * a.kv_heads * max((a.heads // a.kv_heads) // 4, 1)
-        n = min(self.MAX_KEY_SPLITS, max(a.window // 64, 1), max(2048 // max(waves, 1), 1))
+        rep = a.heads // a.kv_heads
+        if int(b.tiles.shape[0]) == b.num_tokens and rep <= 16 and a.dim in (64, 128) and a.vdim in (64, 128):
+            # single rows: a workgroup per (row, kv head) reads at what one CU can (1024 keys of 128 in 13 us), two leave
+            # their gain to the sum over the ranges (window 1024, 4 kv heads, 1 / 2 / 4 / 8 / 16 ranges: 8 rows
+            # 14.0 / 12.5 / 10.5 / 10.4 / 11.6 us, 16 rows 14.4 / 13.3 / 12.6 / 13.6 / 15.1, 32 rows 17.6 / 17.6 / 17.5 / 21.4 / 23.2)
+            n = min(self.MAX_KEY_SPLITS, a.window // 128, 256 // max(b.num_tokens * a.kv_heads, 1))
+            n = n if n > 2 else 1
+        else:
+            waves = int(b.tiles.shape[0]) * a.kv_heads * max(rep // 4, 1)
+            n = min(self.MAX_KEY_SPLITS, max(a.window // 64, 1), max(2048 // max(waves, 1), 1))
         if n <= 1:
             return {}
         need = n * b.num_tokens * a.heads * a.vdim

@@ -310,6 +310,24 @@ def chunk_attn_prefill_ok(dtype: torch.dtype, num_heads: int, num_kv_heads: int,
         and num_heads % num_kv_heads == 0 and num_heads // num_kv_heads <= 16
 
 
+def _prefill_shapes(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens, num_kv_heads, head_dim):
+    """The checks that the prompt attentions share; returns (sequences, blocks, v_dim)."""
+    nb, dv = k_cache.shape[0], v_cache.shape[2]
+    for t, n, shape in ((k_cache, "k_cache", (nb, num_kv_heads, BLOCK_SIZE, head_dim)),
+                        (v_cache, "v_cache", (nb, num_kv_heads, dv, BLOCK_SIZE))):
+        _same(t, q, n)
+        if tuple(t.shape) != shape or not t.is_contiguous():
+            raise ValueError(f"{n} must be contiguous {shape}")
+    if block_tables.dim() != 2 or block_tables.dtype != torch.int32 or not block_tables.is_contiguous():
+        raise ValueError("block_tables must be contiguous int32 [sequences, max_blocks]")
+    S = block_tables.shape[0]
+    for t, n, cnt in ((cu_seqlens, "cu_seqlens", S + 1), (context_lens, "context_lens", S)):
+        _dev(t, n)
+        if t.dtype != torch.int32 or t.numel() != cnt or not t.is_contiguous():
+            raise ValueError(f"{n} must be contiguous int32 [{cnt}]")
+    return S, nb, dv
+
+
 def paged_attn_prefill_ext(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
                            cu_seqlens: torch.Tensor, context_lens: torch.Tensor, max_q_len: int, num_heads: int,
                            num_kv_heads: int, head_dim: int, scale: float, chunk: int = 0, sink: torch.Tensor | None = None,
@@ -325,19 +343,7 @@ def paged_attn_prefill_ext(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     the key size."""
     dt = _dt16(q, "q")
     T = q.shape[0]
-    nb, dv = k_cache.shape[0], v_cache.shape[2]
-    for t, n, shape in ((k_cache, "k_cache", (nb, num_kv_heads, BLOCK_SIZE, head_dim)),
-                        (v_cache, "v_cache", (nb, num_kv_heads, dv, BLOCK_SIZE))):
-        _same(t, q, n)
-        if tuple(t.shape) != shape or not t.is_contiguous():
-            raise ValueError(f"{n} must be contiguous {shape}")
-    if block_tables.dim() != 2 or block_tables.dtype != torch.int32 or not block_tables.is_contiguous():
-        raise ValueError("block_tables must be contiguous int32 [sequences, max_blocks]")
-    S = block_tables.shape[0]
-    for t, n, cnt in ((cu_seqlens, "cu_seqlens", S + 1), (context_lens, "context_lens", S)):
-        _dev(t, n)
-        if t.dtype != torch.int32 or t.numel() != cnt or not t.is_contiguous():
-            raise ValueError(f"{n} must be contiguous int32 [{cnt}]")
+    S, nb, dv = _prefill_shapes(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens, num_kv_heads, head_dim)
     if out is None:
         out = torch.empty((T, num_heads * dv), dtype=q.dtype, device=q.device)
     if out.dtype != q.dtype or tuple(out.shape) != (T, num_heads * dv):
@@ -1256,6 +1262,28 @@ def sigmoid_window_attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
         None if partial is None or num_splits <= 1 else _f32(partial[: num_splits * T * num_heads * dv], "partial",
                                                              num_splits * T * num_heads * dv),
         int(num_splits), dt, _stream()))
+    return out
+
+
+def sigmoid_window_attn_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
+                                cu_seqlens: torch.Tensor, context_lens: torch.Tensor, max_q_len: int, temp: torch.Tensor,
+                                bias: torch.Tensor, gate: torch.Tensor | None, num_heads: int, window: int, scale: float,
+                                out: torch.Tensor | None = None):
+    """sigmoid_window_attn for chunks of many tokens: paged_attn_prefill's walk, K and V staged through LDS once for a
+    tile of queries.  Sizes as chunk_attn_prefill_ok, with keys of 64 or 128."""
+    dt = _dt16(q, "q")
+    T = q.shape[0]
+    G, d = k_cache.shape[1], k_cache.shape[3]
+    S, nb, dv = _prefill_shapes(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens, G, d)
+    if out is None:
+        out = torch.empty((T, num_heads * dv), dtype=q.dtype, device=q.device)
+    if out.dtype != q.dtype or tuple(out.shape) != (T, num_heads * dv):
+        raise ValueError("out must be [tokens, heads * v_dim] in the dtype of q")
+    check(lib.mi355_sigmoid_window_attn_prefill(
+        out.data_ptr(), _rows(out, "out"), q.data_ptr(), _cols(q, "q", num_heads * d), k_cache.data_ptr(), v_cache.data_ptr(),
+        nb, block_tables.data_ptr(), block_tables.shape[1], cu_seqlens.data_ptr(), context_lens.data_ptr(), S, int(max_q_len),
+        num_heads, G, d, dv, float(scale), int(window), _f32(temp, "temp", num_heads), _f32(bias, "bias", num_heads),
+        None if gate is None else _same(gate, q, "gate"), 0 if gate is None else _cols(gate, "gate", num_heads), dt, _stream()))
     return out
 
 
