@@ -862,6 +862,8 @@ int32_t mi355_softcap(void* z, int64_t numel, float cap, int32_t dtype, void* st
  *   causal_conv_silu       y[t, c] = silu(sum_j w[c, j] * x[t - (taps - 1 - j), c]); inputs from before
  *                          the chunk come from the sequence's state slot, zeros before position 0
  *   conv_state_update      state slot <- the last taps - 1 inputs of each sequence (after the conv)
+ *   conv_silu_step         both in one launch, a thread walking a chunk's tokens (decoded tokens): 16-bit rows, 2 to 4
+ *                          taps, channels and x_stride multiples of 8, 16-byte aligned buffers
  *   gated_delta_rule       per token and head, on state S [head_dim, v_dim] (zero at position 0):
  *                          S <- a S; u = b (v - S^T k); S <- S + k u^T; o = S^T q, with k and q made
  *                          unit vectors (q also / sqrt(head_dim)), b = sigmoid(beta),
@@ -895,6 +897,9 @@ int32_t mi355_causal_conv_silu(void* y, const void* x, int64_t x_stride, const v
                                const int32_t* cu_seqlens, const int32_t* state_slots,
                                int64_t num_tokens, int32_t channels, int32_t taps, int32_t dtype,
                                void* stream);
+int32_t mi355_conv_silu_step(void* y, const void* x, int64_t x_stride, const void* weight, float* state,
+                             const int64_t* positions, const int32_t* cu_seqlens, const int32_t* state_slots,
+                             int32_t num_seqs, int32_t channels, int32_t taps, int32_t dtype, void* stream);
 int32_t mi355_conv_state_update(float* state, const void* x, int64_t x_stride,
                                 const int32_t* cu_seqlens, const int32_t* state_slots,
                                 int32_t num_seqs, int32_t channels, int32_t taps, int32_t dtype,

@@ -356,6 +356,78 @@ def test_delta_rule_whole_portions_and_single_tokens(H, G, d, dv, per_channel):
             assert (got - ref).abs().max() <= 3e-5 * ref.abs().max(), (cuts, long_chunks)
 
 
+@pytest.mark.parametrize("C,taps,dtype", [(8, 2, torch.float16), (520, 3, torch.bfloat16), (4096, 4, torch.bfloat16)])
+def test_convolution_step_is_the_two_launches(C, taps, dtype):
+    """One launch for batches of at most a token a chunk: the same numbers to the bit, of the rows and of the states, over
+    chunks of 0, 1 and 3 tokens, at positions inside the first taps (states of slots that begin hold NaN) and beyond."""
+    from mi355_decode import ops
+    from mi355_decode._lib import check, lib
+    g = torch.Generator().manual_seed(C)
+    for lens, first in (([1] * 7, [0, 1, 2, 3, 4, 100, 2]), ([1, 0, 3, 0, 1, 0, 1], [1, 0, 1, 0, 0, 0, 9])):
+        T, S = sum(lens), len(lens)
+        x = torch.randn(T, C + 16, generator=g).to(dtype).cuda()[:, 8: 8 + C]
+        w = torch.randn(C, taps, generator=g).to(dtype).cuda()
+        slots = torch.tensor([5, 0, 3, 1, 2, 6, 4], dtype=torch.int32)
+        state = torch.randn(S + 1, taps - 1, C, generator=g)
+        for s_, p in zip(slots.tolist(), first):
+            state[s_, : max(taps - 1 - p, 0)] = float("nan")
+        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+        seq = torch.repeat_interleave(torch.arange(S, dtype=torch.int32), torch.tensor(lens)).cuda()
+        pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)]).cuda()
+        one, two, slots = state.cuda(), state.cuda(), slots.cuda()
+        y = ops.causal_conv_silu(x, w, one, seq, pos, cu, slots)
+        z, dt, st = torch.empty_like(y), ops._DT[dtype], torch.cuda.current_stream().cuda_stream
+        check(lib.mi355_causal_conv_silu(z.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), two.data_ptr(), seq.data_ptr(),
+                                         pos.data_ptr(), cu.data_ptr(), slots.data_ptr(), T, C, taps, dt, st))
+        check(lib.mi355_conv_state_update(two.data_ptr(), x.data_ptr(), x.stride(0), cu.data_ptr(), slots.data_ptr(), S, C, taps, dt, st))
+        assert torch.isfinite(y).all() and torch.equal(y, z)
+        assert torch.equal(one.view(torch.int32), two.view(torch.int32))
+
+
+@pytest.mark.parametrize("H,G,d,dv,per_channel,dtype", [(2, 1, 64, 64, False, torch.bfloat16), (2, 2, 128, 120, True, torch.bfloat16),
+                                                        (4, 2, 32, 4, True, torch.float16), (1, 1, 20, 17, False, torch.bfloat16),
+                                                        (1, 1, 192, 68, True, torch.float32), (1, 1, 256, 300, False, torch.float16)])
+def test_delta_rule_steps_of_a_mixed_batch(H, G, d, dv, per_channel, dtype):
+    """Chunks of 1, 1, 0, 3 and 2 tokens without a workspace (four columns a lane; a column where v_dim is no multiple of 4),
+    from a state and at position 0 (whose slot holds NaN).  Bound: float32 sums of up to d + 8 products, 2^-24 each."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(d + dv)
+    lens, first = [1, 1, 0, 3, 2], [0, 5, 0, 2, 0]
+    T, S, qk = sum(lens), len(lens), G * d
+    qkv = torch.randn(T, 2 * qk + H * dv, generator=g).to(dtype)
+    beta = torch.randn(T, H, generator=g).to(dtype)
+    decay = torch.randn(T, H * d if per_channel else H, generator=g).to(dtype)
+    a_log, dt_bias = torch.randn(H, generator=g) * 0.5 - 1, torch.randn(decay.shape[1], generator=g) * 0.5
+    state = torch.randn(S, H, d, dv, generator=g)
+    start = state.double()
+    for s in range(S):
+        if first[s] == 0 and lens[s] > 0:
+            state[s] = float("nan")
+            start[s] = 0.0
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)])
+    dev = state.cuda()
+    out = ops.gated_delta_rule(qkv.cuda(), 0, qk, 2 * qk, beta.cuda(), decay.cuda(), a_log.cuda(), dt_bias.cuda(), dev,
+                               cu.to(torch.int32).cuda(), pos.cuda(), torch.arange(S, dtype=torch.int32, device="cuda"), H, G, d, dv,
+                               per_channel=per_channel).cpu()
+    f, rep = qkv.double(), H // G
+    q = (R.unit(f[:, :qk].view(T, G, d)) * d ** -0.5).repeat_interleave(rep, dim=1)
+    k = R.unit(f[:, qk:2 * qk].view(T, G, d)).repeat_interleave(rep, dim=1)
+    v, b = f[:, 2 * qk:].view(T, H, dv), torch.sigmoid(beta.double())
+    z = torch.nn.functional.softplus(decay.double() + dt_bias.double())
+    a = torch.exp(-torch.exp(a_log.double())[None, :, None] * (z.view(T, H, d) if per_channel else z[:, :, None].expand(T, H, d)))
+    bound = 2 * (d + 8) * 2.0 ** -24
+    for s in range(S):
+        M = start[s]
+        for t in range(int(cu[s]), int(cu[s + 1])):
+            M = M * a[t][:, :, None]
+            u = b[t][:, None] * (v[t] - (k[t][:, None, :] @ M).squeeze(1))
+            M = M + k[t][:, :, None] * u[:, None, :]
+            o = (q[t][:, None, :] @ M).squeeze(1)
+            assert (out[t].view(H, dv) - o).abs().max() <= bound * M.abs().max(), (s, t)
+        assert (dev[s].cpu() - M).abs().max() <= bound * M.abs().max(), s
+
+
 @pytest.mark.parametrize("H,G,d,dv,per_channel,dtype", [(2, 1, 64, 64, False, torch.bfloat16), (2, 2, 128, 120, True, torch.bfloat16),
                                                         (4, 2, 128, 128, False, torch.float16), (1, 1, 20, 17, False, torch.bfloat16),
                                                         (1, 1, 192, 16, True, torch.float32), (2, 1, 136, 200, False, torch.float32),

@@ -404,6 +404,56 @@ __global__ __launch_bounds__(256) void conv_state_update_kernel(
   }
 }
 
+// Convolution and state update in one launch, for batches of about a token a chunk: a thread has 8 channels of a chunk,
+// reads their state, walks the tokens and leaves the last inputs behind (no other thread reads those channels).  Bound by
+// the launch: 32 rows of 4096 channels 4.8 us (two launches 5.4 + 5.3).
+template <typename T, int TAPS>
+__global__ __launch_bounds__(64) void conv_silu_step_kernel(
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
+    float* __restrict__ state, const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_seqlens,
+    const int32_t* __restrict__ state_slots, int C) {
+  const int s = blockIdx.x, c8 = (blockIdx.y * 64 + threadIdx.x) * 8;
+  if (c8 >= C) return;
+  const int64_t cs = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s), ce = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s + 1);
+  if (ce <= cs) return;
+  float* st = state + static_cast<int64_t>(MI355_LD(int32_t, state_slots, state_slots + s)) * (TAPS - 1) * C + c8;
+  float wv[TAPS][8], in[TAPS][8];                        // in: the window, oldest first, the token's own input last
+  uint4 wr[TAPS];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) wr[j] = MI355_LD(uint4, w, w + static_cast<int64_t>(c8) * TAPS + 8 * j);
+#pragma unroll
+  for (int j = 0; j < TAPS - 1; ++j) {
+    const float4 a = MI355_LD(float4, state, st + static_cast<int64_t>(j) * C), b = MI355_LD(float4, state, st + static_cast<int64_t>(j) * C + 4);
+    in[j][0] = a.x, in[j][1] = a.y, in[j][2] = a.z, in[j][3] = a.w, in[j][4] = b.x, in[j][5] = b.y, in[j][6] = b.z, in[j][7] = b.w;
+  }
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) unpack8<T>(wr[j], wv[j]);
+  for (int64_t t = cs; t < ce; ++t) {
+    unpack8<T>(MI355_LD(uint4, x, x + t * x_stride + c8), in[TAPS - 1]);
+    const int64_t p = MI355_LD(int64_t, positions, positions + t);
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      if (p - (TAPS - 1 - j) < 0) continue;              // zeros before the start of the sequence
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] += (&wv[0][0])[i * TAPS + j] * in[j][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = acc[i] / (1.0f + expf(-acc[i]));
+    MI355_ST(uint4, y, y + t * C + c8, pack8<T>(acc));
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) in[j][i] = in[j + 1][i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TAPS - 1; ++j) {
+    MI355_ST(float4, state, st + static_cast<int64_t>(j) * C, make_float4(in[j][0], in[j][1], in[j][2], in[j][3]));
+    MI355_ST(float4, state, st + static_cast<int64_t>(j) * C + 4, make_float4(in[j][4], in[j][5], in[j][6], in[j][7]));
+  }
+}
+
 // One wave per (chunk, head, 64 value channels).  Lane j owns column j of the head's state matrix
 // S [d, dv] in registers (D >= d rows, the rest zero) and walks the chunk's tokens in order.  Per
 // token the wave first prepares, in LDS, the unit-length key, the unit-length scaled query and the
@@ -487,6 +537,127 @@ __global__ __launch_bounds__(64) void gated_delta_rule_kernel(
 #pragma unroll
     for (int i = 0; i < D; ++i)
       if (i < d) MI355_ST(float, state, sp + static_cast<int64_t>(i) * dv + col, S[i]);
+  }
+}
+
+// The same for value sizes that are a multiple of 4: one workgroup per (chunk, head, 64 value channels), 16 lanes of four
+// columns each by 16 groups of rows.  A thread holds D / 16 rows of its columns, loaded and stored by 16 bytes and all of
+// them on their way before the key is prepared; S'q = (a S)'q + u (k'q), so that one reduction over the rows serves the
+// removal and the result.  Bound by the state's trip from memory and back: 32 rows, 16 heads of 128 x 128, 13.9 us (4.8 TB/s; a
+// column a lane, one load of 4 bytes behind the other: 20.0), 8 heads with a decay a channel 10.2 (18.5).
+template <typename T, int D>
+__global__ __launch_bounds__(256) void gated_delta_step_kernel(
+    float* __restrict__ o, const typename Elem<T>::S* __restrict__ qkv, int64_t stride, int q_off, int k_off, int v_off,
+    const typename Elem<T>::S* __restrict__ beta, int64_t beta_stride, const typename Elem<T>::S* __restrict__ decay,
+    int64_t decay_stride, const float* __restrict__ a_log, const float* __restrict__ dt_bias, int per_channel,
+    float* __restrict__ state, const int32_t* __restrict__ cu_seqlens, const int64_t* __restrict__ positions,
+    const int32_t* __restrict__ state_slots, int H, int G, int d, int dv) {
+  constexpr int CW = 16, RG = 256 / CW, N = D / RG, V = (D + 63) / 64;
+  __shared__ __attribute__((aligned(16))) float ks[D], qs[D], as[D], sums[4][2][4 * CW];
+  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int cl = tid % CW, rg = tid / CW;
+  const int col = (blockIdx.z * CW + cl) * 4;
+  const bool live = col < dv;                            // (dv % 4 == 0: all four columns or none)
+  const int cc = live ? col : 0;
+  const int g = h / (H / G);
+  const int64_t cs = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s);
+  const int64_t n = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s + 1) - cs;
+  if (n <= 0) return;
+  const int64_t slot = MI355_LD(int32_t, state_slots, state_slots + s);
+  float* sp = state + ((slot * H + h) * d) * dv + cc;
+  const bool fresh = MI355_LD(int64_t, positions, positions + cs) == 0;
+  const float alog = MI355_LD(float, a_log, a_log + h);
+  const float qscale = 1.0f / sqrtf(static_cast<float>(d));
+  const int ch = tid < d ? tid : d - 1;                  // the channel whose decay this thread prepares
+  const int zc = per_channel ? h * d + ch : h;
+  const float bias = MI355_LD(float, dt_bias, dt_bias + zc);
+  float kv[V], qv[V], vj[4], z, bt;
+  auto token = [&](int64_t t) {
+    const typename Elem<T>::S* row = qkv + t * stride;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int c = lane + 64 * i, c1 = c < d ? c : d - 1;
+      kv[i] = MI355_LDF(T, qkv, row + k_off + g * d + c1);
+      qv[i] = MI355_LDF(T, qkv, row + q_off + g * d + c1);
+      kv[i] = c < d ? kv[i] : 0.f, qv[i] = c < d ? qv[i] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) vj[e] = MI355_LDF(T, qkv, row + v_off + h * dv + cc + e);
+    z = MI355_LDF(T, decay, decay + t * decay_stride + zc) + bias;
+    bt = MI355_LDF(T, beta, beta + t * beta_stride + h);
+  };
+  token(cs);
+  __builtin_amdgcn_sched_barrier(0);                     // (loads return in order: the token's values ahead of the state)
+  float4 S[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = j * RG + rg;
+    S[j] = MI355_LD(float4, state, sp + static_cast<int64_t>(i < d ? i : d - 1) * dv);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  for (int64_t r = 0; r < n; ++r) {
+    if (r > 0) {
+      token(cs + r);
+      __syncthreads();                                   // the previous token's reads of ks / qs / as / sums are done
+    }
+    float kk = 0.f, qq = 0.f, kq = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) kk += kv[i] * kv[i], qq += qv[i] * qv[i], kq += kv[i] * qv[i];
+    kk = 1.0f / sqrtf(wave_sum(kk) + 1e-6f);
+    qq = qscale / sqrtf(wave_sum(qq) + 1e-6f);
+    kq = wave_sum(kq) * kk * qq;
+    if (tid < D) {
+      float k1 = 0.f, q1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        if (i == wave) k1 = kv[i], q1 = qv[i];
+      ks[tid] = k1 * kk;
+      qs[tid] = q1 * qq;
+      as[tid] = tid < d ? expf(-expf(alog) * (z > 20.0f ? z : log1pf(expf(z)))) : 1.0f;
+    }
+    const float b = 1.0f / (1.0f + expf(-bt));
+    __syncthreads();
+    float4 dk = make_float4(0.f, 0.f, 0.f, 0.f), dq = dk;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int i = j * RG + rg;
+      if (r == 0 && (fresh || i >= d)) S[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+      const float a = as[i], k1 = ks[i], q1 = qs[i];
+      S[j].x *= a, S[j].y *= a, S[j].z *= a, S[j].w *= a;
+      dk.x += S[j].x * k1, dk.y += S[j].y * k1, dk.z += S[j].z * k1, dk.w += S[j].w * k1;
+      dq.x += S[j].x * q1, dq.y += S[j].y * q1, dq.z += S[j].z * q1, dq.w += S[j].w * q1;
+    }
+    auto over_rows = [](float v) { v += __shfl_xor(v, 16, 64); return v + __shfl_xor(v, 32, 64); };
+    dk = make_float4(over_rows(dk.x), over_rows(dk.y), over_rows(dk.z), over_rows(dk.w));
+    dq = make_float4(over_rows(dq.x), over_rows(dq.y), over_rows(dq.z), over_rows(dq.w));
+    if (lane < CW) {
+      *reinterpret_cast<float4*>(&sums[wave][0][4 * cl]) = dk;
+      *reinterpret_cast<float4*>(&sums[wave][1][4 * cl]) = dq;
+    }
+    __syncthreads();
+    dk = dq = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float4 x = *reinterpret_cast<const float4*>(&sums[w][0][4 * cl]), y = *reinterpret_cast<const float4*>(&sums[w][1][4 * cl]);
+      dk.x += x.x, dk.y += x.y, dk.z += x.z, dk.w += x.w;
+      dq.x += y.x, dq.y += y.y, dq.z += y.z, dq.w += y.w;
+    }
+    const float4 u = make_float4(b * (vj[0] - dk.x), b * (vj[1] - dk.y), b * (vj[2] - dk.z), b * (vj[3] - dk.w));
+    if (live && rg == 0)
+      MI355_ST(float4, o, o + ((cs + r) * H + h) * dv + col,
+               make_float4(dq.x + u.x * kq, dq.y + u.y * kq, dq.z + u.z * kq, dq.w + u.w * kq));
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float k1 = ks[j * RG + rg];
+      S[j].x += k1 * u.x, S[j].y += k1 * u.y, S[j].z += k1 * u.z, S[j].w += k1 * u.w;
+    }
+  }
+  if (live) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int i = j * RG + rg;
+      if (i < d) MI355_ST(float4, state, sp + static_cast<int64_t>(i) * dv, S[j]);
+    }
   }
 }
 
@@ -1139,6 +1310,32 @@ extern "C" int32_t mi355_conv_state_update(float* state, const void* x, int64_t 
   return check_launch("conv_state_update");
 }
 
+extern "C" int32_t mi355_conv_silu_step(void* y, const void* x, int64_t x_stride, const void* weight, float* state,
+                                        const int64_t* positions, const int32_t* cu_seqlens, const int32_t* state_slots,
+                                        int32_t num_seqs, int32_t channels, int32_t taps, int32_t dtype, void* stream) {
+  MI355_REQUIRE(y && x && weight && state && positions && cu_seqlens && state_slots, MI355_ERR_INVALID,
+                "conv_silu_step: null pointer");
+  MI355_REQUIRE(num_seqs >= 0 && channels > 0 && x_stride >= channels, MI355_ERR_INVALID, "conv_silu_step: sizes");
+  MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "conv_silu_step: dtype code %d", dtype);
+  MI355_REQUIRE(taps >= 2 && taps <= 4 && channels % 8 == 0 && x_stride % 8 == 0 && aligned16(x) && aligned16(y) &&
+                    aligned16(weight) && aligned16(state),
+                MI355_ERR_UNSUPPORTED, "conv_silu_step: 2 to 4 taps and rows of whole 16-byte pieces");
+  if (num_seqs == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid(static_cast<unsigned>(num_seqs), static_cast<unsigned>((channels / 8 + 63) / 64));
+#define MI355_CONV_STEP(TT, TAPS)                                                                                    \
+  hipLaunchKernelGGL((conv_silu_step_kernel<TT, TAPS>), grid, dim3(64), 0, s, static_cast<uint16_t*>(y),             \
+                     static_cast<const uint16_t*>(x), x_stride, static_cast<const uint16_t*>(weight), state, positions, \
+                     cu_seqlens, state_slots, channels)
+  if (dtype == MI355_BF16) {
+    if (taps == 2) MI355_CONV_STEP(BF16, 2); else if (taps == 3) MI355_CONV_STEP(BF16, 3); else MI355_CONV_STEP(BF16, 4);
+  } else {
+    if (taps == 2) MI355_CONV_STEP(F16, 2); else if (taps == 3) MI355_CONV_STEP(F16, 3); else MI355_CONV_STEP(F16, 4);
+  }
+#undef MI355_CONV_STEP
+  return check_launch("conv_silu_step");
+}
+
 template <typename TT>
 static void launch_delta(hipStream_t s, float* o, const void* qkv, int64_t stride, int q_off, int k_off, int v_off,
                          const void* beta, int64_t beta_stride, const void* decay, int64_t decay_stride,
@@ -1151,10 +1348,21 @@ static void launch_delta(hipStream_t s, float* o, const void* qkv, int64_t strid
   hipLaunchKernelGGL((gated_delta_rule_kernel<TT, D>), grid, dim3(64), 0, s, o, static_cast<const E*>(qkv), stride, \
                      q_off, k_off, v_off, static_cast<const E*>(beta), beta_stride, static_cast<const E*>(decay),   \
                      decay_stride, a_log, dt_bias, per_channel, state, cu_seqlens, positions, state_slots, H, G, d, dv)
-  if (d <= 32) MI355_DELTA(32);
+  // four columns a lane where the columns of a state row come in whole 16-byte pieces, a column a lane otherwise
+#define MI355_DELTA_STEP(D)                                                                                         \
+  hipLaunchKernelGGL((gated_delta_step_kernel<TT, D>), grid, dim3(256), 0, s, o, static_cast<const E*>(qkv), stride, \
+                     q_off, k_off, v_off, static_cast<const E*>(beta), beta_stride, static_cast<const E*>(decay),   \
+                     decay_stride, a_log, dt_bias, per_channel, state, cu_seqlens, positions, state_slots, H, G, d, dv)
+  if (dv % 4 == 0 && aligned16(state) && aligned16(o)) {
+    if (d <= 32) MI355_DELTA_STEP(32);
+    else if (d <= 64) MI355_DELTA_STEP(64);
+    else if (d <= 128) MI355_DELTA_STEP(128);
+    else MI355_DELTA_STEP(256);
+  } else if (d <= 32) MI355_DELTA(32);
   else if (d <= 64) MI355_DELTA(64);
   else if (d <= 128) MI355_DELTA(128);
   else MI355_DELTA(256);
+#undef MI355_DELTA_STEP
 #undef MI355_DELTA
 }
 

@@ -116,6 +116,7 @@ def _load() -> ctypes.CDLL:
         "mi355_sigmoid_window_attn": (I32, [P, P, I64, P, P, P, I32, P, P, P, P, P, I64, I64, I32, I32, I32, I32, I32,
                                             F, P, I32, P, I32, I32, P]),
         "mi355_causal_conv_silu": (I32, [P, P, I64, P, P, P, P, P, P, I64, I32, I32, I32, P]),
+        "mi355_conv_silu_step": (I32, [P, P, I64, P, P, P, P, P, I32, I32, I32, I32, P]),
         "mi355_conv_state_update": (I32, [P, P, I64, P, P, I32, I32, I32, I32, P]),
         "mi355_gated_delta_rule": (I32, [P, P, I64, I32, I32, I32, P, I64, P, I64, P, P, I32, P, P, P, P, I32, I32, I32,
                                          I32, I32, I64, P, I64, I32, P]),
@@ -203,7 +204,7 @@ EXPORTS = ("mi355_abi_version", "mi355_last_error", "mi355_target_arch",
            "mi355_embed_scale_f32", "mi355_embed_scale_pos_f32", "mi355_gated_act_rows", "mi355_resid_add_f32", "mi355_add_rms_norm_f32", "mi355_rms_norm_mix_f32",
            "mi355_gelu_tanh_and_mul", "mi355_gated_head_rms_norm", "mi355_softcap",
            "mi355_rope_partial_kv_write", "mi355_sigmoid_window_attn", "mi355_sigmoid_window_attn_prefill", "mi355_causal_conv_silu",
-           "mi355_conv_state_update", "mi355_gated_delta_rule", "mi355_gated_delta_rule_workspace",
+           "mi355_conv_state_update", "mi355_conv_silu_step", "mi355_gated_delta_rule", "mi355_gated_delta_rule_workspace",
            "mi355_general_delta_rule", "mi355_general_delta_rule_workspace", "mi355_group_rms_norm_f32",
            "mi355_gated_norm_resid_f32", "mi355_rms_norm_rows", "mi355_tanh_rows", "mi355_latent_kv_write",
            "mi355_latent_q_pack", "mi355_latent_window_attn_tiles",

@@ -1316,6 +1316,13 @@ def causal_conv_silu(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor,
         out = torch.empty(T, C, dtype=x.dtype, device=x.device)
     args = (_idx(cu_seqlens, "cu_seqlens", torch.int32), _idx(state_slots, "state_slots", torch.int32, S))
     st = _f32(state, "state") or x.data_ptr()                # one tap: the state is empty and never read
+    if T <= S and dt != _DT[torch.float32] and 2 <= taps <= 4 and C % 8 == 0 and x.stride(0) % 8 == 0 \
+            and (out.data_ptr() | x.data_ptr() | weight.data_ptr() | st) % 16 == 0:
+        # about a token a chunk (a thread walks a chunk's tokens): one launch, 4.8 us for 32 rows of 4096 against 10.7
+        _idx(tok_seq, "tok_seq", torch.int32, T)
+        check(lib.mi355_conv_silu_step(out.data_ptr(), x.data_ptr(), _cols(x, "x", C), weight.data_ptr(), st,
+                                       _idx(positions, "positions", torch.int64, T), *args, S, C, taps, dt, _stream()))
+        return out
     check(lib.mi355_causal_conv_silu(out.data_ptr(), x.data_ptr(), _cols(x, "x", C), weight.data_ptr(),
                                      st, _idx(tok_seq, "tok_seq", torch.int32, T),
                                      _idx(positions, "positions", torch.int64, T), *args, T, C, taps, dt, _stream()))
