@@ -311,6 +311,49 @@ def test_window_edge_shows_with_one_loud_key(window):
         assert got[inside, 3] > 0.99 and abs(got[outside, 3]) < 1e-6 and got[j0, 3] > 0.99 and got[j0 - 1, 3] == 0
 
 
+@pytest.mark.parametrize("H,G,d,dv,rot,norm,dtype", [
+    (16, 4, 128, 128, 0, True, torch.bfloat16), (3, 1, 40, 24, 16, True, torch.float16), (64, 8, 128, 256, 64, True, torch.bfloat16),
+    (16, 16, 256, 8, 32, True, torch.bfloat16), (16, 4, 128, 128, 64, False, torch.bfloat16), (2, 2, 64, 64, 64, False, torch.float16),
+    (1, 1, 8, 8, 0, False, torch.bfloat16), (8, 0, 128, 128, 128, False, torch.bfloat16)])
+@pytest.mark.parametrize("T", [1, 63, 64, 210])
+def test_rows_rotated_by_vectors_are_the_element_form(H, G, d, dv, rot, norm, dtype, T):
+    """Rows on 16-byte boundaries against the same rows one element off them (which go element by element): the same
+    queries, pages and untouched slots up to one rounding; slots that run through whole pages, break off inside, jump and
+    are missing; G = 0: queries only.  Bound: fp32 sums in another order may
+    move the one rounding of a result to the neighbouring number."""
+    from mi355_decode import ops
+    from mi355_decode.hybrid_runner import rotary_table
+    g = torch.Generator().manual_seed(H + d + T)
+    C = (H + G) * d + G * dv
+    wide = torch.randn(T, C + 40, generator=g).to(dtype)
+    pages = T // 16 + 6
+    slots = torch.cat([torch.arange(32, 32 + T - T // 3), torch.arange(5 + 32 + T, 5 + 32 + T + T // 3)])[:T].clone()
+    slots[T // 2] = -1
+    pos = torch.randint(0, 300, (T,), generator=g)
+    cs = rotary_table(rot, 100.0, 256, "cuda") if rot else torch.zeros(1, device="cuda")
+    wq, wk = torch.rand(max(H * d, 4), generator=g).cuda() + 0.5, torch.rand(max(G * d, 4), generator=g).cuda() + 0.5
+    got = []
+    for shift in (16, 17):
+        x = torch.empty(T, C + 40, dtype=dtype)
+        x[:, shift: shift + C] = wide[:, :C]
+        x = x.cuda()
+        q, k, v = (x[:, shift + o: shift + o + n] for o, n in ((0, H * d), (H * d, G * d), ((H + G) * d, G * dv)))
+        kc = torch.full((pages + T // 16 + 2, max(G, 1), 16, d), 7.0, dtype=dtype, device="cuda")
+        vc = torch.full((pages + T // 16 + 2, max(G, 1), dv, 16), 7.0, dtype=dtype, device="cuda")
+        if norm:
+            ops.row_norm_rope_kv_write(q, k, v, wq[:H * d], wk[:G * d], cs if rot else torch.zeros(256, 0, device="cuda"),
+                                       pos.cuda(), slots.cuda(), kc, vc, H, G, d, dv, 1e-5)
+        elif G:
+            ops.rope_partial_kv_write(q, k, v, cs if rot else torch.zeros(256, 0, device="cuda"), pos.cuda(), slots.cuda(), kc, vc, H, G, d, dv)
+        else:
+            ops.rope_partial_kv_write(q, None, None, cs, pos.cuda(), slots.cuda(), None, None, H, 1, d, dv)
+        got.append([t.float().cpu() for t in (q, kc, vc)])
+    u = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)        # the step between neighbours, relative
+    for a, b in zip(*got):
+        assert (a - b).abs().max() <= u * max(float(b.abs().max()), 1.0), (a - b).abs().max()
+    assert torch.equal(got[0][2], got[1][2])                   # V is moved, not computed
+
+
 def _delta_in_cuts(qkv, beta, decay, a_log, dt_bias, cuts, H, G, d, dv, per_channel, slot=2, slots=4, long_chunks=False):
     from mi355_decode import ops
     T = qkv.shape[0]

@@ -25,6 +25,7 @@
 // + bias) is formed on the fly, and q, k (rotated) and v are all written to the
 // packed 16-bit rows, which then hold what the plain form leaves there.
 #include "common.h"
+#include "kv_rows.h"
 
 namespace mi355 {
 
@@ -143,10 +144,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
 // V heads of a prefill-sized call: one wave per (16 packed tokens, kv head).
 constexpr int kVPitch = 48;   // LDS bytes per head_dim row of the transposed tile: 16 tokens x 2 B + padding, 16-byte aligned
 
-__global__ __launch_bounds__(256) void v_pages_kernel(const uint16_t* __restrict__ qkv, int64_t qkv_stride,
+__global__ __launch_bounds__(256) void v_pages_kernel(const uint16_t* __restrict__ rows, int64_t stride,
                                                       const int64_t* __restrict__ slot_mapping,
                                                       uint16_t* __restrict__ v_cache, int num_blocks, int64_t num_tokens,
-                                                      int num_heads, int num_kv_heads, int head_dim) {
+                                                      int num_kv_heads, int head_dim) {
   constexpr int BS = MI355_BLOCK_SIZE;
   __shared__ __attribute__((aligned(16))) unsigned char lds_all[4 * 256 * kVPitch];   // per wave: head_dim (<= 256) rows
   const int lane = threadIdx.x & 63;
@@ -165,10 +166,10 @@ __global__ __launch_bounds__(256) void v_pages_kernel(const uint16_t* __restrict
     const int64_t slot0 = __shfl(slot, 0, 64);
     const bool in_order = valid && slot == slot0 + t;
     const bool full = __all(in_order) && slot0 >= 0 && (slot0 % BS) == 0 && slot0 + BS <= slots_total;   // wave-uniform
-    const uint16_t* src = qkv + (valid ? tok : 0) * qkv_stride + static_cast<int64_t>(num_heads + num_kv_heads + kvh) * head_dim;
+    const uint16_t* src = rows + (valid ? tok : 0) * stride + static_cast<int64_t>(kvh) * head_dim;
     if (full) {
       for (int piece = p0; piece < pieces; piece += 4) {
-        const uint4 v = MI355_LD(uint4, qkv, src + 8 * piece);
+        const uint4 v = MI355_LD(uint4, rows, src + 8 * piece);
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(256) void v_pages_kernel(const uint16_t* __restrict
     } else if (valid && slot >= 0 && slot < slots_total) {
       uint16_t* dst = v_cache + ((slot / BS) * num_kv_heads + kvh) * static_cast<int64_t>(head_dim) * BS + (slot % BS);
       for (int piece = p0; piece < pieces; piece += 4) {
-        const uint4 v = MI355_LD(uint4, qkv, src + 8 * piece);
+        const uint4 v = MI355_LD(uint4, rows, src + 8 * piece);
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -196,6 +197,14 @@ __global__ __launch_bounds__(256) void v_pages_kernel(const uint16_t* __restrict
       }
     }
   }
+}
+
+void launch_v_pages(const uint16_t* v, int64_t v_stride, const int64_t* slot_mapping, uint16_t* v_cache, int num_blocks,
+                    int64_t num_tokens, int num_kv_heads, int v_dim, hipStream_t s) {
+  const int64_t tiles = ((num_tokens + 15) / 16) * num_kv_heads;
+  const int64_t blocks = (tiles + 3) / 4;
+  hipLaunchKernelGGL(v_pages_kernel, dim3(static_cast<unsigned>(blocks > 8192 ? 8192 : blocks)), dim3(256), 0, s, v, v_stride,
+                     slot_mapping, v_cache, num_blocks, num_tokens, num_kv_heads, v_dim);
 }
 
 template <bool PART>
@@ -249,14 +258,9 @@ static int32_t launch_rope(const char* name, void* qkv, int64_t qkv_stride, cons
                        slot_mapping, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache),
                        num_blocks, num_tokens, num_heads, num_kv_heads, head_dim, partial, num_slabs,
                        slab_stride, static_cast<const uint16_t*>(bias), skip_v);
-  if (skip_v) {
-    const int64_t tiles = ((num_tokens + 15) / 16) * num_kv_heads;
-    int64_t vblocks = (tiles + 3) / 4;
-    if (vblocks > 8192) vblocks = 8192;
-    hipLaunchKernelGGL(v_pages_kernel, dim3(static_cast<unsigned>(vblocks)), dim3(256), 0, s,
-                       static_cast<const uint16_t*>(qkv), qkv_stride, slot_mapping, static_cast<uint16_t*>(v_cache),
-                       num_blocks, num_tokens, num_heads, num_kv_heads, head_dim);
-  }
+  if (skip_v)
+    launch_v_pages(static_cast<const uint16_t*>(qkv) + static_cast<int64_t>(num_heads + num_kv_heads) * head_dim, qkv_stride,
+                   slot_mapping, static_cast<uint16_t*>(v_cache), num_blocks, num_tokens, num_kv_heads, head_dim, s);
   return check_launch(name);
 }
 

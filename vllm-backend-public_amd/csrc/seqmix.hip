@@ -20,6 +20,7 @@
 //                           u = xp + bx; out = S * silu(gp)
 #include "common.h"
 #include "delta_tiles.h"
+#include "kv_rows.h"
 
 namespace mi355 {
 
@@ -1139,6 +1140,16 @@ extern "C" int32_t mi355_rope_partial_kv_write(void* q, int64_t q_stride, const 
   REQ_DTYPE(dtype);
   if (num_tokens == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  KvRows a = {};
+  a.q = static_cast<uint16_t*>(q), a.k = static_cast<const uint16_t*>(k), a.v = static_cast<const uint16_t*>(v);
+  a.q_stride = q_stride, a.k_stride = k_stride, a.v_stride = v_stride, a.cos_sin = cos_sin, a.max_pos = max_pos;
+  a.positions = positions, a.slot_mapping = slot_mapping;
+  a.k_cache = static_cast<uint16_t*>(k_cache), a.v_cache = static_cast<uint16_t*>(v_cache), a.num_tokens = num_tokens;
+  a.H = num_heads, a.G = num_kv_heads, a.d = head_dim, a.dv = v_dim, a.rot = rot_dims;
+  if (dtype != MI355_F32 && kv_rows_ok(a)) {
+    launch_kv_rows<false>(a, dtype, s);
+    return check_launch("rope_partial_kv_write (vectors)");
+  }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((rope_partial_kv_write_kernel<TT>), dim3(num_tokens), dim3(256), 0, s,
                                                   static_cast<Elem<TT>::S*>(q), q_stride,
                                                   static_cast<const Elem<TT>::S*>(k), k_stride,
