@@ -1,6 +1,7 @@
 """Hybrid decoders (the Lozupel design), the parts that need no GPU: the config reader, the order
 of layer runs, the fused weight layout, state-slot bookkeeping in the scheduler, and the float32
 restatement's own invariants (a window edge, a state carried across a cut)."""
+import numpy as np
 import pytest
 import torch
 
@@ -198,3 +199,21 @@ def test_forced_steps_keep_pages_and_slots_straight():
     assert eng.alloc.num_free == 12 and eng.slots.num_free == 3 and not eng.seqs
     with pytest.raises(ValueError):
         eng.forced_step([("z", [99], [0])])                      # outside the vocabulary
+
+
+@pytest.mark.parametrize("rows", [1, 16, 64])
+def test_query_tiles_cover_every_row_once_in_order(rows):
+    from mi355_decode import ops
+    for lens in ([], [0], [1], [rows], [rows + 1, 0, 0, 2 * rows - 1], [0, 70, 3, 0, 129, rows, 0]):
+        cu, want = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64), []
+        for s, n in enumerate(lens):
+            want += [[s, int(cu[s]) + a, min(rows, n - a)] for a in range(0, n, rows)]
+        got = ops.query_tiles(cu, rows)
+        assert got.dtype == np.int32 and got.flags.c_contiguous and got.shape == (len(want), 3) and got.tolist() == want
+
+
+def test_upload_keeps_values_shapes_and_types():
+    from mi355_decode import ops
+    src = [np.arange(5, dtype=np.int64) - 2, np.zeros((0,), np.int32), np.arange(6, dtype=np.int32).reshape(2, 3)[:, ::2], np.zeros((3, 0), np.int64)]
+    for a, t in zip(src, ops.upload("cpu", *src)):
+        assert t.is_contiguous() and tuple(t.shape) == a.shape and t.numpy().dtype == a.dtype and (t.numpy() == a).all()

@@ -207,15 +207,14 @@ class LatentPlan:
         slots = np.concatenate([bt[s, : pages[s]] for s in np.flatnonzero(long)]).astype(np.int64)
         index = (slots[:, None] * BLOCK_SIZE + np.arange(BLOCK_SIZE)).reshape(-1).astype(np.int32)
         tables = np.minimum(first[:, None] + np.arange(max(int(pages.max()), 1))[None, :], max(self.pages - 1, 0)).astype(np.int32)
-        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device, non_blocking=True)     # noqa: E731
-        self.index, self.tables, self.ctx = t(index), t(tables), t(np.where(long, ctx, 0).astype(np.int32))
+        self.index, self.tables, self.ctx = ops.upload(device, index, tables, np.where(long, ctx, 0).astype(np.int32))
         self.short, self._short_tiles = None, {}
         if not long.all():
             ids = np.flatnonzero(~long)
             rows = np.concatenate([np.arange(cu[s], cu[s + 1]) for s in ids])
             self._short_cu = np.concatenate([[0], np.cumsum(lens[ids])])
             seq = np.repeat(np.arange(len(ids)), lens[ids]).astype(np.int32)
-            self.short = (t(rows), t(bt[ids].astype(np.int32)), t(seq))
+            self.short = tuple(ops.upload(device, rows.astype(np.int64), bt[ids].astype(np.int32), seq))
 
     def short_tiles(self, heads: int) -> torch.Tensor:
         if heads not in self._short_tiles:
@@ -1111,26 +1110,23 @@ class HybridRunner(ModelRunner):
         if logit_rows is None:
             return super().run_prefill(token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens,
                                        max_q_len, sampling=sampling, logprobs=logprobs, prompt_logprobs=prompt_logprobs)
-        dev = self.device
-        t = lambda a, dt: torch.from_numpy(np.ascontiguousarray(a)).to(dev, dtype=dt, non_blocking=True)  # noqa: E731
-        resid = self._run_chunks(t(token_ids, torch.int64), t(positions, torch.int64), t(slot_mapping, torch.int64),
-                                 t(block_tables, torch.int32), t(cu_seqlens, torch.int32), t(context_lens, torch.int32),
-                                 max_q_len)
         rows = np.asarray(logit_rows, dtype=np.int64)
+        host = [np.asarray(a, dtype=dt) for a, dt in ((token_ids, np.int64), (positions, np.int64), (slot_mapping, np.int64),
+                                                      (rows, np.int64), (block_tables, np.int32), (cu_seqlens, np.int32),
+                                                      (context_lens, np.int32))]
+        ids, pos, slots, at, tables, cu, ctx = ops.upload(self.device, *host)
+        resid = self._run_chunks(ids, pos, slots, tables, cu, ctx, max_q_len)
         if rows.size == 0:
             torch.cuda.current_stream().synchronize()
             return np.zeros((0, self.V), dtype=np.float32)
-        z = self._logits(resid.index_select(0, t(rows, torch.int64)))
+        z = self._logits(resid.index_select(0, at))
         return z.float().cpu().numpy()
 
     def _run_chunks(self, token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens=None,
                     max_q_len: int = 0) -> torch.Tensor:
-        S = cu_seqlens.numel() - 1
-        lens = (cu_seqlens[1:] - cu_seqlens[:-1]).to(torch.int64)
-        tok_seq = torch.repeat_interleave(torch.arange(S, dtype=torch.int32, device=self.device), lens,
-                                          output_size=int(token_ids.numel()))
-        slots = torch.from_numpy(self._step_state_slots).to(self.device, non_blocking=True)
-        tiles = torch.from_numpy(self._step_tiles).to(self.device, non_blocking=True)
+        lens = self._step_cu[1:] - self._step_cu[:-1]
+        tok_seq, slots, tiles = ops.upload(self.device, np.repeat(np.arange(len(lens), dtype=np.int32), lens),
+                                           self._step_state_slots, self._step_tiles)
         return self._forward(StepBatch(token_ids, positions, slot_mapping, block_tables.contiguous(), cu_seqlens,
                                        tok_seq, slots, tiles, self._step_long, pair_tiles=self._chunk_pair_tiles,
                                        context_lens=None if context_lens is None else context_lens.to(torch.int32).contiguous(),

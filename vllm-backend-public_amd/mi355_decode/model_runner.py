@@ -1011,9 +1011,10 @@ class ModelRunner:
         if prompt_logprobs is not None:
             pk, rows, targets = prompt_logprobs
             score = (int(pk), t(np.asarray(rows), torch.int64), t(np.asarray(targets), torch.int64))
-        nxt, logits = self.prefill(t(token_ids, torch.int64), t(positions, torch.int64), t(slot_mapping, torch.int64),
-                                   t(block_tables, torch.int32), t(cu_seqlens, torch.int32),
-                                   t(context_lens, torch.int32), int(max_q_len),
+        step = ops.upload(dev, *(np.asarray(a, dtype=dt) for a, dt in (
+            (token_ids, np.int64), (positions, np.int64), (slot_mapping, np.int64), (block_tables, np.int32),
+            (cu_seqlens, np.int32), (context_lens, np.int32))))
+        nxt, logits = self.prefill(*step, int(max_q_len),
                                    want_logits=sampling is not None or logprobs >= 0, score=score)
         if sampling is not None:
             self._sample(logits, sampling, nxt)
