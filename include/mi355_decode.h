@@ -833,6 +833,21 @@ int32_t mi355_rms_norm_mix_f32(float* resid, const void* xa, const void* wa, con
                                float alpha, int32_t dtype, void* stream);
 int32_t mi355_gelu_tanh_and_mul(void* out, const void* x, int64_t x_stride, int64_t num_tokens,
                                 int32_t inter, int32_t dtype, void* stream);
+/*
+ * The same on the fp32 slabs [num_slabs][num_tokens][width] (num_slabs 1 .. 8) that a K-split product leaves
+ * (mi355_linear_tiled, partial sums) in place of 16-bit rows: a value is the slabs' sum in slab order, rounded to dtype.
+ * 16-bit dtypes, widths that are multiples of 8 up to 8192 (the mix: 4096), 16-byte aligned buffers.
+ */
+int32_t mi355_add_rms_norm_f32_slabs(void* out, float* resid, const float* partial, int32_t num_slabs, const void* weight,
+                                     int32_t weight_numel, int64_t num_tokens, int32_t width, float eps, int32_t dtype,
+                                     void* stream);
+int32_t mi355_add_layer_norm_f32_slabs(void* out, float* resid, const float* partial, int32_t num_slabs, const void* weight,
+                                       int64_t num_tokens, int32_t width, float eps, int32_t dtype, void* stream);
+int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, int32_t na, const void* wa, const float* pb, int32_t nb,
+                                     const void* wb, int64_t num_tokens, int32_t width, float eps, float alpha, int32_t dtype,
+                                     void* stream);
+int32_t mi355_gelu_tanh_and_mul_slabs(void* out, const float* partial, int32_t num_slabs, int64_t num_tokens, int32_t inter,
+                                      int32_t dtype, void* stream);
 int32_t mi355_gated_head_rms_norm(void* out, int64_t out_stride, const float* o, const void* gate, int64_t gate_stride,
                                   const float* weight, int32_t weight_heads, int64_t num_tokens,
                                   int32_t num_heads, int32_t head_dim, float eps, int32_t activation,

@@ -153,6 +153,27 @@ def test_norms_and_pointwise(dtype):
         assert (out.float().cpu() - ref).abs().max() <= tol * ref.abs().max()
 
 
+@pytest.mark.parametrize("W", [8, 2048, 2056, 4096, 8192])
+@pytest.mark.parametrize("num", [1, 2, 3, 5, 8])
+def test_row_kernels_add_slabs_as_a_launch_of_their_own_would(W, num):
+    """Slabs of a K-split product against the rows that their sum leaves: the same numbers to the bit."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(W + num)
+    for T, dt in ((1, torch.float16), (33, torch.bfloat16)):
+        rn = lambda *s: torch.randn(*s, generator=g).cuda()                  # noqa: E731
+        slabs = lambda n, w: ops.Slabs(rn(n, T, w), n, T, w, dt)             # noqa: E731
+        x, y, wt, w2 = slabs(num, W), slabs(9 - num, W), rn(W).to(dt), rn(W).to(dt)
+        resid = rn(T, W)
+        for fn in (lambda r, a, b: ops.add_rms_norm_f32(r, wt, 1e-5, add=a), lambda r, a, b: ops.add_rms_norm_f32(r, wt[:1], 1e-5, add=a),
+                   lambda r, a, b: ops.add_layer_norm_f32(r, wt, 1e-5, add=a), lambda r, a, b: ops.add_layer_norm_f32(r, None, 1e-5, add=a),
+                   lambda r, a, b: ops.rms_norm_mix_f32(r, a, wt, b, w2, 1e-5, 0.5), lambda r, a, b: ops.rms_norm_mix_f32(r, a, wt, None, None, 1e-5, 0.5)):
+            r1, r2 = resid.clone(), resid.clone()
+            a, b = fn(r1, x, y), fn(r2, x.dense(), y.dense())
+            assert torch.isfinite(r1).all() and torch.equal(r1, r2) and (a is None or torch.equal(a, b))
+        z = slabs(num, 2 * W)
+        assert torch.equal(ops.gelu_tanh_and_mul(z), ops.gelu_tanh_and_mul(z.dense()))
+
+
 def _paged(T, num_pages, seed):
     """A shuffled block table for one sequence of T tokens and its slot mapping."""
     order = np.random.default_rng(seed).permutation(num_pages)[: (T + 15) // 16].astype(np.int32)

@@ -148,9 +148,44 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32_kernel(typename Elem<T>:
   }
 }
 
-template <typename T, int NV>
+// 8 columns of a sub-layer's output, given as 16-bit rows (S = 0) or as the fp32 slabs of a K-split product (n of them, at
+// most S, `slab` numbers apart): added in order and rounded to T, what a launch that writes the rows would leave.  All loads
+// go out before the first is used; those past the n-th repeat it.
+template <typename T, int S>
+struct Rows8 {
+  uint4 raw;
+  float4 a[S > 0 ? S : 1], b[S > 0 ? S : 1];
+  __device__ __forceinline__ void load(const void* rows, int64_t at, int64_t slab, int n) {
+    if (S == 0) {
+      raw = MI355_LD(uint4, rows, static_cast<const uint16_t*>(rows) + at);
+    } else {
+      const float* p = static_cast<const float*>(rows) + at;
+#pragma unroll
+      for (int g = 0; g < S; ++g) {
+        const int64_t off = slab * (g < n ? g : n - 1);
+        a[g] = MI355_LD(float4, rows, p + off), b[g] = MI355_LD(float4, rows, p + off + 4);
+      }
+    }
+  }
+  __device__ __forceinline__ void value(float (&f)[8], int n) const {
+    if (S == 0) {
+      unpack8<T>(raw, f);
+    } else {
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < S; ++g) {
+        const float x[8] = {a[g].x, a[g].y, a[g].z, a[g].w, b[g].x, b[g].y, b[g].z, b[g].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = g < n ? v[j] + x[j] : v[j];
+      }
+      unpack8<T>(pack8<T>(v), f);
+    }
+  }
+};
+
+template <typename T, int NV, int S>
 __global__ __launch_bounds__(256) void add_rms_norm_f32_vec_kernel(uint16_t* __restrict__ out, float* __restrict__ resid,
-                                                                   const uint16_t* __restrict__ add,
+                                                                   const void* __restrict__ add, int num_slabs,
                                                                    const uint16_t* __restrict__ weight, int weight_numel, int W,
                                                                    float eps) {
   __shared__ float scratch[32];
@@ -170,7 +205,9 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32_vec_kernel(uint16_t* __r
       if (weight_numel != 1) wv[i] = MI355_LD(uint4, weight, weight + c);
       if (add != nullptr) {
         float y[8];
-        unpack8<T>(MI355_LD(uint4, add, add + t * W + c), y);
+        Rows8<T, S> rows;
+        rows.load(add, t * W + c, static_cast<int64_t>(gridDim.x) * W, num_slabs);
+        rows.value(y, num_slabs);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[i][j] += y[j];
         store8f(resid, resid + t * W + c, v[i]);
@@ -234,13 +271,14 @@ __global__ __launch_bounds__(256) void add_layer_norm_f32_kernel(typename Elem<T
 }
 
 // 16-bit rows of a multiple of 8 columns, up to 2048 * NV: the row stays in registers between the passes
-template <typename T, int NV>
+template <typename T, int NV, int S>
 __global__ __launch_bounds__(256) void add_layer_norm_f32_vec_kernel(uint16_t* __restrict__ out, float* __restrict__ resid,
-                                                                     const uint16_t* __restrict__ add,
+                                                                     const void* __restrict__ add_, int num_slabs,
                                                                      const int32_t* __restrict__ inv, int top,
                                                                      float row_weight, const uint16_t* __restrict__ weight,
                                                                      int W, float eps) {
   __shared__ float scratch[32];
+  const uint16_t* add = static_cast<const uint16_t*>(add_);
   const int64_t t = blockIdx.x;
   float v[NV][8];
   uint4 wv[NV];
@@ -257,7 +295,9 @@ __global__ __launch_bounds__(256) void add_layer_norm_f32_vec_kernel(uint16_t* _
       b = MI355_LD(float4, resid, resid + t * W + c + 4);
       if (out != nullptr) wv[i] = MI355_LD(uint4, weight, weight + c);
       if (add != nullptr && inv == nullptr) {
-        unpack8<T>(MI355_LD(uint4, add, add + t * W + c), y);
+        Rows8<T, S> rows;
+        rows.load(add_, t * W + c, static_cast<int64_t>(gridDim.x) * W, num_slabs);
+        rows.value(y, num_slabs);
       } else if (add != nullptr) {
         for (int k = 0; k < top; ++k) {
           float f[8];
@@ -333,25 +373,26 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_kernel(float* __restrict
   }
 }
 
-template <typename T, int NV>
-__global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __restrict__ resid, const uint16_t* __restrict__ xa,
+template <typename T, int NV, int S>
+__global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __restrict__ resid, const void* __restrict__ xa, int na,
                                                                    const uint16_t* __restrict__ wa,
-                                                                   const uint16_t* __restrict__ xb,
+                                                                   const void* __restrict__ xb, int nb,
                                                                    const uint16_t* __restrict__ wb, int W, float eps,
                                                                    float alpha) {
   __shared__ float scratch[2][4];
-  const int64_t t = blockIdx.x;
-  uint4 a[NV], b[NV], ga[NV], gb[NV];
-  float v[NV][8], sa = 0.f, sb = 0.f;
+  const int64_t t = blockIdx.x, slab = static_cast<int64_t>(gridDim.x) * W;
+  uint4 ga[NV], gb[NV];
+  Rows8<T, S> a[NV], b[NV];
+  float fa[NV][8], fb[NV][8], v[NV][8], sa = 0.f, sb = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + 256 * i) * 8;
-    a[i] = b[i] = ga[i] = gb[i] = make_uint4(0, 0, 0, 0);
+    ga[i] = gb[i] = make_uint4(0, 0, 0, 0);
     if (c < W) {
-      a[i] = MI355_LD(uint4, xa, xa + t * W + c);
+      a[i].load(xa, t * W + c, slab, na);
       ga[i] = MI355_LD(uint4, wa, wa + c);
       if (xb != nullptr) {
-        b[i] = MI355_LD(uint4, xb, xb + t * W + c);
+        b[i].load(xb, t * W + c, slab, nb);
         gb[i] = MI355_LD(uint4, wb, wb + c);
       }
       load8f(resid, resid + t * W + c, v[i]);
@@ -359,10 +400,13 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __rest
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    float f[8], g[8];
-    unpack8<T>(a[i], f), unpack8<T>(b[i], g);
+    const bool on = (threadIdx.x + 256 * i) * 8 < static_cast<unsigned>(W);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sa += f[j] * f[j], sb += g[j] * g[j];
+    for (int j = 0; j < 8; ++j) fa[i][j] = fb[i][j] = 0.f;
+    if (on) a[i].value(fa[i], na);
+    if (on && xb != nullptr) b[i].value(fb[i], nb);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sa += fa[i][j] * fa[i][j], sb += fb[i][j] * fb[i][j];
   }
   sa = wave_sum(sa), sb = wave_sum(sb);                 // both sums over one barrier
   if ((threadIdx.x & 63) == 0) scratch[0][threadIdx.x >> 6] = sa, scratch[1][threadIdx.x >> 6] = sb;
@@ -375,12 +419,12 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __rest
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + 256 * i) * 8;
     if (c >= W) continue;
-    float f[8], g[8], x[8], y[8];
-    unpack8<T>(a[i], f), unpack8<T>(ga[i], x), unpack8<T>(b[i], g), unpack8<T>(gb[i], y);
+    float x[8], y[8];
+    unpack8<T>(ga[i], x), unpack8<T>(gb[i], y);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      float m = f[j] * ra * x[j];
-      if (xb != nullptr) m += g[j] * rb * y[j];
+      float m = fa[i][j] * ra * x[j];
+      if (xb != nullptr) m += fb[i][j] * rb * y[j];
       v[i][j] += alpha * m;
     }
     store8f(resid, resid + t * W + c, v[i]);
@@ -393,8 +437,8 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
 }
 
 // 16-bit rows, 8 elements per thread (16-byte loads and stores)
-template <typename T>
-__global__ __launch_bounds__(256) void gelu_tanh_and_mul_vec_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+template <typename T, int S>
+__global__ __launch_bounds__(256) void gelu_tanh_and_mul_vec_kernel(uint16_t* __restrict__ out, const void* __restrict__ x, int num_slabs,
                                                                     int64_t x_stride, int64_t num_tokens, int inter) {
   const int vec_per_row = inter >> 3;
   const int64_t total = num_tokens * vec_per_row;
@@ -402,10 +446,11 @@ __global__ __launch_bounds__(256) void gelu_tanh_and_mul_vec_kernel(uint16_t* __
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t row = i / vec_per_row;
     const int v = static_cast<int>(i % vec_per_row);
-    const uint16_t* xr = x + row * x_stride;
+    Rows8<T, S> xg, xu;
+    xg.load(x, row * x_stride + 8 * v, num_tokens * x_stride, num_slabs);
+    xu.load(x, row * x_stride + inter + 8 * v, num_tokens * x_stride, num_slabs);
     float g[8], u[8], y[8];
-    unpack8<T>(MI355_LD(uint4, x, xr + 8 * v), g);
-    unpack8<T>(MI355_LD(uint4, x, xr + inter + 8 * v), u);
+    xg.value(g, num_slabs), xu.value(u, num_slabs);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       y[j] = g[j] * __frcp_rn(1.0f + __expf(-1.5957691216057308f * (g[j] + 0.044715f * g[j] * g[j] * g[j]))) * u[j];
@@ -1013,9 +1058,9 @@ extern "C" int32_t mi355_add_rms_norm_f32(void* out, float* resid, const void* a
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) && aligned16(add) &&
       (weight_numel == 1 || aligned16(weight))) {
-#define MI355_RN(TT, NV)                                                                                                     \
-  hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
-                     resid, static_cast<const uint16_t*>(add), static_cast<const uint16_t*>(weight), weight_numel, width, eps)
+#define MI355_RN(TT, NV)                                                                                                        \
+  hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV, 0>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, add, 0, static_cast<const uint16_t*>(weight), weight_numel, width, eps)
 #define MI355_RN_NV(TT)                      \
   do {                                       \
     if (width <= 2048) MI355_RN(TT, 1);      \
@@ -1047,9 +1092,8 @@ extern "C" int32_t mi355_add_layer_norm_f32(void* out, float* resid, const void*
   if (dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) && aligned16(add) &&
       aligned16(weight)) {
 #define MI355_LN(TT, NV)                                                                                                   \
-  hipLaunchKernelGGL((add_layer_norm_f32_vec_kernel<TT, NV>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
-                     resid, static_cast<const uint16_t*>(add), inv, top, row_weight, static_cast<const uint16_t*>(weight),  \
-                     width, eps)
+  hipLaunchKernelGGL((add_layer_norm_f32_vec_kernel<TT, NV, 0>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, add, 0, inv, top, row_weight, static_cast<const uint16_t*>(weight), width, eps)
 #define MI355_LN_NV(TT)                      \
   do {                                       \
     if (width <= 2048) MI355_LN(TT, 1);      \
@@ -1080,9 +1124,8 @@ extern "C" int32_t mi355_rms_norm_mix_f32(float* resid, const void* xa, const vo
   if (dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(resid) && aligned16(xa) && aligned16(wa) &&
       aligned16(xb) && aligned16(wb)) {
 #define MI355_MIX(TT, NV)                                                                                                \
-  hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV>), dim3(num_tokens), dim3(256), 0, s, resid,                    \
-                     static_cast<const uint16_t*>(xa), static_cast<const uint16_t*>(wa), static_cast<const uint16_t*>(xb), \
-                     static_cast<const uint16_t*>(wb), width, eps, alpha)
+  hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV, 0>), dim3(num_tokens), dim3(256), 0, s, resid, xa, 0,          \
+                     static_cast<const uint16_t*>(wa), xb, 0, static_cast<const uint16_t*>(wb), width, eps, alpha)
 #define MI355_MIX_NV(TT)                      \
   do {                                       \
     if (width <= 2048) MI355_MIX(TT, 1);      \
@@ -1112,11 +1155,11 @@ extern "C" int32_t mi355_gelu_tanh_and_mul(void* out, const void* x, int64_t x_s
   if (dtype != MI355_F32 && inter % 8 == 0 && x_stride % 8 == 0 && aligned16(x) && aligned16(out)) {
     const dim3 grid = stride_grid(num_tokens * (inter / 8));
     if (dtype == MI355_BF16)
-      hipLaunchKernelGGL((gelu_tanh_and_mul_vec_kernel<BF16>), grid, dim3(256), 0, s, static_cast<uint16_t*>(out),
-                         static_cast<const uint16_t*>(x), x_stride, num_tokens, inter);
+      hipLaunchKernelGGL((gelu_tanh_and_mul_vec_kernel<BF16, 0>), grid, dim3(256), 0, s, static_cast<uint16_t*>(out), x, 0, x_stride,
+                         num_tokens, inter);
     else
-      hipLaunchKernelGGL((gelu_tanh_and_mul_vec_kernel<F16>), grid, dim3(256), 0, s, static_cast<uint16_t*>(out),
-                         static_cast<const uint16_t*>(x), x_stride, num_tokens, inter);
+      hipLaunchKernelGGL((gelu_tanh_and_mul_vec_kernel<F16, 0>), grid, dim3(256), 0, s, static_cast<uint16_t*>(out), x, 0, x_stride,
+                         num_tokens, inter);
     return check_launch("gelu_tanh_and_mul");
   }
   MI355_DISPATCH_DTYPE3(dtype, hipLaunchKernelGGL((gelu_tanh_and_mul_kernel<TT>), stride_grid(num_tokens * inter), dim3(256),
@@ -1124,6 +1167,113 @@ extern "C" int32_t mi355_gelu_tanh_and_mul(void* out, const void* x, int64_t x_s
                                                   static_cast<const Elem<TT>::S*>(x), x_stride, num_tokens, inter));
   return check_launch("gelu_tanh_and_mul");
 }
+
+// ---- the norms, the mix and the gate on the fp32 slabs of K-split products (decoded rows): the launch that would add the slabs, 4 to 5 us
+// whatever it adds, falls away.  num_slabs 1 .. 8, slabs [num_slabs][num_tokens][width].
+#define MI355_SLABS(n, CALL) \
+  do {                       \
+    if ((n) <= 2) CALL(2);   \
+    else if ((n) <= 4) CALL(4); \
+    else CALL(8);            \
+  } while (0)
+
+extern "C" int32_t mi355_add_rms_norm_f32_slabs(void* out, float* resid, const float* partial, int32_t num_slabs, const void* weight,
+                                                int32_t weight_numel, int64_t num_tokens, int32_t width, float eps, int32_t dtype,
+                                                void* stream) {
+  MI355_REQUIRE(out && resid && weight && partial, MI355_ERR_INVALID, "add_rms_norm_f32_slabs: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && width > 0 && num_slabs >= 1 && num_slabs <= 8 && (weight_numel == 1 || weight_numel == width),
+                MI355_ERR_INVALID, "add_rms_norm_f32_slabs: sizes");
+  MI355_REQUIRE(dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) && aligned16(partial) &&
+                    (weight_numel == 1 || aligned16(weight)),
+                MI355_ERR_UNSUPPORTED, "add_rms_norm_f32_slabs: 16-bit rows of whole 16-byte pieces, at most 8192 wide");
+  REQ_DTYPE(dtype);
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define MI355_RN(TT, NV, S)                                                                                                     \
+  hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, partial, num_slabs, static_cast<const uint16_t*>(weight), weight_numel, width, eps)
+#define MI355_RN_B(S) \
+  do { if (width <= 2048) MI355_RN(BF16, 1, S); else if (width <= 4096) MI355_RN(BF16, 2, S); else MI355_RN(BF16, 4, S); } while (0)
+#define MI355_RN_H(S) \
+  do { if (width <= 2048) MI355_RN(F16, 1, S); else if (width <= 4096) MI355_RN(F16, 2, S); else MI355_RN(F16, 4, S); } while (0)
+  if (dtype == MI355_BF16) MI355_SLABS(num_slabs, MI355_RN_B); else MI355_SLABS(num_slabs, MI355_RN_H);
+#undef MI355_RN_H
+#undef MI355_RN_B
+#undef MI355_RN
+  return check_launch("add_rms_norm_f32_slabs");
+}
+
+extern "C" int32_t mi355_add_layer_norm_f32_slabs(void* out, float* resid, const float* partial, int32_t num_slabs, const void* weight,
+                                                  int64_t num_tokens, int32_t width, float eps, int32_t dtype, void* stream) {
+  MI355_REQUIRE(out && resid && weight && partial, MI355_ERR_INVALID, "add_layer_norm_f32_slabs: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && width > 0 && num_slabs >= 1 && num_slabs <= 8, MI355_ERR_INVALID, "add_layer_norm_f32_slabs: sizes");
+  MI355_REQUIRE(dtype != MI355_F32 && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) && aligned16(partial) &&
+                    aligned16(weight),
+                MI355_ERR_UNSUPPORTED, "add_layer_norm_f32_slabs: 16-bit rows of whole 16-byte pieces, at most 8192 wide");
+  REQ_DTYPE(dtype);
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define MI355_LN(TT, NV, S)                                                                                                       \
+  hipLaunchKernelGGL((add_layer_norm_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, partial, num_slabs, nullptr, 1, 1.0f, static_cast<const uint16_t*>(weight), width, eps)
+#define MI355_LN_B(S) \
+  do { if (width <= 2048) MI355_LN(BF16, 1, S); else if (width <= 4096) MI355_LN(BF16, 2, S); else MI355_LN(BF16, 4, S); } while (0)
+#define MI355_LN_H(S) \
+  do { if (width <= 2048) MI355_LN(F16, 1, S); else if (width <= 4096) MI355_LN(F16, 2, S); else MI355_LN(F16, 4, S); } while (0)
+  if (dtype == MI355_BF16) MI355_SLABS(num_slabs, MI355_LN_B); else MI355_SLABS(num_slabs, MI355_LN_H);
+#undef MI355_LN_H
+#undef MI355_LN_B
+#undef MI355_LN
+  return check_launch("add_layer_norm_f32_slabs");
+}
+
+extern "C" int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, int32_t na, const void* wa, const float* pb, int32_t nb,
+                                                const void* wb, int64_t num_tokens, int32_t width, float eps, float alpha,
+                                                int32_t dtype, void* stream) {
+  MI355_REQUIRE(resid && pa && wa && pb && wb, MI355_ERR_INVALID, "rms_norm_mix_f32_slabs: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && width > 0 && na >= 1 && na <= 8 && nb >= 1 && nb <= 8, MI355_ERR_INVALID,
+                "rms_norm_mix_f32_slabs: sizes");
+  MI355_REQUIRE(dtype != MI355_F32 && width % 8 == 0 && width <= 4096 && aligned16(resid) && aligned16(pa) && aligned16(wa) &&
+                    aligned16(pb) && aligned16(wb),
+                MI355_ERR_UNSUPPORTED, "rms_norm_mix_f32_slabs: 16-bit rows of whole 16-byte pieces, at most 4096 wide");
+  REQ_DTYPE(dtype);
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int most = na > nb ? na : nb;
+#define MI355_MIX(TT, NV, S)                                                                                               \
+  hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, resid, pa, na,           \
+                     static_cast<const uint16_t*>(wa), pb, nb, static_cast<const uint16_t*>(wb), width, eps, alpha)
+#define MI355_MIX_B(S) do { if (width <= 2048) MI355_MIX(BF16, 1, S); else MI355_MIX(BF16, 2, S); } while (0)
+#define MI355_MIX_H(S) do { if (width <= 2048) MI355_MIX(F16, 1, S); else MI355_MIX(F16, 2, S); } while (0)
+  if (dtype == MI355_BF16) MI355_SLABS(most, MI355_MIX_B); else MI355_SLABS(most, MI355_MIX_H);
+#undef MI355_MIX_H
+#undef MI355_MIX_B
+#undef MI355_MIX
+  return check_launch("rms_norm_mix_f32_slabs");
+}
+
+extern "C" int32_t mi355_gelu_tanh_and_mul_slabs(void* out, const float* partial, int32_t num_slabs, int64_t num_tokens, int32_t inter,
+                                                 int32_t dtype, void* stream) {
+  MI355_REQUIRE(out && partial, MI355_ERR_INVALID, "gelu_tanh_and_mul_slabs: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && inter > 0 && num_slabs >= 1 && num_slabs <= 8, MI355_ERR_INVALID, "gelu_tanh_and_mul_slabs: sizes");
+  MI355_REQUIRE(dtype != MI355_F32 && inter % 8 == 0 && aligned16(partial) && aligned16(out), MI355_ERR_UNSUPPORTED,
+                "gelu_tanh_and_mul_slabs: 16-bit rows of whole 16-byte pieces");
+  REQ_DTYPE(dtype);
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid = stride_grid(num_tokens * (inter / 8));
+#define MI355_GELU(TT, S)                                                                                                  \
+  hipLaunchKernelGGL((gelu_tanh_and_mul_vec_kernel<TT, S>), grid, dim3(256), 0, s, static_cast<uint16_t*>(out), partial,   \
+                     num_slabs, 2ll * inter, num_tokens, inter)
+#define MI355_GELU_B(S) MI355_GELU(BF16, S)
+#define MI355_GELU_H(S) MI355_GELU(F16, S)
+  if (dtype == MI355_BF16) MI355_SLABS(num_slabs, MI355_GELU_B); else MI355_SLABS(num_slabs, MI355_GELU_H);
+#undef MI355_GELU_H
+#undef MI355_GELU_B
+#undef MI355_GELU
+  return check_launch("gelu_tanh_and_mul_slabs");
+}
+#undef MI355_SLABS
 
 extern "C" int32_t mi355_gated_head_rms_norm(void* out, int64_t out_stride, const float* o, const void* gate,
                                              int64_t gate_stride, const float* weight, int32_t weight_heads,

@@ -107,6 +107,10 @@ def _load() -> ctypes.CDLL:
         "mi355_embed_scale_pos_f32": (I32, [P, P, P, P, P, I64, I32, I64, I64, F, I32, P]),
         "mi355_resid_add_f32": (I32, [P, P, P, P, I64, I32, I32, P]),
         "mi355_add_rms_norm_f32": (I32, [P, P, P, P, I32, I64, I32, F, I32, P]),
+        "mi355_add_rms_norm_f32_slabs": (I32, [P, P, P, I32, P, I32, I64, I32, F, I32, P]),
+        "mi355_add_layer_norm_f32_slabs": (I32, [P, P, P, I32, P, I64, I32, F, I32, P]),
+        "mi355_rms_norm_mix_f32_slabs": (I32, [P, P, I32, P, P, I32, P, I64, I32, F, F, I32, P]),
+        "mi355_gelu_tanh_and_mul_slabs": (I32, [P, P, I32, I64, I32, I32, P]),
         "mi355_rms_norm_mix_f32": (I32, [P, P, P, P, P, I64, I32, F, F, I32, P]),
         "mi355_gelu_tanh_and_mul": (I32, [P, P, I64, I64, I32, I32, P]),
         "mi355_gated_head_rms_norm": (I32, [P, I64, P, P, I64, P, I32, I64, I32, I32, F, I32, I32, P]),
@@ -201,7 +205,8 @@ EXPORTS = ("mi355_abi_version", "mi355_last_error", "mi355_target_arch",
            "mi355_allreduce_oneshot_run", "mi355_allreduce_oneshot_run_slabs", "mi355_allreduce_oneshot_run_add_norm", "mi355_allreduce_twoshot_run_add_norm", "mi355_allreduce_oneshot_run_max_keys",
            "mi355_allreduce_oneshot_status",
            "mi355_allreduce_oneshot_status_async", "mi355_allreduce_oneshot_destroy",
-           "mi355_embed_scale_f32", "mi355_embed_scale_pos_f32", "mi355_gated_act_rows", "mi355_resid_add_f32", "mi355_add_rms_norm_f32", "mi355_rms_norm_mix_f32",
+           "mi355_embed_scale_f32", "mi355_embed_scale_pos_f32", "mi355_gated_act_rows", "mi355_resid_add_f32", "mi355_add_rms_norm_f32", "mi355_rms_norm_mix_f32", "mi355_add_rms_norm_f32_slabs", "mi355_add_layer_norm_f32_slabs",
+           "mi355_rms_norm_mix_f32_slabs", "mi355_gelu_tanh_and_mul_slabs",
            "mi355_gelu_tanh_and_mul", "mi355_gated_head_rms_norm", "mi355_softcap",
            "mi355_rope_partial_kv_write", "mi355_sigmoid_window_attn", "mi355_sigmoid_window_attn_prefill", "mi355_causal_conv_silu",
            "mi355_conv_state_update", "mi355_conv_silu_step", "mi355_gated_delta_rule", "mi355_gated_delta_rule_workspace",

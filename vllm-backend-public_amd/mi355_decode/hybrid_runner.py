@@ -102,6 +102,11 @@ class StepBatch:
         self.num_tokens, self.num_seqs = int(ids.numel()), int(cu_seqlens.numel()) - 1
 
 
+def _out_product(r, x: torch.Tensor, w: torch.Tensor):
+    """A sub-layer's last product: HybridRunner.out_linear, or plainly the product for another owner of the sub-layer."""
+    return getattr(r, "out_linear", r.linear)(x, w)
+
+
 class WindowAttention:
     """Sliding-window attention with sigmoid weights over the paged K/V of one layer run."""
 
@@ -126,11 +131,11 @@ class WindowAttention:
                 and q.data_ptr() % 16 == 0 and ops.chunk_attn_prefill_ok(q.dtype, s.heads, s.kv_heads, s.dim, s.vdim):
             o = ops.sigmoid_window_attn_prefill(q, kc, vc, b.block_tables, b.cu_seqlens, b.context_lens, b.max_q_len,
                                                 self.lw.attn_temp, self.lw.attn_bias, g, s.heads, s.window, s.scale)
-            return r.linear(o, self.lw.attn_o_w)
+            return _out_product(r, o, self.lw.attn_o_w)
         o = ops.sigmoid_window_attn(q, kc, vc, b.block_tables, b.tok_seq, b.positions, self.lw.attn_temp,
                                     self.lw.attn_bias, g, s.heads, s.window, s.scale, tiles=b.tiles,
                                     **r.key_splits(b, s))
-        return r.linear(o, self.lw.attn_o_w)
+        return _out_product(r, o, self.lw.attn_o_w)
 
 
 class DeltaMixer:
@@ -159,7 +164,7 @@ class DeltaMixer:
                                  b.positions, b.state_slots, s.heads, s.kv_heads, s.dim, s.vdim,
                                  per_channel=s.per_channel, long_chunks=b.long_chunks)
         on = ops.gated_head_rms_norm(o, gate, lw.head_norm, r.eps, ops.ACT_SIGMOID if s.per_channel else ops.ACT_SILU)
-        return r.linear(on, lw.delta_o_w)
+        return _out_product(r, on, lw.delta_o_w)
 
 
 class GeneralDeltaMixer:
@@ -250,8 +255,8 @@ class LatentAttention:
         gate = col("g") if s.gate else None
         plan = b.latent_plan() if self.expands and b.long_chunks and b.latent_plan is not None else None
         if plan is None or not plan.fits or plan.pages * BLOCK_SIZE * s.heads * (s.dim + s.rot_dim + s.vdim) * 2 > plan.MAX_BYTES:
-            return r.linear(self._on_latents(q, gate, b.positions, b.block_tables, b.tok_seq, b.pair_tiles), lw.o_w)
-        return r.linear(self._expanded(q, gate, b, plan), lw.o_w)
+            return _out_product(r, self._on_latents(q, gate, b.positions, b.block_tables, b.tok_seq, b.pair_tiles), lw.o_w)
+        return _out_product(r, self._expanded(q, gate, b, plan), lw.o_w)
 
     def _expanded(self, q: torch.Tensor, gate: Optional[torch.Tensor], b: StepBatch, plan: LatentPlan) -> torch.Tensor:
         s, lw, r = self.s, self.lw, self.r
@@ -323,7 +328,7 @@ class BlockAttention:
         ops.qk_norm_kv_write(q, k, k, lw.q_norm, lw.k_norm, b.slot_mapping, kc, vc, s.heads, s.kv_heads, s.dim, s.vdim, r.eps)
         o = ops.softmax_bias_attn(q, kc, vc, b.block_tables, b.tok_seq, b.positions, lw.r1, lw.r2, col("g"), s.heads,
                                   s.scale, block=s.block, tiles=b.tiles, num_splits=r.block_key_splits(b, s))
-        return r.linear(o, lw.o_w)
+        return _out_product(r, o, lw.o_w)
 
 
 class RowNormAttention:
@@ -355,7 +360,7 @@ class RowNormAttention:
         else:
             o = ops.softmax_bias_attn(q, kc, vc, b.block_tables, b.tok_seq, b.positions, None, None, None, s.heads, s.scale,
                                       tiles=b.tiles, num_splits=r.block_key_splits(b, s), sink=lw.sink, softcap=s.softcap)
-        return r.linear(o, lw.o_w)
+        return _out_product(r, o, lw.o_w)
 
 
 class RotaryBlockAttention:
@@ -484,7 +489,7 @@ class LimitedFF:
 
     def __call__(self, h: torch.Tensor, b: "StepBatch") -> torch.Tensor:
         gu = self.r.linear(h, self.lw.gate_up_w)
-        return self.r.linear(ops.gated_act_rows(gu[:, : self.ff], gu[:, self.ff:], self.limit), self.lw.down_w)
+        return _out_product(self.r, ops.gated_act_rows(gu[:, : self.ff], gu[:, self.ff:], self.limit), self.lw.down_w)
 
 
 class ExpertRows:
@@ -647,6 +652,7 @@ class HybridRunner(ModelRunner):
                 stack.append(weights.layers[li].table)
         self._tables = {k: torch.stack(v).contiguous() for k, v in stacks.items()}
         latent_of = {}                                  # layer index -> index of its latent pages
+        self._slab_outputs = spec.arrangement == "pre"
         for li, _ in self.runs if spec.arrangement == "sandwich" else ():
             L, lw = spec.layers[li], weights.layers[li]
             if L.kind == "general_delta":
@@ -872,11 +878,12 @@ class HybridRunner(ModelRunner):
                 self._tiled_w[w.data_ptr()] = ops.tile_weights(w)
 
     def linear(self, x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
-               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+               bias: Optional[torch.Tensor] = None, slabs: bool = False) -> torch.Tensor:
         """x @ w.T (+ bias, in the accumulator's float32 ahead of the rounding).  Decode-sized row counts stream the weights once: through the fragment-tiled copy
         (K split over workgroups into fp32 slabs where one pass would leave most of the chip idle, a
         second launch adds the slabs) or, for matrices that have none, row-major through
-        mi355_linear_decode.  A library GEMM otherwise (prefill; float32; odd widths)."""
+        mi355_linear_decode.  A library GEMM otherwise (prefill; float32; odd widths).  slabs: the caller takes
+        ops.Slabs where K is split and adds them itself."""
         M, K = x.shape
         N = w.shape[0]
         ok16 = x.dtype != torch.float32 and x.stride(1) == 1 and (M == 1 or x.stride(0) % 8 == 0) and x.data_ptr() % 16 == 0
@@ -885,11 +892,13 @@ class HybridRunner(ModelRunner):
             plan = ops.plan_linear_tiled(N, K, True, M)
             if plan is not None:
                 tiles, groups = plan
-                if out is None:
+                if out is None and not (slabs and bias is None and groups > 1):
                     out = torch.empty(M, N, dtype=x.dtype, device=x.device)
                 if groups == 1:
                     return ops.linear_tiled(x, tw, N, bias=bias, out=out, tiles_per_wg=tiles)
                 part = ops.linear_tiled(x, tw, N, tiles_per_wg=tiles, k_groups=groups, epilogue=ops.EPI_PARTIAL)
+                if slabs and bias is None:
+                    return ops.Slabs(part, groups, M, N, x.dtype)
                 return ops.sum_slabs(part, groups, out, bias=bias)
         if ok16 and M <= ops.LINEAR_DECODE_MAX_M and K % 32 == 0 and N % 4 == 0:
             return ops.linear_decode(x, w, bias, out=out)
@@ -898,6 +907,11 @@ class HybridRunner(ModelRunner):
         if out is None:
             return torch.mm(x, w.t())
         return torch.mm(x, w.t(), out=out)
+
+    def out_linear(self, x: torch.Tensor, w: torch.Tensor):
+        """A sub-layer's last product.  In the pre arrangement its consumers (the norms that it is added ahead of, the mix)
+        add a K-split product's slabs themselves: 4 to 5 us a launch saved for decoded rows."""
+        return self.linear(x, w, slabs=self._slab_outputs)
 
     def tune(self, bucket: int) -> dict:
         self._modes.setdefault(bucket, {})
@@ -952,7 +966,7 @@ class HybridRunner(ModelRunner):
             wts = torch.full((pending.inv.numel(),), pending.weight, dtype=torch.float32, device=resid.device)
             pending = ops.moe_combine(pending.rows, pending.inv, wts, resid.shape[0], pending.top)
         if weight is None:
-            ops.resid_add_f32(resid, rows=pending)
+            ops.resid_add_f32(resid, rows=ops.dense(pending))
             return None
         return (ops.add_layer_norm_f32 if self.spec.layer_norm else ops.add_rms_norm_f32)(resid, weight, self.eps, add=pending)
 
@@ -976,7 +990,7 @@ class HybridRunner(ModelRunner):
         for ri, (li, t) in enumerate(self.runs):
             L, lw = spec.layers[li], w.layers[li]
             if t is not None and li == spec.loop_start and not spec.loop_plain:    # a pass begins: + embedding output (not the first) + its step vector
-                ops.resid_add_f32(resid, other=x0 if t > 0 else None, rows=pending, vec=w.loop_step[t])
+                ops.resid_add_f32(resid, other=x0 if t > 0 else None, rows=ops.dense(pending), vec=w.loop_step[t])
                 pending = None
             h = self._norm(resid, lw.norm1, pending)       # the add rides in the norm's launch
             pending = None
@@ -996,7 +1010,7 @@ class HybridRunner(ModelRunner):
                 pending = ff(self._norm(resid, lw.norm2, pending))
             elif L.ff:
                 h = self._norm(resid, lw.norm2, pending)
-                pending = self.linear(ops.gelu_tanh_and_mul(self.linear(h, lw.gate_up_w)), lw.down_w)
+                pending = self.out_linear(ops.gelu_tanh_and_mul(self.linear(h, lw.gate_up_w, slabs=True)), lw.down_w)
             if pending is not None and (ri == last or self.layer_trace is not None):
                 self._norm(resid, None, pending)
                 pending = None

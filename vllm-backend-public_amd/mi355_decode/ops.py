@@ -1091,6 +1091,27 @@ def resid_add_f32(resid: torch.Tensor, other: torch.Tensor | None = None, rows: 
     return resid
 
 
+class Slabs:
+    """A K-split product's result as its fp32 slabs [num, rows, width]: the rows are their sum in slab order, rounded to
+    `dtype`.  The norms, the mix and the gate below take it where they take rows (and add the slabs themselves)."""
+
+    __slots__ = ("partial", "num", "rows", "width", "dtype")
+
+    def __init__(self, partial: torch.Tensor, num: int, rows: int, width: int, dtype: torch.dtype):
+        self.partial, self.num, self.rows, self.width, self.dtype = partial, num, rows, width, dtype
+        _check_partial(partial, num, rows, width)
+
+    def dense(self) -> torch.Tensor:
+        return sum_slabs(self.partial, self.num, torch.empty(self.rows, self.width, dtype=self.dtype, device=self.partial.device))
+
+    def fits(self, rows: int, width: int, dtype: torch.dtype, most: int) -> bool:
+        return (self.rows, self.width, self.dtype) == (rows, width, dtype) and width % 8 == 0 and width <= most
+
+
+def dense(x):
+    return x.dense() if isinstance(x, Slabs) else x
+
+
 def add_rms_norm_f32(resid: torch.Tensor, weight: torch.Tensor, eps: float, add: torch.Tensor | None = None,
                      out: torch.Tensor | None = None):
     """resid (float32, in place) += add; returns resid / rms(resid) * weight in the dtype of weight.
@@ -1103,6 +1124,13 @@ def add_rms_norm_f32(resid: torch.Tensor, weight: torch.Tensor, eps: float, add:
         out = torch.empty(T, W, dtype=weight.dtype, device=resid.device)
     if out.dtype != weight.dtype or not out.is_contiguous() or out.shape != resid.shape:
         raise ValueError("out must be contiguous, shaped like resid, in the dtype of weight")
+    if isinstance(add, Slabs):
+        if add.fits(T, W, weight.dtype, 8192) and (out.data_ptr() | resid.data_ptr()) % 16 == 0 \
+                and (weight.numel() == 1 or weight.data_ptr() % 16 == 0):
+            check(lib.mi355_add_rms_norm_f32_slabs(out.data_ptr(), _f32(resid, "resid"), add.partial.data_ptr(), add.num,
+                                                   weight.data_ptr(), weight.numel(), T, W, float(eps), dt, _stream()))
+            return out
+        add = add.dense()
     if add is not None and (add.dtype != weight.dtype or not add.is_contiguous() or add.shape != resid.shape):
         raise ValueError("add must be contiguous, shaped like resid, in the dtype of weight")
     check(lib.mi355_add_rms_norm_f32(out.data_ptr(), _f32(resid, "resid"), None if add is None else add.data_ptr(),
@@ -1117,7 +1145,7 @@ def add_layer_norm_f32(resid: torch.Tensor, weight: torch.Tensor | None, eps: fl
     weight [width]; weight None: the add alone, nothing returned.  inv (int32 [tokens * top]): add holds a
     mixture's rows in expert order, token t's addend is row_weight * sum_k add[inv[t * top + k]]."""
     T, W = resid.shape
-    ref = weight if weight is not None else add
+    ref = weight if weight is not None else dense(add)
     dt = _dt3(ref, "weight")
     if weight is not None and (tuple(weight.shape) != (W,) or not weight.is_contiguous()):
         raise ValueError("weight must be one contiguous row")
@@ -1125,6 +1153,13 @@ def add_layer_norm_f32(resid: torch.Tensor, weight: torch.Tensor | None, eps: fl
         out = torch.empty(T, W, dtype=weight.dtype, device=resid.device)
     if out is not None and (out.dtype != weight.dtype or not out.is_contiguous() or out.shape != resid.shape):
         raise ValueError("out must be contiguous, shaped like resid, in the dtype of weight")
+    if isinstance(add, Slabs):
+        if out is not None and inv is None and add.fits(T, W, weight.dtype, 8192) \
+                and (out.data_ptr() | resid.data_ptr() | weight.data_ptr()) % 16 == 0:
+            check(lib.mi355_add_layer_norm_f32_slabs(out.data_ptr(), _f32(resid, "resid"), add.partial.data_ptr(), add.num,
+                                                     weight.data_ptr(), T, W, float(eps), dt, _stream()))
+            return out
+        add = add.dense()
     if add is not None and (add.dtype != ref.dtype or not add.is_contiguous()
                             or tuple(add.shape) != ((T if inv is None else T * top), W)):
         raise ValueError("add must be contiguous rows in the dtype of weight, one per token or (inv) per routed row")
@@ -1140,6 +1175,14 @@ def rms_norm_mix_f32(resid: torch.Tensor, xa: torch.Tensor, wa: torch.Tensor, xb
                      wb: torch.Tensor | None, eps: float, alpha: float):
     """resid (float32, in place) += alpha * (rmsnorm(xa) * wa + rmsnorm(xb) * wb)."""
     T, W = resid.shape
+    if isinstance(xa, Slabs) and isinstance(xb, Slabs) and xa.fits(T, W, wa.dtype, 4096) and xb.fits(T, W, wb.dtype, 4096) \
+            and wa.dtype == wb.dtype and tuple(wa.shape) == tuple(wb.shape) == (W,) and wa.is_contiguous() and wb.is_contiguous() \
+            and (resid.data_ptr() | wa.data_ptr() | wb.data_ptr()) % 16 == 0:
+        check(lib.mi355_rms_norm_mix_f32_slabs(_f32(resid, "resid"), xa.partial.data_ptr(), xa.num, wa.data_ptr(),
+                                               xb.partial.data_ptr(), xb.num, wb.data_ptr(), T, W, float(eps), float(alpha),
+                                               _dt3(wa, "wa"), _stream()))
+        return resid
+    xa, xb = dense(xa), dense(xb)
     dt = _dt3(xa, "xa")
     for n, t, shape in (("xa", xa, (T, W)), ("wa", wa, (W,)), ("xb", xb, (T, W)), ("wb", wb, (W,))):
         if t is None:
@@ -1154,6 +1197,13 @@ def rms_norm_mix_f32(resid: torch.Tensor, xa: torch.Tensor, wa: torch.Tensor, xb
 
 def gelu_tanh_and_mul(x: torch.Tensor, out: torch.Tensor | None = None):
     """x [tokens, 2 * inter] holding gate | up -> gelu_tanh(gate) * up."""
+    if isinstance(x, Slabs):
+        if x.width % 16 == 0 and out is None:
+            out = torch.empty(x.rows, x.width // 2, dtype=x.dtype, device=x.partial.device)
+            check(lib.mi355_gelu_tanh_and_mul_slabs(out.data_ptr(), x.partial.data_ptr(), x.num, x.rows, x.width // 2, _dt16(out, "out"),
+                                                    _stream()))
+            return out
+        x = x.dense()
     dt = _dt3(x, "x")
     inter = x.shape[1] // 2
     if out is None:
