@@ -308,6 +308,11 @@ def test_window_attention_of_staged_prompts_and_of_single_rows(H, G, d, dv, wind
         near(ops.sigmoid_window_attn(wide[last][:, 16: 16 + H * d], kc, vc, bt, one, pos[last].contiguous(), temp, bias,
                                      gate[last][:, 3:], H, window, 0.3, tiles=tiles, num_splits=n,
                                      partial=torch.full((n * len(new) * H * dv,), float("nan"), device="cuda")), cu[1:] - 1)
+    # results and partial sums off every vector's boundary: the general form
+    odd = torch.empty(len(new) * H * dv + 1, dtype=dt, device="cuda")[1:].view(len(new), H * dv)
+    near(ops.sigmoid_window_attn(wide[last][:, 16: 16 + H * d], kc, vc, bt, one, pos[last].contiguous(), temp, bias, gate[last][:, 3:],
+                                 H, window, 0.3, out=odd, tiles=tiles, num_splits=3,
+                                 partial=torch.full((3 * len(new) * H * dv + 1,), float("nan"), device="cuda")[1:]), cu[1:] - 1)
 
 
 @pytest.mark.parametrize("window", [16, 17, 31, 48])

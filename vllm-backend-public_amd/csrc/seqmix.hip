@@ -22,6 +22,8 @@
 #include "delta_tiles.h"
 #include "kv_rows.h"
 
+#include <type_traits>
+
 namespace mi355 {
 
 constexpr int kPage = MI355_BLOCK_SIZE;
@@ -1084,33 +1086,40 @@ __global__ __launch_bounds__(64 * NW) void sigmoid_window_decode_kernel(
   }
 }
 
-// out = sigmoid(gate) * sum of the key-range partial sums of the two kernels above; four columns a thread, the loads of
-// eight slabs out before the first is used (a load where it was used, an
-// element a thread: 6.5 us for 16 slabs of 32 rows of 2048)
-template <typename T>
+// out = sigmoid(gate) * sum of the key-range partial sums of the two kernels above; V columns a thread (four where the
+// buffers are aligned for it), the loads of eight slabs out before the first is used (a load where it was used, an element a
+// thread: 6.5 us for 16 slabs of 32 rows of 2048)
+template <typename T, int V>
 __global__ __launch_bounds__(256) void window_attn_reduce_kernel(uint16_t* __restrict__ out, const float* __restrict__ partial,
                                                                  const uint16_t* __restrict__ gate, int64_t gate_stride,
                                                                  int64_t rows, int H, int dv, int splits) {
   constexpr int N = 8;
+  typedef typename std::conditional<V == 4, float4, float>::type F;
   const int64_t total = rows * H * dv;
-  for (int64_t i = 4 * (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x); i < total;
-       i += 4 * static_cast<int64_t>(gridDim.x) * blockDim.x) {
+  for (int64_t i = V * (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x); i < total;
+       i += V * static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t th = i / dv;                                       // (dv is a multiple of 16)
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    float v[V] = {};
     for (int z0 = 0; z0 < splits; z0 += N) {
-      float4 f[N];
+      F f[N];
 #pragma unroll
-      for (int k = 0; k < N; ++k) f[k] = MI355_LD(float4, partial, partial + (z0 + k < splits ? z0 + k : splits - 1) * total + i);
+      for (int k = 0; k < N; ++k) f[k] = MI355_LD(F, partial, partial + (z0 + k < splits ? z0 + k : splits - 1) * total + i);
 #pragma unroll
-      for (int k = 0; k < N; ++k) f[k].x = pin_f32(f[k].x);
+      for (int k = 0; k < N; ++k) reinterpret_cast<float*>(&f[k])[0] = pin_f32(reinterpret_cast<const float*>(&f[k])[0]);
 #pragma unroll
-      for (int k = 0; k < N; ++k)
-        if (z0 + k < splits) v.x += f[k].x, v.y += f[k].y, v.z += f[k].z, v.w += f[k].w;
+      for (int k = 0; k < N; ++k) {
+        if (z0 + k >= splits) continue;
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] += reinterpret_cast<const float*>(&f[k])[e];
+      }
     }
     float gt = 1.0f;
     if (gate != nullptr)
       gt = 1.0f / (1.0f + expf(-T::to_f(MI355_LD(uint16_t, gate, gate + (th / H) * gate_stride + th % H))));
-    MI355_ST(uint2, out, out + i, make_uint2(T::pack2(v.x * gt, v.y * gt), T::pack2(v.z * gt, v.w * gt)));
+    if constexpr (V == 4)
+      MI355_ST(uint2, out, out + i, make_uint2(T::pack2(v[0] * gt, v[1] * gt), T::pack2(v[2] * gt, v[3] * gt)));
+    else
+      MI355_ST(uint16_t, out, out + i, T::from_f(v[0] * gt));
   }
 }
 
@@ -1214,7 +1223,13 @@ extern "C" int32_t mi355_sigmoid_window_attn(void* out, const void* q, int64_t q
     const dim3 block(64u * static_cast<unsigned>(waves));
     const int64_t slab = num_tokens * num_heads * v_dim;
     // every row alone in its tile: the decode form, where K and V fill whole MFMA operands
-    const bool single = num_tiles == num_tokens && rep <= 16 && (head_dim == 64 || head_dim == 128) && (v_dim == 64 || v_dim == 128);
+    const bool wide = aligned16(out) && (!split || aligned16(partial));       // results and partial sums by vectors
+    const bool single = num_tiles == num_tokens && rep <= 16 && (head_dim == 64 || head_dim == 128) && (v_dim == 64 || v_dim == 128) && wide;
+#define MI355_WRED(TT, V)                                                                                           \
+  hipLaunchKernelGGL((window_attn_reduce_kernel<TT, V>),                                                            \
+                     dim3(static_cast<unsigned>((slab / V + 255) / 256 > 4096 ? 4096 : (slab / V + 255) / 256)),    \
+                     dim3(256), 0, s, static_cast<uint16_t*>(out), partial, static_cast<const uint16_t*>(gate),     \
+                     gate_stride, num_tokens, num_heads, v_dim, num_splits)
 #define MI355_WDEC(TT, DD, DV, NW)                                                                                   \
   hipLaunchKernelGGL((sigmoid_window_decode_kernel<TT, DD, DV, NW, 2>),                                              \
                      dim3(static_cast<unsigned>(num_tokens), num_kv_heads, split ? num_splits : 1), dim3(64 * NW),   \
@@ -1244,17 +1259,15 @@ extern "C" int32_t mi355_sigmoid_window_attn(void* out, const void* q, int64_t q
     else if (hb == 4) MI355_WMFMA(TT, 4, 4, 8);                                                                     \
     else if (hb == 2) MI355_WMFMA(TT, 2, 4, 8);                                                                     \
     else MI355_WMFMA(TT, 1, 4, 8);                                                                                  \
-    if (split)                                                                                                      \
-      hipLaunchKernelGGL((window_attn_reduce_kernel<TT>),                                                           \
-                         dim3(static_cast<unsigned>((slab + 1023) / 1024 > 4096 ? 4096 : (slab + 1023) / 1024)),        \
-                         dim3(256), 0, s, static_cast<uint16_t*>(out), partial, static_cast<const uint16_t*>(gate), \
-                         gate_stride, num_tokens, num_heads, v_dim, num_splits);                                    \
+    if (split && wide) MI355_WRED(TT, 4);                                                                           \
+    else if (split) MI355_WRED(TT, 1);                                                                              \
   } while (0)
     if (dtype == MI355_BF16) MI355_WMFMA_HB(BF16); else MI355_WMFMA_HB(F16);
 #undef MI355_WMFMA_HB
 #undef MI355_WMFMA
 #undef MI355_WDEC_D
 #undef MI355_WDEC
+#undef MI355_WRED
     return check_launch("sigmoid_window_attn (matrix cores)");
   }
   MI355_DISPATCH_DTYPE3(dtype, launch_window_attn<TT>(s, out, q, q_stride, k_cache, v_cache, block_tables, max_blocks,
