@@ -887,7 +887,7 @@ int32_t mi355_softcap(void* z, int64_t numel, float cap, int32_t dtype, void* st
  *                          [heads * head_dim]); q / k / v are columns q_off / k_off / v_off of qkv rows.
  *                          With a workspace of mi355_gated_delta_rule_workspace(...) floats the form for
  *                          chunks of many tokens runs (tiles of 16 rows on the matrix cores, in fp32; the
- *                          fp32 result rows serve as scratch); without, one state column per lane (decode)
+ *                          fp32 result rows serve as scratch); without, the state in registers, token by token (decode)
  */
 int64_t mi355_gated_delta_rule_workspace(int64_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
                                          int32_t head_dim);
