@@ -654,6 +654,27 @@ def test_sample_spread_over_workgroups(ops, ldt, B, V):
     np.testing.assert_array_equal(ops.sample(wide[:, :V], *args, cut_rows=False).cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("ldt,V", [("bfloat16", 50272), ("float16", 32001), ("float32", 16384), ("bfloat16", 5003)])
+@pytest.mark.parametrize("B", [3, 70])
+def test_sample_top_k_of_the_whole_vocabulary_is_no_cut(ops, ldt, V, B):
+    """top_k of V and beyond: the draw is over the whole row on every way through the sampler (few rows and many, with the
+    hint and without, beside a row with a cut and without one).  Flat rows, whose draws mostly lie past the largest thousand
+    logits.  Exact: the published rule is that such a top_k is off."""
+    rng = np.random.default_rng(V + B)
+    tdt = {"float32": torch.float32, **DT}[ldt]
+    lg = torch.zeros(B, (V + 7) // 8 * 8, dtype=tdt)
+    lg[:, :V] = torch.from_numpy(rng.normal(0, 0.3, (B, V)).astype(np.float32)).to(tdt)
+    temperature, top_p = np.full(B, 1.0, np.float32), np.full(B, 1.0, np.float32)
+    top_k = np.asarray([V, V + 1, 2 ** 31 - 1], np.int32)[np.arange(B) % 3]
+    seeds, steps = rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B, dtype=np.int64)
+    for neighbour in (0, 40):
+        top_k[0] = neighbour if neighbour else V
+        args = [torch.from_numpy(a).cuda() for a in (temperature, top_k, top_p, seeds, steps)]
+        ref = R.sample_topk_topp(lg[:, :V].float().numpy(), temperature, top_k, top_p, seeds, steps)
+        for hint in (True, False) if not neighbour else (True,):
+            np.testing.assert_array_equal(ops.sample(lg.cuda()[:, :V], *args, cut_rows=hint).cpu().numpy(), ref)
+
+
 # --------------------------------------------------------------------------- #
 # random sampling: bit-exact token ids (fixed-order fp32 algorithm on both sides)
 # --------------------------------------------------------------------------- #

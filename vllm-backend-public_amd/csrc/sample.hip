@@ -900,7 +900,7 @@ struct ExactRow {
   float l0;                      // its largest logit
 };
 template <int LDT>
-__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp);
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp, int vocab);
 
 // Replays the picks of stages [0, upto) of a row from its finished histograms [stage][256].  Wave 0 does it alone: it asks
 // for every histogram it will need at once (one memory round trip instead of one per level, each followed by two
@@ -976,17 +976,17 @@ __device__ __forceinline__ ExactState exact_replay(const unsigned long long* his
   return st;
 }
 
-// Rows that need one key only: greedy ones and draws with neither top-k nor top-p.
-__device__ __forceinline__ bool sample_one_key(float temp, int top_k, float top_p) {
-  return !(temp > 0.0f) || (top_k <= 0 && !(top_p < 1.0f));
+// Rows that need one key only: greedy ones and draws with neither top-k nor top-p (a top-k of the whole vocabulary is none).
+__device__ __forceinline__ bool sample_one_key(float temp, int top_k, float top_p, int vocab) {
+  return !(temp > 0.0f) || ((top_k <= 0 || top_k >= vocab) && !(top_p < 1.0f));
 }
 
 template <int LDT>
-__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp) {
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp, int vocab) {
   if (ws == nullptr) return ExactRow{row < kExactRows && g_exact_flag[row] != 0u ? &g_exact_hist[row][0][0] : nullptr,
                                      row < kExactRows ? g_exact_l0[row] : 0.f};
   const uint32_t key = static_cast<uint32_t>(ws[static_cast<int64_t>(row) * kSampleWsHead] >> 32);
-  if (sample_one_key(temp, k, tp) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
+  if (sample_one_key(temp, k, tp, vocab) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
   return ExactRow{ws + static_cast<int64_t>(rows) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256, key_to_logit(key)};
 }
 
@@ -1026,7 +1026,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_hist_kernel(
   const int k = MI355_LD(int32_t, top_k, top_k + row);
   const int K1 = (k > 0 && k < vocab) ? k : 0;
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
-  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp);
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp, vocab);
   if (er.hists == nullptr) return;
   const bool counting = stage < L::NL;
   if (counting ? K1 == 0 : !(tp < 1.0f)) return;       // this selection is off for the row
@@ -1090,7 +1090,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
   const int k = MI355_LD(int32_t, top_k, top_k + row);
   const int K1 = (k > 0 && k < vocab) ? k : 0;
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
-  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp);
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp, vocab);
   if (er.hists == nullptr) return;
   const float l0 = er.l0;
   __shared__ unsigned long long shl[4];
@@ -1222,13 +1222,13 @@ __global__ __launch_bounds__(kSampleThreads) void topk_logits_kernel(
 }
 
 __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __restrict__ temperature,
-                                     const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int n) {
+                                     const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int n, int vocab) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const bool spread = i < kExactRows && g_exact_flag[i] != 0u;      // its token came from the follow-up launches, as a key
   if (spread) g_exact_flag[i] = 0u;
   if (!spread && !sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i),
-                                 MI355_LD(float, top_p, top_p + i)))
+                                 MI355_LD(float, top_p, top_p + i), vocab))
     return;
   const unsigned long long b = static_cast<unsigned long long>(MI355_LD(int64_t, out, out + i));
   MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
@@ -1267,13 +1267,13 @@ __global__ __launch_bounds__(256) void sample_clear_kernel(unsigned long long* _
 
 __global__ void sample_ws_finish_kernel(int64_t* __restrict__ out, const unsigned long long* __restrict__ ws,
                                         const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-                                        const float* __restrict__ top_p, int n) {
+                                        const float* __restrict__ top_p, int n, int vocab) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const unsigned long long* head = ws + static_cast<int64_t>(i) * kSampleWsHead;
   unsigned long long b = head[16];
   const unsigned long long top = head[0];
-  if (!sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i), MI355_LD(float, top_p, top_p + i)) &&
+  if (!sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i), MI355_LD(float, top_p, top_p + i), vocab) &&
       static_cast<uint32_t>(top >> 32) == 0xFFFFFFFFu)
     b = top;                                               // a NaN: its first index
   MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
@@ -1291,7 +1291,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
   __shared__ unsigned long long hist[256];
   const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
   const int k = MI355_LD(int32_t, top_k, top_k + row);
-  if (sample_one_key(temp, k, tp)) {
+  if (sample_one_key(temp, k, tp, vocab)) {
     sample_one_key_pass<LDT>(ws + static_cast<int64_t>(row) * kSampleWsHead + 16, base, vocab, !(temp > 0.0f), temp, static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)),
                              static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row)), blockIdx.x,
                              gridDim.x, chunk_vecs, part, nullptr);
@@ -1347,7 +1347,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const uint64_t seed = static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row));
   const uint64_t step = static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row));
   const bool greedy = !(temp > 0.0f);
-  if (sample_one_key(temp, k, tp)) {
+  if (sample_one_key(temp, k, tp, vocab)) {
     sample_one_key_pass<LDT>(reinterpret_cast<unsigned long long*>(out) + row, base, vocab, greedy, temp, seed, step, blockIdx.y,
                              gridDim.y, chunk_vecs, part, out);
     return;
@@ -1684,7 +1684,7 @@ static int32_t sample_entry(const char* name, int64_t* out_ids, const void* logi
   const int32_t rc2 = check_launch(name);
   if (rc2 != MI355_OK) return rc2;
   hipLaunchKernelGGL(sample_finish_kernel, dim3((num_rows + 255) / 256), dim3(256), 0, s, out_ids, temperature, top_k,
-                     top_p, num_rows);
+                     top_p, num_rows, vocab);
   return check_launch(name);
 }
 }  // namespace mi355
@@ -1753,7 +1753,7 @@ extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logit
   else MI355_SAMPLE_LAUNCH(MI355_F16);
 #undef MI355_SAMPLE_LAUNCH
   hipLaunchKernelGGL(sample_ws_finish_kernel, dim3((num_rows + 255) / 256), dim3(256), 0, s, out_ids, ws, temperature, top_k, top_p,
-                     num_rows);
+                     num_rows, vocab);
   return check_launch(name);
 }
 
