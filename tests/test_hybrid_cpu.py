@@ -217,3 +217,37 @@ def test_upload_keeps_values_shapes_and_types():
     src = [np.arange(5, dtype=np.int64) - 2, np.zeros((0,), np.int32), np.arange(6, dtype=np.int32).reshape(2, 3)[:, ::2], np.zeros((3, 0), np.int64)]
     for a, t in zip(src, ops.upload("cpu", *src)):
         assert t.is_contiguous() and tuple(t.shape) == a.shape and t.numpy().dtype == a.dtype and (t.numpy() == a).all()
+
+
+# what the two forms took, us (staged, by tiles), chunk lengths, keys ahead of every chunk, (heads, kv heads, key size, value size), window
+_WINDOW_SHAPES = [
+    (90, 252, [2048] * 4, 0, (16, 4, 128, 128), 1024), (9, 31, [33] * 32, 0, (16, 4, 128, 128), 1024),
+    (14, 28, [256], 0, (16, 4, 128, 128), 1024), (156, 738, [4096], 0, (16, 16, 128, 128), 4096),
+    (25, 40, [300, 20, 150], 300, (16, 4, 128, 128), 1024), (13, 34, [2048], 0, (8, 8, 64, 64), 128),
+    (636, 256, [1] * 31 + [8000], 0, (16, 4, 128, 128), 1024), (1700, 861, [1] * 31 + [8000], 0, (16, 4, 128, 128), 4096),
+    (134, 75, [1] * 31 + [1000], 1000, (16, 4, 128, 128), 1024), (47, 26, [1] * 31 + [300], 1000, (4, 4, 64, 128), 1024),
+    (99, 82, [512], 3000, (16, 4, 128, 128), 4096), (99, 47, [512], 3000, (8, 1, 128, 128), 4096),
+    (79, 46, [512], 3000, (8, 8, 64, 64), 4096), (38, 30, [128], 1900, (16, 4, 128, 128), 1024),
+]
+
+
+@pytest.mark.parametrize("staged_us,tiles_us,lens,behind,sizes,window", _WINDOW_SHAPES)
+def test_window_attention_takes_the_form_that_was_faster(monkeypatch, staged_us, tiles_us, lens, behind, sizes, window):
+    """The dispatch of a prompt step's window attention at shapes where the two forms are far apart."""
+    from types import SimpleNamespace
+    from mi355_decode import hybrid_runner as HR, ops
+    heads, kv, dim, vdim = sizes
+    called, T = [], sum(lens)
+    monkeypatch.setattr(ops, "rope_partial_kv_write", lambda *a: None)
+    monkeypatch.setattr(ops, "sigmoid_window_attn_prefill", lambda *a, **k: called.append("staged"))
+    monkeypatch.setattr(ops, "sigmoid_window_attn", lambda *a, **k: called.append("tiles"))
+    width = [heads * dim, kv * dim, kv * vdim, heads]
+    seg = {n: (sum(width[:i]), width[i]) for i, n in enumerate(("lq", "lk", "lv", "lg"))}
+    meta = lambda *s, dt=torch.int32: torch.empty(*s, dtype=dt, device="meta")      # noqa: E731
+    runner = SimpleNamespace(k_cache=[None], v_cache=[None], rotary=lambda d, b: None, linear=lambda x, w: x, key_splits=lambda b, s: {})
+    spec = SimpleNamespace(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, window=window, scale=1.0, rot_dims=0, rot_base=1.0)
+    batch = HR.StepBatch(meta(T), meta(T), meta(T), None, meta(len(lens) + 1), meta(T), meta(len(lens)), meta(1, 3), True,
+                         context_lens=meta(len(lens)), max_q_len=max(lens), max_context=max(lens) + behind)
+    HR.WindowAttention(spec, SimpleNamespace(seg=seg, attn_temp=None, attn_bias=None, attn_o_w=None), runner, 0)(
+        meta(T, -(-sum(width) // 8) * 8, dt=torch.bfloat16), batch)
+    assert called == ["staged" if staged_us < tiles_us else "tiles"]

@@ -787,6 +787,50 @@ def test_decode_sized_steps_on_the_tiled_weight_stream():
             assert (np.sqrt((d ** 2).mean(1)) / np.abs(want).std()).max() < 0.08
 
 
+def test_steps_through_the_staged_window_attention(monkeypatch):
+    """What the runner hands the LDS-staged form: a prompt of many tiles, a portion behind earlier keys, a portion beside a
+    single row, against the restatement (bfloat16 activations: the bound of the steps above); one long chunk among single
+    rows goes by tiles.  The forms that ran are asserted."""
+    from mi355_decode import ops
+    eng = _engine("wide", dtype="bfloat16", pages=160, max_model_len=1100)
+    staged, tiles = [], []
+    for name, calls in (("sigmoid_window_attn_prefill", staged), ("sigmoid_window_attn", tiles)):
+        real = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, real=real, calls=calls, **k: (calls.append(1), real(*a, **k))[1])
+    a, b = _tokens("wide", 900, 11), _tokens("wide", 70, 12)
+    got, at = {"a": [], "b": []}, {"a": 0, "b": 0}
+    toks = {"a": a, "b": b}
+
+    def step(form, end=(), **new):
+        staged.clear(), tiles.clear()
+        out = eng.forced_step([(r, toks[r][at[r]: at[r] + n], list(range(n))) for r, n in new.items()], list(end))
+        runs = 2                                                    # the looped parallel layer
+        assert (len(staged), len(tiles)) == ((runs, 0) if form == "staged" else (0, runs)), (new, len(staged), len(tiles))
+        row = 0
+        for r, n in new.items():
+            got[r].append(out[row: row + n])
+            row, at[r] = row + n, at[r] + n
+
+    step("staged", a=530)
+    step("staged", a=171)                                           # behind 530 keys
+    step("staged", a=130, b=1)                                      # beside a single row
+    step("tiles", a=1, b=1)
+    step("staged", a=37, b=50)
+    eng.forced_step([(r, [1], []) for r in "cd"])
+    step("staged", a=1, b=2)
+    staged.clear(), tiles.clear()
+    out = eng.forced_step([("c", [2], []), ("d", [3], []), ("a", a[at["a"]:], list(range(len(a) - at["a"])))], ["a", "c", "d"])
+    assert not staged and len(tiles) == 2                           # 30 rows of 3 x 30: by tiles
+    got["a"].append(out)
+    step("staged", b=16, end=["b"])
+    for r in "ab":
+        assert at[r] + (30 if r == "a" else 0) == len(toks[r])
+        want = _ref("wide", toks[r])
+        d = np.concatenate(got[r]) - want
+        d = d - d.mean(1, keepdims=True)
+        assert (np.sqrt((d ** 2).mean(1)) / np.abs(want).std()).max() < 0.08
+
+
 @pytest.mark.parametrize("name,dtype", [("loop0", "float32"), ("tail", "float32"), ("plain", "bfloat16"), ("wide", "bfloat16")])
 def test_greedy_generation_through_the_engine(name, dtype):
     """LLM.generate: scheduler admission, prefill, then decode steps replayed from HIP graphs with

@@ -83,17 +83,17 @@ class StepBatch:
     """Device-side description of one packed step (see csrc/seqmix.hip)."""
     __slots__ = ("ids", "positions", "slot_mapping", "block_tables", "cu_seqlens", "tok_seq", "state_slots",
                  "num_tokens", "num_seqs", "tiles", "long_chunks", "pair_tiles", "context_lens", "max_q_len", "row_tiles",
-                 "routes", "latent_plan")
+                 "routes", "latent_plan", "max_context")
 
     def __init__(self, ids, positions, slot_mapping, block_tables, cu_seqlens, tok_seq, state_slots, tiles=None,
                  long_chunks=False, pair_tiles=None, context_lens=None, max_q_len=0, row_tiles=None,
-                 latent_plan=None):
+                 latent_plan=None, max_context=0):
         self.routes = {}                              # (experts, top) -> ops.TableRoutes of the step's token ids
         self.latent_plan = latent_plan                # () -> the step's LatentPlan, or None (captured decode steps)
         self.row_tiles = row_tiles                    # rows -> ops.RowTiles of the step, or None (captured decode steps)
-        # every chunk's length of context after the step (int32, on the device) and the longest chunk: what the
-        # LDS-staged prompt attention walks by; None: not known to this step
-        self.context_lens, self.max_q_len = context_lens, int(max_q_len)
+        # every chunk's length of context after the step (int32, on the device), the longest chunk and the longest
+        # context: what the LDS-staged prompt attention walks by; None: not known to this step
+        self.context_lens, self.max_q_len, self.max_context = context_lens, int(max_q_len), int(max_context)
         self.tiles = tiles                            # 16-row query tiles (ops.query_tiles) or None: one wave per row
         self.pair_tiles = pair_tiles                  # heads -> tiles of 16 (row, head) pairs (ops.pair_tiles), or None
         self.long_chunks = long_chunks                # some chunk holds several tokens (prompts and portions)
@@ -105,6 +105,28 @@ class StepBatch:
 def _out_product(r, x: torch.Tensor, w: torch.Tensor):
     """A sub-layer's last product: HybridRunner.out_linear, or plainly the product for another owner of the sub-layer."""
     return getattr(r, "out_linear", r.linear)(x, w)
+
+
+def staged_window_pays(tokens: int, chunks: int, longest: int, context: int, heads: int, kv_heads: int, dim: int,
+                       window: int) -> bool:
+    """Whether the sigmoid window attention of a step's chunks (`longest` rows and `context` keys the largest) goes through
+    LDS once for a workgroup's tile of queries, or by 16-row tiles with their keys spread over workgroups.
+
+    The staged form deals (chunk, kv head, tile) in that order over the XCDs by the longest chunk's tiles: one long chunk
+    among short ones lands on one XCD, so the rows have to fill 2/5 of chunks x longest (31 single rows beside 8000 at
+    16 heads on 4 kv heads of 128, window 1024: 636 us, by tiles 256; beside 1000 behind 1000 keys 134 / 75).  Otherwise it
+    is a workgroup's walk over its keys, one behind the other, against the products of all of them; fitted to 1044 shapes
+    of 1 to 8 query heads a kv head, windows 128 to 4096, 16 to 8192 rows (us): 8 + 27 for every 1024 keys walked, 0.7 for a
+    million (row, head, key); by tiles 20 + 2 a million where groups of 4 heads share K and V, 10 + 2.5 otherwise.
+    Measured, staged / by tiles: 4 x 2048 rows 90 / 252, 32 x 33 rows 9 / 31, 512 rows behind 3000 keys at window 4096
+    99 / 82, at 8 heads on one kv head 99 / 47, 128 rows behind 1900 keys at window 1024 38 / 30."""
+    if 5 * tokens < 2 * chunks * longest:
+        return False
+    keys = min(window, context)
+    products = tokens * heads * max(min(window, context - longest / 2), 1) * 1e-6
+    grouped = heads // kv_heads % 4 == 0
+    by_tiles = 20.0 + 2.0 * products if grouped else 10.0 + 2.5 * products
+    return by_tiles >= max(8.0 + (0.028 if dim > 64 else 0.026) * keys, 0.7 * products)
 
 
 class WindowAttention:
@@ -122,13 +144,9 @@ class WindowAttention:
         kc, vc = r.k_cache[self.ci], r.v_cache[self.ci]
         ops.rope_partial_kv_write(q, k, v, r.rotary(s.rot_dims, s.rot_base), b.positions, b.slot_mapping, kc, vc,
                                   s.heads, s.kv_heads, s.dim, s.vdim)
-        # prompts and portions: K/V steps staged through LDS once for a workgroup's tile of queries.  A workgroup walks
-        # 1024 keys in 22 us however few they are (and starts in 14), so fewer than 32 of them leave it to the form that
-        # spreads a tile's keys: 4 x 2048 rows 88 us against 249, 32 x 33 rows 14 against 34, 256 new rows 14.7 against
-        # 30, 128 new rows behind 1900 keys 37 against 27.
-        groups = max(b.num_tokens * s.heads // 128, b.num_seqs * s.kv_heads)
-        if b.long_chunks and b.context_lens is not None and groups >= 32 and s.dim <= 128 and proj.stride(0) % 8 == 0 \
-                and q.data_ptr() % 16 == 0 and ops.chunk_attn_prefill_ok(q.dtype, s.heads, s.kv_heads, s.dim, s.vdim):
+        if b.long_chunks and b.context_lens is not None and s.dim <= 128 and proj.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0 \
+                and ops.chunk_attn_prefill_ok(q.dtype, s.heads, s.kv_heads, s.dim, s.vdim) \
+                and staged_window_pays(b.num_tokens, b.num_seqs, b.max_q_len, b.max_context, s.heads, s.kv_heads, s.dim, s.window):
             o = ops.sigmoid_window_attn_prefill(q, kc, vc, b.block_tables, b.cu_seqlens, b.context_lens, b.max_q_len,
                                                 self.lw.attn_temp, self.lw.attn_bias, g, s.heads, s.window, s.scale)
             return _out_product(r, o, self.lw.attn_o_w)
@@ -1144,7 +1162,8 @@ class HybridRunner(ModelRunner):
         return self._forward(StepBatch(token_ids, positions, slot_mapping, block_tables.contiguous(), cu_seqlens,
                                        tok_seq, slots, tiles, self._step_long, pair_tiles=self._chunk_pair_tiles,
                                        context_lens=None if context_lens is None else context_lens.to(torch.int32).contiguous(),
-                                       max_q_len=max_q_len, row_tiles=self._chunk_row_tiles, latent_plan=self._chunk_latent_plan))
+                                       max_q_len=max_q_len, row_tiles=self._chunk_row_tiles, latent_plan=self._chunk_latent_plan,
+                                       max_context=np.asarray(self._step_ctx).max(initial=0)))
 
     def prefill(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                 block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
