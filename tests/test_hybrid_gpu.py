@@ -380,6 +380,15 @@ def test_rows_rotated_by_vectors_are_the_element_form(H, G, d, dv, rot, norm, dt
     assert torch.equal(got[0][2], got[1][2])                   # V is moved, not computed
 
 
+@pytest.mark.parametrize("H,G,d,dv,rot,norm,dtype,T", [
+    (16, 16, 128, 128, 0, True, torch.bfloat16, 256), (16, 16, 128, 128, 0, True, torch.bfloat16, 257),
+    (16, 4, 128, 128, 64, False, torch.float16, 1023), (16, 4, 128, 128, 64, False, torch.float16, 1024),
+    (64, 8, 128, 256, 64, True, torch.bfloat16, 261), (8, 8, 64, 64, 64, False, torch.bfloat16, 1040)])
+def test_value_pages_by_rows_and_by_tiles(H, G, d, dv, rot, norm, dtype, T):
+    """Either side of the line between value pages in the rows' workgroups and by tiles of 16 rows."""
+    test_rows_rotated_by_vectors_are_the_element_form(H, G, d, dv, rot, norm, dtype, T)
+
+
 def _delta_in_cuts(qkv, beta, decay, a_log, dt_bias, cuts, H, G, d, dv, per_channel, slot=2, slots=4, long_chunks=False):
     from mi355_decode import ops
     T = qkv.shape[0]

@@ -143,9 +143,12 @@ template <bool NORM>
 static void launch_kv_rows(const KvRows& a, int dtype, hipStream_t s) {
   const int units = (a.H + (a.k != nullptr ? a.G : 0)) * ((a.d - a.rot / 2) / 8);
   const int threads = units >= 512 ? 512 : (units + 63) / 64 * 64;
-  // whole pages of V by tiles where there are some (16 rows that store 2 bytes each meet in a sector), in the row's
-  // workgroup for decoded rows
-  const int inline_v = a.num_tokens < 64 ? 1 : 0;
+  // V pages in the row's workgroup, 2 bytes a store, or by tiles of 16 rows and a kv head (a launch of its own; 16 rows that
+  // store 2 bytes each meet in a sector).  The tiles pay from half a million numbers on, and where rows run on in their pages:
+  // decoded rows lie in pages of their own.  Measured with the rotation, us (in the row / tiles; rows of one run, from its middle,
+  // each in a page of its own): 64 rows of 4 heads of 128 4.2 / 5.8, 4.0 / 7.1, 3.9 / 10.3; 256 rows of 16 heads 6.5 / 5.6,
+  // 6.5 / 7.2, 7.5 / 12.8; 1024 rows of 4 7.9 / 6.9, 8.0 / 8.2, 8.7 / 14.1; 8192 rows of 4 31 / 21, 31 / 23, 40 / 48.
+  const int inline_v = a.num_tokens <= 256 || a.num_tokens * a.G * a.dv < (1 << 19) ? 1 : 0;
 #define MI355_KVR(TT, ROT, N) \
   hipLaunchKernelGGL((kv_rows_vec_kernel<TT, NORM, ROT, N>), dim3(static_cast<unsigned>(a.num_tokens)), dim3(threads), 0, s, a, inline_v)
 #define MI355_KVR_N(TT, ROT)                     \
