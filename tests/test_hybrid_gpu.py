@@ -627,13 +627,13 @@ def test_head_norm_and_gate_rows(H, dv, act):
     assert ((got - want.reshape(T, -1)).abs() <= 2.0 ** -8 * want.reshape(T, -1).abs() + 1e-5).all()
 
 
-@pytest.mark.parametrize("taps", [2, 3, 4])
-def test_convolution_of_long_batches_by_groups_of_rows(taps):
-    """1024 rows and more go four rows a thread: groups that start a chunk, cross into the next or end the batch, chunks that
-    continue from their state.  Tolerance: the 16-bit store, 2^-8 of the result, on float32 sums of `taps` products."""
+@pytest.mark.parametrize("taps,C", [(2, 24), (3, 24), (4, 24), (2, 8192), (3, 8072), (4, 8072), (4, 8064)])
+def test_convolution_of_long_batches_by_groups_of_rows(taps, C):
+    """Rows of many channels go four a thread (here from 8072 channels on), others one: groups that start a chunk, cross into
+    the next or end the batch, chunks that continue from their state.  Tolerance: the 16-bit store, 2^-8 of the result, on float32 sums of `taps` products."""
     from mi355_decode import ops
     g = torch.Generator().manual_seed(taps)
-    lens, first, C = [1, 2, 3, 5, 600, 4, 417, 2], [0, 9, 0, 1, 0, 50, 2, 0], 24
+    lens, first = [1, 2, 3, 5, 600, 4, 417, 5], [0, 9, 0, 1, 0, 50, 2, 0]
     cu = torch.tensor([0] + lens).cumsum(0)
     T, S = int(cu[-1]), len(lens)
     x, w = torch.randn(T, C, generator=g).to(torch.bfloat16), torch.randn(C, taps, generator=g).to(torch.bfloat16)

@@ -310,53 +310,34 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
 // 16-bit rows, 8 channels per thread, the taps a template constant; RT rows a thread, whose weights (four times the
 // bytes of a row's inputs) and inputs it then loads once for all of them.  Rows too near the start of their
 // chunk, or a group across chunks, go row by row.  Bound by the trips to L2 for prompts: 8192 rows of 4096 channels and 4 taps
-// 67 us with a row a thread, 43 with 4.
+// 65 us with a row a thread, 45 with 4.
 template <typename T, int TAPS, int RT>
 __global__ __launch_bounds__(256) void causal_conv_silu_vec_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
     const float* __restrict__ state, const int32_t* __restrict__ tok_seq, const int64_t* __restrict__ positions,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ state_slots, int64_t num_tokens, int C) {
   const int vec_per_row = C >> 3;
-  const int64_t total = (num_tokens + RT - 1) / RT * vec_per_row;
+  const int64_t total = (RT == 1 ? num_tokens : (num_tokens + RT - 1) / RT) * vec_per_row;
   for (int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; idx < total;
        idx += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t t0 = idx / vec_per_row * RT;
     const int c8 = static_cast<int>(idx % vec_per_row) * 8;
-    const int rows = static_cast<int>(num_tokens - t0 < RT ? num_tokens - t0 : RT);
     float wv[TAPS][8];                                  // weights of the 8 channels: 8 * TAPS contiguous values
+    auto weights = [&]() {
 #pragma unroll
-    for (int j = 0; j < TAPS; ++j) unpack8<T>(MI355_LD(uint4, w, w + static_cast<int64_t>(c8) * TAPS + 8 * j), wv[j]);
+      for (int j = 0; j < TAPS; ++j) unpack8<T>(MI355_LD(uint4, w, w + static_cast<int64_t>(c8) * TAPS + 8 * j), wv[j]);
+    };
     auto finish = [&](int64_t t, float (&acc)[8]) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = acc[i] / (1.0f + expf(-acc[i]));
       MI355_ST(uint4, y, y + t * C + c8, pack8<T>(acc));
     };
-    const int s0 = MI355_LD(int32_t, tok_seq, tok_seq + t0);
-    const int64_t cs0 = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s0);
-    if (RT > 1 && rows == RT && t0 - cs0 >= TAPS - 1 && MI355_LD(int32_t, tok_seq, tok_seq + t0 + RT - 1) == s0) {
-      uint4 raw[RT + TAPS - 1];
-#pragma unroll
-      for (int r = 0; r < RT + TAPS - 1; ++r) raw[r] = MI355_LD(uint4, x, x + (t0 - (TAPS - 1) + r) * x_stride + c8);
-#pragma unroll
-      for (int u = 0; u < RT; ++u) {
-        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < TAPS; ++j) {
-          float xv[8];
-          unpack8<T>(raw[u + j], xv);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[i] += (&wv[0][0])[i * TAPS + j] * xv[i];
-        }
-        finish(t0 + u, acc);
-      }
-      continue;
-    }
-    for (int u = 0; u < rows; ++u) {
-      const int64_t t = t0 + u;
+    auto row = [&](int64_t t, bool first) {             // any row, by itself
       const int s = MI355_LD(int32_t, tok_seq, tok_seq + t);
       const int64_t cs = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s);
       const int64_t p = MI355_LD(int64_t, positions, positions + t);
       const float* st = state + static_cast<int64_t>(MI355_LD(int32_t, state_slots, state_slots + s)) * (TAPS - 1) * C;
+      if (first) weights();                             // (behind the row's own loads, which its other loads wait for)
       float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) {
@@ -375,6 +356,33 @@ __global__ __launch_bounds__(256) void causal_conv_silu_vec_kernel(
         for (int i = 0; i < 8; ++i) acc[i] += (&wv[0][0])[i * TAPS + j] * xv[i];
       }
       finish(t, acc);
+    };
+    if constexpr (RT == 1) {
+      row(t0, true);
+    } else {
+      weights();
+      const int rows = static_cast<int>(num_tokens - t0 < RT ? num_tokens - t0 : RT);
+      const int s0 = MI355_LD(int32_t, tok_seq, tok_seq + t0);
+      const int64_t cs0 = MI355_LD(int32_t, cu_seqlens, cu_seqlens + s0);
+      if (rows == RT && t0 - cs0 >= TAPS - 1 && MI355_LD(int32_t, tok_seq, tok_seq + t0 + RT - 1) == s0) {
+        uint4 raw[RT + TAPS - 1];
+#pragma unroll
+        for (int r = 0; r < RT + TAPS - 1; ++r) raw[r] = MI355_LD(uint4, x, x + (t0 - (TAPS - 1) + r) * x_stride + c8);
+#pragma unroll
+        for (int u = 0; u < RT; ++u) {
+          float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < TAPS; ++j) {
+            float xv[8];
+            unpack8<T>(raw[u + j], xv);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] += (&wv[0][0])[i * TAPS + j] * xv[i];
+          }
+          finish(t0 + u, acc);
+        }
+        continue;
+      }
+      for (int u = 0; u < rows; ++u) row(t0 + u, false);
     }
   }
 }
@@ -1289,8 +1297,12 @@ extern "C" int32_t mi355_causal_conv_silu(void* y, const void* x, int64_t x_stri
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype != MI355_F32 && taps >= 2 && taps <= 4 && channels % 8 == 0 && x_stride % 8 == 0 && aligned16(x) &&
       aligned16(y) && aligned16(weight) && aligned16(state)) {
-    const bool few = num_tokens < 1024;                  // (decoded rows: chunks of their own, and workgroups for every CU)
-    const int64_t vecs = (few ? num_tokens : (num_tokens + 3) / 4) * (channels / 8);
+    // four rows a thread where that leaves four waves for every SIMD; below, the waves that hide the trips to memory are
+    // worth more.  Measured with 4 taps, us, a row / four rows a thread: 8192 rows of 1024 channels (2^18 threads of four)
+    // 21.5 / 18.1, of 256 9.4 / 13.9; 1024 rows of 8192 21.4 / 19.1, of 4096 14.6 / 14.4, of 1024 8.2 / 11.6.
+    const int64_t fours = (num_tokens + 3) / 4 * (channels / 8);
+    const bool few = fours < (1 << 18);
+    const int64_t vecs = few ? num_tokens * (channels / 8) : fours;
     const dim3 vgrid(static_cast<unsigned>((vecs + 255) / 256 > 65536 ? 65536 : (vecs + 255) / 256));
 #define MI355_CONV_RT(TT, TAPS, RT)                                                                                   \
   hipLaunchKernelGGL((causal_conv_silu_vec_kernel<TT, TAPS, RT>), vgrid, dim3(256), 0, s, static_cast<uint16_t*>(y),  \
