@@ -391,3 +391,34 @@ def test_prompt_logprobs_cover_every_prompt_token_once_across_chunks():
             assert lp == -(p[j - 1] * 1000 + p[j]) / 1e6       # scored by the row of token j-1 against token j
             assert [t for t, _ in top] == [p[j], p[j] + 1]
     assert runner.scored_rows == sum(len(p) - 1 for i, p in enumerate(ps) if i != 2)
+
+
+@pytest.mark.parametrize("params,cut_rows,short_cuts", [
+    ([(0.0, 5, 0.5), (1.0, 0, 1.0), (1.0, 1000, 1.0)], False, False),          # greedy, plain, a top-k of everything
+    ([(1.0, 50, 1.0), (0.7, 256, 1.0)], True, False),                           # top-k alone: spread is the faster way
+    ([(1.0, 40, 0.9), (0.0, 0, 0.5), (1.0, 0, 1.0)], True, True),
+    ([(1.0, 40, 0.9), (1.0, 257, 1.0)], True, False),
+    ([(1.0, 40, 0.9), (1.0, 0, 0.95)], True, False)])                           # a top-p alone: its masses take a whole row
+def test_what_the_runner_says_of_a_batchs_cuts(monkeypatch, params, cut_rows, short_cuts):
+    from types import SimpleNamespace
+    import torch
+    from mi355_decode import model_runner, ops
+    seen = {}
+    monkeypatch.setattr(ops, "sample", lambda *a, **k: seen.update(k))
+    n = len(params)
+    model_runner.ModelRunner._sample(SimpleNamespace(device="cpu"), torch.zeros(n, 1000), {
+        "temperature": np.float32([p[0] for p in params]), "top_k": np.int32([p[1] for p in params]),
+        "top_p": np.float32([p[2] for p in params]), "seeds": np.zeros(n, np.int64), "steps": np.zeros(n, np.int64)}, torch.zeros(n))
+    assert (seen["cut_rows"], seen["short_cuts"]) == (cut_rows, short_cuts)
+
+
+@pytest.mark.parametrize("dtype,rows,short_cuts,spread_us,single_us", [
+    ("bfloat16", 32, True, 45, 44), ("bfloat16", 64, True, 62, 44), ("float16", 42, True, 65, 47), ("float32", 32, True, 100, 54),
+    ("bfloat16", 64, False, 77, 104), ("float16", 42, False, 62, 108), ("float32", 16, False, 64, 113), ("bfloat16", 65, False, None, None)])
+def test_a_draw_is_spread_where_that_is_faster(dtype, rows, short_cuts, spread_us, single_us):
+    """152064 logits: top-k of 40 with top-p (short_cuts), and a mix of cuts."""
+    import torch
+    from mi355_decode import ops
+    want = spread_us is not None and spread_us < 1.05 * single_us
+    assert ops.sample_spreads(rows, 152064, getattr(torch, dtype), short_cuts) == want
+    assert not ops.sample_spreads(rows, ops.SAMPLE_SPREAD_VOCAB - 1, getattr(torch, dtype), short_cuts)

@@ -654,6 +654,20 @@ def test_sample_spread_over_workgroups(ops, ldt, B, V):
     np.testing.assert_array_equal(ops.sample(wide[:, :V], *args, cut_rows=False).cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("ldt,B", [("bfloat16", 32), ("bfloat16", 33), ("float16", 5), ("float32", 5)])
+def test_sample_of_short_cuts_is_the_same_either_way(ops, ldt, B):
+    """The caller's word that every cut is short moves rows to another way through the sampler and no token."""
+    rng = np.random.default_rng(B)
+    V = 16384
+    lg = torch.from_numpy(np.round(rng.normal(0, 3, (B, V)), 1).astype(np.float32)).to({"float32": torch.float32, **DT}[ldt])   # (ties)
+    temperature, top_k = rng.choice([0.0, 0.8, 1.2], B).astype(np.float32), rng.choice([1, 40, 256], B).astype(np.int32)
+    top_p, seeds, steps = rng.choice([1.0, 0.9, 0.3], B).astype(np.float32), rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B)
+    args = [torch.from_numpy(a).cuda() for a in (temperature, top_k, top_p, seeds, steps)]
+    ref = R.sample_topk_topp(lg.float().numpy(), temperature, top_k, top_p, seeds, steps)
+    for short in (True, False):
+        np.testing.assert_array_equal(ops.sample(lg.cuda(), *args, short_cuts=short).cpu().numpy(), ref)
+
+
 @pytest.mark.parametrize("ldt,V", [("bfloat16", 50272), ("float16", 32001), ("float32", 16384), ("bfloat16", 5003)])
 @pytest.mark.parametrize("B", [3, 70])
 def test_sample_top_k_of_the_whole_vocabulary_is_no_cut(ops, ldt, V, B):

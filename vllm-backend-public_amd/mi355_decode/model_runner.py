@@ -914,20 +914,22 @@ class ModelRunner:
         buffer, one copy; without (a prefill, which waits for its result anyway) array by array."""
         n = logits.shape[0]
         tk, tpp, tmp = (np.asarray(sampling[k]) for k in ("top_k", "top_p", "temperature"))
-        cut = bool(((tmp > 0) & (((tk > 0) & (tk < logits.shape[1])) | (tpp < 1))).any())   # any row with an active top-k / top-p
+        cuts = (tmp > 0) & (((tk > 0) & (tk < logits.shape[1])) | (tpp < 1))                # rows with an active top-k / top-p
+        short = cuts.any() and ((tk > 0) & (tk <= ops.SAMPLE_SHORT_CUT))[cuts].all() and (tpp[cuts] < 1).any()
+        hints = {"cut_rows": bool(cuts.any()), "short_cuts": bool(short)}
         if stage is not None:
             seeds, steps, temp, top_p, top_k = self.h_samp_np[stage]
             seeds[:n], steps[:n] = sampling["seeds"], sampling["steps"]
             temp[:n], top_p[:n], top_k[:n] = sampling["temperature"], sampling["top_p"], sampling["top_k"]
             self.d_samp.copy_(self.h_samp[stage], non_blocking=True)
             d_seeds, d_steps, d_temp, d_top_p, d_top_k = self.d_samp_views
-            ops.sample(logits, d_temp[:n], d_top_k[:n], d_top_p[:n], d_seeds[:n], d_steps[:n], out=out, cut_rows=cut)
+            ops.sample(logits, d_temp[:n], d_top_k[:n], d_top_p[:n], d_seeds[:n], d_steps[:n], out=out, **hints)
             return
         dev = self.device
         t = lambda a, dt: torch.from_numpy(a).to(dev, dtype=dt, non_blocking=True)  # noqa: E731
         ops.sample(logits, t(sampling["temperature"], torch.float32), t(sampling["top_k"], torch.int32),
                    t(sampling["top_p"], torch.float32), t(sampling["seeds"], torch.int64),
-                   t(sampling["steps"], torch.int64), out=out, cut_rows=cut)
+                   t(sampling["steps"], torch.int64), out=out, **hints)
 
     def _logprobs(self, logits: torch.Tensor, chosen: torch.Tensor, k: int) -> torch.Tensor:
         """[rows, 1 + 2k] float32 on the device: log-probability of the chosen token, then the k

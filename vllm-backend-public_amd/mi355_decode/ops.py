@@ -602,17 +602,34 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
 
 # Rows with a cut are spread over many workgroups (a pass per 8 key bits and cut: 2 x 2 for bfloat16, 2 x 3 for float16,
 # 2 x 4 for float32) up to this many rows times passes, from this vocabulary on; more rows fill the chip with a workgroup
-# each.  Measured, us a call (spread / a workgroup each), 128256 bfloat16 logits: 32 rows top-p 41 / 95, 64 rows top-p 54 / 95, top-k
-# 38 / 41; 128 rows top-p 82 / 99, top-k 53 / 45; float32, 64 rows top-k 75 / 55, 16 rows 40 / 49; a vocabulary of 1000: 28 / 20.
-SAMPLE_SPREAD_PASSES, SAMPLE_SPREAD_VOCAB = 128, 16384
+# each.  Measured, us a call (spread / a workgroup each), 50272 and 152064 logits:
+#   a mix of cuts, some top-p alone   bfloat16 32 rows 36 / 66, 45 / 104, 64 rows 44 / 67, 77 / 104; float16 42 rows 49 / 70,
+#                                     62 / 108; float32 16 rows 50 / 73, 64 / 113, 32 rows 61 / 74, 82 / 113
+#   top-k of 50 alone                 bfloat16 64 rows 30 / 33, 40 / 44; float16 42 rows 31 / 36, 42 / 47; float32 16 rows 34 / 40, 41 / 54
+#   top-k of 40 and top-p             bfloat16 32 rows 34 / 33, 45 / 44, 64 rows 42 / 33, 62 / 44; float16 4 rows 37 / 35, 42 / 46,
+#                                     42 rows 49 / 36, 65 / 47; float32 4 rows 46 / 40, 53 / 53, 32 rows 80 / 41, 100 / 54
+# (of 256 and top-p: bfloat16 64 rows 44 / 41, 64 / 54).  A workgroup each is slow where it has to add up the masses of a whole row;
+# where every row's top-k leaves it a short list, the spread form's passes for the top-p are what costs: a caller that
+# knows so says it, and only bfloat16 batches of up to 32 rows are then spread.
+SAMPLE_SPREAD_PASSES, SAMPLE_SPREAD_VOCAB, SAMPLE_SHORT_CUT = 128, 16384, 256
 _KEY_PASSES = {torch.bfloat16: 2, torch.float16: 3, torch.float32: 4}
 
 
+def sample_spreads(rows: int, vocab: int, dtype: torch.dtype, short_cuts: bool = False) -> bool:
+    """Whether `sample` spreads rows with a cut over many workgroups (see above)."""
+    if short_cuts and (dtype != torch.bfloat16 or rows > 32):
+        return False
+    return rows * _KEY_PASSES[dtype] <= SAMPLE_SPREAD_PASSES and vocab >= SAMPLE_SPREAD_VOCAB
+
+
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
-           seeds: torch.Tensor, steps: torch.Tensor, out: torch.Tensor | None = None, cut_rows: bool = True):
+           seeds: torch.Tensor, steps: torch.Tensor, out: torch.Tensor | None = None, cut_rows: bool = True,
+           short_cuts: bool = False):
     """Per-row sampling (greedy where temperature <= 0).  temperature/top_p float32 [B], top_k int32 [B],
     seeds/steps int64 [B], all on the device.  cut_rows=False: the caller knows that no row has an active
-    top-k / top-p, so the follow-up launches that serve rows with huge kept sets are left out (same tokens)."""
+    top-k / top-p, so the follow-up launches that serve rows with huge kept sets are left out (same tokens).
+    short_cuts=True: the caller knows that every row with a cut has a top-k of at most SAMPLE_SHORT_CUT and some a top-p
+    with it (the way that is faster for those; same tokens)."""
     _dev(logits, "logits")
     if logits.dtype not in _DT:
         raise TypeError(f"logits dtype {logits.dtype} not supported")
@@ -626,7 +643,7 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
         out = torch.empty(B, dtype=torch.int64, device=logits.device)
     args = (out.data_ptr(), logits.data_ptr(), _rows(logits, "logits"), B, V, _DT[logits.dtype], temperature.data_ptr(),
             top_k.data_ptr(), top_p.data_ptr(), seeds.data_ptr(), steps.data_ptr())
-    if cut_rows and B * _KEY_PASSES[logits.dtype] <= SAMPLE_SPREAD_PASSES and V >= SAMPLE_SPREAD_VOCAB:
+    if cut_rows and sample_spreads(B, V, logits.dtype, short_cuts):
         ws = torch.empty(lib.mi355_sample_workspace(B, _DT[logits.dtype]), dtype=torch.uint8, device=logits.device)
         check(lib.mi355_sample_topk_topp_ws(*args, ws.data_ptr(), ws.numel(), _stream()))
     else:
