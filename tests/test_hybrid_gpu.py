@@ -506,6 +506,34 @@ def test_delta_rule_steps_of_a_mixed_batch(H, G, d, dv, per_channel, dtype):
         assert (dev[s].cpu() - M).abs().max() <= bound * M.abs().max(), s
 
 
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_delta_rule_of_short_portions_goes_token_by_token(monkeypatch, per_channel):
+    """Portions of a few rows take no workspace and no tiles, longer ones do, with the batch's longest chunk given and
+    bounded; the same numbers either way (float32 sums of up to d + 8 products in another order)."""
+    from mi355_decode import ops
+    H, G, d, dv, short = 2, 1, 64, 64, 6 if per_channel else 3
+    g = torch.Generator().manual_seed(3)
+    asked, size = [], ops.lib.mi355_gated_delta_rule_workspace
+    monkeypatch.setattr(ops.lib, "mi355_gated_delta_rule_workspace", lambda *a: (asked.append(a), size(*a))[1])
+    for lens, given, tiles in (([short], 0, False), ([short + 1], 0, True), ([1] * 5 + [short], 0, False), ([1] * 5 + [short + 1], 0, True),
+                               ([short] * 4, 0, True), ([short] * 4, short, False), ([short + 1] * 4, short + 1, True)):
+        T, S = sum(lens), len(lens)
+        qkv = torch.randn(T, 2 * G * d + H * dv, generator=g).bfloat16().cuda()
+        beta, decay = torch.randn(T, H, generator=g).bfloat16().cuda(), torch.randn(T, H * d if per_channel else H, generator=g).bfloat16().cuda()
+        a_log, dt_bias = torch.randn(H, generator=g).cuda() * 0.5 - 1, torch.randn(decay.shape[1], generator=g).cuda()
+        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+        pos, slots = torch.cat([torch.arange(3, 3 + n) for n in lens]).cuda(), torch.arange(S, dtype=torch.int32, device="cuda")
+        state, outs = torch.randn(S, H, d, dv, generator=g), []
+        for kw in ({"long_chunks": True, "longest": given}, {"long_chunks": False}):
+            asked.clear()
+            st = state.cuda()
+            outs.append((ops.gated_delta_rule(qkv, 0, G * d, 2 * G * d, beta, decay, a_log, dt_bias, st, cu, pos, slots, H, G, d, dv,
+                                              per_channel=per_channel, **kw), st))
+            assert len(asked) == (1 if tiles and kw["long_chunks"] else 0), (lens, kw)
+        for a, b in zip(*outs):
+            assert (a - b).abs().max() <= 2 * (d + 8) * 2.0 ** -24 * outs[1][1].abs().max() * max(lens)
+
+
 @pytest.mark.parametrize("H,G,d,dv,per_channel,dtype", [(2, 1, 64, 64, False, torch.bfloat16), (2, 2, 128, 120, True, torch.bfloat16),
                                                         (4, 2, 128, 128, False, torch.float16), (1, 1, 20, 17, False, torch.bfloat16),
                                                         (1, 1, 192, 16, True, torch.float32), (2, 1, 136, 200, False, torch.float32),

@@ -180,7 +180,7 @@ class DeltaMixer:
             gate = proj[:, seg["g"][0]: seg["g"][0] + vv]
         o = ops.gated_delta_rule(y, 0, qk, 2 * qk, beta, decay, lw.a_log, lw.dt_bias, rec_state, b.cu_seqlens,
                                  b.positions, b.state_slots, s.heads, s.kv_heads, s.dim, s.vdim,
-                                 per_channel=s.per_channel, long_chunks=b.long_chunks)
+                                 per_channel=s.per_channel, long_chunks=b.long_chunks, longest=b.max_q_len)
         on = ops.gated_head_rms_norm(o, gate, lw.head_norm, r.eps, ops.ACT_SIGMOID if s.per_channel else ops.ACT_SILU)
         return _out_product(r, on, lw.delta_o_w)
 

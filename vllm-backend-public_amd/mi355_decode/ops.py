@@ -1402,16 +1402,21 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
                      a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
                      positions: torch.Tensor, state_slots: torch.Tensor, num_heads: int, num_kv_heads: int,
                      head_dim: int, v_dim: int, per_channel: bool = False, out: torch.Tensor | None = None,
-                     long_chunks: bool = False):
+                     long_chunks: bool = False, longest: int = 0):
     """The gated delta rule over packed chunks.  qkv [tokens, C] holds q (kv_heads x head_dim) at column
     q_off, k at k_off, v (heads x v_dim) at v_off; beta [tokens, heads] and decay [tokens, heads] or
     [tokens, heads * head_dim] are raw projection outputs (column slices are fine); a_log [heads] and
     dt_bias (decay's width) float32; state float32 [slots, heads, head_dim, v_dim].
     Returns o float32 [tokens, heads, v_dim].  long_chunks: the batch holds chunks of many tokens -- take
-    the form that goes by tiles of 16 rows (it allocates a float32 workspace; not for graphs)."""
+    the form that goes by tiles of 16 rows (it allocates a float32 workspace; not for graphs), unless the longest chunk
+    (`longest`; 0: as many rows as the batch has beyond one a chunk) is so short that token by token is faster."""
     dt = _dt3(qkv, "qkv")
     T = qkv.shape[0]
     S = cu_seqlens.numel() - 1
+    # Two launches of tiles take 12 to 20 us however few rows there are, a token 2 behind the first one's 8.  Measured, us
+    # (token by token / tiles): a chunk of 2 rows at 16 heads of 128 9.4 / 12.9, of 3 11.4 / 12.9, of 4 13.4 / 12.9; 8 heads with
+    # a decay a channel 9.4 / 18.4, of 4 13.3 / 18.7, of 6 17.6 / 18.6, of 8 21.6 / 18.8; 32 chunks of 2 12.8 / 35.1.
+    long_chunks = long_chunks and (longest or T - S + 1) > (6 if per_channel else 3)
     width = num_heads * head_dim if per_channel else num_heads
     if tuple(state.shape[1:]) != (num_heads, head_dim, v_dim):
         raise ValueError("state must be [slots, heads, head_dim, v_dim]")
