@@ -506,6 +506,30 @@ def test_delta_rule_steps_of_a_mixed_batch(H, G, d, dv, per_channel, dtype):
         assert (dev[s].cpu() - M).abs().max() <= bound * M.abs().max(), s
 
 
+@pytest.mark.parametrize("rows", [128, 129])
+@pytest.mark.parametrize("d,dv", [(32, 32), (20, 64)])
+def test_delta_rule_of_many_small_heads(rows, d, dv):
+    """Either side of the line between four columns a lane and one (1024 workgroups of small states), one token each against
+    the recurrence in float64.  Bound: float32 sums of up to d + 8 products, 2^-24 each."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(rows + d)
+    H = 8
+    qkv = torch.randn(rows, 2 * H * d + H * dv, generator=g).bfloat16()
+    beta, decay = torch.randn(rows, H, generator=g).bfloat16(), torch.randn(rows, H, generator=g).bfloat16()
+    a_log, dt_bias, state = torch.randn(H, generator=g) * 0.5 - 1, torch.randn(H, generator=g), torch.randn(rows, H, d, dv, generator=g)
+    dev = state.cuda()
+    out = ops.gated_delta_rule(qkv.cuda(), 0, H * d, 2 * H * d, beta.cuda(), decay.cuda(), a_log.cuda(), dt_bias.cuda(), dev,
+                               torch.arange(rows + 1, dtype=torch.int32, device="cuda"), torch.full((rows,), 5, device="cuda"),
+                               torch.arange(rows, dtype=torch.int32, device="cuda"), H, H, d, dv).cpu()
+    f = qkv.double()
+    q, k = (R.unit(f[:, i * H * d:(i + 1) * H * d].view(rows, H, d)) for i in (0, 1))
+    v, a = f[:, 2 * H * d:].view(rows, H, dv), torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(decay.double() + dt_bias.double()))
+    M = state.double() * a[..., None, None]
+    M = M + k[..., None] * (torch.sigmoid(beta.double())[..., None] * (v - (k[:, :, None, :] @ M)[:, :, 0]))[:, :, None, :]
+    want, bound = (q[:, :, None, :] @ M)[:, :, 0] * d ** -0.5, 2 * (d + 8) * 2.0 ** -24 * M.abs().max()
+    assert (dev.cpu() - M).abs().max() <= bound and (out.view_as(want) - want).abs().max() <= bound
+
+
 @pytest.mark.parametrize("per_channel", [False, True])
 def test_delta_rule_of_short_portions_goes_token_by_token(monkeypatch, per_channel):
     """Portions of a few rows take no workspace and no tiles, longer ones do, with the batch's longest chunk given and
