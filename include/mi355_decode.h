@@ -885,12 +885,15 @@ int32_t mi355_softcap(void* z, int64_t numel, float cap, int32_t dtype, void* st
  *                          a = exp(-exp(a_log[h]) * softplus(decay + dt_bias)), one per head
  *                          (per_channel 0) or one per key channel (per_channel 1: decay rows
  *                          [heads * head_dim]); q / k / v are columns q_off / k_off / v_off of qkv rows.
- *                          With a workspace of mi355_gated_delta_rule_workspace(...) floats the form for
+ *                          With a workspace of mi355_gated_delta_rule_workspace_form(...) floats
+ *                          (mi355_gated_delta_rule_workspace: enough for either kind of decay) the form for
  *                          chunks of many tokens runs (tiles of 16 rows on the matrix cores, in fp32; the
  *                          fp32 result rows serve as scratch); without, the state in registers, token by token (decode)
  */
 int64_t mi355_gated_delta_rule_workspace(int64_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
                                          int32_t head_dim);
+int64_t mi355_gated_delta_rule_workspace_form(int64_t num_tokens, int32_t num_heads, int32_t head_dim,
+                                              int32_t per_channel);
 int32_t mi355_rope_partial_kv_write(void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                     const void* v, int64_t v_stride, const float* cos_sin,
                                     int32_t max_pos, const int64_t* positions,

@@ -531,14 +531,50 @@ def test_delta_rule_of_many_small_heads(rows, d, dv):
 
 
 @pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("d", [20, 128, 256])
+def test_delta_rule_keeps_to_its_workspace(d, per_channel):
+    """The tile form in a workspace of just the size that its kind of decay asks for, between two guards: the guards hold, the
+    numbers are those of a workspace for either kind; a float less is refused."""
+    from mi355_decode import ops
+    from mi355_decode._lib import Mi355Error, check, lib
+    g = torch.Generator().manual_seed(d)
+    H, G, dv, lens = 2, 1, 48, [17, 16, 5, 33]
+    T, S = sum(lens), len(lens)
+    qkv = torch.randn(T, 2 * G * d + H * dv, generator=g).bfloat16().cuda()
+    beta, decay = torch.randn(T, H, generator=g).bfloat16().cuda(), torch.randn(T, H * d if per_channel else H, generator=g).bfloat16().cuda()
+    a_log, dt_bias = torch.randn(H, generator=g).cuda(), torch.randn(decay.shape[1], generator=g).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    pos, slots = torch.cat([torch.arange(3, 3 + n) for n in lens]).cuda(), torch.arange(S, dtype=torch.int32, device="cuda")
+    state, guard, got = torch.randn(S, H, d, dv, generator=g), 256, []
+    form, either = lib.mi355_gated_delta_rule_workspace_form(T, H, d, int(per_channel)), lib.mi355_gated_delta_rule_workspace(T, H, G, d)
+    assert form == either if per_channel else 2 * form < either
+
+    def run(floats, told):
+        room = torch.full((floats + 2 * guard,), 7.5, device="cuda")
+        st, o = state.cuda(), torch.empty(T, H, dv, device="cuda")
+        check(lib.mi355_gated_delta_rule(
+            o.data_ptr(), qkv.data_ptr(), qkv.shape[1], 0, G * d, 2 * G * d, beta.data_ptr(), H, decay.data_ptr(), decay.shape[1],
+            a_log.data_ptr(), dt_bias.data_ptr(), int(per_channel), st.data_ptr(), cu.data_ptr(), pos.data_ptr(), slots.data_ptr(), S, H, G,
+            d, dv, T, room[guard:].data_ptr(), told, ops._DT[torch.bfloat16], torch.cuda.current_stream().cuda_stream))
+        assert (room[:guard] == 7.5).all() and (room[guard + floats:] == 7.5).all()
+        got.append((o, st))
+
+    run(form, form)
+    run(either, either)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    with pytest.raises(Mi355Error, match="workspace"):
+        run(form, form - 1)
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
 def test_delta_rule_of_short_portions_goes_token_by_token(monkeypatch, per_channel):
     """Portions of a few rows take no workspace and no tiles, longer ones do, with the batch's longest chunk given and
     bounded; the same numbers either way (float32 sums of up to d + 8 products in another order)."""
     from mi355_decode import ops
     H, G, d, dv, short = 2, 1, 64, 64, 6 if per_channel else 3
     g = torch.Generator().manual_seed(3)
-    asked, size = [], ops.lib.mi355_gated_delta_rule_workspace
-    monkeypatch.setattr(ops.lib, "mi355_gated_delta_rule_workspace", lambda *a: (asked.append(a), size(*a))[1])
+    asked, size = [], ops.lib.mi355_gated_delta_rule_workspace_form
+    monkeypatch.setattr(ops.lib, "mi355_gated_delta_rule_workspace_form", lambda *a: (asked.append(a), size(*a))[1])
     for lens, given, tiles in (([short], 0, False), ([short + 1], 0, True), ([1] * 5 + [short], 0, False), ([1] * 5 + [short + 1], 0, True),
                                ([short] * 4, 0, True), ([short] * 4, short, False), ([short + 1] * 4, short + 1, True)):
         T, S = sum(lens), len(lens)

@@ -18,8 +18,8 @@ struct DeltaTiles {
   int q_off, k_off, v_off, per_channel, S, H, G, d, dv;
 };
 
-// floats of workspace
-int64_t delta_tiles_workspace(int64_t rows, int H, int d);
+// floats of workspace: a decay per head needs about a third of what one per channel does
+int64_t delta_tiles_workspace(int64_t rows, int H, int d, bool per_channel);
 // dtype: an mi355_dtype code; d at most 256
 void launch_delta_tiles(const DeltaTiles& a, int dtype, hipStream_t stream);
 

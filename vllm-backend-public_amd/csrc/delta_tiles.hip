@@ -34,21 +34,25 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __bui
 // padded key channels: a multiple of the 4 waves' 16-row blocks
 __host__ __device__ __forceinline__ int padded(int d) { return (d + 63) & ~63; }
 
-// workspace: W [rows][H][dp] | P [rows][H][16] | q, k, e [rows + 16][H][dp] each:
-//   a decay per channel   e^G q | e^(G_end - G) k | e^G_end (a tile's, at its first row)
+// workspace: W [rows][H][dp] | P [rows][H][16] | q | k | e, of `plane` floats each:
+//   a decay per channel   [rows + 16][H][dp] e^G q | e^(G_end - G) k | e^G_end (a tile's, at its first row)
 //   a decay per head      [H][rows + 16] factors of the raw query and key, e^G / (|q| sqrt(d)) and e^(G_end - G) / |k|,
 //                         and e^G_end (a tile's, at its first row)
 struct Layout {
   float *w, *p, *q, *k, *e;
 };
-__host__ __device__ __forceinline__ Layout layout(float* ws, int64_t rows, int H, int dp) {
+__host__ __device__ __forceinline__ int64_t plane(bool per_channel, int64_t rows, int H, int dp) {
+  return (rows + C) * H * (per_channel ? dp : 1);
+}
+template <bool PC>
+__device__ __forceinline__ Layout layout(float* ws, int64_t rows, int H, int dp) {
   const int64_t n = rows * H;
   Layout l;
   l.w = ws;
   l.p = l.w + n * dp;
   l.q = l.p + n * C;
-  l.k = l.q + (n + static_cast<int64_t>(H) * C) * dp;
-  l.e = l.k + (n + static_cast<int64_t>(H) * C) * dp;
+  l.k = l.q + plane(PC, rows, H, dp);
+  l.e = l.k + plane(PC, rows, H, dp);
   return l;
 }
 
@@ -236,7 +240,7 @@ __global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int
     part[wave][1][i * C + li] = y;
   }
   __syncthreads();
-  const Layout l = layout(a.ws, a.rows, a.H, dp);
+  const Layout l = layout<PC>(a.ws, a.rows, a.H, dp);
   const int64_t at0 = row0 * a.H + h;                     // (row, head) of the tile's first row; a row further: + H
   {
     float u = 0.f, y = 0.f;
@@ -329,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void delta_tiles_walk_kernel(DeltaTiles a, 
   if (len <= 0) return;
   const int col = cg * 16 + li, c0 = wave * 16 * DT, cw = c0 + 4 * DT * kg, ck = c0 + DT * li;
   const bool live = col < dv;
-  const Layout l = layout(a.ws, a.rows, a.H, dp);
+  const Layout l = layout<PC>(a.ws, a.rows, a.H, dp);
   [[maybe_unused]] const void* kv_base = PC ? static_cast<const void*>(a.ws) : a.qkv;
   float* sp = a.state + ((static_cast<int64_t>(MI355_LD(int32_t, a.state_slots, a.state_slots + s)) * a.H + h) * d) * dv + col;
   const bool fresh = MI355_LD(int64_t, a.positions, a.positions + cs) == 0;
@@ -522,7 +526,9 @@ void launch(const DeltaTiles& a, hipStream_t stream) {
 
 }  // namespace
 
-int64_t delta_tiles_workspace(int64_t rows, int H, int d) { return (rows + C) * H * (4 * static_cast<int64_t>(padded(d)) + C); }
+int64_t delta_tiles_workspace(int64_t rows, int H, int d, bool per_channel) {
+  return rows * H * (padded(d) + C) + 3 * plane(per_channel, rows, H, padded(d));
+}
 
 void launch_delta_tiles(const DeltaTiles& a, int dtype, hipStream_t stream) {
   MI355_DISPATCH_DTYPE3(dtype, {

@@ -1409,7 +1409,12 @@ static void launch_delta(hipStream_t s, float* o, const void* qkv, int64_t strid
 extern "C" int64_t mi355_gated_delta_rule_workspace(int64_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
                                                     int32_t head_dim) {
   (void)num_kv_heads;
-  return delta_tiles_workspace(num_tokens, num_heads, head_dim);
+  return delta_tiles_workspace(num_tokens, num_heads, head_dim, true);
+}
+
+extern "C" int64_t mi355_gated_delta_rule_workspace_form(int64_t num_tokens, int32_t num_heads, int32_t head_dim,
+                                                         int32_t per_channel) {
+  return delta_tiles_workspace(num_tokens, num_heads, head_dim, per_channel != 0);
 }
 
 extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t stride, int32_t q_off, int32_t k_off,
@@ -1432,7 +1437,7 @@ extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t str
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (workspace != nullptr && num_tokens > 0) {
     // the form for chunks of many tokens: tiles of 16 rows on the matrix cores
-    const int64_t need = mi355_gated_delta_rule_workspace(num_tokens, num_heads, num_kv_heads, head_dim);
+    const int64_t need = mi355_gated_delta_rule_workspace_form(num_tokens, num_heads, head_dim, per_channel);
     MI355_REQUIRE(workspace_floats >= need && aligned16(workspace), MI355_ERR_INVALID,
                   "gated_delta_rule: workspace of %lld floats, %lld needed, 16-byte aligned",
                   static_cast<long long>(workspace_floats), static_cast<long long>(need));

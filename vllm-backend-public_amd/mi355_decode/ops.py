@@ -1427,7 +1427,7 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
         out = torch.empty(T, num_heads, v_dim, dtype=torch.float32, device=qkv.device)
     ws = None
     if long_chunks and T > 0:
-        ws = torch.empty(lib.mi355_gated_delta_rule_workspace(T, num_heads, num_kv_heads, head_dim), dtype=torch.float32,
+        ws = torch.empty(lib.mi355_gated_delta_rule_workspace_form(T, num_heads, head_dim, int(per_channel)), dtype=torch.float32,
                          device=qkv.device)
     check(lib.mi355_gated_delta_rule(
         _f32(out, "out", T * num_heads * v_dim), qkv.data_ptr(), qkv.shape[1], q_off, k_off, v_off,
