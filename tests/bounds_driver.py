@@ -429,9 +429,10 @@ def sampler_rows():
             seeds = torch.arange(B, dtype=torch.int64).cuda()
             steps = torch.arange(B, dtype=torch.int64).cuda() * 3
             out = torch.empty(B, dtype=torch.int64, device="cuda")
+            ws = torch.empty(lib.mi355_sample_workspace(B, ops._DT[dt]), dtype=torch.uint8, device="cuda")
             torch.cuda.synchronize()
             bounds.sync_allocations()
-            ops.sample(lgd, temp, top_k, top_p, seeds, steps, out=out)
+            ops.sample(lgd, temp, top_k, top_p, seeds, steps, out=out, workspace=ws)
             torch.cuda.synchronize()
             rep = bounds.report()
             assert rep is None, (str(dt), B, V, rep)
@@ -441,10 +442,38 @@ def sampler_rows():
     return done
 
 
+def sampler_workspace_control():
+    """The spread sampler told that its workspace is larger than the tensor: what lies past the end is refused, and named."""
+    from mi355_decode import ops
+    B, V = 4, 16384
+    g = torch.Generator(device="cpu").manual_seed(5)
+    logits, code = torch.randn(B, V, generator=g).cuda(), ops._DT[torch.float32]
+    args = [torch.tensor(v, dtype=d, device="cuda") for v, d in (([0.7] * B, torch.float32), ([40] * B, torch.int32), ([0.9] * B, torch.float32),
+                                                                 (list(range(B)), torch.int64), (list(range(B)), torch.int64))]
+    out, need = torch.empty(B, dtype=torch.int64, device="cuda"), lib.mi355_sample_workspace(B, code)
+    found = []
+    # the last rows' ranges' masses fall off the end; the last row's histograms too
+    words = 8 * B * (32 + 8 * 256)                    # keys and histograms of float32 rows
+    for held in (words + 8 * 256, words - 8 * 256):
+        ws = torch.empty(held, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        bounds.sync_allocations()
+        rc = lib.mi355_sample_topk_topp_ws(out.data_ptr(), logits.data_ptr(), V, B, V, code, *[a.data_ptr() for a in args], ws.data_ptr(),
+                                           need, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, rc
+        rep = bounds.report()
+        assert rep is not None and rep["refused"] > 0 and rep["unknown_base"] == 0, rep
+        assert rep["file"].endswith("sample.hip") and rep["base"] == ws.data_ptr() and rep["address"] + rep["bytes"] > ws.data_ptr() + held, rep
+        bounds.clear()
+        found.append(rep["refused"])
+    return found
+
+
 if __name__ == "__main__":
     assert bounds.enabled(), "not the bounds-checking build: set MI355_DECODE_LIB"
     res = {"negative_control": negative_control()}
     res["sampler"] = sampler_rows()
+    res["sampler_workspace_control"] = sampler_workspace_control()
     res["rank_steps"] = rank_steps()
     res["engine"] = engine_generation()
     res["sandwich"] = sandwich_generation()

@@ -32,7 +32,7 @@ def test_no_access_leaves_its_allocation():
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
     res = json.loads(p.stdout.strip().splitlines()[-1])
     print(json.dumps(res, indent=1))
-    assert res["negative_control"]["refused"] > 0
+    assert res["negative_control"]["refused"] > 0 and min(res["sampler_workspace_control"]) > 0
     assert len(res["rank_steps"]) == 18 and len(res["engine"]) == 3 and len(res["sampler"]) == 12
     assert len(res["sandwich"]) == 2 and len(res["block_mixers"]) == 2 and len(res["parallel_layers"]) == 2
     assert len(res["post_norms"]) == 2 and len(res["table_mixtures"]) == 2

@@ -888,8 +888,7 @@ __device__ __forceinline__ void radix_pick_regs(const unsigned long long (&h4)[4
 // last: the masses of the last stage, for every column range by itself (how many tokens of the key at which the
 // top-p prefix ends lie in the ranges ahead follows from them: such tokens weigh the same).
 // best: the order-preserving key of the row's largest logit and its inverted index (a NaN on top); without a
-// workspace, in the library's own scratch, for the rows whose flag is up.  Either scratch is addressed by row, stage and
-// range alone, never by a value, and accessed plainly: a workspace allocated for one call is not in a bounds list.
+// workspace, in the library's own scratch, for the rows whose flag is up (accessed plainly: it is in no bounds list).
 constexpr int kSampleWsHead = 32;
 __host__ __device__ __forceinline__ int64_t sample_ws_words(int64_t rows, int stages) { return rows * (kSampleWsHead + stages * 256); }
 constexpr int kSampleWsThreads = 256;                       // of a workgroup of this way
@@ -907,8 +906,8 @@ __device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, 
 // workgroup barriers -- a third of the follow-up launches' time), picks level after level with shuffles only and
 // hands the state to the workgroup through LDS (shl scratch).  upto = 2 * NL: the full state.
 template <int LDT>
-__device__ __forceinline__ ExactState exact_replay(const unsigned long long* hists, int upto, int K1, float tp, float temp,
-                                                   float l0, unsigned long long* shl) {
+__device__ __forceinline__ ExactState exact_replay(const unsigned long long* ws, const unsigned long long* hists, int upto, int K1,
+                                                   float tp, float temp, float l0, unsigned long long* shl) {
   using L = ExactLevels<LDT>;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   ExactState st;
@@ -919,7 +918,10 @@ __device__ __forceinline__ ExactState exact_replay(const unsigned long long* his
     for (int s_ = 0; s_ < 2 * L::NL; ++s_) {
       const bool on = s_ < upto && (s_ < L::NL ? K1 > 0 : tp < 1.0f);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) h[s_][j] = on ? hists[s_ * 256 + 255 - 4 * lane - j] : 0ull;
+      for (int j = 0; j < 4; ++j) {
+        const unsigned long long* at = hists + s_ * 256 + 255 - 4 * lane - j;
+        h[s_][j] = !on ? 0ull : ws != nullptr ? MI355_LD(unsigned long long, ws, at) : *at;
+      }
     }
     // top-k: stages 0 .. NL-1
     if (K1 > 0) {
@@ -985,7 +987,7 @@ template <int LDT>
 __device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp, int vocab) {
   if (ws == nullptr) return ExactRow{row < kExactRows && g_exact_flag[row] != 0u ? &g_exact_hist[row][0][0] : nullptr,
                                      row < kExactRows ? g_exact_l0[row] : 0.f};
-  const uint32_t key = static_cast<uint32_t>(ws[static_cast<int64_t>(row) * kSampleWsHead] >> 32);
+  const uint32_t key = static_cast<uint32_t>(MI355_LD(unsigned long long, ws, ws + static_cast<int64_t>(row) * kSampleWsHead) >> 32);
   if (sample_one_key(temp, k, tp, vocab) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
   return ExactRow{ws + static_cast<int64_t>(rows) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256, key_to_logit(key)};
 }
@@ -1037,7 +1039,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_hist_kernel(
   __shared__ float list[kListed];
   __shared__ int listed;
   const int tid = threadIdx.x;
-  const ExactState st = exact_replay<LDT>(er.hists, stage, K1, tp, temp, l0, shl);
+  const ExactState st = exact_replay<LDT>(ws, er.hists, stage, K1, tp, temp, l0, shl);
   const int shift = 24 - 8 * (counting ? stage : stage - L::NL);
   if (tid < 256) hist[tid] = 0ull;
   __syncthreads();
@@ -1073,9 +1075,11 @@ __global__ __launch_bounds__(kSampleThreads) void exact_hist_kernel(
   }
   __syncthreads();
   if (tid < 256) {
-    if (hist[tid] != 0ull) atomicAdd(er.hists + stage * 256 + tid, hist[tid]);
+    unsigned long long* bin = er.hists + stage * 256 + tid;
+    if (hist[tid] != 0ull && (ws == nullptr || MI355_OK_AT(ws, bin, 8))) atomicAdd(bin, hist[tid]);
     if (ws != nullptr && stage == 2 * L::NL - 1)
-      ws[sample_ws_words(rows, 2 * L::NL) + (static_cast<int64_t>(row) * ranges + range) * 256 + tid] = hist[tid];
+      MI355_ST(unsigned long long, ws,
+               ws + sample_ws_words(rows, 2 * L::NL) + (static_cast<int64_t>(row) * ranges + range) * 256 + tid, hist[tid]);
   }
 }
 
@@ -1096,7 +1100,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
   __shared__ unsigned long long shl[4];
   __shared__ int eq_base[kSampleThreads / 64 + 1];
   __shared__ unsigned long long part[kSampleThreads / 64];
-  const ExactState st = exact_replay<LDT>(er.hists, 2 * L::NL, K1, tp, temp, l0, shl);
+  const ExactState st = exact_replay<LDT>(ws, er.hists, 2 * L::NL, K1, tp, temp, l0, shl);
   const void* base = LDT == MI355_F32 ? static_cast<const void*>(static_cast<const float*>(logits) + row * stride)
                                       : static_cast<const void*>(static_cast<const uint16_t*>(logits) + row * stride);
   // tokens at the cut key in the column ranges before this one (only when top-p cuts inside that tie): counted
@@ -1105,7 +1109,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
   if (st.take != ~0ull && range != 0 && ws != nullptr) {
     const unsigned long long* last = ws + sample_ws_words(rows, 2 * L::NL) + static_cast<int64_t>(row) * ranges * 256 +
                                      ((st.Tp >> L::kLastShift) & 255u);
-    unsigned long long m = tid < range ? last[tid * 256] : 0ull;
+    unsigned long long m = tid < range ? MI355_LD(unsigned long long, ws, last + tid * 256) : 0ull;
     m = wave_sum64(m);                                   // (at most 64 ranges: the first wave has them all)
     if (tid == 0) part[0] = m / sample_mass(key_to_logit(st.Tp), l0, temp);
     __syncthreads();
@@ -1134,7 +1138,7 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
   __syncthreads();
   best = sample_reduce_max(best, part);
   unsigned long long* key = ws != nullptr ? ws + static_cast<int64_t>(row) * kSampleWsHead + 16 : reinterpret_cast<unsigned long long*>(out) + row;
-  if (tid == 0 && best != 0ull && (ws != nullptr || MI355_OK_AT(out, key, 8))) atomicMax(key, best);
+  if (tid == 0 && best != 0ull && MI355_OK_AT((ws != nullptr ? static_cast<const void*>(ws) : out), key, 8)) atomicMax(key, best);
 }
 
 // ---- the k most likely tokens of a row (the `logprobs` / `top_logprobs` lists of the completion routes): an
@@ -1235,8 +1239,8 @@ __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __r
 }
 
 // One pass, one key: the row is cut into column ranges, every workgroup merges the best key of its
-// range into *key (cleared ahead; of `buffer`, or null: in the sampler's own scratch) with a 64-bit atomic max -- order-free, so the same on every launch --
-// and a later launch turns it into the index.
+// range into *key (of `buffer`, cleared ahead) with a 64-bit atomic max -- order-free, so the same on every launch -- and a
+// later launch turns it into the index.
 template <int LDT>
 __device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, const void* base, int vocab, bool greedy, float temp,
                                                     uint64_t seed, uint64_t step, int range, int ranges, int chunk_vecs,
@@ -1250,7 +1254,7 @@ __device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, con
   else
     best = sample_full_vocab<LDT>(base, vocab, v0, v1, tail, temp, seed, step);
   best = sample_reduce_max(best, part);
-  if (threadIdx.x == 0 && best != 0ull && (buffer == nullptr || MI355_OK_AT(buffer, key, 8))) atomicMax(key, best);
+  if (threadIdx.x == 0 && best != 0ull && MI355_OK_AT(buffer, key, 8)) atomicMax(key, best);
 }
 
 // ---- sampling with a caller's workspace: every row spread over all of its workgroups.  The list way above keeps a row
@@ -1262,7 +1266,7 @@ __device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, con
 // 32 rows of 128256 bf16 logits with a mix of cuts: 94 us a call, here 40 (the draws of uncut rows and the launches' gaps).
 __global__ __launch_bounds__(256) void sample_clear_kernel(unsigned long long* __restrict__ ws, int64_t words) {
   const int64_t i = 2 * (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x);
-  if (i + 1 < words) *reinterpret_cast<uint4*>(ws + i) = make_uint4(0u, 0u, 0u, 0u);
+  if (i + 1 < words) MI355_ST(uint4, ws, ws + i, make_uint4(0u, 0u, 0u, 0u));
 }
 
 __global__ void sample_ws_finish_kernel(int64_t* __restrict__ out, const unsigned long long* __restrict__ ws,
@@ -1271,8 +1275,8 @@ __global__ void sample_ws_finish_kernel(int64_t* __restrict__ out, const unsigne
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const unsigned long long* head = ws + static_cast<int64_t>(i) * kSampleWsHead;
-  unsigned long long b = head[16];
-  const unsigned long long top = head[0];
+  unsigned long long b = MI355_LD(unsigned long long, ws, head + 16);
+  const unsigned long long top = MI355_LD(unsigned long long, ws, head);
   if (!sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i), MI355_LD(float, top_p, top_p + i), vocab) &&
       static_cast<uint32_t>(top >> 32) == 0xFFFFFFFFu)
     b = top;                                               // a NaN: its first index
@@ -1294,7 +1298,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
   if (sample_one_key(temp, k, tp, vocab)) {
     sample_one_key_pass<LDT>(ws + static_cast<int64_t>(row) * kSampleWsHead + 16, base, vocab, !(temp > 0.0f), temp, static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)),
                              static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row)), blockIdx.x,
-                             gridDim.x, chunk_vecs, part, nullptr);
+                             gridDim.x, chunk_vecs, part, ws);
     return;
   }
   const bool counts = k > 0 && k < vocab;
@@ -1312,9 +1316,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
   });
   best = sample_reduce_max(best, part);                  // (its barrier also ends the counting)
   unsigned long long* top = ws + static_cast<int64_t>(row) * kSampleWsHead;
-  if (tid == 0 && best != 0ull) atomicMax(top, best);
+  if (tid == 0 && best != 0ull && MI355_OK_AT(ws, top, 8)) atomicMax(top, best);
   if (counts && tid < 256 && hist[tid] != 0ull) {
-    atomicAdd(ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256 + tid, hist[tid]);
+    unsigned long long* bin = ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256 + tid;
+    if (MI355_OK_AT(ws, bin, 8)) atomicAdd(bin, hist[tid]);
   }
 }
 

@@ -624,12 +624,13 @@ def sample_spreads(rows: int, vocab: int, dtype: torch.dtype, short_cuts: bool =
 
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
            seeds: torch.Tensor, steps: torch.Tensor, out: torch.Tensor | None = None, cut_rows: bool = True,
-           short_cuts: bool = False):
+           short_cuts: bool = False, workspace: torch.Tensor | None = None):
     """Per-row sampling (greedy where temperature <= 0).  temperature/top_p float32 [B], top_k int32 [B],
     seeds/steps int64 [B], all on the device.  cut_rows=False: the caller knows that no row has an active
     top-k / top-p, so the follow-up launches that serve rows with huge kept sets are left out (same tokens).
     short_cuts=True: the caller knows that every row with a cut has a top-k of at most SAMPLE_SHORT_CUT and some a top-p
-    with it (the way that is faster for those; same tokens)."""
+    with it (the way that is faster for those; same tokens).  workspace: uint8, lib.mi355_sample_workspace(B, dtype code)
+    bytes or more, for rows that are spread over workgroups (None: allocated for the call)."""
     _dev(logits, "logits")
     if logits.dtype not in _DT:
         raise TypeError(f"logits dtype {logits.dtype} not supported")
@@ -644,8 +645,12 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     args = (out.data_ptr(), logits.data_ptr(), _rows(logits, "logits"), B, V, _DT[logits.dtype], temperature.data_ptr(),
             top_k.data_ptr(), top_p.data_ptr(), seeds.data_ptr(), steps.data_ptr())
     if cut_rows and sample_spreads(B, V, logits.dtype, short_cuts):
-        ws = torch.empty(lib.mi355_sample_workspace(B, _DT[logits.dtype]), dtype=torch.uint8, device=logits.device)
-        check(lib.mi355_sample_topk_topp_ws(*args, ws.data_ptr(), ws.numel(), _stream()))
+        if workspace is None:
+            workspace = torch.empty(lib.mi355_sample_workspace(B, _DT[logits.dtype]), dtype=torch.uint8, device=logits.device)
+        _dev(workspace, "workspace")
+        if workspace.dtype != torch.uint8 or not workspace.is_contiguous():
+            raise ValueError("workspace must be contiguous uint8")
+        check(lib.mi355_sample_topk_topp_ws(*args, workspace.data_ptr(), workspace.numel(), _stream()))
     else:
         check(lib.mi355_sample_topk_topp_hinted(*args, 1 if cut_rows else 0, _stream()))
     return out
