@@ -410,6 +410,65 @@ def table_mixture_generation():
     return out
 
 
+def window_and_delta_generation():
+    """A hybrid decoder of the Lozupel design (sigmoid window attention, the gated delta rule with a decay per head and per
+    channel, short convolutions, a loop): portions and prompts long enough for the tiled and staged forms, single rows, a mixed
+    batch, then generation, in bfloat16 (head sizes of the vector forms, K-split products) and in float32."""
+    from mi355_decode import weights as W
+    from mi355_decode.config import EngineArgs, ModelConfig
+    from mi355_decode.llm import build_engine
+    from mi355_decode.sampling_params import SamplingParams
+
+    def left(heads, kv, dim, vdim, window, rot):
+        return {"heads": heads, "kv_heads": kv, "dim": dim, "vdim": vdim, "mask": {"size": window}, "rot": {"dims": rot, "base": 10000.0},
+                "scale": 0.2}
+
+    def right(heads, kv, dim, vdim, conv):
+        return {"heads": heads, "kv_heads": kv, "dim": dim, "vdim": vdim, "conv": conv}
+    cfg = ModelConfig.from_dict({
+        "architecture": "Lozupel", "embedding": {"scale": 1.0}, "width": 512, "vocab": 300, "norm": {"eps": 1e-6}, "logit_softcap": 20.0,
+        "loop": {"start": 0, "stop": 2, "times": 2},
+        "layers": [{"type": "parallel", "mixer": {"left": left(8, 2, 64, 128, 40, 32), "right": right(4, 2, 64, 128, 4)},
+                    "mlp": {"kind": "dense", "ff": 1024}},
+                   {"type": "delta", "mixer": right(8, 4, 64, 64, 3), "mlp": {"kind": "dense", "ff": 512}},
+                   {"type": "parallel", "mixer": {"left": left(3, 3, 24, 40, 33, 8), "right": right(4, 2, 24, 17, 2)}, "mlp": None}]})
+    state = W.hybrid_synthetic_state(cfg, seed=3)
+    rng = np.random.default_rng(1)
+    out = []
+    for dtype in ("bfloat16", "float32"):
+        bounds.clear()
+        eng = build_engine(EngineArgs(model="windows", dtype=dtype, max_num_seqs=4, max_model_len=640,
+                                      num_gpu_blocks_override=96, gpu_memory_utilization=0.0, max_num_batched_tokens=1 << 20),
+                           state_dict=state, model_config=cfg)
+
+        def run(tag):
+            toks = {r: rng.integers(0, 300, n).tolist() for r, n in (("a", 560), ("b", 137), ("c", 2))}
+            eng.forced_step([(tag + "a", toks["a"][:500], [499]), (tag + "c", toks["c"][:1], [0])])
+            eng.forced_step([(tag + "a", toks["a"][500:502], [1]), (tag + "b", toks["b"][:133], []), (tag + "c", toks["c"][1:], [0])],
+                            [tag + "c"])
+            for i in range(4):
+                eng.forced_step([(tag + "a", toks["a"][502 + i:503 + i], [0]), (tag + "b", toks["b"][133 + i:134 + i], [0])])
+            eng.forced_step([(tag + "a", toks["a"][506:], [])], [tag + "a", tag + "b"])
+            for i, n in enumerate((5, 70, 17)):
+                eng.add_request(f"{tag}g{i}", rng.integers(0, 300, n).tolist(),
+                                SamplingParams(max_tokens=10, temperature=0.0 if i else 0.8, seed=i, ignore_eos=True))
+            n = 0
+            while eng.has_unfinished():
+                n += sum(len(o.new_token_ids) for o in eng.step())
+            return n
+
+        run("warm"), run("again")                     # (the second finds every segment that the third will want)
+        n = bounds.sync_allocations(granularity="segment")
+        toks = run("checked")
+        rep = bounds.report()
+        assert rep is None or rep["refused"] == 0, (dtype, rep)
+        out.append(f"{dtype}:{toks} tokens:{n} segments:{rep['unknown_base'] if rep else 0} accesses with an unlisted base")
+        del eng
+        gc.collect()
+        torch.cuda.empty_cache()
+    return out
+
+
 def sampler_rows():
     """The sampling launch on exactly sized logits (no slack behind the last row), every kind of
     row in one call: greedy, whole-vocabulary draw, top-k / top-p cuts, an all-tied row (the list
@@ -481,4 +540,5 @@ if __name__ == "__main__":
     res["parallel_layers"] = parallel_layer_generation()
     res["post_norms"] = post_norm_generation()
     res["table_mixtures"] = table_mixture_generation()
+    res["windows_and_deltas"] = window_and_delta_generation()
     print(json.dumps(res))
