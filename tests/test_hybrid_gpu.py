@@ -174,6 +174,22 @@ def test_row_kernels_add_slabs_as_a_launch_of_their_own_would(W, num):
         assert torch.equal(ops.gelu_tanh_and_mul(z), ops.gelu_tanh_and_mul(z.dense()))
 
 
+def test_slabs_that_no_row_kernel_takes_are_added_once(monkeypatch):
+    """An add without a norm and rows wider than the row kernels': one launch adds the slabs, and the numbers are its rows'."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(2)
+    added, add = [], ops.sum_slabs
+    monkeypatch.setattr(ops, "sum_slabs", lambda *a, **k: (added.append(1), add(*a, **k))[1])
+    for W, weight in ((64, False), (8200, True), (8200, False)):
+        x, resid = ops.Slabs(torch.randn(2, 5, W, generator=g).cuda(), 2, 5, W, torch.bfloat16), torch.randn(5, W, generator=g).cuda()
+        w, rows, r1, r2 = torch.randn(W, generator=g).bfloat16().cuda() if weight else None, x.dense(), resid.clone(), resid.clone()
+        added.clear()
+        a = ops.add_layer_norm_f32(r1, w, 1e-5, add=x)
+        assert len(added) == 1
+        b = ops.add_layer_norm_f32(r2, w, 1e-5, add=rows)
+        assert torch.equal(r1, r2) and (torch.equal(a, b) if weight else a is None or torch.equal(a, b))
+
+
 def _paged(T, num_pages, seed):
     """A shuffled block table for one sequence of T tokens and its slot mapping."""
     order = np.random.default_rng(seed).permutation(num_pages)[: (T + 15) // 16].astype(np.int32)

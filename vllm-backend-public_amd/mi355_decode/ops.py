@@ -1167,7 +1167,9 @@ def add_layer_norm_f32(resid: torch.Tensor, weight: torch.Tensor | None, eps: fl
     weight [width]; weight None: the add alone, nothing returned.  inv (int32 [tokens * top]): add holds a
     mixture's rows in expert order, token t's addend is row_weight * sum_k add[inv[t * top + k]]."""
     T, W = resid.shape
-    ref = weight if weight is not None else dense(add)
+    if weight is None:
+        add = dense(add)
+    ref = weight if weight is not None else add
     dt = _dt3(ref, "weight")
     if weight is not None and (tuple(weight.shape) != (W,) or not weight.is_contiguous()):
         raise ValueError("weight must be one contiguous row")
