@@ -563,8 +563,7 @@ __global__ __launch_bounds__(D) void paged_attn_merge_kernel(uint16_t* __restric
   const float* ml = part_ml + row * num_splits * 2;
   const float* po = part_o + row * num_splits * D + d;
   // N splits a turn, all of a turn's loads out before the first is used (one trip to memory); a turn after the first
-  // rescales what is there.  (A load where it was used took 7.1 us for 16 splits of 32 heads; so 4.6, what an empty
-  // launch takes under the same profiler.)
+  // rescales what is there.  (A load where it was used took 7.1 us for 16 splits of 32 heads; so 4.6.)
   float mg = -INFINITY, acc = 0.f, lsum = 0.f;
   for (int s0 = 0; s0 < num_splits; s0 += N) {
     float2 m[N];

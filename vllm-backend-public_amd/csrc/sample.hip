@@ -216,6 +216,9 @@ constexpr int kSampleThreads = 1024;
 constexpr int kSampleGuessRank = 1024;   // the LDS list is built around the row's 1024 largest logits (or its top_k, if smaller)
 constexpr int kSampleCap = 4096;         // candidates at or above the threshold guess that LDS holds (4 a thread)
 
+// The top-k that cuts, 0: none (off, or of the whole vocabulary).
+__device__ __forceinline__ int active_top_k(int top_k, int vocab) { return top_k > 0 && top_k < vocab ? top_k : 0; }
+
 // NaN sorts on top, as in argmax_key: a row that holds a NaN yields the index of its first NaN
 // from greedy and from random sampling alike
 __device__ __forceinline__ uint32_t sample_key(float v) {
@@ -889,6 +892,11 @@ __device__ __forceinline__ void radix_pick_regs(const unsigned long long (&h4)[4
 // top-p prefix ends lie in the ranges ahead follows from them: such tokens weigh the same).
 // best: the order-preserving key of the row's largest logit and its inverted index (a NaN on top); without a
 // workspace, in the library's own scratch, for the rows whose flag is up (accessed plainly: it is in no bounds list).
+#ifdef MI355_BOUNDS
+#define MI355_SCRATCH_LD(ws, p) ((ws) != nullptr ? MI355_LD(unsigned long long, (ws), (p)) : *(p))
+#else
+#define MI355_SCRATCH_LD(ws, p) (*(p))
+#endif
 constexpr int kSampleWsHead = 32;
 __host__ __device__ __forceinline__ int64_t sample_ws_words(int64_t rows, int stages) { return rows * (kSampleWsHead + stages * 256); }
 constexpr int kSampleWsThreads = 256;                       // of a workgroup of this way
@@ -899,7 +907,7 @@ struct ExactRow {
   float l0;                      // its largest logit
 };
 template <int LDT>
-__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp, int vocab);
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int K1, float tp);
 
 // Replays the picks of stages [0, upto) of a row from its finished histograms [stage][256].  Wave 0 does it alone: it asks
 // for every histogram it will need at once (one memory round trip instead of one per level, each followed by two
@@ -919,8 +927,7 @@ __device__ __forceinline__ ExactState exact_replay(const unsigned long long* ws,
       const bool on = s_ < upto && (s_ < L::NL ? K1 > 0 : tp < 1.0f);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const unsigned long long* at = hists + s_ * 256 + 255 - 4 * lane - j;
-        h[s_][j] = !on ? 0ull : ws != nullptr ? MI355_LD(unsigned long long, ws, at) : *at;
+        h[s_][j] = on ? MI355_SCRATCH_LD(ws, hists + s_ * 256 + 255 - 4 * lane - j) : 0ull;
       }
     }
     // top-k: stages 0 .. NL-1
@@ -978,17 +985,17 @@ __device__ __forceinline__ ExactState exact_replay(const unsigned long long* ws,
   return st;
 }
 
-// Rows that need one key only: greedy ones and draws with neither top-k nor top-p (a top-k of the whole vocabulary is none).
-__device__ __forceinline__ bool sample_one_key(float temp, int top_k, float top_p, int vocab) {
-  return !(temp > 0.0f) || ((top_k <= 0 || top_k >= vocab) && !(top_p < 1.0f));
+// Rows that need one key only: greedy ones and draws with neither an active top-k (active_top_k) nor a top-p.
+__device__ __forceinline__ bool sample_one_key(float temp, int K1, float top_p) {
+  return !(temp > 0.0f) || (K1 == 0 && !(top_p < 1.0f));
 }
 
 template <int LDT>
-__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int k, float tp, int vocab) {
+__device__ __forceinline__ ExactRow exact_row(unsigned long long* ws, int rows, int row, float temp, int K1, float tp) {
   if (ws == nullptr) return ExactRow{row < kExactRows && g_exact_flag[row] != 0u ? &g_exact_hist[row][0][0] : nullptr,
                                      row < kExactRows ? g_exact_l0[row] : 0.f};
   const uint32_t key = static_cast<uint32_t>(MI355_LD(unsigned long long, ws, ws + static_cast<int64_t>(row) * kSampleWsHead) >> 32);
-  if (sample_one_key(temp, k, tp, vocab) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
+  if (sample_one_key(temp, K1, tp) || key == 0xFFFFFFFFu) return ExactRow{nullptr, 0.f};      // (a NaN: its index is known)
   return ExactRow{ws + static_cast<int64_t>(rows) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256, key_to_logit(key)};
 }
 
@@ -1025,10 +1032,9 @@ __global__ __launch_bounds__(kSampleThreads) void exact_hist_kernel(
   using L = ExactLevels<LDT>;
   const int row = ws != nullptr ? blockIdx.y : blockIdx.x, range = ws != nullptr ? blockIdx.x : blockIdx.y;
   const int rows = ws != nullptr ? gridDim.y : gridDim.x, ranges = ws != nullptr ? gridDim.x : gridDim.y;
-  const int k = MI355_LD(int32_t, top_k, top_k + row);
-  const int K1 = (k > 0 && k < vocab) ? k : 0;
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
-  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp, vocab);
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, K1, tp);
   if (er.hists == nullptr) return;
   const bool counting = stage < L::NL;
   if (counting ? K1 == 0 : !(tp < 1.0f)) return;       // this selection is off for the row
@@ -1091,10 +1097,9 @@ __global__ __launch_bounds__(kSampleThreads) void exact_final_kernel(
   using L = ExactLevels<LDT>;
   const int row = ws != nullptr ? blockIdx.y : blockIdx.x, range = ws != nullptr ? blockIdx.x : blockIdx.y;
   const int rows = ws != nullptr ? gridDim.y : gridDim.x, ranges = ws != nullptr ? gridDim.x : gridDim.y, tid = threadIdx.x;
-  const int k = MI355_LD(int32_t, top_k, top_k + row);
-  const int K1 = (k > 0 && k < vocab) ? k : 0;
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
   const float tp = MI355_LD(float, top_p, top_p + row), temp = MI355_LD(float, temperature, temperature + row);
-  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, k, tp, vocab);
+  const ExactRow er = exact_row<LDT>(ws, rows, row, temp, K1, tp);
   if (er.hists == nullptr) return;
   const float l0 = er.l0;
   __shared__ unsigned long long shl[4];
@@ -1231,8 +1236,8 @@ __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __r
   if (i >= n) return;
   const bool spread = i < kExactRows && g_exact_flag[i] != 0u;      // its token came from the follow-up launches, as a key
   if (spread) g_exact_flag[i] = 0u;
-  if (!spread && !sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i),
-                                 MI355_LD(float, top_p, top_p + i), vocab))
+  if (!spread && !sample_one_key(MI355_LD(float, temperature, temperature + i), active_top_k(MI355_LD(int32_t, top_k, top_k + i), vocab),
+                                 MI355_LD(float, top_p, top_p + i)))
     return;
   const unsigned long long b = static_cast<unsigned long long>(MI355_LD(int64_t, out, out + i));
   MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
@@ -1277,7 +1282,8 @@ __global__ void sample_ws_finish_kernel(int64_t* __restrict__ out, const unsigne
   const unsigned long long* head = ws + static_cast<int64_t>(i) * kSampleWsHead;
   unsigned long long b = MI355_LD(unsigned long long, ws, head + 16);
   const unsigned long long top = MI355_LD(unsigned long long, ws, head);
-  if (!sample_one_key(MI355_LD(float, temperature, temperature + i), MI355_LD(int32_t, top_k, top_k + i), MI355_LD(float, top_p, top_p + i), vocab) &&
+  if (!sample_one_key(MI355_LD(float, temperature, temperature + i), active_top_k(MI355_LD(int32_t, top_k, top_k + i), vocab),
+                      MI355_LD(float, top_p, top_p + i)) &&
       static_cast<uint32_t>(top >> 32) == 0xFFFFFFFFu)
     b = top;                                               // a NaN: its first index
   MI355_ST(int64_t, out, out + i, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
@@ -1294,14 +1300,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
   __shared__ unsigned long long part[kSampleThreads / 64];
   __shared__ unsigned long long hist[256];
   const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
-  const int k = MI355_LD(int32_t, top_k, top_k + row);
-  if (sample_one_key(temp, k, tp, vocab)) {
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
+  if (sample_one_key(temp, K1, tp)) {
     sample_one_key_pass<LDT>(ws + static_cast<int64_t>(row) * kSampleWsHead + 16, base, vocab, !(temp > 0.0f), temp, static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)),
                              static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row)), blockIdx.x,
                              gridDim.x, chunk_vecs, part, ws);
     return;
   }
-  const bool counts = k > 0 && k < vocab;
+  const bool counts = K1 > 0;
   if (counts) {
     if (tid < 256) hist[tid] = 0ull;
     __syncthreads();
@@ -1347,18 +1353,17 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   __shared__ int sh[4];
 
   const float temp = MI355_LD(float, temperature, temperature + row);
-  int k = MI355_LD(int32_t, top_k, top_k + row);
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
   const float tp = MI355_LD(float, top_p, top_p + row);
   const uint64_t seed = static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row));
   const uint64_t step = static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row));
   const bool greedy = !(temp > 0.0f);
-  if (sample_one_key(temp, k, tp, vocab)) {
+  if (sample_one_key(temp, K1, tp)) {
     sample_one_key_pass<LDT>(reinterpret_cast<unsigned long long*>(out) + row, base, vocab, greedy, temp, seed, step, blockIdx.y,
                              gridDim.y, chunk_vecs, part, out);
     return;
   }
   if (blockIdx.y != 0) return;
-  const int K1 = (k > 0 && k < vocab) ? k : 0;          // an active top-k
   const uint32_t row_hash = sample_hash(seed, step);
 
   // ---- 1. one pass: every thread's two largest logits (for the threshold guess), the row maximum,

@@ -983,9 +983,9 @@ __global__ __launch_bounds__(1024) void mingru_scan_kernel(
 // memory to registers as MFMA operands (paged_attn_decode.hip's layout) and STG steps of a wave are in flight.  The
 // weights are not normalised: the waves' sums, and the key ranges', simply add up.  gridDim.z > 1: fp32 sums without
 // the gate to slab z of `partial`.  Bound by what
-// one CU draws from memory: 32 rows, 16 heads of 128 on 4 kv heads, 1024 keys each, 17.6 us without ranges, 13 with two and
-// the sum's launch behind it (the tile form, 15 of a tile's 16 rows empty and V by 8 bytes: 34 and 6 for the sum).  Eight
-// waves a workgroup in place of four: 18.0.
+// one CU draws from memory: 32 rows, 16 heads of 128 on 4 kv heads, 1024 keys each, 17.6 us without ranges (21.9 in a decode
+// step), 13 with two and the sum's launch behind it (the tile form, 15 of a tile's 16 rows empty and V by 8 bytes: 34 and 6
+// for the sum).  Eight waves a workgroup in place of four: 18.0.
 template <typename T, int D, int DV, int NW, int STG>
 __global__ __launch_bounds__(64 * NW) void sigmoid_window_decode_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ k_cache,

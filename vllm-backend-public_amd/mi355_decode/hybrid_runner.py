@@ -840,7 +840,10 @@ class HybridRunner(ModelRunner):
         if int(b.tiles.shape[0]) == b.num_tokens and rep <= 16 and a.dim in (64, 128) and a.vdim in (64, 128):
             # single rows: a workgroup per (row, kv head) reads at what one CU can (1024 keys of 128 in 13 us), two leave
             # their gain to the sum over the ranges (window 1024, 4 kv heads, 1 / 2 / 4 / 8 / 16 ranges: 8 rows
-            # 14.0 / 12.5 / 10.5 / 10.4 / 11.6 us, 16 rows 14.4 / 13.3 / 12.6 / 13.6 / 15.1, 32 rows 17.6 / 17.6 / 17.5 / 21.4 / 23.2)
+            # 14.0 / 12.5 / 10.5 / 10.4 / 11.6 us, 16 rows 14.4 / 13.3 / 12.6 / 13.6 / 15.1, 32 rows 17.6 / 17.6 / 17.5 / 21.4 / 23.2;
+            # in a step, where other launches have emptied the caches, the 32 rows take 21.9).  The rule against the tile form
+            # with its up to 16 ranges, 1 to 64 rows, windows 128 to 4096, 1 to 16 kv heads, 64 and 128 wide: nowhere slower
+            # (32 rows of one kv head 12.2 / 25.6, at window 4096 21.3 / 49.1; of 16 kv heads 47.0 / 52.2, 193 / 205)
             n = min(self.MAX_KEY_SPLITS, a.window // 128, 256 // max(b.num_tokens * a.kv_heads, 1))
             n = n if n > 2 else 1
         else:

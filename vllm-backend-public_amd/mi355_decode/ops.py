@@ -647,9 +647,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     if cut_rows and sample_spreads(B, V, logits.dtype, short_cuts):
         if workspace is None:
             workspace = torch.empty(lib.mi355_sample_workspace(B, _DT[logits.dtype]), dtype=torch.uint8, device=logits.device)
-        _dev(workspace, "workspace")
-        if workspace.dtype != torch.uint8 or not workspace.is_contiguous():
-            raise ValueError("workspace must be contiguous uint8")
+        elif not workspace.is_cuda or workspace.dtype != torch.uint8 or not workspace.is_contiguous():
+            raise ValueError("workspace must be contiguous uint8 on the GPU")
         check(lib.mi355_sample_topk_topp_ws(*args, workspace.data_ptr(), workspace.numel(), _stream()))
     else:
         check(lib.mi355_sample_topk_topp_hinted(*args, 1 if cut_rows else 0, _stream()))
