@@ -445,7 +445,7 @@ def test_delta_rule_whole_portions_and_single_tokens(H, G, d, dv, per_channel):
     a_log, dt_bias = torch.randn(H, generator=g) * 0.5 - 1, torch.randn(decay.shape[1], generator=g) * 0.5
     ref = _delta_ref(qkv, beta, decay, a_log, dt_bias, H, G, d, dv, per_channel)
     for cuts in ([T], [1] * T, [2, 3, 1, 17, 2, 16]):
-        for long_chunks in (False, True):             # one column per lane; tiles of 16 rows (single tokens: always the former)
+        for long_chunks in (False, True):             # token by token; tiles of 16 rows (portions of a few rows: the former)
             got = _delta_in_cuts(qkv, beta, decay, a_log, dt_bias, cuts, H, G, d, dv, per_channel, long_chunks=long_chunks)
             assert (got - ref).abs().max() <= 3e-5 * ref.abs().max(), (cuts, long_chunks)
 
