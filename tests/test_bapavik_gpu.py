@@ -226,6 +226,50 @@ def test_table_mixture_of_ungated_experts(dtype, E, top, T, W, F):
         H.EXPERT_GEMM_MIN_ROWS = keep
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])      # half an ulp of the largest number, and sums
+@pytest.mark.parametrize("counts,N,K", [((1, 128, 129, 255), 12288, 128), ((0, 256, 257, 384, 385, 0), 4104, 192), ((640, 0, 511, 513), 2816, 320),
+                                        ((1030,) * 7 + (900,), 1536, 128)])
+def test_expert_products_by_wide_tiles(dtype, tol, counts, N, K):
+    """Rows that end a tile of 256 or 128 early, fill it, or just spill over; experts without rows, outputs and steps of K
+    that do not fill the last tile; gathered rows and rows in place, with and without the activation."""
+    from mi355_decode import ops
+    g = torch.Generator(device="cuda").manual_seed(N)
+    E, rows = len(counts), sum(counts)
+    w = (torch.randn(E, N, K, generator=g, device="cuda") * K ** -0.5).to(dtype)
+    x = torch.randn(rows, K, generator=g, device="cuda").to(dtype)
+    perm = torch.randperm(rows, generator=g, device="cuda").to(torch.int32)
+    c = torch.tensor(counts)
+    off = torch.cat([torch.zeros(1, dtype=torch.long), c.cumsum(0)]).to(torch.int32).cuda()
+    start = torch.cat([torch.zeros(1, dtype=torch.long), (-(-c // ops.MOE_TILE_ROWS)).cumsum(0)]).to(torch.int32).cuda()
+    for p in (None, perm):
+        xs = x if p is None else x[p.long()]
+        want = torch.cat([xs[a:b].float() @ w[e].float().t() for e, (a, b) in enumerate(zip(off[:-1].tolist(), off[1:].tolist()))])
+        _near(ops.expert_gemm(x, w, off, start, rows, perm=p), want, tol)
+    _near(ops.expert_gemm(x, w, off, start, rows, perm=perm, relu2=True), want.clamp(min=0) ** 2, 3 * tol)
+
+
+@pytest.mark.parametrize("rows", [3000, 3073, 4096 + 17])
+def test_products_per_head_by_wide_tiles(rows):
+    from mi355_decode import ops
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    H, N, K, C = 17, 128, 256, 64
+    w = (torch.randn(H, N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    src = torch.randn(rows + 9, K + C, generator=g, device="cuda").bfloat16()
+    index = torch.randint(0, rows + 9, (rows,), generator=g, device="cuda").to(torch.int32)
+    x, pages = src[index.long()], -(-rows // 16)
+    want = (x[:, :K].float() @ w.view(H * N, K).float().t()).view(rows, H, N)
+    out = torch.full((pages, H, 16, N + C), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.head_gemm(src, 0, w, out, H * 16 * (N + C), N + C, 16 * (N + C), rows, index=index, copy=C)
+    got = out.permute(0, 2, 1, 3).reshape(pages * 16, H, N + C)
+    _near(got[:rows, :, :N], want, 4e-3)
+    assert torch.equal(got[:rows, :, N:], x[:, None, K:].expand(rows, H, C)) and (got[rows:] == 7.0).all()
+    out = torch.full((pages, H, N, 16), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.head_gemm(src, 0, w, out, H * N * 16, 0, N * 16, rows, index=index, transposed=True)
+    got = out.permute(0, 3, 1, 2).reshape(pages * 16, H, N)
+    _near(got[:rows], want, 4e-3)
+    assert (got[rows:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3)])
 @pytest.mark.parametrize("rows", [1, 15, 33, 64, 65, 200])
 @pytest.mark.parametrize("H,N,K", [(3, 64, 32), (2, 200, 136), (5, 12, 8), (1, 132, 512)])

@@ -220,6 +220,28 @@ __device__ __forceinline__ void bounds_store(const void* base, void* p, const W&
 #define MI355_OK_AT(base, p, bytes) true
 #endif
 
+// 16 bytes a lane from global memory straight into LDS, without a register in between: lane i's go to `lds` + 16 i (`lds`
+// the same for the whole wave).  They count as vector memory loads (wait_vm); whoever reads them waits for the
+// loads of every wave that brought a part, and then at a barrier.
+__device__ __forceinline__ void lds_dma16(const void* base, const void* p, void* lds) {
+#ifdef MI355_BOUNDS
+  reinterpret_cast<uint4*>(lds)[threadIdx.x & 63] = bounds_load<uint4>(base, p, __LINE__);
+#else
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p, (__attribute__((address_space(3))) void*)lds, 16,
+                                   0, 0);
+#endif
+}
+// waits until at most N of this wave's vector memory operations are out (they end in the order they were sent)
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+#ifdef MI355_BOUNDS
+  __builtin_amdgcn_s_waitcnt(0);                    // (there the writes to LDS are the wave's own)
+#else
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+#endif
+}
+
 // ---- element access for kernels that keep some tensors in 32 bits --------------------------------
 // F32 joins BF16 / F16 as a storage type for the kernels whose arithmetic is fp32 throughout and
 // whose activations may be stored in 16 or in 32 bits (the residual stream, recurrent state and

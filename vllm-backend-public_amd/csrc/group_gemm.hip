@@ -197,8 +197,426 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GroupGemmArgs a) {
   }
 }
 
+
+// ---- tiles of 256 x 256: a persistent workgroup of 8 waves a CU -------------------------------------------------------
+// What bounds the kernel above at many rows is not the matrix cores: a 128 x 128 tile asks L2 for 64 bytes a clock and CU
+// at their full rate, as much as comes.  256 x 256 halves that, and the loads go straight to LDS (lds_dma16).
+//
+// Waves 0-3 and 4-7 are two groups, one wave of each on a SIMD, half a phase apart: while one group reads its fragments
+// and sends loads, the other has the matrix cores; a barrier after every phase keeps them so.  A step is 64 columns of K
+// in four phases: fragments of the wave's first 64 rows and of its 64 outputs (16 reads), their products, fragments of the
+// other 64 rows (8 reads), their products.  Two images of 64 KB in LDS: the loads of step t + 2 overwrite what both groups have
+// read of step t -- the first rows and W after the second read phase, the other rows a step later -- and have four
+// phases to land.  Loads run on into the next tile, so that a tile's first loads travel under the end of the one ahead;
+// the results' stores travel under the next tile's first phases (wait_vm counts them where a whole tile was stored).
+//
+// Row tiles of 256 leave more padding than 128 where the groups' rows are few or end unevenly: an expert's last 1 .. 128
+// rows, or all rows if that is the shorter plan for the rounds of workgroups (below), go as tiles of 128 x 256, half the
+// phases a step, three images of 48 KB.
+//
+// Measured in bf16: 32844 rows of 32 experts 2048 -> 1536 195 us (1060 TFLOP/s of the products asked for), 1536 -> 2048
+// 205 us; by tiles of 128 x 128 351 and 326 us on the same card.  One plain product of 8192^3 runs at 1510 TFLOP/s here.
+constexpr int kWideThreads = 512, kWideMaxGroups = 512;
+
+// Fragments of one read phase.  By instructions of our own, each block with its wait: the compiler cannot tell which loads
+// into LDS a read depends on and would wait for all of them.  X rows 16 apart (2048 bytes); W rows of fragment j at
+// (j >> 1) * 32 + (j & 1) * 4, so that a lane's outputs of two fragments are 8 adjacent ones.
+__device__ __forceinline__ void wide_read_xw(uint32_t x0, uint32_t x1, uint32_t w0, uint32_t w1, uint4 (&x)[2][4], uint4 (&w)[2][4]) {
+  asm volatile(
+      "ds_read_b128 %0, %16\n ds_read_b128 %1, %16 offset:2048\n ds_read_b128 %2, %16 offset:4096\n ds_read_b128 %3, %16 offset:6144\n"
+      "ds_read_b128 %8, %18\n ds_read_b128 %9, %18 offset:512\n ds_read_b128 %10, %18 offset:4096\n ds_read_b128 %11, %18 offset:4608\n"
+      "ds_read_b128 %4, %17\n ds_read_b128 %5, %17 offset:2048\n ds_read_b128 %6, %17 offset:4096\n ds_read_b128 %7, %17 offset:6144\n"
+      "ds_read_b128 %12, %19\n ds_read_b128 %13, %19 offset:512\n ds_read_b128 %14, %19 offset:4096\n ds_read_b128 %15, %19 offset:4608\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[0][2]), "=&v"(x[0][3]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[1][2]), "=&v"(x[1][3]),
+        "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[0][2]), "=&v"(w[0][3]), "=&v"(w[1][0]), "=&v"(w[1][1]), "=&v"(w[1][2]), "=&v"(w[1][3])
+      : "v"(x0), "v"(x1), "v"(w0), "v"(w1)
+      : "memory");
+}
+__device__ __forceinline__ void wide_read_x(uint32_t x0, uint32_t x1, uint4 (&x)[2][4]) {      // the 64 rows behind those
+  asm volatile(
+      "ds_read_b128 %0, %8 offset:8192\n ds_read_b128 %1, %8 offset:10240\n ds_read_b128 %2, %8 offset:12288\n"
+      "ds_read_b128 %3, %8 offset:14336\n ds_read_b128 %4, %9 offset:8192\n ds_read_b128 %5, %9 offset:10240\n"
+      "ds_read_b128 %6, %9 offset:12288\n ds_read_b128 %7, %9 offset:14336\n s_waitcnt lgkmcnt(0)"
+      : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[0][2]), "=&v"(x[0][3]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[1][2]), "=&v"(x[1][3])
+      : "v"(x0), "v"(x1)
+      : "memory");
+}
+__device__ __forceinline__ int wide_read_int(const int* p) {
+  int v;
+  asm volatile("ds_read_b32 %0, %1\n s_waitcnt lgkmcnt(0)"
+               : "=&v"(v)
+               : "v"(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) int*)p)))
+               : "memory");
+  return v;
+}
+
+// per: outputs of a group that lie side by side in y (experts: all n; heads: a head's); a.n: outputs of a row tile
+template <typename T, bool TRANS>
+__global__ __launch_bounds__(kWideThreads, 2) void group_gemm_wide_kernel(GroupGemmArgs a, int per) {
+  constexpr int kFull = 512 * kBK, kHalf = 384 * kBK;                  // an image: X rows | 256 W rows
+  __shared__ __attribute__((aligned(16))) uint16_t lds[3 * kHalf];
+  __shared__ int first[4][kWideMaxGroups + 1];                         // rows | tiles of 256 | of 128 beside them | of 128 alone
+  static_assert(3 * kHalf >= 2 * kFull, "one buffer for both kinds of tiles");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, kk = lane >> 4;
+  const int ntn = (a.n + 255) / 256, W = gridDim.x;
+  const bool experts = a.offsets != nullptr;
+  // without experts: groups of 1024 rows of the one matrix, whose tiles run side by side on an XCD
+  const int groups = experts ? a.groups : static_cast<int>((a.rows + 1023) >> 10);
+  int tiles[3];                                                        // row tiles of the three kinds
+  if (experts) {
+    if (wave == 0) {
+      int sum[3] = {0, 0, 0};
+      for (int base = 0; base < groups; base += 64) {
+        const int e = base + lane, c = e < groups ? e : groups - 1;
+        const int lo = MI355_LD(int32_t, a.offsets, a.offsets + c), hi = MI355_LD(int32_t, a.offsets, a.offsets + c + 1);
+        const int rows = e < groups ? hi - lo : 0, last = rows & 255;
+        int v[3] = {(rows >> 8) + (last > 128), last > 0 && last <= 128, (rows + 127) >> 7};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+#pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(v[q], o, 64);
+            if (lane >= o) v[q] += up;
+          }
+          v[q] += sum[q];
+          if (e < groups) first[1 + q][e + 1] = v[q];
+          sum[q] = __builtin_amdgcn_readlane(v[q], 63);
+        }
+        if (e < groups) first[0][e] = lo;
+        if (e == groups - 1) first[0][groups] = hi;
+      }
+      if (lane < 3) first[1 + lane][0] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 3; ++q) tiles[q] = __builtin_amdgcn_readfirstlane(first[1 + q][groups]);
+  } else {
+    const int rows = static_cast<int>(a.rows), last = rows & 255;
+    tiles[0] = (rows >> 8) + (last > 128), tiles[1] = last > 0 && last <= 128, tiles[2] = (rows + 127) >> 7;
+  }
+  // The plan of fewer rounds, in tiles of 128 rows (16 % slower by the row: 1269 against 1445 TFLOP/s in their steps):
+  // workgroups that have no tile of a last partial round take two of the small ones meanwhile.
+  bool halves;
+  {
+    const int f = tiles[0] * ntn, h = tiles[1] * ntn, part = f % W;
+    const int more = part > 0 ? max(h - 2 * (W - part), 0) : h;
+    const int mixed = 2 * ((f + W - 1) / W) + (more + W - 1) / W;
+    halves = 29 * ((tiles[2] * ntn + W - 1) / W) < 25 * mixed;
+  }
+  // XCD c takes the c-th contiguous part of the tiles, its workgroups in turn
+  const int nx = min(W, 8), xcd = blockIdx.x % nx, mine = blockIdx.x / nx, wgs = (W - xcd + nx - 1) / nx;
+  struct Tile {
+    int m0, hi, n0, g;
+  };
+  // tile u of kind q (1: 256 rows, 2: 128 rows beside them, 3: 128 rows alone): a group's row tiles in turn, then the next outputs
+  auto place = [&](int q, int u) {
+    Tile t;
+    const int size = q == 1 ? 256 : 128;
+    int at, n;                                                         // first row tile of the group, its number of them
+    if (experts) {
+      t.g = -1;
+      at = n = 0;
+      for (int base = 0; base < groups; base += 64) {                  // the group whose tiles hold u: the last that starts by it
+        const int e = min(base + lane, groups);
+        const int lo = wide_read_int(&first[q][e]);
+        const int c = __popcll(__ballot(base + lane < groups && lo * ntn <= u));
+        if (c > 0) t.g = base + c - 1, at = __builtin_amdgcn_readlane(lo, c - 1);
+        if (c < 64) break;
+      }
+      n = __builtin_amdgcn_readfirstlane(wide_read_int(&first[q][t.g + 1])) - at;
+      t.m0 = __builtin_amdgcn_readfirstlane(wide_read_int(&first[0][t.g]));
+      t.hi = __builtin_amdgcn_readfirstlane(wide_read_int(&first[0][t.g + 1]));
+    } else {
+      const int row_tiles = q == 2 ? tiles[1] : q == 1 ? tiles[0] : tiles[2], most = 1024 / size;
+      const int c = u / (most * ntn);
+      at = c * most, n = min(row_tiles - at, most);
+      t.g = 0, t.m0 = c << 10, t.hi = static_cast<int>(a.rows);
+    }
+    const int local = u - at * ntn;
+    t.n0 = local / n * 256;
+    // (a small tile beside large ones holds the group's last rows)
+    if (q == 2) t.m0 = t.m0 + ((t.hi - t.m0 - 1) & ~255);
+    else t.m0 += local % n * size;
+    return t;
+  };
+  const int r = tid >> 3;                                              // row of a 64-row piece this thread brings
+  const uint32_t sx = ((tid & 7) ^ ((r >> 1) & 7)) * 16, sw = ((tid & 7) ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) * 16;
+  const char* xb = reinterpret_cast<const char*>(a.x);
+  auto x_at = [&](const Tile& t, int row) {                            // byte offset of a row of the tile (past its end: its last)
+    int64_t p = t.m0 + row < t.hi ? t.m0 + row : t.hi - 1;
+    if (a.perm != nullptr) p = MI355_LD(int32_t, a.perm, a.perm + p) / a.top;
+    p = p < 0 ? 0 : (p >= a.x_rows ? a.x_rows - 1 : p);
+    return static_cast<uint32_t>(p * a.x_stride) * 2u + sx;
+  };
+  auto w_at = [&](const Tile& t, int row) {
+    const int n = t.n0 + row < a.n ? t.n0 + row : a.n - 1;
+    return static_cast<uint32_t>(n) * static_cast<uint32_t>(a.k) * 2u + sw;
+  };
+  auto w_base = [&](const Tile& t) { return reinterpret_cast<const char*>(a.w + t.g * a.w_group); };
+  const int steps = a.k / kBK;                                         // (two at least, no remainder)
+  const int rb = ((li >> 2) << 3) | (li & 3);                          // W row of this lane in a fragment
+  const int fx = (li >> 1) & 7, fw = ((rb >> 1) & 1) | (((rb >> 3) & 3) << 1), wn = (wave & 3) * 64;
+  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)lds));
+  f32x4 acc[2][4][4];
+  uint4 xf[2][4], wf[2][4];
+  auto clear = [&]() {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto products = [&](f32x4 (&c)[4][4]) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[i][j] = TRANS ? T::mfma(xf[ks][i], wf[ks][j], c[i][j]) : T::mfma(wf[ks][j], xf[ks][i], c[i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // results of the wave's 64 rows from m on; whole: no row or output past the end
+  auto emit = [&](const f32x4 (&c)[4][4], int m0, const Tile& t, bool whole) {
+    const int nb = t.n0 + wn, in = nb % per;                           // (a wave's 64 outputs lie in one group)
+    uint16_t* y = a.y + (t.g + nb / per) * a.y_group;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (TRANS) {                                                     // rows m .. m + 3 of output n
+        const int m = m0 + 16 * i + 4 * kk;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int n = (j >> 1) * 32 + (j & 1) * 4 + rb;
+          uint16_t* p = y + static_cast<int64_t>(m >> 4) * a.y_block + static_cast<int64_t>(in + n) * 16 + (m & 15);
+          const f32x4 v = c[i][j];
+          if (whole || (m + 3 < t.hi && nb + n < a.n)) {
+            MI355_ST(uint2, a.y, p, make_uint2(T::pack2(v[0], v[1]), T::pack2(v[2], v[3])));
+          } else if (nb + n < a.n) {
+            for (int e = 0; e < 4 && m + e < t.hi; ++e) MI355_ST(uint16_t, a.y, p + e, T::from_f(v[e]));
+          }
+        }
+      } else {                                                         // outputs n .. n + 7 of row m
+        const int m = m0 + 16 * i + li;
+        uint16_t* row = y + static_cast<int64_t>(m >> 4) * a.y_block + (m & 15) * a.y_stride + in;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          float v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            v[e] = c[i][2 * s + (e >> 2)][e & 3];
+            if (a.relu2) {                                             // (of the product as a 16-bit buffer would hold it)
+              v[e] = fmaxf(round_f<T>(v[e]), 0.f);
+              v[e] *= v[e];
+            }
+          }
+          const int n = s * 32 + kk * 8;
+          if (whole || (m < t.hi && nb + n < a.n)) MI355_ST(uint4, a.y, row + n, pack8<T>(v));
+        }
+      }
+    }
+  };
+  constexpr int S = TRANS ? 16 : 8;                                    // stores of 64 whole rows
+  if (!halves) {
+    const int total = tiles[0] * ntn, lo = static_cast<int>(static_cast<int64_t>(total) * xcd / nx),
+              end = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / nx);
+    int u = lo + mine;
+    if (u < end) {
+      const int wm = (wave >> 2) * 128;
+      const uint32_t x0 = base + ((wm + li) * kBK + ((kk ^ fx) << 3)) * 2, x1 = base + ((wm + li) * kBK + (((4 + kk) ^ fx) << 3)) * 2;
+      const uint32_t w0 = base + ((256 + wn + rb) * kBK + ((kk ^ fw) << 3)) * 2,
+                     w1 = base + ((256 + wn + rb) * kBK + (((4 + kk) ^ fw) << 3)) * 2;
+      uint32_t o1[6], o2[2];                                           // this thread's pieces: X rows 0 .. 63 of each 128 and W | the other X rows
+      const char* wb;
+      int at1 = 0, at2 = 0;
+      auto aim1 = [&](const Tile& t) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) o1[j] = x_at(t, j * 128 + r);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o1[2 + j] = w_at(t, j * 64 + r);
+        wb = w_base(t);
+        at1 = 0;
+      };
+      auto aim2 = [&](const Tile& t) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) o2[j] = x_at(t, 64 + j * 128 + r);
+        at2 = 0;
+      };
+      auto issue1 = [&](int img) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) lds_dma16(a.x, xb + at1 + o1[j], &lds[img * kFull + (j * 128 + wave * 8) * kBK]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lds_dma16(a.w, wb + at1 + o1[2 + j], &lds[img * kFull + (256 + j * 64 + wave * 8) * kBK]);
+        at1 += 2 * kBK;
+      };
+      auto issue2 = [&](int img) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) lds_dma16(a.x, xb + at2 + o2[j], &lds[img * kFull + (64 + j * 128 + wave * 8) * kBK]);
+        at2 += 2 * kBK;
+      };
+      Tile cur = place(1, u);
+      aim1(cur), aim2(cur);
+      issue1(0), issue2(0), issue1(1);
+      wait_vm<8>();
+      __builtin_amdgcn_s_barrier();
+      if (wave >= 4) __builtin_amdgcn_s_barrier();                     // the second group: a phase behind
+      int img = 0;
+      bool stored = false;                                             // 2 S stores went out ahead of the loads waited for
+      while (true) {
+        const bool more = u + wgs < end;
+        const Tile nxt = place(1, more ? u + wgs : u);                 // (none: loads that nobody reads)
+        clear();
+        for (int t = 0; t < steps; ++t) {
+          const uint32_t o = img * (kFull * 2);
+          wide_read_xw(x0 + o, x1 + o, w0 + o, w1 + o, xf, wf);
+          if (t == steps - 1) aim2(nxt);
+          issue2(img ^ 1);
+          if (stored) wait_vm<8 + 2 * S>(); else wait_vm<8>();
+          __builtin_amdgcn_s_barrier();
+          products(acc[0]);
+          __builtin_amdgcn_s_barrier();
+          wide_read_x(x0 + o, x1 + o, xf);
+          if (t == steps - 2) aim1(nxt);
+          issue1(img);
+          if (stored) wait_vm<8 + 2 * S>(); else wait_vm<8>();
+          stored = false;
+          __builtin_amdgcn_s_barrier();
+          products(acc[1]);
+          __builtin_amdgcn_s_barrier();
+          img ^= 1;
+        }
+        stored = cur.m0 + 256 <= cur.hi && cur.n0 + 256 <= a.n;
+        if (stored) emit(acc[0], cur.m0 + wm, cur, true), emit(acc[1], cur.m0 + wm + 64, cur, true);
+        else emit(acc[0], cur.m0 + wm, cur, false), emit(acc[1], cur.m0 + wm + 64, cur, false);
+        if (!more) break;
+        u += wgs, cur = nxt;
+      }
+      if (wave < 4) __builtin_amdgcn_s_barrier();
+      wait_vm<0>();                                                    // (the last loads into LDS: it is used again, or given back)
+      __builtin_amdgcn_s_barrier();
+    }
+  }
+  // ---- tiles of 128 x 256
+  const int kind = halves ? 3 : 2, total = tiles[kind - 1] * ntn;
+  const int lo = static_cast<int>(static_cast<int64_t>(total) * xcd / nx), end = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / nx);
+  int turn = mine;                                                     // first those that had one large tile less
+  if (!halves) {
+    const int f = tiles[0] * ntn;
+    const int had = static_cast<int>(static_cast<int64_t>(f) * (xcd + 1) / nx) - static_cast<int>(static_cast<int64_t>(f) * xcd / nx);
+    turn = (mine + wgs - had % wgs) % wgs;
+  }
+  int u = lo + turn;
+  if (u >= end) return;
+  const int wm = (wave >> 2) * 64;
+  const uint32_t x0 = base + ((wm + li) * kBK + ((kk ^ fx) << 3)) * 2, x1 = base + ((wm + li) * kBK + (((4 + kk) ^ fx) << 3)) * 2;
+  const uint32_t w0 = base + ((128 + wn + rb) * kBK + ((kk ^ fw) << 3)) * 2, w1 = base + ((128 + wn + rb) * kBK + (((4 + kk) ^ fw) << 3)) * 2;
+  uint32_t o1[6];
+  const char* wb;
+  int at1 = 0;
+  auto aim = [&](const Tile& t) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) o1[j] = x_at(t, j * 64 + r);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o1[2 + j] = w_at(t, j * 64 + r);
+    wb = w_base(t);
+    at1 = 0;
+  };
+  auto issue = [&](int img) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) lds_dma16(a.x, xb + at1 + o1[j], &lds[img * kHalf + (j * 64 + wave * 8) * kBK]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lds_dma16(a.w, wb + at1 + o1[2 + j], &lds[img * kHalf + (128 + j * 64 + wave * 8) * kBK]);
+    at1 += 2 * kBK;
+  };
+  Tile cur = place(kind, u);
+  aim(cur);
+  issue(0), issue(1);
+  wait_vm<6>();
+  __builtin_amdgcn_s_barrier();
+  if (wave >= 4) __builtin_amdgcn_s_barrier();
+  int img = 0;
+  bool stored = false;
+  while (true) {
+    const bool more = u + wgs < end;
+    const Tile nxt = place(kind, more ? u + wgs : u);
+    clear();
+    for (int t = 0; t < steps; ++t) {
+      const uint32_t o = img * (kHalf * 2);
+      wide_read_xw(x0 + o, x1 + o, w0 + o, w1 + o, xf, wf);
+      if (t == steps - 2) aim(nxt);
+      issue(img == 0 ? 2 : img - 1);                                   // step t + 2: what both groups have read of step t - 1
+      if (stored) wait_vm<6 + S>(); else wait_vm<6>();
+      stored = false;
+      __builtin_amdgcn_s_barrier();
+      products(acc[0]);
+      __builtin_amdgcn_s_barrier();
+      img = img == 2 ? 0 : img + 1;
+    }
+    stored = cur.m0 + 128 <= cur.hi && cur.n0 + 256 <= a.n;
+    if (stored) emit(acc[0], cur.m0 + wm, cur, true); else emit(acc[0], cur.m0 + wm, cur, false);
+    if (!more) break;
+    u += wgs, cur = nxt;
+  }
+  if (wave < 4) __builtin_amdgcn_s_barrier();
+  wait_vm<0>();
+}
+
+// The columns that follow every group's outputs, copied from the group's row of x (a.copy a multiple of 8)
+template <typename T>
+__global__ __launch_bounds__(256) void group_copy_kernel(GroupGemmArgs a) {
+  const int per = a.copy >> 3;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, m = i / per;
+  if (m >= a.rows) return;
+  int64_t row = a.perm != nullptr ? MI355_LD(int32_t, a.perm, a.perm + m) : m;
+  row = row < 0 ? 0 : (row >= a.x_rows ? a.x_rows - 1 : row);
+  const int c = static_cast<int>(i % per) * 8;
+  const uint4 v = MI355_LD(uint4, a.x, a.x + row * a.x_stride + a.k + c);
+  uint16_t* to = a.y + (m >> 4) * a.y_block + (m & 15) * a.y_stride + a.n + c;
+  for (int g = blockIdx.y; g < a.groups; g += gridDim.y) MI355_ST(uint4, a.y, to + g * a.y_group, v);
+}
+
+// What the wide tiles take: whole steps of K, 16-byte stores, byte offsets of 32 bits
+static bool wide_fits(const GroupGemmArgs& a, bool trans, bool experts) {
+  const int64_t w_rows = experts ? a.n : static_cast<int64_t>(a.n) * a.groups;
+  if (a.k % kBK != 0 || a.k < 2 * kBK || a.x_rows * a.x_stride * 2 >= (1ll << 32) || w_rows * a.k * 2 >= (1ll << 32) || a.rows >= (1 << 30) ||
+      w_rows >= (1 << 30))
+    return false;
+  if (a.n % 8 != 0 || a.y_stride % 8 != 0 || a.y_block % 8 != 0 || a.y_group % 8 != 0) return false;
+  if (experts) return a.groups <= kWideMaxGroups;
+  return a.x_group == 0 && a.n % 64 == 0 && a.w_group == static_cast<int64_t>(a.n) * a.k && (!trans || a.copy == 0);
+}
+
+// Where the wide tiles are the faster ones (bf16, us, 128 x 128 tiles / wide; 12 and less are the host's).  They need about
+// half a round of 128 x 128 tiles on two workgroups a CU: 32 experts 512 -> 512 of 200 rows 13.7 / 15.6, of 384 rows 18.9 / 17.4,
+// 8 experts 512 -> 1536 of 200 rows 13.4 / 16.0, of 384 17.6 / 16.7, 2048 -> 4096 of 128 rows 42 / 33.  Experts of few rows stream their
+// weights, and a tile's 128 rows then are mostly padding: 32 experts 2048 -> 4096 of 64 rows 123 / 132, of 128 rows 172 / 154; 128
+// experts 2048 -> 512 of 128 rows 94 / 110, of 200 rows 104 / 95.  Outputs that fill little of their last 256 lose it again:
+// 32 experts 2048 -> 320 of 1030 rows 78 / 80.  Heads (16 of 512 -> 128, with 64 copied columns, which are a launch of their own
+// here): 2000 rows 16.0 / 17.8, 3000 20.1 / 19.4, 8224 48.8 / 40.9; of 128 inputs 4000 rows 14.4 / 18.0.
+static bool wide_pays(const GroupGemmArgs& a, bool experts) {
+  const int64_t n = experts ? a.n : static_cast<int64_t>(a.n) * a.groups;
+  if (4 * ((n + 255) & ~255ll) > 5 * n) return false;
+  if (!experts) return a.k >= 256 && a.rows * n >= 384ll * 128 * 128;
+  return a.rows >= (a.groups <= 64 ? 96ll : 160ll) * a.groups && (a.rows + 64ll * a.groups) * n >= 288ll * 128 * 128;
+}
+
 template <typename T>
 static void launch_group_gemm(const GroupGemmArgs& a, bool trans, int64_t tiles_m, int bm, hipStream_t s) {
+  const bool experts = a.offsets != nullptr;
+  if (bm == 128 && wide_fits(a, trans, experts) && wide_pays(a, experts)) {
+    GroupGemmArgs b = a;
+    if (!experts) b.n = a.n * a.groups, b.groups = 1;
+    const int64_t most = (a.rows / 128 + b.groups) * ((b.n + 255) / 256);
+    const dim3 grid(static_cast<unsigned>(most < 256 ? most : 256));
+    if (trans) hipLaunchKernelGGL((group_gemm_wide_kernel<T, true>), grid, dim3(kWideThreads), 0, s, b, a.n);
+    else hipLaunchKernelGGL((group_gemm_wide_kernel<T, false>), grid, dim3(kWideThreads), 0, s, b, a.n);
+    if (a.copy > 0)
+      hipLaunchKernelGGL(group_copy_kernel<T>, dim3(static_cast<unsigned>((a.rows * (a.copy >> 3) + 255) / 256), 2), dim3(256), 0, s, a);
+    return;
+  }
 #define MI355_GG(BM, BN, MW, TR)                                                                                   \
   hipLaunchKernelGGL((group_gemm_kernel<T, BM, BN, MW, TR>), dim3(static_cast<unsigned>(tiles_m * ((a.n + BN - 1) / BN))), \
                      dim3(256), 0, s, a)
