@@ -654,6 +654,52 @@ def test_sample_spread_over_workgroups(ops, ldt, B, V):
     np.testing.assert_array_equal(ops.sample(wide[:, :V], *args, cut_rows=False).cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("B,V", [(1, 16384), (16, 70001), (17, 33333), (63, 16389), (64, 152064), (9, 5), (40, 64), (5, 262144)])
+def test_sample_from_counts_of_values(ops, monkeypatch, B, V):
+    """bfloat16 rows counted by value, against the launches per eight key bits (a workspace of the size those need) and the
+    restatement: rows of nearly all values there are, of one value, of ties past what a workgroup lists, NaN and
+    infinities, cuts by top-k alone, by top-p alone and by both, vocabularies that end inside a vector."""
+    from mi355_decode._lib import lib
+    monkeypatch.setattr(ops, "SAMPLE_SPREAD_VOCAB", 0)
+    rng = np.random.default_rng(V + B)
+    lg = torch.from_numpy((12 - 1.5 * np.log(rng.integers(1, V + 1, (B, V))) + 0.5 * rng.normal(size=(B, V))).astype(np.float32)).bfloat16()
+    top_k, top_p = rng.choice([0, 1, 40, 5000], B).astype(np.int32), rng.choice([1.0, 0.95, 0.4, 1e-6], B).astype(np.float32)
+    temperature = rng.choice([0.0, 0.7, 1.0, 30.0], B, p=[0.1, 0.3, 0.3, 0.3]).astype(np.float32)
+    for r in range(B):
+        kind = (r + B) % 8
+        if kind == 0:                                       # values of every size and sign (their differences in mass: temperature)
+            lg[r] = torch.from_numpy(np.arange(V, dtype=np.int64) * 40503 % 65536).to(torch.int32).to(torch.int16).view(torch.bfloat16)
+            lg[r][lg[r].isnan()] = 0.5
+            lg[r][lg[r].abs() > 3e38] = -0.0
+            temperature[r] = 1e38
+        elif kind == 1:
+            lg[r] = 1.5
+        elif kind == 2:
+            lg[r] = torch.from_numpy(rng.choice([0.0, -0.0, 2.0], V).astype(np.float32)).bfloat16()
+            top_k[r], top_p[r] = 0, 0.6
+        elif kind == 3:
+            lg[r, rng.integers(0, V, 3)] = float("nan")
+        elif kind == 4:
+            lg[r] = -float("inf")
+            lg[r, V // 2:] = -1.0
+        elif kind == 5:
+            lg[r, -1] = float("inf")
+    seeds, steps = rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B, dtype=np.int64)
+    wide = torch.zeros(B, (V + 7) // 8 * 8, dtype=torch.bfloat16, device="cuda")
+    wide[:, :V] = lg.cuda()
+    args = [torch.from_numpy(a).cuda() for a in (temperature, top_k, top_p, seeds, steps)]
+    ws = torch.full((lib.mi355_sample_workspace(B, 0),), 0xA5, dtype=torch.uint8, device="cuda")
+    passes = torch.empty(8 * (B * (32 + 4 * 256) + (2048 + B) * 256), dtype=torch.uint8, device="cuda")
+    if B * V < 3_000_000:
+        np.testing.assert_array_equal(ops.sample(wide[:, :V], *args, workspace=ws).cpu().numpy(),
+                                      R.sample_topk_topp(lg.float().numpy(), temperature, top_k, top_p, seeds, steps))
+    for _ in range(2):                                      # (what a call leaves in the workspace is of no account to the next)
+        got = ops.sample(wide[:, :V], *args, workspace=ws)
+        assert torch.equal(got, ops.sample(wide[:, :V], *args, cut_rows=False))
+    if passes.numel() < ws.numel():
+        assert torch.equal(got, ops.sample(wide[:, :V], *args, workspace=passes))
+
+
 @pytest.mark.parametrize("ldt,B", [("bfloat16", 32), ("bfloat16", 33), ("float16", 5), ("float32", 5)])
 def test_sample_of_short_cuts_is_the_same_either_way(ops, ldt, B):
     """The caller's word that every cut is short moves rows to another way through the sampler and no token."""

@@ -1247,9 +1247,9 @@ __global__ void sample_finish_kernel(int64_t* __restrict__ out, const float* __r
 // range into *key (of `buffer`, cleared ahead) with a 64-bit atomic max -- order-free, so the same on every launch -- and a
 // later launch turns it into the index.
 template <int LDT>
-__device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, const void* base, int vocab, bool greedy, float temp,
-                                                    uint64_t seed, uint64_t step, int range, int ranges, int chunk_vecs,
-                                                    unsigned long long* part, const void* buffer) {
+__device__ __forceinline__ unsigned long long sample_one_key_best(const void* base, int vocab, bool greedy, float temp, uint64_t seed,
+                                                                  uint64_t step, int range, int ranges, int chunk_vecs,
+                                                                  unsigned long long* part) {
   const int v0 = range * chunk_vecs, v1 = v0 + chunk_vecs;
   const bool tail = range == ranges - 1;
   unsigned long long best = 0ull;
@@ -1258,7 +1258,13 @@ __device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, con
                               [&](float f, int i) { best = umax64(best, argmax_key(f, static_cast<uint32_t>(i))); });
   else
     best = sample_full_vocab<LDT>(base, vocab, v0, v1, tail, temp, seed, step);
-  best = sample_reduce_max(best, part);
+  return sample_reduce_max(best, part);                   // (thread 0)
+}
+template <int LDT>
+__device__ __forceinline__ void sample_one_key_pass(unsigned long long* key, const void* base, int vocab, bool greedy, float temp,
+                                                    uint64_t seed, uint64_t step, int range, int ranges, int chunk_vecs,
+                                                    unsigned long long* part, const void* buffer) {
+  const unsigned long long best = sample_one_key_best<LDT>(base, vocab, greedy, temp, seed, step, range, ranges, chunk_vecs, part);
   if (threadIdx.x == 0 && best != 0ull && MI355_OK_AT(buffer, key, 8)) atomicMax(key, best);
 }
 
@@ -1327,6 +1333,356 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
     unsigned long long* bin = ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead + static_cast<int64_t>(row) * 2 * ExactLevels<LDT>::NL * 256 + tid;
     if (MI355_OK_AT(ws, bin, 8)) atomicAdd(bin, hist[tid]);
   }
+}
+
+// ---- bf16 logits with a caller's workspace: three launches.  A 16-bit logit has 65536 values, so a row is its counts of
+// them, and everything a cut needs -- the k-th largest key, the mass of what is left (a value's mass times its count), the
+// key at which the nucleus ends -- follows from the counts without another look at the row:
+//   sample_count   a workgroup per (row, part of its columns) counts its logits by key in LDS (65536 counters of 16 bits)
+//                  and writes the lines of 32 counters that hold any, with a byte a line that says so
+//   sample_pick    a workgroup a row adds up the counts of all parts (a few hundred lines: a trained model's logits have
+//                  some thousand values) and selects by prefix sums
+//   sample_draw    every row spread over many workgroups, those without a cut too (their pass is arithmetic: two logarithms a
+//                  logit); the last one to end turns the row's best key into the token
+// What bounds the launch per eight key bits (exact_hist_kernel) is the launches: seven for bf16, each of 3 to 12 us for a pass of
+// about 1 us.  32 rows of 128256 logits with a mix of cuts: 40 us a call that way, here 26 (count 6.5, pick 9, draw 10); top-p
+// alone 42 / 26, top-k of 50 alone 31 / 19; 4 rows 30 / 21, 64 rows 51 / 35, 32 rows of 32000 31 / 21; nowhere slower, 1 to 64 rows.
+// fp16 keeps the passes: its rows have some ten thousand values, and the pick then takes them in several batches (16 rows
+// with a top-p 38 us by passes, 48 by counts).
+constexpr int kCountRows = 64;                              // rows up to which a row has four parts and more
+constexpr int kCountParts = 16;                             // most parts of a row
+constexpr int kCountLines = 2048;                           // lines of 32 counters, 64 bytes each
+// parts of a row: 256 workgroups (a CU holds one: 128 KB of counters)
+__host__ __device__ __forceinline__ int count_parts(int rows) { return rows >= 64 ? 4 : rows <= 16 ? kCountParts : 256 / rows; }
+// workspace, in 64-bit words: [rows] x 32 (the draw's key at 0, the cut's key and how many tokens with it stay at 1 and 2,
+// such tokens ahead of every part (32 bits each) from 3 on, workgroups done at 16) | flags [rows][parts][2048 bytes] |
+// counters [rows][parts][65536] of 16 bits
+__host__ __device__ __forceinline__ int64_t count_ws_words(int64_t rows) {
+  return rows * (kSampleWsHead + count_parts(static_cast<int>(rows)) * static_cast<int64_t>(kCountLines / 8 + 16384));
+}
+
+// the order-preserving key of a 16-bit logit (a NaN on top, -0 as +0), and back to its 32-bit key
+template <int LDT>
+__device__ __forceinline__ uint32_t key16(uint32_t raw) {
+  if ((raw & 0x7FFFu) > (LDT == MI355_BF16 ? 0x7F80u : 0x7C00u)) return 0xFFFFu;
+  if (raw == 0x8000u) raw = 0u;
+  return raw & 0x8000u ? ~raw & 0xFFFFu : raw | 0x8000u;
+}
+template <int LDT>
+__device__ __forceinline__ float key16_logit(uint32_t key) {
+  const uint16_t raw = static_cast<uint16_t>(key & 0x8000u ? key ^ 0x8000u : ~key);
+  return LDT == MI355_BF16 ? BF16::to_f(raw) : F16::to_f(raw);
+}
+
+template <int LDT>
+__global__ __launch_bounds__(kSampleThreads) void sample_count_kernel(
+    unsigned long long* __restrict__ ws, const uint16_t* __restrict__ logits, int64_t stride, int vocab,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int part_vecs) {
+  __shared__ __attribute__((aligned(16))) uint32_t counts[32768];      // two keys a word
+  const int row = blockIdx.y, part = blockIdx.x, parts = gridDim.x, tid = threadIdx.x, lane = tid & 63;
+  if (part == 0 && tid == 0) {
+    unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
+    MI355_ST(unsigned long long, ws, head, 0ull);
+    MI355_ST(unsigned long long, ws, head + 16, 0ull);
+  }
+  if (sample_one_key(MI355_LD(float, temperature, temperature + row), active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab),
+                     MI355_LD(float, top_p, top_p + row)))
+    return;
+  const uint16_t* base = logits + row * stride;
+  const int v0 = part * part_vecs, v1 = min(v0 + part_vecs, vocab >> 3);
+  auto count = [&](uint32_t raw) {
+    const uint32_t k = key16<LDT>(raw);
+    atomicAdd(&counts[k >> 1], 1u << ((k & 1u) * 16u));                // (a part has fewer than 65536 logits)
+  };
+  for (int i = tid; i < 8192; i += kSampleThreads) reinterpret_cast<uint4*>(counts)[i] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  for (int v = v0 + tid; v < v1; v += kSampleThreads) {
+    const uint4 raw = MI355_LD(uint4, logits, base + 8 * v);
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) count(w[j] & 0xFFFFu), count(w[j] >> 16);
+  }
+  if (part == parts - 1)
+    for (int i = (vocab & ~7) + tid; i < vocab; i += kSampleThreads) count(MI355_LD(uint16_t, logits, base + i));
+  __syncthreads();
+  uint8_t* flags = reinterpret_cast<uint8_t*>(ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead) +
+                   (static_cast<int64_t>(row) * parts + part) * kCountLines;
+  unsigned long long* lines = ws + static_cast<int64_t>(gridDim.y) * (kSampleWsHead + parts * (kCountLines / 8)) +
+                              (static_cast<int64_t>(row) * parts + part) * 16384;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {                                        // four lanes a line
+    const int piece = tid + kSampleThreads * j;
+    const uint4 c = reinterpret_cast<const uint4*>(counts)[piece];
+    const unsigned long long any = __ballot((c.x | c.y | c.z | c.w) != 0u);
+    const bool used = ((any >> (lane & ~3)) & 15ull) != 0ull;
+    if (used) MI355_ST(uint4, ws, lines + 2 * piece, c);
+    if ((lane & 3) == 0) MI355_ST(uint8_t, ws, flags + (piece >> 2), static_cast<uint8_t>(used));
+  }
+}
+
+// Inclusive prefix sum over the workgroup (16 waves), and the whole sum.  scratch: 16 words; all threads call it.
+__device__ __forceinline__ unsigned long long block_scan64(unsigned long long v, unsigned long long* scratch, unsigned long long& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  v = wave_scan64(v, [](unsigned long long a, unsigned long long b) { return a + b; });
+  __syncthreads();                                                     // scratch may still be read from a previous call
+  if (lane == 63) scratch[wave] = v;
+  __syncthreads();
+  unsigned long long before = 0ull;
+  total = 0ull;
+#pragma unroll
+  for (int w = 0; w < kSampleThreads / 64; ++w) {
+    const unsigned long long s = scratch[w];
+    if (w < wave) before += s;
+    total += s;
+  }
+  return v + before;
+}
+
+template <int LDT>
+__global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(
+    unsigned long long* __restrict__ ws, int parts, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const float* __restrict__ top_p) {
+  __shared__ unsigned long long scratch[kSampleThreads / 64], found[2];
+  __shared__ uint16_t used[kCountLines];                               // the row's lines that hold any, from the highest keys down
+  const int row = blockIdx.x, tid = threadIdx.x;
+  unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
+  const uint8_t* flags = reinterpret_cast<const uint8_t*>(ws + static_cast<int64_t>(gridDim.x) * kSampleWsHead) +
+                         static_cast<int64_t>(row) * parts * kCountLines;
+  const uint16_t* counters = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(gridDim.x) * (kSampleWsHead + parts * (kCountLines / 8))) +
+                             static_cast<int64_t>(row) * parts * 65536;
+  // lines in use, highest first: thread t looks at lines 2047 - 2t and 2046 - 2t
+  const int hi = kCountLines - 1 - 2 * tid;
+  uint32_t mine = 0u;
+#pragma unroll
+  for (int c = 0; c < kCountParts; ++c) mine |= MI355_LD(uint16_t, ws, flags + (c < parts ? c : 0) * kCountLines + hi - 1);
+  const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
+  if (sample_one_key(temp, K1, tp)) return;                            // (its flags were not written)
+  unsigned long long lines, at = block_scan64((mine >> 8 & 1u) + (mine & 1u), scratch, lines);
+  if (mine & 1u) used[--at] = static_cast<uint16_t>(hi - 1);
+  if (mine >> 8 & 1u) used[--at] = static_cast<uint16_t>(hi);
+  __syncthreads();
+  const int items = static_cast<int>(lines) * 4;                       // an item: 8 keys of a line
+  // The counts of an item by key, highest first; its highest key.  No branch around a load: all of eight parts' are on
+  // their way together (a line that a part has not written holds anything: its flag clears it).
+  auto load_item = [&](int item, uint32_t (&n)[8]) -> uint32_t {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) n[e] = 0u;
+    if (item >= items) return 0u;
+    const int line = used[item >> 2], piece = line * 4 + 3 - (item & 3);
+    for (int c0 = 0; c0 < parts; c0 += 8) {
+      uint4 q[8];
+      uint32_t on[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int c = c0 + j < parts ? c0 + j : parts - 1;
+        on[j] = MI355_LD(uint8_t, ws, flags + c * kCountLines + line);
+        q[j] = MI355_LD(uint4, ws, counters + c * 65536 + piece * 8);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t keep = on[j] != 0u && c0 + j < parts ? 0xFFFFFFFFu : 0u;
+        const uint32_t w[4] = {q[j].w & keep, q[j].z & keep, q[j].y & keep, q[j].x & keep};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) n[2 * e] += w[e] >> 16, n[2 * e + 1] += w[e] & 0xFFFFu;
+      }
+    }
+    return static_cast<uint32_t>(piece * 8 + 7);
+  };
+  uint32_t n[8];
+  uint32_t top = load_item(tid, n);
+  auto sum8 = [&]() { return static_cast<unsigned long long>(n[0] + n[1] + n[2] + n[3] + n[4] + n[5] + n[6] + n[7]); };
+  // batches of 1024 items (one, unless the row has more than 8192 values' worth of lines)
+  auto batch = [&](int b) {
+    if (items > kSampleThreads) top = load_item(b * kSampleThreads + tid, n);
+  };
+  const int batches = (items + kSampleThreads - 1) / kSampleThreads;
+  if (tid < 64) {                                                      // the row's largest key: of its first line's four items
+    uint32_t k = 0u;
+#pragma unroll
+    for (int e = 7; e >= 0; --e) k = n[e] != 0u ? top - e : k;
+    const unsigned long long most = wave_max64(k);
+    if (tid == 0) found[0] = most;
+  }
+  __syncthreads();
+  const uint32_t best_key = static_cast<uint32_t>(found[0]);
+  const float l0 = key16_logit<LDT>(best_key);
+  uint32_t Tk = 0u;                                                    // keys of 16 bits
+  if (K1 > 0) {
+    const unsigned long long need = static_cast<unsigned long long>(K1);
+    unsigned long long carry = 0ull;
+    for (int b = 0; b < batches; ++b) {
+      batch(b);
+      unsigned long long total, end = block_scan64(sum8(), scratch, total) + carry, run = end - sum8();
+      if (run < need && need <= end) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (run < need && run + n[e] >= need) found[1] = top - e;
+          run += n[e];
+        }
+      }
+      carry += total;
+      if (carry >= need) break;
+    }
+    __syncthreads();
+    Tk = static_cast<uint32_t>(found[1]);
+    __syncthreads();
+  }
+  uint32_t Tp = Tk;
+  unsigned long long take = ~0ull;
+  if (tp < 1.0f) {
+    unsigned long long m[8], sum, Z = 0ull, end = 0ull;
+    auto masses = [&]() {
+      sum = 0ull;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        m[e] = n[e] != 0u && top - e >= Tk ? n[e] * sample_mass(key16_logit<LDT>(top - e), l0, temp) : 0ull;
+        sum += m[e];
+      }
+    };
+    for (int b = 0; b < batches; ++b) {
+      batch(b);
+      masses();
+      unsigned long long total;
+      end = block_scan64(sum, scratch, total);
+      Z += total;
+    }
+    const unsigned long long P = mass_threshold(tp, Z);
+    unsigned long long carry = 0ull;
+    for (int b = 0; b < batches; ++b) {
+      unsigned long long total = Z;
+      if (batches > 1) {
+        batch(b);
+        masses();
+        end = block_scan64(sum, scratch, total);
+      }
+      unsigned long long run = carry + end - sum;
+      if (run < P && P <= carry + end) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (run < P && run + m[e] >= P) found[0] = P - run, found[1] = top - e;
+          run += m[e];
+        }
+      }
+      carry += total;
+      if (carry >= P) break;
+    }
+    __syncthreads();
+    Tp = static_cast<uint32_t>(found[1]);
+    const unsigned long long need = found[0], Fp = sample_mass(key16_logit<LDT>(Tp), l0, temp);
+    take = Fp > 0ull ? (need + Fp - 1ull) / Fp : ~0ull;
+  }
+  if (tid == 0) {
+    // (a NaN: everything stays, and the draw's first pass is the greedy one)
+    MI355_ST(unsigned long long, ws, head + 1, best_key == 0xFFFFu ? 0xFFFFull : static_cast<unsigned long long>(Tp));
+    MI355_ST(unsigned long long, ws, head + 2, take);
+  }
+  if (take != ~0ull && tid < 64) {                                     // tokens at the cut key in the parts ahead of each
+    unsigned long long c = 0ull;
+    if (tid < parts && MI355_LD(uint8_t, ws, flags + tid * kCountLines + (Tp >> 5)) != 0) c = MI355_LD(uint16_t, ws, counters + tid * 65536 + Tp);
+    const unsigned long long upto = wave_scan64(c, [](unsigned long long x, unsigned long long y) { return x + y; });
+    if (tid < parts) MI355_ST(uint32_t, ws, reinterpret_cast<uint32_t*>(head + 3) + tid, static_cast<uint32_t>(upto - c));
+  }
+}
+
+template <int LDT>
+__global__ __launch_bounds__(kSampleWsThreads) void sample_draw_kernel(
+    int64_t* __restrict__ out, unsigned long long* __restrict__ ws, const uint16_t* __restrict__ logits, int64_t stride, int vocab,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
+    const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps, int part_vecs, int chunk_vecs) {
+  __shared__ unsigned long long part_best[kSampleThreads / 64];
+  __shared__ int eq_base[kSampleThreads / 64 + 1], ties[2], listed[kSampleWsThreads];
+  const int row = blockIdx.y, range = blockIdx.x, ranges = gridDim.x, tid = threadIdx.x;
+  const float temp = MI355_LD(float, temperature, temperature + row);
+  const uint64_t seed = static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)), step = static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row));
+  const uint16_t* base = logits + row * stride;
+  unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
+  const bool one = sample_one_key(temp, active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab), MI355_LD(float, top_p, top_p + row));
+  const uint32_t Tp = static_cast<uint32_t>(MI355_LD(unsigned long long, ws, head + 1));       // (written for rows with a cut)
+  unsigned long long best = 0ull;
+  if (one || Tp == 0xFFFFu) {
+    best = sample_one_key_best<LDT>(base, vocab, !one || !(temp > 0.0f), temp, seed, step, range, ranges, chunk_vecs, part_best);
+  } else {
+    const unsigned long long take = MI355_LD(unsigned long long, ws, head + 2);
+    const int v0 = range * chunk_vecs, v1 = min(v0 + chunk_vecs, vocab >> 3);
+    const uint32_t row_hash = sample_hash(seed, step);
+    // one look: what stays for sure is drawn, the cut key's tokens are listed
+    if (tid < 2) ties[tid] = 0;
+    __syncthreads();
+    auto look = [&](uint32_t raw, int i) {
+      const uint32_t k = key16<LDT>(raw);
+      if (k > Tp || (k == Tp && take == ~0ull)) {
+        best = umax64(best, gumbel_key(key16_logit<LDT>(k), static_cast<uint32_t>(i), temp, row_hash));
+      } else if (k == Tp) {
+        const int at = atomicAdd(&ties[0], 1);
+        if (at < kSampleWsThreads) listed[at] = i;
+      }
+    };
+    for (int v = v0 + tid; v < v1; v += kSampleWsThreads) {
+      const uint4 raw = MI355_LD(uint4, logits, base + 8 * v);
+      const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) look(w[j] & 0xFFFFu, 8 * v + 2 * j), look(w[j] >> 16, 8 * v + 2 * j + 1);
+    }
+    if (range == ranges - 1)
+      for (int i = (vocab & ~7) + tid; i < vocab; i += kSampleWsThreads) look(MI355_LD(uint16_t, logits, base + i), i);
+    __syncthreads();
+    const int num = ties[0];
+    if (num > 0) {                                                     // ranked: behind those of the part ahead of this range
+      // (the vectors past the row's last whole one belong to the last part, wherever this range begins)
+      const int part = min(v0 / part_vecs, count_parts(gridDim.y) - 1);
+      int c = 0;
+#pragma unroll 4
+      for (int v = part * part_vecs + tid; v < v0; v += kSampleWsThreads) {
+        const uint4 raw = MI355_LD(uint4, logits, base + 8 * v);
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c += (key16<LDT>(w[j] & 0xFFFFu) == Tp) + (key16<LDT>(w[j] >> 16) == Tp);
+      }
+      if (c != 0) atomicAdd(&ties[1], c);
+      __syncthreads();
+      const unsigned long long before = static_cast<unsigned long long>(ties[1]) + MI355_LD(uint32_t, ws, reinterpret_cast<const uint32_t*>(head + 3) + part);
+      const float l = key16_logit<LDT>(Tp);
+      if (num <= kSampleWsThreads) {
+        if (tid < num) {
+          const int i = listed[tid];
+          unsigned long long rank = before;
+          for (int j = 0; j < num; ++j) rank += listed[j] < i ? 1 : 0;
+          if (rank < take) best = umax64(best, gumbel_key(l, static_cast<uint32_t>(i), temp, row_hash));
+        }
+      } else if (before < take) {
+        ordered_kept_pass<LDT>(base, vocab, v0, v0 + chunk_vecs, range == ranges - 1, sample_key(l), take, before, eq_base, [&](float f, int i) {
+          best = umax64(best, gumbel_key(f, static_cast<uint32_t>(i), temp, row_hash));
+        });
+      }
+      __syncthreads();
+    }
+    best = sample_reduce_max(best, part_best);
+  }
+  if (tid == 0 && MI355_OK_AT(ws, head, 8) && MI355_OK_AT(ws, head + 16, 8)) {
+    // The key is in memory when its atomic's answer is here, so that the count that follows needs no fence (a fence of
+    // the device writes a whole L2 back: 38 us for the 2000 workgroups of 32 rows, here 12).
+    const unsigned long long was = atomicMax(head, best);
+    asm volatile("s_waitcnt vmcnt(0)" ::"v"(was) : "memory");
+    if (atomicAdd(head + 16, 1ull) == static_cast<unsigned long long>(ranges) - 1ull) {
+      const unsigned long long b = atomicMax(head, 0ull);
+      MI355_ST(int64_t, out, out + row, static_cast<int64_t>(0xFFFFFFFFu - static_cast<uint32_t>(b & 0xFFFFFFFFull)));
+    }
+  }
+}
+
+template <int LDT>
+static int32_t launch_counted(const char* name, int64_t* out, unsigned long long* ws, const void* logits, int64_t stride, int rows, int vocab,
+                              const float* temperature, const int32_t* top_k, const float* top_p, const int64_t* seeds, const int64_t* steps,
+                              int chunks, int chunk_vecs, hipStream_t s) {
+  const int parts = count_parts(rows), part_vecs = ((vocab >> 3) + parts - 1) / parts + (vocab < 8);
+  const uint16_t* p = static_cast<const uint16_t*>(logits);
+  hipLaunchKernelGGL((sample_count_kernel<LDT>), dim3(parts, rows), dim3(kSampleThreads), 0, s, ws, p, stride, vocab, temperature, top_k, top_p,
+                     part_vecs);
+  hipLaunchKernelGGL((sample_pick_kernel<LDT>), dim3(rows), dim3(kSampleThreads), 0, s, ws, parts, vocab, temperature, top_k, top_p);
+  hipLaunchKernelGGL((sample_draw_kernel<LDT>), dim3(chunks, rows), dim3(kSampleWsThreads), 0, s, out, ws, p, stride, vocab, temperature, top_k,
+                     top_p, seeds, steps, part_vecs, chunk_vecs);
+  return check_launch(name);
 }
 
 template <int LDT>
@@ -1716,11 +2072,17 @@ extern "C" int32_t mi355_sample_topk_topp_hinted(int64_t* out_ids, const void* l
                              logits_dtype, temperature, top_k, top_p, seeds, steps, cut_rows, stream);
 }
 
+static int64_t sample_passes_bytes(int64_t rows, int stages) {
+  return 8 * (mi355::sample_ws_words(rows, stages) + (mi355::kSampleWsGroups + rows) * 256);
+}
+
 extern "C" int64_t mi355_sample_workspace(int32_t num_rows, int32_t logits_dtype) {
   using namespace mi355;
   const int stages = 2 * (logits_dtype == MI355_F32 ? ExactLevels<MI355_F32>::NL : logits_dtype == MI355_BF16 ? ExactLevels<MI355_BF16>::NL
                                                                                                              : ExactLevels<MI355_F16>::NL);
-  return num_rows > 0 ? 8 * (sample_ws_words(num_rows, stages) + (static_cast<int64_t>(kSampleWsGroups) + num_rows) * 256) : 0;
+  if (num_rows <= 0) return 0;
+  const int64_t passes = sample_passes_bytes(num_rows, stages);
+  return logits_dtype == MI355_BF16 && num_rows <= kCountRows && 8 * count_ws_words(num_rows) > passes ? 8 * count_ws_words(num_rows) : passes;
 }
 
 extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logits, int64_t logits_stride, int32_t num_rows,
@@ -1732,7 +2094,9 @@ extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logit
   MI355_REQUIRE(temperature && top_k && top_p && seeds && steps, MI355_ERR_INVALID, "%s: null pointer", name);
   const int32_t rc = check_logits(name, out_ids, logits, logits_stride, num_rows, vocab, logits_dtype, 0);
   if (rc != MI355_OK || num_rows == 0) return rc;
-  const int64_t need = mi355_sample_workspace(num_rows, logits_dtype);
+  const int stages = 2 * (logits_dtype == MI355_F32 ? ExactLevels<MI355_F32>::NL : logits_dtype == MI355_BF16 ? ExactLevels<MI355_BF16>::NL
+                                                                                                             : ExactLevels<MI355_F16>::NL);
+  const int64_t need = sample_passes_bytes(num_rows, stages);
   MI355_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), MI355_ERR_INVALID,
                 "%s: workspace of %lld bytes, %lld needed, 16-byte aligned", name, static_cast<long long>(workspace_bytes),
                 static_cast<long long>(need));
@@ -1744,6 +2108,12 @@ extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logit
   chunks = chunks > 64 ? 64 : chunks;
   const int chunk_vecs = ((nvec + chunks * kSampleWsThreads - 1) / (chunks * kSampleWsThreads) + (nvec == 0)) * kSampleWsThreads;
   chunks = nvec > chunk_vecs ? (nvec + chunk_vecs - 1) / chunk_vecs : 1;
+  // counts of 16 bits (a part of a row: at most 65535 logits), and room for them
+  if (logits_dtype == MI355_BF16 && num_rows <= kCountRows && workspace_bytes >= 8 * count_ws_words(num_rows) &&
+      ((vocab >> 3) / count_parts(num_rows) + 2) * 8 <= 65535) {
+    return launch_counted<MI355_BF16>(name, out_ids, ws, logits, logits_stride, num_rows, vocab, temperature, top_k, top_p, seeds, steps, chunks,
+                                      chunk_vecs, s);
+  }
   const int64_t words = sample_ws_words(num_rows, 2 * (logits_dtype == MI355_F32 ? 4 : logits_dtype == MI355_BF16 ? 2 : 3));
   const int64_t threads = words / 2;                     // (two words each)
   hipLaunchKernelGGL(sample_clear_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s, ws, words);

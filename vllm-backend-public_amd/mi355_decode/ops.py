@@ -608,7 +608,8 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
 #   top-k of 50 alone                 bfloat16 64 rows 30 / 33, 40 / 44; float16 42 rows 31 / 36, 42 / 47; float32 16 rows 34 / 40, 41 / 54
 #   top-k of 40 and top-p             bfloat16 32 rows 34 / 33, 45 / 44, 64 rows 42 / 33, 62 / 44; float16 4 rows 37 / 35, 42 / 46,
 #                                     42 rows 49 / 36, 65 / 47; float32 4 rows 46 / 40, 53 / 53, 32 rows 80 / 41, 100 / 54
-# (of 256 and top-p: bfloat16 64 rows 44 / 41, 64 / 54).  A workgroup each is slow where it has to add up the masses of a whole row;
+# (of 256 and top-p: bfloat16 64 rows 44 / 41, 64 / 54).  bfloat16 rows have since been counted by value instead (a mix of cuts
+# 32 rows 21 / 60 at 32000 logits, 26 / 97 at 128256, 64 rows 24 / 60, 35 / 99; top-k of 40 and top-p 32 rows 27 / 44).  A workgroup each is slow where it has to add up the masses of a whole row;
 # where every row's top-k leaves it a short list, the spread form's passes for the top-p are what costs: a caller that
 # knows so says it, and only bfloat16 batches of up to 32 rows are then spread.
 SAMPLE_SPREAD_PASSES, SAMPLE_SPREAD_VOCAB, SAMPLE_SHORT_CUT = 128, 16384, 256
