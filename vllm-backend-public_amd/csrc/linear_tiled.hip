@@ -89,7 +89,11 @@ __global__ __launch_bounds__(NW * 64) void linear_tiled_kernel(
   constexpr int ROWB = KSL * 2 + 32;       // padded LDS row (bytes)
   constexpr int XBUF = ROWS * ROWB;
   constexpr int G = KSL / 32 / U;          // register groups per phase (8, 4 or 2)
-  constexpr int D = 2;                     // ring depth: one group computing, one in flight; deeper rings measured no faster (more outstanding requests only lengthen the memory queues) and cost registers
+  // Ring depth: one group computing, one in flight; deeper rings measured no faster (more outstanding requests only lengthen
+  // the memory queues) and cost registers.  But for fp8 weights at 17 .. 32 rows: their groups are half the bytes, and two
+  // waves a SIMD with two row blocks each leave the stream waiting (3584 -> 37888 at 24 rows, us: 40.4 with two groups,
+  // 34.1 with four; up to 16 rows, four waves a SIMD, 25.9 / 27.3; at 64 rows the products bind, 31.0 / 32.0).
+  constexpr int D = W8 && MT == 2 ? 4 : 2;
   constexpr int PU = G >= D ? 1 : D / G;   // phases per main-loop iteration: ring slots stay compile-time
   const int ubase = phases_total / static_cast<int>(gridDim.y), urem = phases_total % static_cast<int>(gridDim.y);
   const int P = ubase + (static_cast<int>(blockIdx.y) < urem ? 1 : 0);
