@@ -846,6 +846,19 @@ int32_t mi355_add_layer_norm_f32_slabs(void* out, float* resid, const float* par
 int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, int32_t na, const void* wa, const float* pb, int32_t nb,
                                      const void* wb, int64_t num_tokens, int32_t width, float eps, float alpha, int32_t dtype,
                                      void* stream);
+/*
+ * An update of the residual and the norm that reads it next, in one launch:
+ *   resid_add_norm_f32      resid += other (fp32 rows) + rows + vec (one row), each may be null, in this order; then
+ *                           out = resid / rms(resid) * weight (one number or one per column)
+ *   rms_norm_mix_norm_f32   rms_norm_mix_f32, then the same
+ * num_slabs, na, nb: 0: 16-bit rows, 1 .. 8: fp32 slabs (na and nb both or neither).  16-bit dtypes, widths and alignment as above.
+ */
+int32_t mi355_resid_add_norm_f32(void* out, const void* weight, int32_t weight_numel, float* resid, const float* other,
+                                 const void* rows, int32_t num_slabs, const void* vec, int64_t num_tokens, int32_t width,
+                                 float eps, int32_t dtype, void* stream);
+int32_t mi355_rms_norm_mix_norm_f32(void* out, const void* weight, int32_t weight_numel, float* resid, const void* xa,
+                                    int32_t na, const void* wa, const void* xb, int32_t nb, const void* wb, int64_t num_tokens,
+                                    int32_t width, float eps, float alpha, int32_t dtype, void* stream);
 int32_t mi355_gelu_tanh_and_mul_slabs(void* out, const float* partial, int32_t num_slabs, int64_t num_tokens, int32_t inter,
                                       int32_t dtype, void* stream);
 int32_t mi355_gated_head_rms_norm(void* out, int64_t out_stride, const float* o, const void* gate, int64_t gate_stride,

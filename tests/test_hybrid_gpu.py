@@ -1029,3 +1029,45 @@ def test_served_from_a_model_directory(tmp_path):
             proc.wait(timeout=20)
         except subprocess.TimeoutExpired:
             os.killpg(proc.pid, signal.SIGKILL)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,W,num", [(1, 8, 0), (3, 2048, 0), (5, 2056, 8), (2, 4096, 2), (7, 8192, 0), (33, 264, 3)])
+def test_residual_update_and_its_norm_in_one_launch(dtype, T, W, num):
+    """The same bits as the launches one after the other: plain rows and slabs, each addend there and absent, a weight of one
+    number and of one per column; widths past the one-launch form (slabs of 8192, float32) take those launches."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(W + T)
+    rnd = lambda *s: torch.randn(*s, generator=g).cuda()                      # noqa: E731
+    part = (lambda: ops.Slabs(rnd(num, T, W), num, T, W, dtype)) if num else (lambda: rnd(T, W).to(dtype))
+    x, other, vec = rnd(T, W), rnd(T, W), rnd(W).to(dtype)
+    for weight in (rnd(1).to(dtype), rnd(W).to(dtype)):
+        for o, rows, v in ((other, part(), vec), (None, part(), vec), (other, None, None), (None, None, vec), (other, part(), None)):
+            want, got = x.clone(), x.clone()
+            ops.resid_add_f32(want, other=o, rows=ops.dense(rows), vec=v)
+            h = ops.add_rms_norm_f32(want, weight, 1e-6)
+            assert torch.equal(ops.resid_add_norm_f32(got, weight, 1e-6, other=o, rows=rows, vec=v), h) and torch.equal(got, want)
+        want, got, mix = x.clone(), x.clone(), (part(), rnd(W).to(dtype), part(), rnd(W).to(dtype), 1e-6, 0.5)
+        ops.rms_norm_mix_f32(want, *mix)
+        h = ops.add_rms_norm_f32(want, weight, 1e-6)
+        assert torch.equal(ops.rms_norm_mix_norm_f32(got, *mix, weight), h) and torch.equal(got, want)
+    want, got, w32 = x.clone(), x.clone(), rnd(W)
+    ops.resid_add_f32(want, rows=other)
+    assert torch.equal(ops.resid_add_norm_f32(got, w32, 1e-6, rows=other), ops.add_rms_norm_f32(want, w32, 1e-6))
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(4104, 1024), (2048, 2048), (6208, 512), (264, 1024), (4096, 2048)])
+def test_rows_of_products_split_over_waves(M, N, K):
+    """Either side of the lines between K split over workgroups and over waves: one rounding of the fp32 sum, with a bias."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(N + M)
+    x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    bias = torch.randn(N, generator=g).bfloat16().cuda()
+    plan = ops.plan_linear_rows(N, K, M)
+    if plan is None:
+        assert M > 64 or K % 1024 or (M > 32 and N <= 4096)
+        return
+    got = ops.linear_tiled(x, ops.tile_weights(w), N, bias=bias, tiles_per_wg=plan[0])
+    want = x.double() @ w.double().t() + bias.double()
+    assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4).all()

@@ -187,7 +187,8 @@ template <typename T, int NV, int S>
 __global__ __launch_bounds__(256) void add_rms_norm_f32_vec_kernel(uint16_t* __restrict__ out, float* __restrict__ resid,
                                                                    const void* __restrict__ add, int num_slabs,
                                                                    const uint16_t* __restrict__ weight, int weight_numel, int W,
-                                                                   float eps) {
+                                                                   float eps, const float* __restrict__ other,
+                                                                   const uint16_t* __restrict__ vec) {
   __shared__ float scratch[32];
   const int64_t t = blockIdx.x;
   float v[NV][8];
@@ -203,15 +204,25 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32_vec_kernel(uint16_t* __r
     if (c < W) {
       load8f(resid, resid + t * W + c, v[i]);
       if (weight_numel != 1) wv[i] = MI355_LD(uint4, weight, weight + c);
+      float x0[8] = {}, step[8] = {};                     // a loop's input and step vector, ahead of and behind the addend
+      if (other != nullptr) load8f(other, other + t * W + c, x0);
+      if (vec != nullptr) unpack8<T>(MI355_LD(uint4, vec, vec + c), step);
       if (add != nullptr) {
         float y[8];
         Rows8<T, S> rows;
         rows.load(add, t * W + c, static_cast<int64_t>(gridDim.x) * W, num_slabs);
         rows.value(y, num_slabs);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] += y[j];
-        store8f(resid, resid + t * W + c, v[i]);
+        for (int j = 0; j < 8; ++j) v[i][j] = (other != nullptr ? v[i][j] + x0[j] : v[i][j]) + y[j];
+      } else if (other != nullptr) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] += x0[j];
       }
+      if (vec != nullptr) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] += step[j];
+      }
+      if (add != nullptr || other != nullptr || vec != nullptr) store8f(resid, resid + t * W + c, v[i]);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
@@ -378,16 +389,17 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __rest
                                                                    const uint16_t* __restrict__ wa,
                                                                    const void* __restrict__ xb, int nb,
                                                                    const uint16_t* __restrict__ wb, int W, float eps,
-                                                                   float alpha) {
-  __shared__ float scratch[2][4];
+                                                                   float alpha, uint16_t* __restrict__ out,
+                                                                   const uint16_t* __restrict__ weight, int weight_numel) {
+  __shared__ float scratch[3][4];
   const int64_t t = blockIdx.x, slab = static_cast<int64_t>(gridDim.x) * W;
-  uint4 ga[NV], gb[NV];
+  uint4 ga[NV], gb[NV], gn[NV];
   Rows8<T, S> a[NV], b[NV];
   float fa[NV][8], fb[NV][8], v[NV][8], sa = 0.f, sb = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + 256 * i) * 8;
-    ga[i] = gb[i] = make_uint4(0, 0, 0, 0);
+    ga[i] = gb[i] = gn[i] = make_uint4(0, 0, 0, 0);
     if (c < W) {
       a[i].load(xa, t * W + c, slab, na);
       ga[i] = MI355_LD(uint4, wa, wa + c);
@@ -396,8 +408,10 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __rest
         gb[i] = MI355_LD(uint4, wb, wb + c);
       }
       load8f(resid, resid + t * W + c, v[i]);
+      if (out != nullptr && weight_numel != 1) gn[i] = MI355_LD(uint4, weight, weight + c);
     }
   }
+  const float g1 = out != nullptr && weight_numel == 1 ? T::to_f(MI355_LD(uint16_t, weight, weight)) : 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const bool on = (threadIdx.x + 256 * i) * 8 < static_cast<unsigned>(W);
@@ -428,6 +442,29 @@ __global__ __launch_bounds__(256) void rms_norm_mix_f32_vec_kernel(float* __rest
       v[i][j] += alpha * m;
     }
     store8f(resid, resid + t * W + c, v[i]);
+  }
+  if (out == nullptr) return;
+  // the next sub-layer's norm of the row, which is here in registers
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if ((threadIdx.x + 256 * i) * 8 >= static_cast<unsigned>(W)) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += v[i][j] * v[i][j];
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) scratch[2][threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float r = 1.0f / sqrtf((scratch[2][0] + scratch[2][1] + scratch[2][2] + scratch[2][3]) / static_cast<float>(W) + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (threadIdx.x + 256 * i) * 8;
+    if (c >= W) continue;
+    float f[8];
+    unpack8<T>(gn[i], f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = v[i][j] * r * (weight_numel == 1 ? g1 : f[j]);
+    MI355_ST(uint4, out, out + t * W + c, pack8<T>(f));
   }
 }
 
@@ -1060,7 +1097,7 @@ extern "C" int32_t mi355_add_rms_norm_f32(void* out, float* resid, const void* a
       (weight_numel == 1 || aligned16(weight))) {
 #define MI355_RN(TT, NV)                                                                                                        \
   hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV, 0>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
-                     resid, add, 0, static_cast<const uint16_t*>(weight), weight_numel, width, eps)
+                     resid, add, 0, static_cast<const uint16_t*>(weight), weight_numel, width, eps, nullptr, nullptr)
 #define MI355_RN_NV(TT)                      \
   do {                                       \
     if (width <= 2048) MI355_RN(TT, 1);      \
@@ -1125,7 +1162,7 @@ extern "C" int32_t mi355_rms_norm_mix_f32(float* resid, const void* xa, const vo
       aligned16(xb) && aligned16(wb)) {
 #define MI355_MIX(TT, NV)                                                                                                \
   hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV, 0>), dim3(num_tokens), dim3(256), 0, s, resid, xa, 0,          \
-                     static_cast<const uint16_t*>(wa), xb, 0, static_cast<const uint16_t*>(wb), width, eps, alpha)
+                     static_cast<const uint16_t*>(wa), xb, 0, static_cast<const uint16_t*>(wb), width, eps, alpha, nullptr, nullptr, 1)
 #define MI355_MIX_NV(TT)                      \
   do {                                       \
     if (width <= 2048) MI355_MIX(TT, 1);      \
@@ -1191,7 +1228,7 @@ extern "C" int32_t mi355_add_rms_norm_f32_slabs(void* out, float* resid, const f
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define MI355_RN(TT, NV, S)                                                                                                     \
   hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
-                     resid, partial, num_slabs, static_cast<const uint16_t*>(weight), weight_numel, width, eps)
+                     resid, partial, num_slabs, static_cast<const uint16_t*>(weight), weight_numel, width, eps, nullptr, nullptr)
 #define MI355_RN_B(S) \
   do { if (width <= 2048) MI355_RN(BF16, 1, S); else if (width <= 4096) MI355_RN(BF16, 2, S); else MI355_RN(BF16, 4, S); } while (0)
 #define MI355_RN_H(S) \
@@ -1242,7 +1279,7 @@ extern "C" int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, i
   const int most = na > nb ? na : nb;
 #define MI355_MIX(TT, NV, S)                                                                                               \
   hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, resid, pa, na,           \
-                     static_cast<const uint16_t*>(wa), pb, nb, static_cast<const uint16_t*>(wb), width, eps, alpha)
+                     static_cast<const uint16_t*>(wa), pb, nb, static_cast<const uint16_t*>(wb), width, eps, alpha, nullptr, nullptr, 1)
 #define MI355_MIX_B(S) do { if (width <= 2048) MI355_MIX(BF16, 1, S); else MI355_MIX(BF16, 2, S); } while (0)
 #define MI355_MIX_H(S) do { if (width <= 2048) MI355_MIX(F16, 1, S); else MI355_MIX(F16, 2, S); } while (0)
   if (dtype == MI355_BF16) MI355_SLABS(most, MI355_MIX_B); else MI355_SLABS(most, MI355_MIX_H);
@@ -1250,6 +1287,76 @@ extern "C" int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, i
 #undef MI355_MIX_B
 #undef MI355_MIX
   return check_launch("rms_norm_mix_f32_slabs");
+}
+
+// The residual's update and the norm that reads it, in one launch: 32 rows of 2048, where a launch is 4 to 5 us whatever it
+// does, and prompts, whose residual (fp32) would be read back (8192 rows: mix 34 and norm 26 us in two launches).
+extern "C" int32_t mi355_resid_add_norm_f32(void* out, const void* weight, int32_t weight_numel, float* resid, const float* other,
+                                            const void* rows, int32_t num_slabs, const void* vec, int64_t num_tokens, int32_t width,
+                                            float eps, int32_t dtype, void* stream) {
+  MI355_REQUIRE(out && weight && resid, MI355_ERR_INVALID, "resid_add_norm_f32: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && width > 0 && num_slabs >= 0 && num_slabs <= 8 && (rows != nullptr || num_slabs == 0) &&
+                    (weight_numel == 1 || weight_numel == width),
+                MI355_ERR_INVALID, "resid_add_norm_f32: sizes");
+  MI355_REQUIRE((dtype == MI355_BF16 || dtype == MI355_F16) && width % 8 == 0 && width <= 8192 && aligned16(out) && aligned16(resid) &&
+                    aligned16(other) && aligned16(rows) && aligned16(vec) && (weight_numel == 1 || aligned16(weight)),
+                MI355_ERR_UNSUPPORTED, "resid_add_norm_f32: 16-bit rows of whole 16-byte pieces, at most 8192 wide");
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define MI355_RN(TT, NV, S)                                                                                                     \
+  hipLaunchKernelGGL((add_rms_norm_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, static_cast<uint16_t*>(out), \
+                     resid, rows, num_slabs, static_cast<const uint16_t*>(weight), weight_numel, width, eps, other,             \
+                     static_cast<const uint16_t*>(vec))
+#define MI355_RN_B(S) \
+  do { if (width <= 2048) MI355_RN(BF16, 1, S); else if (width <= 4096) MI355_RN(BF16, 2, S); else MI355_RN(BF16, 4, S); } while (0)
+#define MI355_RN_H(S) \
+  do { if (width <= 2048) MI355_RN(F16, 1, S); else if (width <= 4096) MI355_RN(F16, 2, S); else MI355_RN(F16, 4, S); } while (0)
+  if (num_slabs == 0) {
+    if (dtype == MI355_BF16) MI355_RN_B(0); else MI355_RN_H(0);
+  } else if (dtype == MI355_BF16) {
+    MI355_SLABS(num_slabs, MI355_RN_B);
+  } else {
+    MI355_SLABS(num_slabs, MI355_RN_H);
+  }
+#undef MI355_RN_H
+#undef MI355_RN_B
+#undef MI355_RN
+  return check_launch("resid_add_norm_f32");
+}
+
+extern "C" int32_t mi355_rms_norm_mix_norm_f32(void* out, const void* weight, int32_t weight_numel, float* resid, const void* xa,
+                                               int32_t na, const void* wa, const void* xb, int32_t nb, const void* wb, int64_t num_tokens,
+                                               int32_t width, float eps, float alpha, int32_t dtype, void* stream) {
+  MI355_REQUIRE(out && weight && resid && xa && wa && xb && wb, MI355_ERR_INVALID, "rms_norm_mix_norm_f32: null pointer");
+  MI355_REQUIRE(num_tokens >= 0 && width > 0 && na >= 0 && na <= 8 && nb >= 0 && nb <= 8 && (na == 0) == (nb == 0) &&
+                    (weight_numel == 1 || weight_numel == width),
+                MI355_ERR_INVALID, "rms_norm_mix_norm_f32: sizes");
+  MI355_REQUIRE((dtype == MI355_BF16 || dtype == MI355_F16) && width % 8 == 0 && width <= (na == 0 ? 8192 : 4096) && aligned16(out) &&
+                    aligned16(resid) && aligned16(xa) && aligned16(wa) && aligned16(xb) && aligned16(wb) &&
+                    (weight_numel == 1 || aligned16(weight)),
+                MI355_ERR_UNSUPPORTED, "rms_norm_mix_norm_f32: 16-bit rows of whole 16-byte pieces, at most 8192 wide (slabs: 4096)");
+  if (num_tokens == 0) return MI355_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int most = na > nb ? na : nb;
+#define MI355_MIX(TT, NV, S)                                                                                               \
+  hipLaunchKernelGGL((rms_norm_mix_f32_vec_kernel<TT, NV, S>), dim3(num_tokens), dim3(256), 0, s, resid, xa, na,           \
+                     static_cast<const uint16_t*>(wa), xb, nb, static_cast<const uint16_t*>(wb), width, eps, alpha,        \
+                     static_cast<uint16_t*>(out), static_cast<const uint16_t*>(weight), weight_numel)
+#define MI355_MIX_B(S) do { if (width <= 2048) MI355_MIX(BF16, 1, S); else MI355_MIX(BF16, 2, S); } while (0)
+#define MI355_MIX_H(S) do { if (width <= 2048) MI355_MIX(F16, 1, S); else MI355_MIX(F16, 2, S); } while (0)
+  if (most == 0) {
+    if (width <= 4096) { if (dtype == MI355_BF16) MI355_MIX_B(0); else MI355_MIX_H(0); }
+    else if (dtype == MI355_BF16) MI355_MIX(BF16, 4, 0);
+    else MI355_MIX(F16, 4, 0);
+  } else if (dtype == MI355_BF16) {
+    MI355_SLABS(most, MI355_MIX_B);
+  } else {
+    MI355_SLABS(most, MI355_MIX_H);
+  }
+#undef MI355_MIX_H
+#undef MI355_MIX_B
+#undef MI355_MIX
+  return check_launch("rms_norm_mix_norm_f32");
 }
 
 extern "C" int32_t mi355_gelu_tanh_and_mul_slabs(void* out, const float* partial, int32_t num_slabs, int64_t num_tokens, int32_t inter,

@@ -83,12 +83,14 @@ class StepBatch:
     """Device-side description of one packed step (see csrc/seqmix.hip)."""
     __slots__ = ("ids", "positions", "slot_mapping", "block_tables", "cu_seqlens", "tok_seq", "state_slots",
                  "num_tokens", "num_seqs", "tiles", "long_chunks", "pair_tiles", "context_lens", "max_q_len", "row_tiles",
-                 "routes", "latent_plan", "max_context")
+                 "routes", "latent_plan", "max_context", "keep_tail", "tail")
 
     def __init__(self, ids, positions, slot_mapping, block_tables, cu_seqlens, tok_seq, state_slots, tiles=None,
                  long_chunks=False, pair_tiles=None, context_lens=None, max_q_len=0, row_tiles=None,
                  latent_plan=None, max_context=0):
         self.routes = {}                              # (experts, top) -> ops.TableRoutes of the step's token ids
+        # keep_tail: the last sub-layer's output may be left off the residual, in `tail`: the final norm adds it to the rows that have logits
+        self.keep_tail, self.tail = False, None
         self.latent_plan = latent_plan                # () -> the step's LatentPlan, or None (captured decode steps)
         self.row_tiles = row_tiles                    # rows -> ops.RowTiles of the step, or None (captured decode steps)
         # every chunk's length of context after the step (int32, on the device), the longest chunk and the longest
@@ -913,6 +915,8 @@ class HybridRunner(ModelRunner):
             plan = ops.plan_linear_tiled(N, K, True, M)
             if plan is not None:
                 tiles, groups = plan
+                if groups > 1 and not (slabs and bias is None):
+                    tiles, groups = ops.plan_linear_rows(N, K, M) or plan
                 if out is None and not (slabs and bias is None and groups > 1):
                     out = torch.empty(M, N, dtype=x.dtype, device=x.device)
                 if groups == 1:
@@ -1011,32 +1015,41 @@ class HybridRunner(ModelRunner):
         for ri, (li, t) in enumerate(self.runs):
             L, lw = spec.layers[li], w.layers[li]
             if t is not None and li == spec.loop_start and not spec.loop_plain:    # a pass begins: + embedding output (not the first) + its step vector
-                ops.resid_add_f32(resid, other=x0 if t > 0 else None, rows=ops.dense(pending), vec=w.loop_step[t])
-                pending = None
-            h = self._norm(resid, lw.norm1, pending)       # the add rides in the norm's launch
+                if spec.layer_norm or isinstance(pending, ExpertRows):
+                    ops.resid_add_f32(resid, other=x0 if t > 0 else None, rows=ops.dense(pending), vec=w.loop_step[t])
+                    h = self._norm(resid, lw.norm1)
+                else:
+                    h = ops.resid_add_norm_f32(resid, lw.norm1, self.eps, other=x0 if t > 0 else None, rows=pending, vec=w.loop_step[t])
+            else:
+                h = self._norm(resid, lw.norm1, pending)   # the add rides in the norm's launch
             pending = None
             proj = self.linear(h, lw.in_w)
-            mixer, ff = self.mixers[ri], self.ffs[ri]
+            mixer, ff, normed = self.mixers[ri], self.ffs[ri], False
             if not isinstance(mixer, tuple):
                 pending = mixer(proj, b)
             elif mixer[0] is not None:
                 attn, delta = mixer
-                ops.rms_norm_mix_f32(resid, attn(proj, b), lw.attn_out_norm, delta(proj, b), lw.delta_out_norm,
-                                     self.eps, 0.5)
+                mix = (resid, attn(proj, b), lw.attn_out_norm, delta(proj, b), lw.delta_out_norm, self.eps, 0.5)
+                if (ff is not None or L.ff) and not spec.layer_norm:
+                    h, normed = ops.rms_norm_mix_norm_f32(*mix, lw.norm2), True
+                else:
+                    ops.rms_norm_mix_f32(*mix)
             else:
                 pending = mixer[1](proj, b)
-            if isinstance(ff, (LimitedFF, TableMoE)):
-                pending = ff(self._norm(resid, lw.norm2, pending), b)
-            elif ff is not None:
-                pending = ff(self._norm(resid, lw.norm2, pending))
-            elif L.ff:
+            if (ff is not None or L.ff) and not normed:
                 h = self._norm(resid, lw.norm2, pending)
+            if isinstance(ff, (LimitedFF, TableMoE)):
+                pending = ff(h, b)
+            elif ff is not None:
+                pending = ff(h)
+            elif L.ff:
                 pending = self.out_linear(ops.gelu_tanh_and_mul(self.linear(h, lw.gate_up_w, slabs=True)), lw.down_w)
-            if pending is not None and (ri == last or self.layer_trace is not None):
+            if pending is not None and (self.layer_trace is not None or (ri == last and not b.keep_tail)):
                 self._norm(resid, None, pending)
                 pending = None
             if self.layer_trace is not None:
                 self.layer_trace.append(resid.clone())
+        b.tail = pending
         return resid
 
     def _forward_parallel(self, b: StepBatch) -> torch.Tensor:
@@ -1103,14 +1116,24 @@ class HybridRunner(ModelRunner):
                 self.layer_trace.append(resid.clone())
         return resid
 
-    def _logits(self, resid: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """Final norm, head and soft cap over the given residual rows."""
+    @staticmethod
+    def _tail_rows(tail, at: torch.Tensor):
+        """A StepBatch.tail of the packed rows `at` alone."""
+        if tail is None:
+            return None
+        if isinstance(tail, ExpertRows):
+            rows = tail.rows.index_select(0, tail.inv.view(-1, tail.top).index_select(0, at).view(-1))
+            return ExpertRows(rows, torch.arange(rows.shape[0], dtype=torch.int32, device=rows.device), tail.top, tail.weight)
+        return ops.dense(tail).index_select(0, at)
+
+    def _logits(self, resid: torch.Tensor, out: Optional[torch.Tensor] = None, tail=None) -> torch.Tensor:
+        """Final norm, head and soft cap over the given residual rows (+ their last sub-layer's output `tail`)."""
         if self.spec.arrangement == "sandwich":
             h = ops.group_rms_norm_f32(resid, self.w.final_norm, self.spec.norm_groups, self.eps, dtype=self.dtype)
         elif self.spec.arrangement == "post":
             h = ops.group_rms_norm_f32(resid, self.w.final_norm, 1, self.eps, dtype=self.dtype)
         else:
-            h = self._norm(resid, self.w.final_norm)
+            h = self._norm(resid, self.w.final_norm, tail)
         z = self.linear(h, self.head_w, out=out)
         if self.spec.logit_softcap:
             ops.softcap(z, self.spec.logit_softcap)
@@ -1124,8 +1147,9 @@ class HybridRunner(ModelRunner):
                           self._dec_cu[:b + 1], self._dec_seq[:b], self.row_extra[:b], self._dec_tiles[:b],
                           pair_tiles=lambda heads: self._decode_pair_tiles(heads)[: b * (-(-heads // 16))],
                           context_lens=self.ctx[:b])
+        batch.keep_tail = True
         resid = self._forward(batch)
-        self._logits(resid, out=self.logits_rows[:b])
+        self._logits(resid, out=self.logits_rows[:b], tail=batch.tail)
         self.greedy(self.logits[:b], self.next_ids[:b], ids_out=self.ids[:b])
 
     def run_prefill(self, token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens, max_q_len: int,
@@ -1150,38 +1174,42 @@ class HybridRunner(ModelRunner):
                                                       (rows, np.int64), (block_tables, np.int32), (cu_seqlens, np.int32),
                                                       (context_lens, np.int32))]
         ids, pos, slots, at, tables, cu, ctx = ops.upload(self.device, *host)
-        resid = self._run_chunks(ids, pos, slots, tables, cu, ctx, max_q_len)
+        resid, tail = self._run_chunks(ids, pos, slots, tables, cu, ctx, max_q_len)
         if rows.size == 0:
             torch.cuda.current_stream().synchronize()
             return np.zeros((0, self.V), dtype=np.float32)
-        z = self._logits(resid.index_select(0, at))
+        z = self._logits(resid.index_select(0, at), tail=self._tail_rows(tail, at))
         return z.float().cpu().numpy()
 
     def _run_chunks(self, token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens=None,
-                    max_q_len: int = 0) -> torch.Tensor:
+                    max_q_len: int = 0):
+        """The residual of every row, and what its last sub-layer has still to add to it (StepBatch.tail)."""
         lens = self._step_cu[1:] - self._step_cu[:-1]
         tok_seq, slots, tiles = ops.upload(self.device, np.repeat(np.arange(len(lens), dtype=np.int32), lens),
                                            self._step_state_slots, self._step_tiles)
-        return self._forward(StepBatch(token_ids, positions, slot_mapping, block_tables.contiguous(), cu_seqlens,
-                                       tok_seq, slots, tiles, self._step_long, pair_tiles=self._chunk_pair_tiles,
-                                       context_lens=None if context_lens is None else context_lens.to(torch.int32).contiguous(),
-                                       max_q_len=max_q_len, row_tiles=self._chunk_row_tiles, latent_plan=self._chunk_latent_plan,
-                                       max_context=np.asarray(self._step_ctx).max(initial=0)))
+        b = StepBatch(token_ids, positions, slot_mapping, block_tables.contiguous(), cu_seqlens,
+                      tok_seq, slots, tiles, self._step_long, pair_tiles=self._chunk_pair_tiles,
+                      context_lens=None if context_lens is None else context_lens.to(torch.int32).contiguous(),
+                      max_q_len=max_q_len, row_tiles=self._chunk_row_tiles, latent_plan=self._chunk_latent_plan,
+                      max_context=np.asarray(self._step_ctx).max(initial=0))
+        b.keep_tail = True
+        return self._forward(b), b.tail
 
     def prefill(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                 block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
                 max_q_len: int, want_logits: bool = True, score=None):
         """As ModelRunner.prefill: packed prompts (or prompt chunks), eager."""
-        resid = self._run_chunks(token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens, max_q_len)
+        resid, tail = self._run_chunks(token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens, max_q_len)
         if score is not None:
             k, srows, targets = score
             parts = []
             for a in range(0, srows.numel(), 1024):
-                lg = self._logits(resid.index_select(0, srows[a:a + 1024]))
+                at = srows[a:a + 1024]
+                lg = self._logits(resid.index_select(0, at), tail=self._tail_rows(tail, at))
                 parts.append(self._logprobs(lg, targets[a:a + 1024], k))
             self.prompt_scores = torch.cat(parts, dim=0)
         rows = (cu_seqlens[1:] - 1).to(torch.int64)
-        logits = self._logits(resid.index_select(0, rows))
+        logits = self._logits(resid.index_select(0, rows), tail=self._tail_rows(tail, rows))
         nxt = torch.empty(logits.shape[0], dtype=torch.int64, device=self.device)
         self.greedy(logits, nxt)
         return nxt, (logits if want_logits else None)

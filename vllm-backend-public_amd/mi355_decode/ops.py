@@ -722,6 +722,20 @@ def plan_linear_tiled(N: int, K: int, split_k: bool, M: int = 32):
     return None
 
 
+def plan_linear_rows(N: int, K: int, M: int):
+    """(tiles_per_wg, 1) where 16-bit rows cost less with K split over the waves of a workgroup than over workgroups with
+    a second launch that adds the slabs (2 us, and 4 to 5 in a step of small launches), or None.  Measured on 512 .. 24576 x
+    512 .. 8192 (us, slabs and their sum / across waves): 4 waves a tile 6208 x 2048 9.1 / 7.4 at 16 rows, 12.4 / 10.7 at 64,
+    8192 x 8192 26.0 / 25.1; 8 waves a tile 2048 x 1024 5.6 / 3.6, 2048 x 2048 6.2 / 5.0 at 16 rows, 6.6 / 5.9 at 32.  Longer K in
+    fewer tiles is one long walk: 2048 x 4096 7.6 / 7.9 at 16 rows, 10.4 / 14.8 at 64."""
+    tiles_total = (N + 15) // 16
+    if M <= 32:
+        code = 304 if tiles_total > 256 else 308 if K <= 2048 else 0
+    else:
+        code = 304 if M <= 64 and (tiles_total > 256 or K <= max(512, N // 2)) else 0
+    return (code, 1) if code and K % tiled_slice_width(M, code) == 0 else None
+
+
 def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: bool = False):
     """Every (tiles_per_wg, k_groups) worth timing for linear_tiled on an [N, K] weight and M rows:
     both workgroup shapes that every kernel form (fp8, fused epilogues) is built for, K split into
@@ -1217,6 +1231,60 @@ def rms_norm_mix_f32(resid: torch.Tensor, xa: torch.Tensor, wa: torch.Tensor, xb
                                      None if xb is None else xb.data_ptr(), None if wb is None else wb.data_ptr(),
                                      T, W, float(eps), float(alpha), dt, _stream()))
     return resid
+
+
+def _norm_rides(resid: torch.Tensor, weight: torch.Tensor, parts, most: int) -> bool:
+    """Whether the launches below take these: 16-bit rows (or slabs) like resid's on 16-byte boundaries."""
+    T, W = resid.shape
+    if weight.dtype not in (torch.bfloat16, torch.float16) or W % 8 or W > most or not weight.is_contiguous() \
+            or weight.numel() not in (1, W) or not resid.is_contiguous() or resid.data_ptr() % 16 \
+            or (weight.numel() != 1 and weight.data_ptr() % 16):
+        return False
+    for p in parts:
+        if isinstance(p, Slabs):
+            if not p.fits(T, W, weight.dtype, most):
+                return False
+        elif p.dtype != weight.dtype or tuple(p.shape) != (T, W) or not p.is_contiguous() or p.data_ptr() % 16:
+            return False
+    return True
+
+
+def _part(p):
+    return (None, 0) if p is None else (p.partial.data_ptr(), p.num) if isinstance(p, Slabs) else (p.data_ptr(), 0)
+
+
+def resid_add_norm_f32(resid: torch.Tensor, weight: torch.Tensor, eps: float, other: torch.Tensor | None = None,
+                       rows: torch.Tensor | None = None, vec: torch.Tensor | None = None) -> torch.Tensor:
+    """resid_add_f32 (rows: plain or Slabs), then add_rms_norm_f32 of the sum: one launch where the types and sizes allow."""
+    T, W = resid.shape
+    if T and _norm_rides(resid, weight, [] if rows is None else [rows], 8192) \
+            and (vec is None or (vec.dtype == weight.dtype and vec.numel() == W and vec.is_contiguous() and vec.data_ptr() % 16 == 0)) \
+            and (other is None or other.data_ptr() % 16 == 0):
+        out = torch.empty(T, W, dtype=weight.dtype, device=resid.device)
+        p, n = _part(rows)
+        check(lib.mi355_resid_add_norm_f32(out.data_ptr(), weight.data_ptr(), weight.numel(), _f32(resid, "resid"),
+                                           None if other is None else _f32(other, "other", T * W), p, n,
+                                           None if vec is None else vec.data_ptr(), T, W, float(eps), _dt16(weight, "weight"), _stream()))
+        return out
+    resid_add_f32(resid, other=other, rows=dense(rows), vec=vec)
+    return add_rms_norm_f32(resid, weight, eps)
+
+
+def rms_norm_mix_norm_f32(resid: torch.Tensor, xa, wa: torch.Tensor, xb, wb: torch.Tensor, eps: float, alpha: float,
+                          weight: torch.Tensor) -> torch.Tensor:
+    """rms_norm_mix_f32, then add_rms_norm_f32 of the sum with `weight`: one launch where the types and sizes allow."""
+    T, W = resid.shape
+    slabs = isinstance(xa, Slabs)
+    if T and slabs == isinstance(xb, Slabs) and _norm_rides(resid, weight, [xa, xb], 4096 if slabs else 8192) \
+            and all(w.dtype == weight.dtype and tuple(w.shape) == (W,) and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in (wa, wb)):
+        out = torch.empty(T, W, dtype=weight.dtype, device=resid.device)
+        (pa, na), (pb, nb) = _part(xa), _part(xb)
+        check(lib.mi355_rms_norm_mix_norm_f32(out.data_ptr(), weight.data_ptr(), weight.numel(), _f32(resid, "resid"), pa, na,
+                                              wa.data_ptr(), pb, nb, wb.data_ptr(), T, W, float(eps), float(alpha),
+                                              _dt16(weight, "weight"), _stream()))
+        return out
+    rms_norm_mix_f32(resid, xa, wa, xb, wb, eps, alpha)
+    return add_rms_norm_f32(resid, weight, eps)
 
 
 def gelu_tanh_and_mul(x: torch.Tensor, out: torch.Tensor | None = None):
