@@ -847,6 +847,33 @@ int32_t mi355_rms_norm_mix_f32_slabs(float* resid, const float* pa, int32_t na, 
                                      const void* wb, int64_t num_tokens, int32_t width, float eps, float alpha, int32_t dtype,
                                      void* stream);
 /*
+ * A gated delta rule's mixer for rows that are a sequence's next token each (row s: state_slots[s], positions[s]), from the
+ * input projection to the gated, normed heads: conv_silu_step, the low-rank decay and gate (a2, g2 [heads * 128][rank]; both
+ * null: a decay a head and a gate per column straight from the projection), gated_delta_rule and gated_head_rms_norm in
+ * one launch.  Columns of a projection row: q | k | v at qkv_off, the removal rate at beta_off, the decay at a_off, the
+ * gate at g_off.  16-bit storage, heads of 128 x 128, one or two to a key head, 2 to 4 taps, rank a multiple of 32.
+ */
+int32_t mi355_delta_decode(void* out, int64_t out_stride, const void* proj, int64_t proj_stride, int32_t qkv_off,
+                           int32_t beta_off, int32_t a_off, int32_t g_off, const void* conv_w, float* conv_state, int32_t taps,
+                           const void* a2, const void* g2, int32_t rank, const float* a_log, const float* dt_bias,
+                           const float* norm_w, int32_t norm_heads, int32_t act, float eps, float* state,
+                           const int64_t* positions, const int32_t* state_slots, int32_t num_rows, int32_t num_heads,
+                           int32_t num_kv_heads, int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream);
+/*
+ * The same beside a sliding-window attention with sigmoid weights of the same rows (sigmoid_window_attn of single rows, keys and
+ * values of 128, at most 7 query heads a kv head; attn_out [num_rows][attn_heads * 128]) in one launch; two heads a key head.
+ */
+int32_t mi355_window_delta_decode(void* attn_out, const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                  const int32_t* block_tables, int32_t max_blocks, const int32_t* tok_seq, const float* temp,
+                                  const float* bias, const void* gate, int64_t gate_stride, int32_t attn_heads,
+                                  int32_t attn_kv_heads, int32_t window, float scale, void* out, int64_t out_stride,
+                                  const void* proj, int64_t proj_stride, int32_t qkv_off, int32_t beta_off, int32_t a_off,
+                                  int32_t g_off, const void* conv_w, float* conv_state, int32_t taps, const void* a2,
+                                  const void* g2, int32_t rank, const float* a_log, const float* dt_bias, const float* norm_w,
+                                  int32_t norm_heads, int32_t act, float eps, float* state, const int64_t* positions,
+                                  const int32_t* state_slots, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads,
+                                  int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream);
+/*
  * An update of the residual and the norm that reads it next, in one launch:
  *   resid_add_norm_f32      resid += other (fp32 rows) + rows + vec (one row), each may be null, in this order; then
  *                           out = resid / rms(resid) * weight (one number or one per column)

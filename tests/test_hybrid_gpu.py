@@ -1071,3 +1071,78 @@ def test_rows_of_products_split_over_waves(M, N, K):
     got = ops.linear_tiled(x, ops.tile_weights(w), N, bias=bias, tiles_per_wg=plan[0])
     want = x.double() @ w.double().t() + bias.double()
     assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4).all()
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3)])
+@pytest.mark.parametrize("B,H,G,taps,rank", [(1, 2, 1, 4, 0), (5, 16, 8, 4, 0), (3, 3, 3, 2, 0), (33, 8, 4, 4, 128), (2, 4, 4, 3, 32), (4, 2, 1, 2, 64)])
+def test_delta_mixer_of_single_tokens_in_one_launch(dtype, tol, B, H, G, taps, rank):
+    """Against the launches one after the other, over three steps: fresh sequences and ones inside their first taps beside
+    long ones, states and pages of other slots left alone.  Rounding of the convolution, the decay and the gate sits at the
+    same places; the sums over the rows of a state run in another order."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(B + H)
+    d, slots = 128, B + 2
+    C, seg, at = (2 * G + H) * d, {}, 8
+    for n, w in (("q", G * d), ("k", G * d), ("v", H * d), ("b", H), ("a1", rank) if rank else ("a", H), ("g1", rank) if rank else ("g", H * d)):
+        at = -(-at // 8) * 8 if n not in ("k", "v") else at
+        seg[n], at = (at, w), at + w
+    width = -(-at // 8) * 8
+    rnd = lambda *s: torch.randn(*s, generator=g)                              # noqa: E731
+    conv_w, norm_w = (rnd(C, taps) * 0.5).to(dtype).cuda(), (rnd(d) * 0.2 + 1).cuda()
+    a2, g2 = ((rnd(H * d, rank) * rank ** -0.5).to(dtype).cuda() for _ in range(2)) if rank else (None, None)
+    a_log, dt_bias = (rnd(H) * 0.3).cuda(), rnd(H * d if rank else H).cuda()
+    cs, st = rnd(slots, taps - 1, C).cuda(), (rnd(slots, H, d, d) * 0.3).cuda()
+    order = torch.randperm(slots, generator=g)[:B].to(torch.int32).cuda()
+    cu, seq = torch.arange(B + 1, dtype=torch.int32).cuda(), torch.arange(B, dtype=torch.int32).cuda()
+    cs2, st2, idle = cs.clone(), st.clone(), [i for i in range(slots) if i not in order.tolist()]
+    act = ops.ACT_SIGMOID if rank else ops.ACT_SILU
+    for step in range(3):
+        pos = torch.tensor([(0, 1, 2, 50)[i % 4] + step for i in range(B)]).cuda()
+        proj = rnd(B, width).to(dtype).cuda()
+        col = lambda n: proj[:, seg[n][0]: seg[n][0] + seg[n][1]]              # noqa: E731
+        assert ops.delta_decode_ok(proj, seg, H, G, d, d, taps, a2, g2)
+        got = ops.delta_decode(proj, seg, conv_w, cs2, a_log, dt_bias, norm_w, 1e-6, act, st2, pos, order, H, G, d, d, a2=a2, g2=g2)
+        y = ops.causal_conv_silu(proj[:, seg["q"][0]: seg["q"][0] + C], conv_w, cs, seq, pos, cu, order)
+        decay, gate = (col("a"), col("g")) if not rank else ((col("a1").float() @ a2.float().t()).to(dtype), (col("g1").float() @ g2.float().t()).to(dtype))
+        o = ops.gated_delta_rule(y, 0, G * d, 2 * G * d, col("b"), decay, a_log, dt_bias, st, cu, pos, order, H, G, d, d, per_channel=bool(rank))
+        want = ops.gated_head_rms_norm(o, gate, norm_w, 1e-6, act)
+        assert torch.equal(cs, cs2) and torch.equal(st[idle], st2[idle])
+        assert (st - st2).abs().max() <= tol * st.abs().max()
+        err = (got.float() - want.float()).abs().max() / want.float().abs().max()
+        assert err <= tol, float(err)
+
+
+@pytest.mark.parametrize("B,H,G,rank,heads,kv,window", [(1, 2, 1, 0, 4, 1, 100), (33, 8, 4, 128, 16, 4, 1024), (3, 4, 2, 32, 7, 1, 31), (5, 2, 1, 0, 6, 6, 2000)])
+def test_window_attention_beside_the_delta_mixer(B, H, G, rank, heads, kv, window):
+    """The launch of both against the two alone: the recurrence to the bit, the attention within the rounding of its keys'
+    weights to 16 bits and of its result (its waves take other keys)."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(window)
+    d, C = 128, (2 * G + H) * 128
+    rnd = lambda *s: torch.randn(*s, generator=g)                              # noqa: E731
+    seg, at = {}, 0
+    for n, w in (("q", G * d), ("k", G * d), ("v", H * d), ("a1", rank) if rank else ("g", H * d), ("g1", rank) if rank else ("a", H), ("b", H),
+                 ("lg", heads), ("lq", heads * d)):
+        at = -(-at // 8) * 8
+        seg[n], at = (at, w), at + w
+    proj = rnd(B, -(-at // 8) * 8).bfloat16().cuda()
+    low = {n: (rnd(H * d, rank) * rank ** -0.5).bfloat16().cuda() for n in ("a2", "g2")} if rank else {}
+    conv_w, norm_w, a_log, dt_bias = (rnd(C, 4) * 0.5).bfloat16().cuda(), rnd(d).cuda(), rnd(H).cuda(), rnd(H * d if rank else H).cuda()
+    cs, st = rnd(B, 3, C).cuda(), (rnd(B, H, d, d) * 0.3).cuda()
+    slots = torch.randperm(B, generator=g).to(torch.int32).cuda()
+    pos = torch.tensor([(0, 40, 2500, window)[i % 4] for i in range(B)]).cuda()
+    nb = 157 + 1
+    kc, vc = rnd(nb * B, kv, 16, d).bfloat16().cuda(), rnd(nb * B, kv, d, 16).bfloat16().cuda()
+    bt = torch.randperm(nb * B, generator=g).to(torch.int32).view(B, nb).cuda()
+    seq = torch.arange(B, dtype=torch.int32).cuda()
+    col = lambda n: proj[:, seg[n][0]: seg[n][0] + seg[n][1]]                  # noqa: E731
+    temp, bias = rnd(heads).abs().cuda(), rnd(heads).cuda()
+    args = lambda c, s: (proj, seg, conv_w, c, a_log, dt_bias, norm_w, 1e-6, ops.ACT_SILU, s, pos, slots, H, G, d, d)      # noqa: E731
+    c1, s1, c2, s2 = cs.clone(), st.clone(), cs.clone(), st.clone()
+    want_on = ops.delta_decode(*args(c1, s1), **low)
+    tiles = torch.stack([seq, seq, torch.ones_like(seq)], dim=1).contiguous()
+    want = ops.sigmoid_window_attn(col("lq"), kc, vc, bt, seq, pos, temp, bias, col("lg"), heads, window, 0.1, tiles=tiles)
+    got, on = ops.delta_decode(*args(c2, s2), **low, attention=dict(q=col("lq"), k_cache=kc, v_cache=vc, block_tables=bt, tok_seq=seq, temp=temp,
+                                                                    bias=bias, gate=col("lg"), num_heads=heads, window=window, scale=0.1))
+    assert torch.equal(on, want_on) and torch.equal(c1, c2) and torch.equal(s1, s2)
+    assert (got.float() - want.float()).abs().max() <= 2.0 ** -7 * want.float().abs().max()

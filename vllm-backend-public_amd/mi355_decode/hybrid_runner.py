@@ -137,7 +137,8 @@ class WindowAttention:
     def __init__(self, spec, lw, runner, cache_index: int):
         self.s, self.lw, self.r, self.ci = spec, lw, runner, cache_index
 
-    def __call__(self, proj: torch.Tensor, b: StepBatch) -> torch.Tensor:
+    def _rows(self, proj: torch.Tensor, b: StepBatch):
+        """Queries (rotated), gate and pages, the step's keys and values written to them."""
         s, seg, r = self.s, self.lw.seg, self.r
         q = proj[:, seg["lq"][0]: seg["lq"][0] + seg["lq"][1]]
         k = proj[:, seg["lk"][0]: seg["lk"][0] + seg["lk"][1]]
@@ -146,6 +147,24 @@ class WindowAttention:
         kc, vc = r.k_cache[self.ci], r.v_cache[self.ci]
         ops.rope_partial_kv_write(q, k, v, r.rotary(s.rot_dims, s.rot_base), b.positions, b.slot_mapping, kc, vc,
                                   s.heads, s.kv_heads, s.dim, s.vdim)
+        return q, g, kc, vc
+
+    def beside(self, delta: "DeltaMixer", proj: torch.Tensor, b: StepBatch):
+        """Both mixers of a step of single tokens by one launch, or None: where the window is one that a workgroup walks at
+        once (16 waves of 32 keys, twice) or the rows are so many that their keys are not spread over workgroups."""
+        s, d, lw = self.s, delta.s, self.lw
+        if not delta.one_launch(proj, b) or s.dim != 128 or s.vdim != 128 or s.heads // s.kv_heads > 7 or d.heads != 2 * d.kv_heads \
+                or lw.seg["lq"][0] % 8 or (s.window > 1024 and self.r.key_splits(b, s)):
+            return None
+        q, g, kc, vc = self._rows(proj, b)
+        rows, on = delta.step(proj, b, attention=dict(q=q, k_cache=kc, v_cache=vc, block_tables=b.block_tables, tok_seq=b.tok_seq,
+                                                      temp=lw.attn_temp, bias=lw.attn_bias, gate=g, num_heads=s.heads,
+                                                      window=s.window, scale=s.scale))
+        return _out_product(self.r, rows, lw.attn_o_w), _out_product(self.r, on, lw.delta_o_w)
+
+    def __call__(self, proj: torch.Tensor, b: StepBatch) -> torch.Tensor:
+        s, r = self.s, self.r
+        q, g, kc, vc = self._rows(proj, b)
         if b.long_chunks and b.context_lens is not None and s.dim <= 128 and proj.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0 \
                 and ops.chunk_attn_prefill_ok(q.dtype, s.heads, s.kv_heads, s.dim, s.vdim) \
                 and staged_window_pays(b.num_tokens, b.num_seqs, b.max_q_len, b.max_context, s.heads, s.kv_heads, s.dim, s.window):
@@ -164,8 +183,25 @@ class DeltaMixer:
     def __init__(self, spec, lw, runner, state_index: int):
         self.s, self.lw, self.r, self.si = spec, lw, runner, state_index
 
+    def _low(self) -> dict:
+        return {"a2": self.lw.a2_w, "g2": self.lw.g2_w} if self.s.per_channel else {"a2": None, "g2": None}
+
+    def one_launch(self, proj: torch.Tensor, b: StepBatch) -> bool:
+        """Whether `step` serves the batch: single tokens, at the sizes that the launch is built for."""
+        s = self.s
+        return not b.long_chunks and b.num_tokens == b.num_seqs and b.max_q_len <= 1 and ops.delta_decode_ok(
+            proj, self.lw.seg, s.heads, s.kv_heads, s.dim, s.vdim, self.lw.conv_w.shape[1], **self._low())
+
+    def step(self, proj: torch.Tensor, b: StepBatch, attention: Optional[dict] = None):
+        s, lw, r = self.s, self.lw, self.r
+        return ops.delta_decode(proj, lw.seg, lw.conv_w, r.conv_state[self.si], lw.a_log, lw.dt_bias, lw.head_norm, r.eps,
+                                ops.ACT_SIGMOID if s.per_channel else ops.ACT_SILU, r.rec_state[self.si], b.positions, b.state_slots,
+                                s.heads, s.kv_heads, s.dim, s.vdim, attention=attention, **self._low())
+
     def __call__(self, proj: torch.Tensor, b: StepBatch) -> torch.Tensor:
         s, lw, seg, r = self.s, self.lw, self.lw.seg, self.r
+        if self.one_launch(proj, b):
+            return _out_product(r, self.step(proj, b), lw.delta_o_w)
         qk, vv = s.kv_heads * s.dim, s.heads * s.vdim
         q0 = seg["q"][0]
         if seg["k"][0] != q0 + qk or seg["v"][0] != q0 + 2 * qk:
@@ -1009,7 +1045,9 @@ class HybridRunner(ModelRunner):
             resid = ops.embed_scale_f32(w.embed, b.ids, spec.embed_scale)
         for (experts, _), tables in self._tables.items():   # the expert orders of all layers, by one launch per kind of mixture
             b.routes[(experts, tables.shape[2])] = ops.TableRoutes(tables, b.ids, experts)
-        x0 = resid.clone() if spec.loop_times > 1 and not spec.loop_plain else None
+        # (not a copy of resid: a copy in a graph is no kernel and stops the queue, 16 us ahead of and behind it)
+        x0 = None if spec.loop_times <= 1 or spec.loop_plain else resid.clone() if spec.bigram is not None or self._pos_freq is not None \
+            else ops.embed_scale_f32(w.embed, b.ids, spec.embed_scale)
         pending = None                                 # a sub-layer output not yet added to the residual
         last = len(self.runs) - 1
         for ri, (li, t) in enumerate(self.runs):
@@ -1029,7 +1067,8 @@ class HybridRunner(ModelRunner):
                 pending = mixer(proj, b)
             elif mixer[0] is not None:
                 attn, delta = mixer
-                mix = (resid, attn(proj, b), lw.attn_out_norm, delta(proj, b), lw.delta_out_norm, self.eps, 0.5)
+                left, right = attn.beside(delta, proj, b) or (attn(proj, b), delta(proj, b))
+                mix = (resid, left, lw.attn_out_norm, right, lw.delta_out_norm, self.eps, 0.5)
                 if (ff is not None or L.ff) and not spec.layer_norm:
                     h, normed = ops.rms_norm_mix_norm_f32(*mix, lw.norm2), True
                 else:

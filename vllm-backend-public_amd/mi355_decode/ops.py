@@ -1514,6 +1514,63 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
     return out
 
 
+def delta_decode_ok(proj: torch.Tensor, seg: dict, num_heads: int, num_kv_heads: int, head_dim: int, v_dim: int, taps: int,
+                    a2: torch.Tensor | None, g2: torch.Tensor | None) -> bool:
+    """Whether delta_decode takes a mixer whose parts lie at seg's (offset, width) in rows of proj."""
+    if proj.dtype not in (torch.bfloat16, torch.float16) or proj.stride(1) != 1 or proj.data_ptr() % 16 or proj.stride(0) % 8 \
+            or head_dim != 128 or v_dim != 128 or num_heads // num_kv_heads > 2 or not 2 <= taps <= 4:
+        return False
+    if a2 is None:
+        return seg["g"][0] % 4 == 0
+    rank = a2.shape[1]
+    return g2.shape[1] == rank and rank % 32 == 0 and seg["a1"][0] % 8 == 0 and seg["g1"][0] % 8 == 0 \
+        and (a2.data_ptr() | g2.data_ptr()) % 16 == 0 and a2.is_contiguous() and g2.is_contiguous()
+
+
+def delta_decode(proj: torch.Tensor, seg: dict, conv_w: torch.Tensor, conv_state: torch.Tensor, a_log: torch.Tensor,
+                 dt_bias: torch.Tensor, norm_w: torch.Tensor, eps: float, activation: int, state: torch.Tensor,
+                 positions: torch.Tensor, state_slots: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, v_dim: int,
+                 a2: torch.Tensor | None = None, g2: torch.Tensor | None = None, attention: dict | None = None):
+    """causal_conv_silu, the products with a2 and g2 (a decay a channel), gated_delta_rule and gated_head_rms_norm for rows
+    that are one token of a sequence each, in one launch.  seg: (offset, width) of the columns q, k, v (adjacent), b and
+    a, g or a1, g1 in proj's rows.  attention: sigmoid_window_attn's arguments (q, k_cache, v_cache, block_tables, tok_seq, temp,
+    bias, gate, num_heads, window, scale) of an attention of the same rows that the launch takes along; its rows come first then."""
+    S, (H, G) = proj.shape[0], (num_heads, num_kv_heads)
+    C, taps = conv_w.shape
+    low = a2 is not None
+    if seg["k"][0] != seg["q"][0] + G * head_dim or seg["v"][0] != seg["k"][0] + G * head_dim or C != 2 * G * head_dim + H * v_dim:
+        raise ValueError("q | k | v must be adjacent, conv_w [their columns, taps]")
+    if tuple(state.shape[1:]) != (H, head_dim, v_dim) or tuple(conv_state.shape[1:]) != (taps - 1, C) or not conv_w.is_contiguous():
+        raise ValueError("state must be [slots, heads, head_dim, v_dim], conv_state [slots, taps - 1, channels]")
+    if low and (a2.shape[0] != H * head_dim or g2.shape[0] != H * v_dim):
+        raise ValueError("a2 and g2 must be [heads * dim, rank]")
+    out = torch.empty(S, H * v_dim, dtype=proj.dtype, device=proj.device)
+    wh = H if norm_w.numel() == H * v_dim and H > 1 else 1
+    off = lambda n, w: seg[n][0] if seg[n][0] + w <= proj.shape[1] else -1                       # noqa: E731
+    rank = a2.shape[1] if low else 0
+    launch, attn = lib.mi355_delta_decode, ()
+    if attention is not None:
+        at = attention
+        q, kc, vc, bt, gate, nh = at["q"], at["k_cache"], at["v_cache"], at["block_tables"], at["gate"], at["num_heads"]
+        if kc.shape[3] != 128 or vc.shape[2] != 128 or bt.dim() != 2 or bt.dtype != torch.int32 or not bt.is_contiguous():
+            raise ValueError("pages of 128 keys and values, block_tables contiguous int32 [chunks, max_blocks]")
+        rows = torch.empty(S, nh * 128, dtype=proj.dtype, device=proj.device)
+        launch = lib.mi355_window_delta_decode
+        attn = (rows.data_ptr(), _same(q, proj, "q"), _cols(q, "q", nh * 128), _same(kc, proj, "k_cache"), _same(vc, proj, "v_cache"),
+                bt.data_ptr(), bt.shape[1], _idx(at["tok_seq"], "tok_seq", torch.int32, S), _f32(at["temp"], "temp", nh),
+                _f32(at["bias"], "bias", nh), None if gate is None else _same(gate, proj, "gate"),
+                0 if gate is None else _cols(gate, "gate", nh), nh, kc.shape[1], int(at["window"]), float(at["scale"]))
+    check(launch(
+        *attn, out.data_ptr(), out.stride(0), proj.data_ptr(), proj.stride(0), off("q", C), off("b", H),
+        off("a1" if low else "a", rank if low else H), off("g1" if low else "g", rank if low else H * v_dim),
+        _same(conv_w, proj, "conv_w"), _f32(conv_state, "conv_state"), taps,
+        _same(a2, proj, "a2") if low else None, _same(g2, proj, "g2") if low else None, rank,
+        _f32(a_log, "a_log", H), _f32(dt_bias, "dt_bias", H * head_dim if low else H), _f32(norm_w, "norm_w", wh * v_dim), wh,
+        int(activation), float(eps), _f32(state, "state"), _idx(positions, "positions", torch.int64, S),
+        _idx(state_slots, "state_slots", torch.int32, S), S, H, G, head_dim, v_dim, _dt16(proj, "proj"), _stream()))
+    return out if attention is None else (rows, out)
+
+
 def general_delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, decay_bias: torch.Tensor,
                        rate: torch.Tensor, rate_bias: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
                        positions: torch.Tensor, state_slots: torch.Tensor, num_heads: int, head_dim: int,
