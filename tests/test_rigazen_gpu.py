@@ -502,11 +502,15 @@ def _mem_in_cuts(c, cap, cuts, tiled, rows=None, eps=1e-5, slot=1):
     return torch.cat(outs)
 
 
-def _mem_ref(c, cap, eps=1e-5):
+def _mem_ref_rows(c, cap):
     H, d = c["q"].shape[1:]
     z = c["x"].double() @ c["w"].double().T + c["b"].double()
     a, b = R.mlstm_gates(z[:, :H], z[:, H:], cap)
-    o, _ = R.mlstm_memory(c["q"].double() * d ** -0.5, c["k"].double(), c["v"].double(), a, b)
+    return R.mlstm_memory(c["q"].double() * d ** -0.5, c["k"].double(), c["v"].double(), a, b)[0]
+
+
+def _mem_ref(c, cap, eps=1e-5):
+    o = _mem_ref_rows(c, cap)
     return R.head_norm_gate(o, c["norm"].double(), c["g"].double(), eps).float()
 
 
@@ -528,6 +532,35 @@ def test_matrix_memory_in_both_forms(H, d, dv, W, cap, ib, fb):
     ref = _mem_ref(c, cap)
     for cuts, tiled in (([100, 50], True), ([1] * T, False), ([40, 2, 2, 60], True)):
         _near(_mem_in_cuts(c, cap, cuts, tiled), ref, 1e-2)
+
+
+@pytest.mark.parametrize("cuts", [[1], [16, 1], [63, 2], [64], [65, 64], [31, 1, 33, 200], [300]])
+@pytest.mark.parametrize("pad", [8, 4])
+def test_matrix_memory_of_stored_bf16_numbers_keeps_float32(cuts, pad):
+    """Heads of 128 x 128 in bfloat16 enter the products as they are stored, what is float32 as three parts; the same numbers
+    given in float32 take the general kernels, as do rows off 16 bytes (pad 4).  Each sum has at most 192 terms behind 32 steps
+    of accumulation a tile: 224 roundings of 2^-24, 1.4e-5, on either side."""
+    from mi355_decode import ops
+    H, d, cap, T = 3, 128, 15.0, sum(cuts)
+    c = _mem_case(T, H, d, d, 64, seed=T + pad, ib=-8.0, fb=5.0, dtype=torch.bfloat16)
+    z = (c["x"] @ c["w"].float().t()).cuda()
+    ref = _mem_ref_rows(c, cap)
+    states = []
+    for dtype in (torch.bfloat16, torch.float32):
+        state = torch.full((3, H, ops.linear_attn_state_floats(d, d, True)), 1e30, device="cuda")
+        mst, outs, at = torch.full((3, H), 1e30, device="cuda"), [], 0
+        for n in cuts:
+            s = slice(at, at + n)
+            buf = torch.cat([torch.zeros(n, pad, dtype=torch.bfloat16)] + [c[e][s].reshape(n, -1) for e in "qkv"], 1).to(dtype).cuda()
+            q, k, v = (buf[:, pad + i * H * d: pad + (i + 1) * H * d] for i in range(3))
+            outs.append(ops.mlstm_chunks(q, k, v, d ** -0.5, z[s].contiguous(), c["b"].float().cuda(), cap, state, mst, *_chunk(at, n, 1), H, d, d,
+                                         ops.RowTiles([0, n], 64, "cuda")))
+            at += n
+        assert (state[0] == 1e30).all() and (state[2] == 1e30).all(), "another slot was touched"
+        states.append(state[1].cpu())
+        got = torch.cat(outs).cpu().double()
+        assert float(((got - ref).norm(dim=-1) / ref.norm(dim=-1)).max()) < 2.8e-5
+    assert float((states[0] - states[1]).abs().max() / states[1].abs().max()) < 2.8e-5
 
 
 def test_matrix_memory_over_long_prompts():

@@ -426,6 +426,280 @@ __global__ __launch_bounds__(512) void la_out_kernel(
   }
 }
 
+// ---- 2 and 4 of the matrix memory for bf16 heads of 128 x 128 and tiles of 64 rows: its queries, keys and values enter as
+// they are stored, and what is fp32 -- the weighted keys, the state, the weights of P -- is split into three bf16 parts that
+// hold all of its 24 bits (split3), so that every product of a part with a stored number is exact and the sums are fp32 as
+// before.  Three 16x16x32 instructions then do in 48 cycles what eight of 16x16x4 do in 256.  What bounds them now is the states:
+// 134 MB written, rewritten by the scan and read for 8192 rows of 16 heads.  Measured there: states 98 -> 57 us, outputs 184 -> 92.
+// (fp16 parts could not hold the exponents; the constant decay's rows go through silu first and are no longer 16 bits.)
+// Parts are cut off, not rounded: a large number's first part stays finite.
+__device__ __forceinline__ void split3(float x, float y, uint32_t (&p)[3]) {      // two numbers -> their parts, packed
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
+    p[u] = a >> 16 | (b & 0xFFFF0000u);
+    x -= __uint_as_float(a & 0xFFFF0000u), y -= __uint_as_float(b & 0xFFFF0000u);
+  }
+}
+constexpr int kMemD = 128, kMemC = 64;
+constexpr int kMemT = kMemC + 8, kMemR = kMemD + 8;     // row strides in LDS of transposed and plain tiles: 16 rows of 16 bytes on all banks
+
+__global__ __launch_bounds__(256, 4) void la_states_mem_kernel(
+    float* __restrict__ ws, const uint16_t* __restrict__ k, int64_t k_stride, const uint16_t* __restrict__ v, int64_t v_stride,
+    const float* __restrict__ ga, const double* __restrict__ gf, const float* __restrict__ gm, const float* __restrict__ mstart,
+    const int32_t* __restrict__ tiles, LaDims D, int64_t total_rows, int64_t num_tiles) {
+  // half a tile at a time, so that four workgroups share a CU: one's stores travel under the others' products
+  constexpr int HC = kMemC / 2, L = HC + 8;
+  __shared__ __attribute__((aligned(16))) uint16_t Kt[3][kMemD * L], Vt[kMemD * L];              // [channel][row]
+  const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, kk = lane >> 4;
+  const int64_t row0 = MI355_LD(int32_t, tiles, tiles + 3 * tile + 1);
+  const int n = MI355_LD(int32_t, tiles, tiles + 3 * tile + 2);
+  const int64_t at = h * total_rows + row0;
+  const int r = 2 * (tid & 15), c = 8 * (tid >> 4);     // a pair of rows by 8 channels a thread
+  uint4 kr[2][2], vr[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int i = HC * t + r + e, ic = i < n ? i : n - 1;
+      kr[t][e] = MI355_LD(uint4, k, k + (row0 + ic) * k_stride + h * kMemD + c);
+      vr[t][e] = MI355_LD(uint4, v, v + (row0 + ic) * v_stride + h * kMemD + c);
+    }
+  const double Fe = MI355_LD(double, gf, gf + at + n - 1), me = MI355_LD(float, gm, gm + at + n - 1);
+  float w[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int i = HC * t + r + e, ic = i < n ? i : n - 1;
+      const double x = Fe - MI355_LD(double, gf, gf + at + ic) + static_cast<double>(MI355_LD(float, ga, ga + at + ic)) - me;
+      w[t][e] = i < n ? expf(static_cast<float>(x)) : 0.f;             // (rows past the end: keys of zero)
+    }
+  if (tid == 0) {                                       // the factor on the tile's incoming state, for la_scan
+    const double m0 = MI355_LD(float, mstart, mstart + static_cast<int64_t>(tile) * D.H + h);
+    MI355_ST(float, ws, ws + num_tiles * D.H * D.us + static_cast<int64_t>(tile) * D.H + h, expf(static_cast<float>(Fe + m0 - me)));
+  }
+  // wave: 32 channels of the keys by all of the values; a lane's four numbers are adjacent values of one channel
+  f32x4 acc[2][8], sum[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (t > 0) __syncthreads();                         // the first half has been read
+    float k0[8], k1[8];
+    unpack8<BF16>(kr[t][0], k0), unpack8<BF16>(kr[t][1], k1);
+    const uint32_t v0[4] = {vr[t][0].x, vr[t][0].y, vr[t][0].z, vr[t][0].w}, v1[4] = {vr[t][1].x, vr[t][1].y, vr[t][1].z, vr[t][1].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int to = (c + e) * L + r;
+      uint32_t p[3];
+      split3(k0[e] * w[t][0], k1[e] * w[t][1], p);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) *reinterpret_cast<uint32_t*>(&Kt[u][to]) = p[u];
+      const uint32_t a = v0[e >> 1] >> (16 * (e & 1)), b = v1[e >> 1] >> (16 * (e & 1));
+      *reinterpret_cast<uint32_t*>(&Vt[to]) = (a & 0xFFFFu) | b << 16;
+    }
+    __syncthreads();
+    uint4 kf[2][3];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        kf[i][u] = *reinterpret_cast<const uint4*>(&Kt[u][(wave * 32 + 16 * i + li) * L + 8 * kk]);
+        sum[i] = BF16::mfma(ones, kf[i][u], sum[i]);
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint4 vf = *reinterpret_cast<const uint4*>(&Vt[(16 * j + li) * L + 8 * kk]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) acc[i][j] = BF16::mfma(vf, kf[i][u], acc[i][j]);
+    }
+  }
+  float* U = ws + (static_cast<int64_t>(tile) * D.H + h) * D.us;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int ch = wave * 32 + 16 * i + li;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      MI355_ST(float4, ws, U + ch * kMemD + 16 * j + 4 * kk, make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]));
+    if (kk == 0) MI355_ST(float, ws, U + kMemD * kMemD + ch, sum[i][0]);
+  }
+}
+
+__global__ __launch_bounds__(512, 2) void la_out_mem_kernel(
+    float* __restrict__ o, const float* __restrict__ ws, const uint16_t* __restrict__ q, int64_t q_stride,
+    const uint16_t* __restrict__ k, int64_t k_stride, const uint16_t* __restrict__ v, int64_t v_stride, float q_scale,
+    const float* __restrict__ ga, const double* __restrict__ gf, const float* __restrict__ gm, const float* __restrict__ mstart,
+    const int32_t* __restrict__ tiles, LaDims D, int64_t total_rows) {
+  __shared__ __attribute__((aligned(16))) uint16_t Qs[kMemC * kMemR], Vt[kMemD * kMemT];
+  __shared__ __attribute__((aligned(16))) uint16_t KP[3 * kMemC * kMemT];       // the keys, then the parts of P
+  __shared__ double Fr[kMemC];
+  __shared__ float ar[kMemC], mr[kMemC], er[kMemC], dr[kMemC], psum[4][kMemC], nv[kMemD];
+  static_assert(3 * kMemC * kMemT >= kMemC * kMemR, "the keys fit where P goes");
+  const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, kk = lane >> 4;
+  const int64_t row0 = MI355_LD(int32_t, tiles, tiles + 3 * tile + 1);
+  const int n = MI355_LD(int32_t, tiles, tiles + 3 * tile + 2);
+  const float* S = ws + (static_cast<int64_t>(tile) * D.H + h) * D.us;
+  // ---- all loads out: rows of q and k, pairs of rows of v, this wave's 16 columns of the incoming state
+  uint4 qr[2], kr[2], vr[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int i = (tid >> 4) + 32 * e, c = 8 * (tid & 15), ic = i < n ? i : n - 1;
+    qr[e] = MI355_LD(uint4, q, q + (row0 + ic) * q_stride + h * kMemD + c);
+    kr[e] = MI355_LD(uint4, k, k + (row0 + ic) * k_stride + h * kMemD + c);
+    const int j = 2 * (tid & 31) + e;
+    vr[e] = MI355_LD(uint4, v, v + (row0 + (j < n ? j : n - 1)) * v_stride + h * kMemD + 8 * (tid >> 5));
+  }
+  float st[4][8];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) st[ks][e] = MI355_LD(float, ws, S + (32 * ks + 8 * kk + e) * kMemD + 16 * wave + li);
+  if (tid < kMemC) {
+    const int i = tid < n ? tid : n - 1;
+    const int64_t at = h * total_rows + row0 + i;
+    const double F = MI355_LD(double, gf, gf + at), m0 = MI355_LD(float, mstart, mstart + static_cast<int64_t>(tile) * D.H + h);
+    const float m = MI355_LD(float, gm, gm + at);
+    Fr[tid] = F, ar[tid] = MI355_LD(float, ga, ga + at), mr[tid] = m;
+    er[tid] = expf(static_cast<float>(F + m0 - static_cast<double>(m)));
+  } else if (tid < kMemC + kMemD) {
+    nv[tid - kMemC] = MI355_LD(float, ws, S + kMemD * kMemD + tid - kMemC);
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int i = (tid >> 4) + 32 * e, c = 8 * (tid & 15);
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(&Qs[i * kMemR + c]) = i < n ? qr[e] : zero;
+    *reinterpret_cast<uint4*>(&KP[i * kMemR + c]) = i < n ? kr[e] : zero;
+  }
+  {
+    const int j = 2 * (tid & 31), c = 8 * (tid >> 5);
+    const uint32_t v0[4] = {vr[0].x, vr[0].y, vr[0].z, vr[0].w}, v1[4] = {vr[1].x, vr[1].y, vr[1].z, vr[1].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t a = v0[e >> 1] >> (16 * (e & 1)), b = v1[e >> 1] >> (16 * (e & 1));
+      *reinterpret_cast<uint32_t*>(&Vt[(c + e) * kMemT + j]) = (j < n ? a & 0xFFFFu : 0u) | (j + 1 < n ? b << 16 : 0u);
+    }
+  }
+  __syncthreads();
+  // ---- P = (Q K^T) under the decay weights: blocks on and below the diagonal, and the two above it that a step of 32 columns meets
+  float p[2][4];
+  int pi[2], pj[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int blk = wave + 8 * t;
+    int bi = 0, bj = blk;
+    if (blk < 10) {
+      while (bj > bi) bj -= ++bi;                       // blk = bi (bi + 1) / 2 + bj
+    } else {
+      bi = blk == 10 ? 0 : 2, bj = bi + 1;
+    }
+    pi[t] = bi, pj[t] = bj;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[t][r] = 0.f;
+    if (blk >= 10) continue;
+    f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      x = BF16::mfma(*reinterpret_cast<const uint4*>(&Qs[(16 * bi + li) * kMemR + 32 * ks + 8 * kk]),
+                     *reinterpret_cast<const uint4*>(&KP[(16 * bj + li) * kMemR + 32 * ks + 8 * kk]), x);
+    const int j = 16 * bj + li;
+    const double Fj = Fr[j], aj = ar[j];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * bi + 4 * kk + r;
+      if (j <= i && i < n) p[t][r] = expf(static_cast<float>(Fr[i] - Fj + aj - static_cast<double>(mr[i]))) * (x[r] * q_scale);
+      float sum = p[t][r];
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
+      if (li == 0) psum[bj][i] = sum;
+    }
+  }
+  // n . q of every row, 8 lanes a row
+  float nq = 0.f;
+  {
+    const int i = tid >> 3, c = 16 * (tid & 7);
+    float f[8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      unpack8<BF16>(*reinterpret_cast<const uint4*>(&Qs[i * kMemR + c + 8 * u]), f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nq += nv[c + 8 * u + e] * (f[e] * q_scale);
+    }
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) nq += __shfl_xor(nq, off, 64);
+  }
+  // the state's parts: the left operand of the products, this wave's columns as its rows
+  uint4 sf[4][3];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    uint32_t s[4][3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split3(st[ks][2 * e], st[ks][2 * e + 1], s[e]);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) sf[ks][u] = make_uint4(s[0][u], s[1][u], s[2][u], s[3][u]);
+  }
+  __syncthreads();                                      // the keys have been read, the sums of P written
+  if ((tid & 7) == 0) {
+    const int i = tid >> 3;
+    float sum = er[i] * nq;
+    for (int b = 0; b <= i >> 4; ++b) sum += psum[b][i];
+    dr[i] = 1.0f / (fmaxf(fabsf(sum), expf(-mr[i])) + 1e-6f);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (wave + 8 * t >= 12) continue;
+#pragma unroll
+    for (int r = 0; r < 4; r += 2) {
+      uint32_t s[3];
+      split3(p[t][r], p[t][r + 1], s);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        uint16_t* to = &KP[(u * kMemC + 16 * pi[t] + 4 * kk + r) * kMemT + 16 * pj[t] + li];
+        to[0] = static_cast<uint16_t>(s[u] & 0xFFFFu), to[kMemT] = static_cast<uint16_t>(s[u] >> 16);
+      }
+    }
+  }
+  __syncthreads();
+  const uint4 vf[2] = {*reinterpret_cast<const uint4*>(&Vt[(16 * wave + li) * kMemT + 8 * kk]),
+                       *reinterpret_cast<const uint4*>(&Vt[(16 * wave + li) * kMemT + 32 + 8 * kk])};
+  const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+  for (int bi = 0; bi < 4; ++bi) {
+    const int i = 16 * bi + li;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const uint4 qf = *reinterpret_cast<const uint4*>(&Qs[i * kMemR + 32 * ks + 8 * kk]);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) acc = BF16::mfma(sf[ks][u], qf, acc);
+    }
+    const float e = er[i] * q_scale;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] *= e;
+#pragma unroll
+    for (int ks = 0; ks <= bi >> 1; ++ks) {
+      const uint4 vu = 2 * ks + 1 <= bi || kk < 2 ? vf[ks] : none;      // (values of the block above the diagonal: no row's to see)
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        acc = BF16::mfma(vu, *reinterpret_cast<const uint4*>(&KP[(u * kMemC + i) * kMemT + 32 * ks + 8 * kk]), acc);
+    }
+    const float f = dr[i];
+    if (i < n)
+      MI355_ST(float4, o, o + ((row0 + i) * D.H + h) * kMemD + 16 * wave + 4 * kk,
+               make_float4(acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f));
+  }
+}
+
 // ---- chunks of a few tokens: one workgroup per (chunk, head), the state updated in place
 struct LaStepMem {                // matrix memory only: what its gates, norm and output gate read
   const float* x;                 // fp32 rows the gate projections read
@@ -670,6 +944,17 @@ extern "C" int32_t mi355_linear_attn_chunks(float* o, const void* q, int64_t q_s
   const dim3 grid(num_tiles, num_heads);
   const size_t lds_states = la_states_lds(tile_rows, head_dim, v_dim), lds_out = la_out_lds(tile_rows, head_dim, v_dim);
   const dim3 sgrid((D.us / 4 + 255) / 256, num_heads, num_seqs);
+  if (mem && dtype == MI355_BF16 && vec && head_dim == kMemD && v_dim == kMemD && tile_rows == kMemC && aligned16(o)) {
+    hipLaunchKernelGGL(la_states_mem_kernel, grid, dim3(256), 0, s, workspace, static_cast<const uint16_t*>(k), k_stride,
+                       static_cast<const uint16_t*>(v), v_stride, log_in, log_decay_sum, running_max, tile_max, tiles, D, num_tokens,
+                       static_cast<int64_t>(num_tiles));
+    hipLaunchKernelGGL(la_scan_kernel, sgrid, dim3(256), 0, s, workspace, state, cu_seqlens, positions, state_slots, tile_start, D,
+                       static_cast<int64_t>(num_tiles));
+    hipLaunchKernelGGL(la_out_mem_kernel, grid, dim3(512), 0, s, o, workspace, static_cast<const uint16_t*>(q), q_stride,
+                       static_cast<const uint16_t*>(k), k_stride, static_cast<const uint16_t*>(v), v_stride, q_scale, log_in, log_decay_sum,
+                       running_max, tile_max, tiles, D, num_tokens);
+    return check_launch("linear_attn_chunks (bf16)");
+  }
 #define MI355_LA(TT, MM)                                                                                                       \
   do {                                                                                                                         \
     typedef Elem<TT>::S E;                                                                                                     \
