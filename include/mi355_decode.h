@@ -577,6 +577,9 @@ int32_t mi355_untile_weights_fp8(void* dst, const void* src_tiled, const float* 
  *               (mi355_fused_add_rms_norm_partial, mi355_rope_kv_write_partial,
  *               mi355_sum_slabs, mi355_silu_and_mul_slabs)
  *               add the slabs in order, so results do not depend on scheduling.
+ *   epilogue 5: weights tiled as they are, gate rows ahead of up rows; y[M, N/2] =
+ *               round(gelu_tanh(round(gate)) * round(up))    (304, M <= 64, N % 32 == 0,
+ *               no bias, rows on 8-byte boundaries)
  * Same role as mi355_linear_decode (the engine's decode GEMMs, --max-num-seqs,
  * vllm_templates.py:53) with the weight layout chosen for this chip.
  */

@@ -1073,6 +1073,27 @@ def test_rows_of_products_split_over_waves(M, N, K):
     assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(32, 1024), (96, 2048), (2080, 512), (8192, 2048), (8224, 1024)])
+def test_gelu_in_the_product(dtype, M, N, K):
+    """Gate and up rounded to 16 bits ahead of the gate, one rounding after it, as by two launches: a 16-bit number of either
+    may fall the other way (2^-8 or 2^-11 of it; GELU's slope is below 1.13 and its value at least a tenth of the gate's
+    above -1.3: beyond, the gate's own half ulp counts against |gate up|)."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(N + M)
+    x, w = torch.randn(M, K, generator=g).to(dtype).cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).cuda()
+    if K % ops.tiled_slice_width(M, 304):
+        assert not ops.gelu_in_product(N, K, M)
+        return
+    assert ops.gelu_in_product(N, K, M) == (N <= 8192)
+    got = ops.linear_tiled(x, ops.tile_weights(w), N, tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL).double()
+    gate, up = (x.double() @ w.double().t()).split(N // 2, dim=1)
+    want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert ((got - want).abs() <= 4 * eps * (gate * up).abs() + 1e-5).all()
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3)])
 @pytest.mark.parametrize("B,H,G,taps,rank", [(1, 2, 1, 4, 0), (5, 16, 8, 4, 0), (3, 3, 3, 2, 0), (33, 8, 4, 4, 128), (2, 4, 4, 3, 32), (4, 2, 1, 2, 64)])
 def test_delta_mixer_of_single_tokens_in_one_launch(dtype, tol, B, H, G, taps, rank):

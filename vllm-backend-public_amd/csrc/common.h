@@ -98,6 +98,11 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
   return s * u;
 }
 
+// GELU in its tanh form, g sigmoid(2 sqrt(2 / pi) (g + 0.044715 g^3))
+__device__ __forceinline__ float gelu_tanh_fast(float g) {
+  return g * __frcp_rn(1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)));
+}
+
 // 8 packed 16-bit words <-> 8 floats
 template <typename T>
 __device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {

@@ -28,6 +28,8 @@
 //                 2u+1): act = round(round(silu(round(gate))) * round(up))
 //   EPI_PARTIAL   fp32 partial sums to slab [kgroup][M][N] (K split over
 //                 workgroups; the consumer kernel adds the slabs in order)
+//   EPI_GELU_MUL  (K split over waves only) rows 0 .. N/2 are gates, the others their ups:
+//                 round(gelu_tanh(round(gate)) * round(up))
 //   EPI_REDUCE_STORE / EPI_REDUCE_RESID   K split over workgroups, finished in the
 //                 same launch: every workgroup writes its slab, then takes a ticket
 //                 from a per-column-group counter; the workgroup that draws the last
@@ -47,7 +49,7 @@ namespace mi355 {
 constexpr int kTU = 4;  // k-steps per register group
 constexpr int kMaxRows = 256;  // rows of x a launch takes: one or two row blocks of up to 128
 
-enum { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_PARTIAL = 2, EPI_REDUCE_STORE = 3, EPI_REDUCE_RESID = 4 };
+enum { EPI_STORE = 0, EPI_SILU_MUL = 1, EPI_PARTIAL = 2, EPI_REDUCE_STORE = 3, EPI_REDUCE_RESID = 4, EPI_GELU_MUL = 5 };
 
 constexpr int kSumsqRows = 32;  // row pitch of the sum-of-squares tables ([column group][32])
 
@@ -678,7 +680,8 @@ __global__ __launch_bounds__(512) void linear_tiled_kw_kernel(
   constexpr int D = 2;
   constexpr int PU = GL >= D ? 1 : D / GL;     // phases per main-loop iteration: ring slots stay compile-time
   static_assert(G % KW == 0 && GL >= 1 && (PU * GL) % D == 0, "ring slots must repeat every main-loop iteration");
-  static_assert(EPI != EPI_SILU_MUL || TPG % 2 == 0, "gate and up tiles of a column block share a workgroup");
+  constexpr bool GATED = EPI == EPI_SILU_MUL || EPI == EPI_GELU_MUL;
+  static_assert(!GATED || TPG % 2 == 0, "gate and up tiles of a column block share a workgroup");
   static_assert(2 * XBUF >= NW * MT * 4 * 64 * 4, "the reduction reuses the x buffers");
   static_assert(NT % (KSL / 8) == 0, "a thread must keep one column of the x slice");
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * XBUF];
@@ -691,7 +694,8 @@ __global__ __launch_bounds__(512) void linear_tiled_kw_kernel(
   const int tl = wave / KW, kq = wave % KW;
   const int c = lane & 15, h = lane >> 4;
   const int tile_raw = blockIdx.x * TPG + tl;
-  const int tile = min(tile_raw, tiles_total - 1);
+  // (gates and ups in halves: the tiles of a pair lie half a matrix apart)
+  const int tile = min(EPI == EPI_GELU_MUL ? (tile_raw >> 1) + (tile_raw & 1) * (tiles_total >> 1) : tile_raw, tiles_total - 1);
   const int kgroup = blockIdx.y;
   MI355_ROW_BLOCK();
 
@@ -778,7 +782,7 @@ __global__ __launch_bounds__(512) void linear_tiled_kw_kernel(
   // ---- the partial accumulators of a tile meet in LDS (the x buffers are dead): [wave][m-tile][r][lane]
   __syncthreads();
   float* red = reinterpret_cast<float*>(lds);
-  const bool lead = kq == 0 && (EPI != EPI_SILU_MUL || (tl & 1) == 0);
+  const bool lead = kq == 0 && (!GATED || (tl & 1) == 0);
   if (!lead) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -794,7 +798,7 @@ __global__ __launch_bounds__(512) void linear_tiled_kw_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[m][r] += red[(((wave + j) * MT + m) * 4 + r) * 64 + lane];
 
-  if (EPI == EPI_SILU_MUL) {                             // this wave: the gate tile; waves wave + KW ...: the up tile
+  if (GATED) {                                           // this wave: the gate tile; waves wave + KW ...: the up tile
     if (tile_raw + 1 >= tiles_total) return;
     const int F = N >> 1;
     const int j0 = (tile_raw >> 1) * 16 + 4 * h;
@@ -808,7 +812,8 @@ __global__ __launch_bounds__(512) void linear_tiled_kw_kernel(
         float up = 0.f;
 #pragma unroll
         for (int j = 0; j < KW; ++j) up += red[(((wave + KW + j) * MT + m) * 4 + r) * 64 + lane];
-        o[r] = silu_mul<T>(round_f<T>(acc[m][r]), round_f<T>(up));
+        const float g = round_f<T>(acc[m][r]), u = round_f<T>(up);
+        o[r] = EPI == EPI_GELU_MUL ? gelu_tanh_fast(g) * u : silu_mul<T>(g, u);
       }
       uint16_t* yp = y + static_cast<int64_t>(mm) * y_stride + j0;
       if (j0 + 3 < F) {
@@ -1113,6 +1118,9 @@ static bool launch_cfg_kw(int epi, dim3 grid, hipStream_t s, MI355_LT_PARAMS) {
   if constexpr (KW <= 4) {
     if (epi == EPI_SILU_MUL) { MI355_LTKW(EPI_SILU_MUL); return true; }
   }
+  if constexpr (KW == 4 && KSL * (MT < 2 ? 2 : MT) == 2048) {        // (code 304)
+    if (epi == EPI_GELU_MUL) { MI355_LTKW(EPI_GELU_MUL); return true; }
+  }
 #undef MI355_LTKW
   return false;
 }
@@ -1148,7 +1156,7 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
   MI355_REQUIRE(M >= 0 && M <= kMaxRows, MI355_ERR_UNSUPPORTED, "%s: M %d outside [0, %d]", name, M, kMaxRows);
   MI355_REQUIRE(M <= 128 || (!norm && !reduce), MI355_ERR_UNSUPPORTED,
                 "%s: the norm prologue and the in-launch reduction are built for up to 128 rows (M %d)", name, M);
-  MI355_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_REDUCE_RESID, MI355_ERR_INVALID, "%s: unknown epilogue %d",
+  MI355_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_GELU_MUL, MI355_ERR_INVALID, "%s: unknown epilogue %d",
                 name, epilogue);
   // tiles_per_wg: 4 or 8 tiles (= waves) per workgroup; +100 selects the narrow x slice.  The slice is
   // 1024 (narrow: 512) wide up to 32 rows and halves with every doubling of the rows, so that the
@@ -1177,6 +1185,9 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
                 "402; up to 128 rows: 302)", name, tiles_per_wg % 100, (tiles_per_wg % 100) * 128, M, ksl);
   MI355_REQUIRE(!kws || epilogue != EPI_SILU_MUL || tiles_per_wg % 100 <= 4, MI355_ERR_UNSUPPORTED,
                 "%s: the SwiGLU epilogue needs the gate and up tiles in one workgroup: at most 4 waves per tile", name);
+  MI355_REQUIRE(epilogue != EPI_GELU_MUL || (tiles_per_wg == 304 && M <= 64 && N % 32 == 0 && bias == nullptr && y_stride % 4 == 0 &&
+                                             (reinterpret_cast<uintptr_t>(y) & 7) == 0), MI355_ERR_UNSUPPORTED,
+                "%s: the GELU epilogue is built for tiles_per_wg 304, up to 64 rows, N %% 32 == 0, no bias and rows on 8-byte boundaries", name);
   MI355_REQUIRE(!two || (M > 32 && !norm && !reduce), MI355_ERR_UNSUPPORTED,
                 "%s: two tiles per wave (tiles_per_wg %d) is built for 33 rows and more and epilogues 0-2", name, tiles_per_wg);
   MI355_REQUIRE(N > 0 && K > 0 && K % ksl == 0, MI355_ERR_UNSUPPORTED,
@@ -1209,8 +1220,9 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
                       M <= 32,
                   MI355_ERR_INVALID,
                   "%s: residual (16-byte aligned, stride >= N, multiple of 8), sumsq_out and M <= 32 needed", name);
-  if (epilogue == EPI_STORE || epilogue == EPI_SILU_MUL || epilogue == EPI_REDUCE_STORE)
-    MI355_REQUIRE(y && y_stride >= (epilogue == EPI_SILU_MUL ? N / 2 : N) &&
+  const bool gated = epilogue == EPI_SILU_MUL || epilogue == EPI_GELU_MUL;
+  if (epilogue == EPI_STORE || gated || epilogue == EPI_REDUCE_STORE)
+    MI355_REQUIRE(y && y_stride >= (gated ? N / 2 : N) &&
                       (epilogue != EPI_REDUCE_STORE || (aligned16(y) && y_stride % 8 == 0)),
                   MI355_ERR_INVALID, "%s: y missing, misaligned or y_stride too small", name);
   if (epilogue == EPI_SILU_MUL)
@@ -1321,7 +1333,7 @@ extern "C" int32_t mi355_linear_tiled(void* y, int64_t y_stride, void* partial, 
                                       void* stream) {
   using namespace mi355;
   const char* name = "mi355_linear_tiled";
-  MI355_REQUIRE(epilogue == EPI_STORE || epilogue == EPI_SILU_MUL || epilogue == EPI_PARTIAL, MI355_ERR_INVALID,
+  MI355_REQUIRE(epilogue == EPI_STORE || epilogue == EPI_SILU_MUL || epilogue == EPI_PARTIAL || epilogue == EPI_GELU_MUL, MI355_ERR_INVALID,
                 "%s: unknown epilogue %d", name, epilogue);
   return linear_tiled_launch(name, y, y_stride, static_cast<float*>(partial), x, x_stride, w_tiled, bias, M, N, K,
                              tiles_per_wg, k_groups, epilogue, FusedArgs{}, dtype, stream);

@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_and_mul_vec_kernel(uint16_t* __
     xg.value(g, num_slabs), xu.value(u, num_slabs);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      y[j] = g[j] * __frcp_rn(1.0f + __expf(-1.5957691216057308f * (g[j] + 0.044715f * g[j] * g[j] * g[j]))) * u[j];
+      y[j] = gelu_tanh_fast(g[j]) * u[j];
     MI355_ST(uint4, out, out + row * inter + 8 * v, pack8<T>(y));
   }
 }

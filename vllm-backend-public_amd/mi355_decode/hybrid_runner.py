@@ -969,6 +969,14 @@ class HybridRunner(ModelRunner):
             return torch.mm(x, w.t())
         return torch.mm(x, w.t(), out=out)
 
+    def gelu_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """gelu_tanh(gate) * up of x @ w.T, gate rows of w ahead of up rows; in one launch where that is the faster way."""
+        tw = self._tiled_w.get(w.data_ptr())
+        if tw is not None and tw.dtype == x.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 \
+                and ops.gelu_in_product(w.shape[0], w.shape[1], x.shape[0]):
+            return ops.linear_tiled(x, tw, w.shape[0], tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL)
+        return ops.gelu_tanh_and_mul(self.linear(x, w, slabs=True))
+
     def out_linear(self, x: torch.Tensor, w: torch.Tensor):
         """A sub-layer's last product.  In the pre arrangement its consumers (the norms that it is added ahead of, the mix)
         add a K-split product's slabs themselves: 4 to 5 us a launch saved for decoded rows."""
@@ -1082,7 +1090,7 @@ class HybridRunner(ModelRunner):
             elif ff is not None:
                 pending = ff(h)
             elif L.ff:
-                pending = self.out_linear(ops.gelu_tanh_and_mul(self.linear(h, lw.gate_up_w, slabs=True)), lw.down_w)
+                pending = self.out_linear(self.gelu_linear(h, lw.gate_up_w), lw.down_w)
             if pending is not None and (self.layer_trace is not None or (ri == last and not b.keep_tail)):
                 self._norm(resid, None, pending)
                 pending = None

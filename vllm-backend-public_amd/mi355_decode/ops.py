@@ -656,7 +656,7 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     return out
 
 
-EPI_STORE, EPI_SILU_MUL, EPI_PARTIAL, EPI_REDUCE_STORE, EPI_REDUCE_RESID = 0, 1, 2, 3, 4
+EPI_STORE, EPI_SILU_MUL, EPI_PARTIAL, EPI_REDUCE_STORE, EPI_REDUCE_RESID, EPI_GELU_MUL = 0, 1, 2, 3, 4, 5
 SUMSQ_ROWS = 32                      # row pitch of the sum-of-squares tables
 LINEAR_TILED_MAX_M = 256             # beyond 128 rows: two row blocks of one launch
 
@@ -734,6 +734,14 @@ def plan_linear_rows(N: int, K: int, M: int):
     else:
         code = 304 if M <= 64 and (tiles_total > 256 or K <= max(512, N // 2)) else 0
     return (code, 1) if code and K % tiled_slice_width(M, code) == 0 else None
+
+
+def gelu_in_product(N: int, K: int, M: int) -> bool:
+    """Whether gelu_tanh(gate) * up of an [N, K] product (gate rows ahead of up rows) costs less in the product's own epilogue
+    (EPI_GELU_MUL, a workgroup a tile of gates and its ups) than in a launch behind it.  While one round of workgroups
+    covers the matrix and a wave's quarter of K is short (us, two launches / one: 8192 x 2048 10.7 / 8.9 at 16 rows, 11.5 / 10.1 at
+    32, 14.6 / 13.1 at 64; 4096 x 1024 6.9 / 5.0, 9.2 / 7.6 at 64).  Beyond: 16384 x 2048 16.9 / 18.6 at 32 rows, 4096 x 4096 11.8 / 12.8."""
+    return M <= 64 and N % 32 == 0 and N <= 8192 and K <= 2048 and K % tiled_slice_width(M, 304) == 0
 
 
 def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: bool = False):
@@ -833,7 +841,7 @@ def linear_tiled(x: torch.Tensor, w_tiled: torch.Tensor, N: int, bias: torch.Ten
                  out: torch.Tensor | None = None, partial: torch.Tensor | None = None, tiles_per_wg: int = 0,
                  k_groups: int = 1, epilogue: int = EPI_STORE):
     """y = x @ W.T on fragment-tiled weights (M <= 256).  Returns `out`
-    ([M, N], or [M, N/2] with the SwiGLU epilogue) or `partial` ([k_groups, M, N] fp32)."""
+    ([M, N], or [M, N/2] with the SwiGLU and GELU epilogues) or `partial` ([k_groups, M, N] fp32)."""
     dt = _dt16(x, "x")
     _dev(w_tiled, "w_tiled")
     M, K = x.shape
@@ -852,7 +860,7 @@ def linear_tiled(x: torch.Tensor, w_tiled: torch.Tensor, N: int, bias: torch.Ten
         p_ptr = partial.data_ptr()
         ret = partial
     else:
-        width = N // 2 if epilogue == EPI_SILU_MUL else N
+        width = N // 2 if epilogue in (EPI_SILU_MUL, EPI_GELU_MUL) else N
         if out is None:
             out = torch.empty((M, width), dtype=x.dtype, device=x.device)
         elif out.dtype != x.dtype or tuple(out.shape) != (M, width):
