@@ -190,6 +190,26 @@ def test_expert_orders_from_tables(E, top, V, T, L):
         assert torch.equal(want[perm], torch.repeat_interleave(torch.arange(E), counts).to(torch.int32))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts", [[1], [0, 16, 0, 1], [17, 3, 33, 0]])
+@pytest.mark.parametrize("N,K", [(16, 32), (48, 96), (80, 128), (64, 416), (16, 512), (208, 1664), (32, 2112)])
+def test_expert_rows_with_inputs_split_over_waves(dtype, counts, N, K):
+    """Waves without a whole step of inputs, remainders behind the last step, experts without rows, and row blocks that end
+    anywhere: one rounding of the fp32 sum."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(N + K)
+    rows, E = sum(counts), len(counts)
+    x, w = torch.randn(rows, K, generator=g).to(dtype), (torch.randn(E, N, K, generator=g) * K ** -0.5).to(dtype)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    perm = torch.randperm(rows, generator=g).to(torch.int32)
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for p in (None, perm):
+        got = ops.moe_linear_rows(x.cuda(), w.cuda(), off.cuda(), rows, perm=None if p is None else p.cuda()).cpu().double()
+        xs = (x if p is None else x[p.long()]).double()
+        want = torch.cat([xs[off[e]: off[e + 1]] @ w[e].double().t() for e in range(E)])
+        assert ((got - want).abs() <= eps * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("E,top,T,W,F", [(4, 1, 600, 64, 96), (6, 2, 37, 96, 64), (5, 3, 300, 72, 40), (3, 2, 9, 90, 30), (9, 2, 1, 32, 16),
                                          (2, 1, 500, 136, 200)])

@@ -457,18 +457,25 @@ __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(uint16_t* __restr
   }
 }
 
+// A workgroup 16 outputs of an expert, its four waves a quarter of the inputs each (sums added in wave order): a wave with all
+// inputs of 16 outputs walks 64 KB one stage behind the other, and a few experts leave most of the chip without a wave.
+// Rows of x are read by the lanes that have one: with 1 to 4 rows an expert 12 to 15 of 16 lanes would fetch what nobody
+// reads, as many bytes through the cache as the weights.  32 experts of 2048 -> 1536 / 1536 -> 2048, 4 a token, bf16, us: 1 token
+// 19.9 / 9.4 -> 10.0 / 9.4, 5 tokens 30.9 / 32.3 -> 17.0 / 20.1, 32 tokens 41.6 / 39.9 -> 36.8 / 37.1 (5.3 TB/s), 200 tokens 101.7 / 92.4 ->
+// 85.9 / 85.0; either change alone: the split 40.5 / 43.1 at 32 tokens, the lanes 45.3 / 40.2.
 template <typename T>
 __global__ __launch_bounds__(256) void moe_down_mfma_kernel(uint16_t* __restrict__ y, const uint16_t* __restrict__ a,
                                                             const uint16_t* __restrict__ w_down,
                                                             const int32_t* __restrict__ offsets,
                                                             const int32_t* __restrict__ perm, int top, int relu2, int W, int F) {
+  __shared__ f32x4 part[3][64];
   const int e = blockIdx.y, lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
-  const int c0 = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 16;
-  if (c0 >= W) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c0 = blockIdx.x * 16;
   const int lo = MI355_LD(int32_t, offsets, offsets + e), hi = MI355_LD(int32_t, offsets, offsets + e + 1);
   const uint16_t* wd = w_down + (static_cast<int64_t>(e) * W + c0 + li) * F + 8 * kk;
   for (int p0 = lo; p0 < hi; p0 += 16) {
-    const uint16_t* ar = a + input_row(perm, top, p0 + li < hi ? p0 + li : p0) * F + 8 * kk;
+    const bool mine = p0 + li < hi;                       // (a column past the expert's last row may hold anything)
+    const uint16_t* ar = a + input_row(perm, top, mine ? p0 + li : p0) * F + 8 * kk;
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, acc2 = f32x4{0.f, 0.f, 0.f, 0.f};     // two chains of products in turn
     // bound by the weights' way from HBM: stages of 4 k-steps, the next one's loads in flight while one is multiplied
     // (32 experts of 1536 x 2048 in bf16, 201 MB: 51 us with a k-step's loads in flight, 40 with these; 2 a stage 45, 6 or 8
@@ -477,12 +484,13 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(uint16_t* __restrict
     struct Stage {
       uint4 w[U], x[U];
     };
-    Stage s0, s1;
+    Stage s0 = {}, s1 = {};
     auto load = [&](Stage& st, int i) {
 #pragma unroll
-      for (int j = 0; j < U; ++j) {
-        st.w[j] = MI355_LD(uint4, w_down, wd + (i * U + j) * 32);
-        st.x[j] = MI355_LD(uint4, a, ar + (i * U + j) * 32);
+      for (int j = 0; j < U; ++j) st.w[j] = MI355_LD(uint4, w_down, wd + (i * U + j) * 32);
+      if (mine) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) st.x[j] = MI355_LD(uint4, a, ar + (i * U + j) * 32);
       }
     };
     auto mma = [&](const Stage& st) {
@@ -492,10 +500,10 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(uint16_t* __restrict
         acc2 = T::mfma(st.w[j + 1], st.x[j + 1], acc2);
       }
     };
-    const int n = F / (32 * U);
-    if (n > 0) {
-      load(s0, 0);
-      int i = 0;
+    const int all = F / (32 * U), n = all * (wave + 1) / 4;
+    int i = all * wave / 4;
+    if (i < n) {
+      load(s0, i);
       for (; i + 2 < n; i += 2) {
         load(s1, i + 1);
         mma(s0);
@@ -510,13 +518,21 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(uint16_t* __restrict
         mma(s0);
       }
     }
-    for (int s = n * 32 * U; s < F; s += 64) {
+    for (int s = wave == 3 ? all * 32 * U : F; s < F; s += 64) {
       acc = T::mfma(MI355_LD(uint4, w_down, wd + s), MI355_LD(uint4, a, ar + s), acc);
       if (s + 32 < F) acc2 = T::mfma(MI355_LD(uint4, w_down, wd + s + 32), MI355_LD(uint4, a, ar + s + 32), acc2);
     }
+    acc += acc2;
+    if (wave > 0) part[wave - 1][lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 0; w < 3; ++w) acc += part[w][lane];
+    }
+    __syncthreads();                                      // (the next 16 rows' sums)
+    if (wave > 0) continue;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      acc[r] += acc2[r];
       if (relu2) acc[r] = relu2_f(round_f<T>(acc[r]));        // (of the product as a 16-bit buffer would hold it)
     }
     if (p0 + li < hi)
@@ -716,7 +732,7 @@ static int32_t launch_moe_linear_rows(const char* name, void* y, const void* x, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>((out_width + 3) / 4), static_cast<unsigned>(experts));
   if (dtype != MI355_F32 && in_width % 32 == 0 && out_width % 16 == 0 && aligned16(x) && aligned16(w) && aligned16(y)) {
-    const dim3 mgrid(static_cast<unsigned>((out_width / 16 + 3) / 4), static_cast<unsigned>(experts));
+    const dim3 mgrid(static_cast<unsigned>(out_width / 16), static_cast<unsigned>(experts));
     if (dtype == MI355_BF16)
       hipLaunchKernelGGL((moe_down_mfma_kernel<BF16>), mgrid, dim3(256), 0, s, static_cast<uint16_t*>(y),
                          static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), offsets, perm, top, relu2, out_width,
