@@ -557,8 +557,10 @@ class ExpertRows:
         self.rows, self.inv, self.top, self.weight = rows, inv, top, weight
 
 
-# from this many rows per expert on, tiles of 128 rows through LDS; below, one pass over each expert's weights
-EXPERT_GEMM_MIN_ROWS = 32
+# From this many rows per expert on, tiles of 128 rows through LDS; below, one pass over each expert's weights for every 16 of its
+# rows (32 experts, 2048 -> 1536 / 1536 -> 2048, us: 8 rows each 42.9 / 42.2 by passes and 47.6 / 44.5 by tiles, 12 rows 53.2 / 54.3 and
+# 53.2 / 45.6, 16 rows 64.0 / 61.5 and 51.8 / 45.0, 31 rows 105 / 103 and 52 / 46; 16 experts of 4096 -> 3072 12 rows 91.0 and 87.6)
+EXPERT_GEMM_MIN_ROWS = 12
 
 
 class TableMoE:
@@ -585,7 +587,8 @@ class MoEFeedForward:
     """Mixture of experts: fp32 routing, rows sorted by expert, the expert products, the weighted sum
     (which also takes in identity experts and a gated shared expert where the design has them)."""
 
-    GROUPED_MIN_ROWS = 512          # from this many routed rows on (and EXPERT_GEMM_MIN_ROWS per expert) products by row tiles
+    GROUPED_MIN_ROWS = 512          # from this many routed rows on, and TILE_MIN_ROWS per expert, products by row tiles
+    TILE_MIN_ROWS = 32
 
     def __init__(self, spec, lw, runner):
         self.s, self.lw, self.r = spec, lw, runner
@@ -624,7 +627,7 @@ class MoEFeedForward:
                                  group_max=s.group_score == "max", weight_scale=s.weight_scale, experts=s.outputs,
                                  chosen_softmax=s.score == "chosen_softmax")
         rows = T * s.top
-        tiled = rows >= max(self.GROUPED_MIN_ROWS, EXPERT_GEMM_MIN_ROWS * E) and ops.expert_gemm_ok(h.dtype, h.shape[1], s.ff)
+        tiled = rows >= max(self.GROUPED_MIN_ROWS, self.TILE_MIN_ROWS * E) and ops.expert_gemm_ok(h.dtype, h.shape[1], s.ff)
         offsets, perm, inv, start = ops.moe_sort(ids, s.outputs, tiles=True)
         extra = {}
         if s.identity:
