@@ -932,12 +932,16 @@ int32_t mi355_softcap(void* z, int64_t numel, float cap, int32_t dtype, void* st
  *                          With a workspace of mi355_gated_delta_rule_workspace_form(...) floats
  *                          (mi355_gated_delta_rule_workspace: enough for either kind of decay) the form for
  *                          chunks of many tokens runs (tiles of 16 rows on the matrix cores, in fp32; the
- *                          fp32 result rows serve as scratch); without, the state in registers, token by token (decode)
+ *                          fp32 result rows serve as scratch); without, the state in registers, token by token (decode).
+ *                          With one of mi355_gated_delta_rule_workspace_chunks(...) floats (0: not for these sizes) bf16
+ *                          rows on 16 bytes, 64 a sequence on average and more, go by chunks of 64 rows
  */
 int64_t mi355_gated_delta_rule_workspace(int64_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
                                          int32_t head_dim);
 int64_t mi355_gated_delta_rule_workspace_form(int64_t num_tokens, int32_t num_heads, int32_t head_dim,
                                               int32_t per_channel);
+int64_t mi355_gated_delta_rule_workspace_chunks(int64_t num_tokens, int32_t num_seqs, int32_t num_heads,
+                                                int32_t num_kv_heads, int32_t head_dim, int32_t per_channel);
 int32_t mi355_rope_partial_kv_write(void* q, int64_t q_stride, const void* k, int64_t k_stride,
                                     const void* v, int64_t v_stride, const float* cos_sin,
                                     int32_t max_pos, const int64_t* positions,

@@ -590,6 +590,13 @@ def single_launches():
         w, x, off = rnd(E, N, K, m=K ** -0.5), rnd(E * per, K), i32([per * e for e in range(E + 1)])
         want = torch.cat([x[per * e: per * e + per].float() @ w[e].float().t() for e in range(E)])
         checked(f"moe_linear_rows {E}x{N}x{K}", lambda: ops.moe_linear_rows(x, w, off, E * per), want)
+    # the delta rule by chunks of 64 rows: chunks that end early, columns that are not 16, a sequence that goes on
+    H, G, d, dv, lens = 3, 1, 128, 40, (65, 130, 1, 120)
+    T = sum(lens)
+    x, pos = rnd(T, 2 * G * d + H * dv), torch.cat([torch.arange(a, a + n) for a, n in zip((0, 9, 4, 0), lens)]).cuda()
+    args = (x, 0, G * d, 2 * G * d, rnd(T, H), rnd(T, H), f32(H), f32(H), f32(4, H, d, dv), i32(np.concatenate([[0], np.cumsum(lens)])), pos,
+            i32([2, 0, 3, 1]), H, G, d, dv)
+    checked("gated_delta_rule by chunks", lambda: ops.gated_delta_rule(*args, long_chunks=True))
     # the matrix memory's bf16 products: tiles that end early, a sequence that goes on
     H, d, lens, at = 2, 128, (130, 64, 3), (0, 70, 5)
     T, cu = sum(lens), np.concatenate([[0], np.cumsum(lens)])

@@ -1,4 +1,4 @@
-// The gated delta rule over tiles of 16 rows (delta_tiles.hip), called by mi355_gated_delta_rule.
+// The gated delta rule over tiles of 16 rows (delta_tiles.hip) and chunks of 64 (delta_chunks.hip), called by mi355_gated_delta_rule.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,5 +22,10 @@ struct DeltaTiles {
 int64_t delta_tiles_workspace(int64_t rows, int H, int d, bool per_channel);
 // dtype: an mi355_dtype code; d at most 256
 void launch_delta_tiles(const DeltaTiles& a, int dtype, hipStream_t stream);
+
+// floats of workspace of the form by chunks, 0 where it is not for these sizes; whether it takes these operands
+int64_t delta_chunks_workspace(int64_t rows, int S, int H, int G, int d, bool per_channel);
+bool delta_chunks_ok(const DeltaTiles& a, int dtype);
+void launch_delta_chunks(const DeltaTiles& a, hipStream_t stream);
 
 }  // namespace mi355

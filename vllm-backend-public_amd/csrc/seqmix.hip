@@ -1308,6 +1308,11 @@ extern "C" int64_t mi355_gated_delta_rule_workspace_form(int64_t num_tokens, int
   return delta_tiles_workspace(num_tokens, num_heads, head_dim, per_channel != 0);
 }
 
+extern "C" int64_t mi355_gated_delta_rule_workspace_chunks(int64_t num_tokens, int32_t num_seqs, int32_t num_heads,
+                                                           int32_t num_kv_heads, int32_t head_dim, int32_t per_channel) {
+  return delta_chunks_workspace(num_tokens, num_seqs, num_heads, num_kv_heads, head_dim, per_channel != 0);
+}
+
 extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t stride, int32_t q_off, int32_t k_off,
                                           int32_t v_off, const void* beta, int64_t beta_stride, const void* decay,
                                           int64_t decay_stride, const float* a_log, const float* dt_bias,
@@ -1340,6 +1345,11 @@ extern "C" int32_t mi355_gated_delta_rule(float* o, const void* qkv, int64_t str
     a.ws = workspace, a.rows = num_tokens;
     a.q_off = q_off, a.k_off = k_off, a.v_off = v_off, a.per_channel = per_channel;
     a.S = num_seqs, a.H = num_heads, a.G = num_kv_heads, a.d = head_dim, a.dv = v_dim;
+    const int64_t chunks = delta_chunks_workspace(num_tokens, num_seqs, num_heads, num_kv_heads, head_dim, per_channel != 0);
+    if (chunks > 0 && workspace_floats >= chunks && delta_chunks_ok(a, dtype)) {
+      launch_delta_chunks(a, s);
+      return check_launch("gated_delta_rule (chunks)");
+    }
     launch_delta_tiles(a, dtype, s);
     return check_launch("gated_delta_rule (tiles)");
   }

@@ -126,6 +126,7 @@ def _load() -> ctypes.CDLL:
                                          I32, I32, I64, P, I64, I32, P]),
         "mi355_gated_delta_rule_workspace": (I64, [I64, I32, I32, I32]),
         "mi355_gated_delta_rule_workspace_form": (I64, [I64, I32, I32, I32]),
+        "mi355_gated_delta_rule_workspace_chunks": (I64, [I64, I32, I32, I32, I32, I32]),
         "mi355_general_delta_rule_workspace": (I64, [I64, I32, I32]),
         "mi355_general_delta_rule": (I32, [P, P, I64, P, I64, P, I64, P, I64, P, P, I64, P, P, P, P, P, I32, I32, I32, I64,
                                            I32, P, I64, I32, P]),
@@ -218,7 +219,7 @@ EXPORTS = ("mi355_abi_version", "mi355_last_error", "mi355_target_arch",
            "mi355_gelu_tanh_and_mul", "mi355_gated_head_rms_norm", "mi355_softcap",
            "mi355_rope_partial_kv_write", "mi355_sigmoid_window_attn", "mi355_sigmoid_window_attn_prefill", "mi355_causal_conv_silu",
            "mi355_conv_state_update", "mi355_conv_silu_step", "mi355_gated_delta_rule", "mi355_gated_delta_rule_workspace",
-           "mi355_gated_delta_rule_workspace_form",
+           "mi355_gated_delta_rule_workspace_form", "mi355_gated_delta_rule_workspace_chunks",
            "mi355_general_delta_rule", "mi355_general_delta_rule_workspace", "mi355_group_rms_norm_f32",
            "mi355_gated_norm_resid_f32", "mi355_rms_norm_rows", "mi355_tanh_rows", "mi355_latent_kv_write",
            "mi355_latent_q_pack", "mi355_latent_window_attn_tiles",

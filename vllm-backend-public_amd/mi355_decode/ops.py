@@ -1494,7 +1494,7 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
     [tokens, heads * head_dim] are raw projection outputs (column slices are fine); a_log [heads] and
     dt_bias (decay's width) float32; state float32 [slots, heads, head_dim, v_dim].
     Returns o float32 [tokens, heads, v_dim].  long_chunks: the batch holds chunks of many tokens -- take
-    the form that goes by tiles of 16 rows (it allocates a float32 workspace; not for graphs), unless the longest chunk
+    the form that goes by tiles of 16 rows, or chunks of 64 (it allocates a float32 workspace; not for graphs), unless the longest chunk
     (`longest`; 0: as many rows as the batch has beyond one a chunk) is so short that token by token is faster."""
     dt = _dt3(qkv, "qkv")
     T = qkv.shape[0]
@@ -1513,8 +1513,10 @@ def gated_delta_rule(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, beta
         out = torch.empty(T, num_heads, v_dim, dtype=torch.float32, device=qkv.device)
     ws = None
     if long_chunks and T > 0:
-        ws = torch.empty(lib.mi355_gated_delta_rule_workspace_form(T, num_heads, head_dim, int(per_channel)), dtype=torch.float32,
-                         device=qkv.device)
+        floats = lib.mi355_gated_delta_rule_workspace_form(T, num_heads, head_dim, int(per_channel))
+        if qkv.dtype == torch.bfloat16:
+            floats = max(floats, lib.mi355_gated_delta_rule_workspace_chunks(T, S, num_heads, num_kv_heads, head_dim, int(per_channel)))
+        ws = torch.empty(floats, dtype=torch.float32, device=qkv.device)
     check(lib.mi355_gated_delta_rule(
         _f32(out, "out", T * num_heads * v_dim), qkv.data_ptr(), qkv.shape[1], q_off, k_off, v_off,
         _same(beta, qkv, "beta"), _cols(beta, "beta", num_heads), _same(decay, qkv, "decay"), _cols(decay, "decay", width),
