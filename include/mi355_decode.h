@@ -1052,6 +1052,13 @@ int32_t mi355_latent_kv_write(void* cache, void* cache_t, const void* x, int64_t
                               const int64_t* slot_mapping, int64_t num_tokens, int32_t rank,
                               int32_t rot, int32_t rot_dims, int32_t interleaved, float eps,
                               int32_t dtype, void* stream);
+/* latent_kv_write, and in the same launch of every head of q the columns that latent_q_pack rotates (without an absorbed part) */
+int32_t mi355_latent_kv_write_q(void* cache, void* cache_t, const void* x, int64_t x_stride, const float* norm_weight,
+                                const float* cos_sin, int32_t max_pos, const int64_t* positions,
+                                const int64_t* slot_mapping, void* q_packed, const void* q, int64_t q_stride,
+                                int32_t q_head_width, int32_t q_rot_offset, int64_t num_tokens, int32_t num_heads,
+                                int32_t rank, int32_t rot, int32_t rot_dims, int32_t interleaved, float eps, int32_t dtype,
+                                void* stream);
 /*
  * The matrix-core form of latent_window_attn (16-bit storage, rank a multiple of 16 up to 512,
  * rank + rot a multiple of 8 up to 640), same result.

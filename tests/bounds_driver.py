@@ -597,6 +597,16 @@ def single_launches():
     args = (x, 0, G * d, 2 * G * d, rnd(T, H), rnd(T, H), f32(H), f32(H), f32(4, H, d, dv), i32(np.concatenate([[0], np.cumsum(lens)])), pos,
             i32([2, 0, 3, 1]), H, G, d, dv)
     checked("gated_delta_rule by chunks", lambda: ops.gated_delta_rule(*args, long_chunks=True))
+    # the latent attention with keys staged: contexts that end inside a step, splits without a key
+    lens, H = (40, 1, 97), 5
+    need = [-(-n // 16) for n in lens]
+    bt = torch.zeros(3, 7, dtype=torch.int32, device="cuda")
+    for s, n in enumerate(need):
+        bt[s, :n] = torch.arange(sum(need[:s]), sum(need[:s]) + n)
+    cache, pos = rnd(sum(need), 16, 576), torch.tensor([n - 1 for n in lens]).cuda()
+    q, tiles, cache_t = rnd(3, H, 576), torch.from_numpy(ops.pair_tiles(np.arange(4), H)).cuda(), cache[:, :, :512].transpose(1, 2).contiguous()
+    for n in (1, 4):
+        checked(f"latent attention staged {n}", lambda: ops.latent_window_attn_tiles(q, cache, cache_t, bt, tiles, pos, None, None, 1 << 30, 0.1, num_splits=n))
     # the matrix memory's bf16 products: tiles that end early, a sequence that goes on
     H, d, lens, at = 2, 128, (130, 64, 3), (0, 70, 5)
     T, cu = sum(lens), np.concatenate([[0], np.cumsum(lens)])

@@ -632,6 +632,63 @@ def test_latent_attention_in_float32(H, d, r, dv, rank, base):
         _near(_latent_in_cuts(full, st, h, torch.float32, cuts)[0], want, 3e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,lens,rows,splits,window,gated", [(16, [1, 31, 32, 33], 1, 1, 1 << 30, False), (16, [64, 65, 127, 300], 1, 3, 1 << 30, True),
+                                                             (3, [96, 161], 1, 16, 1 << 30, True), (17, [200, 90], 5, 2, 70, False),
+                                                             (40, [1100], 2, 4, 1 << 30, False), (16, [97] * 1030, 1, 1, 1 << 30, False)])
+def test_latent_attention_with_keys_staged(dtype, H, lens, rows, splits, window, gated):
+    """A latent of 512 + 64 by steps of 32 keys: contexts around a step, more splits than steps, windows that begin inside a step, tiles
+    that are not full, a launch of more tiles than are staged; pages in no order with NaN behind every context.  Against float64; bound:
+    weights and results are rounded to 16 bits (2^-9 each in bf16, 2^-12 in fp16) of latents whose weights sum to 1 at most."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(len(lens) + H)
+    need = [-(-n // 16) for n in lens]
+    order, at = torch.randperm(sum(need), generator=g), 0
+    cache = torch.full((sum(need), 16, 576), float("nan"), dtype=dtype)
+    bt = torch.zeros(len(lens), max(need) + 2, dtype=torch.int32)
+    keys = [torch.randn(n, 576, generator=g).to(dtype) for n in lens]
+    for s, n in enumerate(lens):
+        bt[s, :need[s]] = order[at:at + need[s]].to(torch.int32)
+        at += need[s]
+        cache[bt[s, torch.arange(n) // 16].long(), torch.arange(n) % 16] = keys[s]
+    T = len(lens) * rows
+    pos = torch.tensor([n - rows + r for n in lens for r in range(rows)])
+    q = (torch.randn(T, H, 576, generator=g) * 0.3).to(dtype)
+    sink, gate = (torch.randn(H, generator=g), torch.randn(T, H, generator=g).to(dtype)) if gated else (None, None)
+    dev = lambda t: None if t is None else t.cuda()       # noqa: E731
+    tiles = torch.from_numpy(ops.pair_tiles(np.arange(0, T + 1, rows), H)).cuda()
+    got = ops.latent_window_attn_tiles(q.cuda(), cache.cuda(), cache[:, :, :512].transpose(1, 2).contiguous().cuda(), bt.cuda(), tiles, pos.cuda(),
+                                       dev(sink), dev(gate), window, 0.07, num_splits=splits).transpose(0, 1).cpu()
+    for t in range(0, T, 1 if T < 100 else 97):
+        k = keys[t // rows].double()
+        lo, p = max(0, int(pos[t]) - window + 1), int(pos[t])
+        e = torch.exp(q[t].double() @ k[lo:p + 1].t() * 0.07)
+        w = e / (e.sum(1, keepdim=True) + (torch.exp(sink.double())[:, None] if gated else 0.0))
+        want = (w @ k[lo:p + 1, :512]) * (torch.sigmoid(gate[t].double())[:, None] if gated else 1.0)
+        eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+        assert (got[t] - want).abs().max() <= (2 * eps + 1e-5) * k[lo:p + 1, :512].abs().max(), t
+
+
+def test_latents_written_with_the_queries_rotated():
+    """One launch for the latents of a step and the rotated part of its queries: the numbers of the two, also for rows that are not
+    stored, and nothing else of the packed queries."""
+    from mi355_decode import ops
+    from mi355_decode.hybrid_runner import rotary_table
+    g = torch.Generator().manual_seed(1)
+    for T, H, rank, rot, dtype in ((5, 6, 32, 8, torch.bfloat16), (1, 1, 512, 64, torch.float16), (3, 17, 20, 70, torch.float32)):
+        x, q = torch.randn(T, rank + rot, generator=g).to(dtype).cuda(), torch.randn(T, H * (24 + rot), generator=g).to(dtype).cuda()
+        w, pos, table = torch.randn(rank, generator=g).cuda(), torch.arange(3, 3 + T).cuda(), rotary_table(rot, 300.0, 40, "cuda", exact=True)
+        slots = torch.tensor([7, -1, 20, 31, 4][:T]).cuda()
+        pages = [(torch.zeros(2, 16, rank + rot, dtype=dtype, device="cuda"), torch.zeros(2, rank, 16, dtype=dtype, device="cuda")) for _ in range(2)]
+        qe = [torch.full((T, H, rank + rot), 7.0, dtype=dtype, device="cuda") for _ in range(2)]
+        args = lambda i: (x, w, table, pos, slots, pages[i][0], rank, rot, 1e-5)       # noqa: E731
+        ops.latent_kv_write(*args(0), cache_t=pages[0][1], interleaved=True)
+        ops.latent_q_pack(None, q, 24 + rot, 24, rot, table, pos, interleaved=True, out=qe[0])
+        ops.latent_kv_write(*args(1), cache_t=pages[1][1], interleaved=True, query=(q, 24 + rot, 24, qe[1]))
+        assert torch.equal(qe[0], qe[1]) and torch.equal(pages[0][0], pages[1][0]) and torch.equal(pages[0][1], pages[1][1])
+        assert (qe[1][:, :, :rank] == 7.0).all() and (qe[1][:, :, rank:] != 7.0).any()
+
+
 @pytest.mark.parametrize("H,d,r,dv,rank,base", [(3, 16, 8, 24, 32, 500.0), (8, 64, 16, 48, 64, 1e4), (5, 24, 8, 40, 272, 1e4), (7, 13, 6, 9, 22, 77.0),
                                                 (17, 32, 32, 16, 112, 1e5), (3, 20, 4, 12, 48, 100.0), (17, 64, 64, 64, 512, 1e4), (5, 24, 8, 40, 192, 1e4),
                                                 (2, 16, 8, 24, 128, 1e3), (33, 16, 64, 8, 256, 1e4), (3, 16, 128, 16, 512, 1e4)])

@@ -314,14 +314,19 @@ class LatentAttention:
         s, lw, r = self.s, self.lw, self.r
         col = lambda n: proj[:, lw.seg[n][0]: lw.seg[n][0] + lw.seg[n][1]]     # noqa: E731
         (cache, cache_t), table = r.latent_cache[self.ci], r.rotary(s.rot_dims, s.rot_base, exact=s.interleaved)
-        if self.writes:
-            ops.latent_kv_write(col("dkv"), lw.dkv_norm, table, b.positions, b.slot_mapping, cache, s.kv_rank, s.rot_dim,
-                                r.eps, cache_t=cache_t, interleaved=s.interleaved)
         q = col("q") if s.q_direct else r.linear(ops.rms_norm_rows(col("dq"), lw.dq_norm, r.eps), lw.uq_w)
         gate = col("g") if s.gate else None
         plan = b.latent_plan() if self.expands and b.long_chunks and b.latent_plan is not None else None
-        if plan is None or not plan.fits or plan.pages * BLOCK_SIZE * s.heads * (s.dim + s.rot_dim + s.vdim) * 2 > plan.MAX_BYTES:
-            return _out_product(r, self._on_latents(q, gate, b.positions, b.block_tables, b.tok_seq, b.pair_tiles), lw.o_w)
+        on_latents = plan is None or not plan.fits or plan.pages * BLOCK_SIZE * s.heads * (s.dim + s.rot_dim + s.vdim) * 2 > plan.MAX_BYTES
+        qe = None
+        if on_latents and self.writes and self.head_gemm and cache_t is not None and b.pair_tiles is not None:
+            qe = torch.empty(q.shape[0], s.heads, s.kv_rank + s.rot_dim, dtype=q.dtype, device=q.device)
+        if self.writes:
+            ops.latent_kv_write(col("dkv"), lw.dkv_norm, table, b.positions, b.slot_mapping, cache, s.kv_rank, s.rot_dim,
+                                r.eps, cache_t=cache_t, interleaved=s.interleaved,
+                                query=None if qe is None else (q, s.dim + s.rot_dim, s.dim, qe))
+        if on_latents:
+            return _out_product(r, self._on_latents(q, gate, b.positions, b.block_tables, b.tok_seq, b.pair_tiles, qe), lw.o_w)
         return _out_product(r, self._expanded(q, gate, b, plan), lw.o_w)
 
     def _expanded(self, q: torch.Tensor, gate: Optional[torch.Tensor], b: StepBatch, plan: LatentPlan) -> torch.Tensor:
@@ -345,8 +350,8 @@ class LatentAttention:
             o.index_copy_(0, plan.short[0], rest)
         return o
 
-    def _on_latents(self, q, gate, positions, block_tables, tok_seq, pair_tiles) -> torch.Tensor:
-        """The concatenated heads [tokens, heads * vdim]."""
+    def _on_latents(self, q, gate, positions, block_tables, tok_seq, pair_tiles, qe=None) -> torch.Tensor:
+        """The concatenated heads [tokens, heads * vdim].  qe: packed queries that hold their rotated part already."""
         s, lw, r = self.s, self.lw, self.r
         (cache, cache_t), table = r.latent_cache[self.ci], r.rotary(s.rot_dims, s.rot_base, exact=s.interleaved)
         T, H, hw, R, dq = q.shape[0], s.heads, s.dim + s.rot_dim, s.kv_rank, s.kv_rank + s.rot_dim
@@ -357,9 +362,10 @@ class LatentAttention:
             tiles = pair_tiles(H)
             n = min(16, max(s.window // 64, 1), max(ops.latent_tile_workgroups(R, s.rot_dim) // max(int(tiles.shape[0]), 1), 1))
         if matrix_cores and self.head_gemm:
-            qe = torch.empty(T, H, dq, dtype=q.dtype, device=q.device)
+            if qe is None:
+                qe = torch.empty(T, H, dq, dtype=q.dtype, device=q.device)
+                ops.latent_q_pack(None, q, hw, s.dim, s.rot_dim, table, positions, interleaved=s.interleaved, out=qe)
             ops.head_gemm(q, hw, lw.uk_t, qe, 16 * H * dq, H * dq, dq, T)
-            ops.latent_q_pack(None, q, hw, s.dim, s.rot_dim, table, positions, interleaved=s.interleaved, out=qe)
             ol = torch.empty(T, H, R, dtype=q.dtype, device=q.device)
             ops.latent_window_attn_tiles(qe, cache, cache_t, block_tables, tiles, positions, lw.sink, gate, s.window, s.scale,
                                          num_splits=n, out=ol.transpose(0, 1))

@@ -1676,23 +1676,31 @@ def tanh_rows(x: torch.Tensor):
 
 def latent_kv_write(x: torch.Tensor, norm_weight: torch.Tensor, cos_sin: torch.Tensor, positions: torch.Tensor,
                     slot_mapping: torch.Tensor, cache: torch.Tensor, rank: int, rot: int, eps: float,
-                    cache_t: torch.Tensor | None = None, interleaved: bool = False):
+                    cache_t: torch.Tensor | None = None, interleaved: bool = False, query: tuple | None = None):
     """x [tokens, rank + rot] (a column slice is fine): the first rank columns RMS-normed with norm_weight
     (float32), the last rot rotated by the table cos_sin [max_pos, rot_dims] (coordinates i, i + rot_dims / 2, or
     neighbours if interleaved), both into the row's slot of
-    cache [blocks, 16, rank + rot]; the latent also into cache_t [blocks, rank, 16] if given."""
+    cache [blocks, 16, rank + rot]; the latent also into cache_t [blocks, rank, 16] if given.  query (q, q_head_width,
+    q_rot_offset, out): in the same launch latent_q_pack(None, q, ..., out=out)."""
     dt = _dt3(x, "x")
     T = x.shape[0]
     if cache.dim() != 3 or tuple(cache.shape[1:]) != (BLOCK_SIZE, rank + rot) or not cache.is_contiguous():
         raise ValueError("latent pages must be contiguous [blocks, 16, rank + rot]")
     if cache_t is not None and (tuple(cache_t.shape) != (cache.shape[0], rank, BLOCK_SIZE) or not cache_t.is_contiguous()):
         raise ValueError("the channel-major latent pages must be contiguous [blocks, rank, 16]")
-    check(lib.mi355_latent_kv_write(_same(cache, x, "cache"), None if cache_t is None else _same(cache_t, x, "cache_t"),
-                                    x.data_ptr(), _cols(x, "x", rank + rot),
-                                    _f32(norm_weight, "norm_weight", rank), _f32(cos_sin, "cos_sin") or x.data_ptr(),
-                                    max(cos_sin.shape[0], 1), _idx(positions, "positions", torch.int64, T),
-                                    _idx(slot_mapping, "slot_mapping", torch.int64, T), T, rank, rot, cos_sin.shape[1],
-                                    int(bool(interleaved)), float(eps), dt, _stream()))
+    args = (_same(cache, x, "cache"), None if cache_t is None else _same(cache_t, x, "cache_t"), x.data_ptr(), _cols(x, "x", rank + rot),
+            _f32(norm_weight, "norm_weight", rank), _f32(cos_sin, "cos_sin") or x.data_ptr(), max(cos_sin.shape[0], 1),
+            _idx(positions, "positions", torch.int64, T), _idx(slot_mapping, "slot_mapping", torch.int64, T))
+    tail = (rank, rot, cos_sin.shape[1], int(bool(interleaved)), float(eps), dt, _stream())
+    if query is None:
+        check(lib.mi355_latent_kv_write(*args, T, *tail))
+        return
+    q, q_head_width, q_rot_offset, out = query
+    H = out.shape[1]
+    if tuple(out.shape) != (T, H, rank + rot) or not out.is_contiguous() or q.shape[0] != T:
+        raise ValueError("out must be contiguous [tokens, heads, rank + rot] and q have as many rows")
+    check(lib.mi355_latent_kv_write_q(*args, _same(out, x, "out"), _same(q, x, "q"), _cols(q, "q", H * q_head_width), q_head_width, q_rot_offset,
+                                      T, H, *tail))
 
 
 def pair_tiles(cu_seqlens, num_heads: int) -> "np.ndarray":
