@@ -590,23 +590,6 @@ def single_launches():
         w, x, off = rnd(E, N, K, m=K ** -0.5), rnd(E * per, K), i32([per * e for e in range(E + 1)])
         want = torch.cat([x[per * e: per * e + per].float() @ w[e].float().t() for e in range(E)])
         checked(f"moe_linear_rows {E}x{N}x{K}", lambda: ops.moe_linear_rows(x, w, off, E * per), want)
-    # the delta rule by chunks of 64 rows: chunks that end early, columns that are not 16, a sequence that goes on
-    H, G, d, dv, lens = 3, 1, 128, 40, (65, 130, 1, 120)
-    T = sum(lens)
-    x, pos = rnd(T, 2 * G * d + H * dv), torch.cat([torch.arange(a, a + n) for a, n in zip((0, 9, 4, 0), lens)]).cuda()
-    args = (x, 0, G * d, 2 * G * d, rnd(T, H), rnd(T, H), f32(H), f32(H), f32(4, H, d, dv), i32(np.concatenate([[0], np.cumsum(lens)])), pos,
-            i32([2, 0, 3, 1]), H, G, d, dv)
-    checked("gated_delta_rule by chunks", lambda: ops.gated_delta_rule(*args, long_chunks=True))
-    # the latent attention with keys staged: contexts that end inside a step, splits without a key
-    lens, H = (40, 1, 97), 5
-    need = [-(-n // 16) for n in lens]
-    bt = torch.zeros(3, 7, dtype=torch.int32, device="cuda")
-    for s, n in enumerate(need):
-        bt[s, :n] = torch.arange(sum(need[:s]), sum(need[:s]) + n)
-    cache, pos = rnd(sum(need), 16, 576), torch.tensor([n - 1 for n in lens]).cuda()
-    q, tiles, cache_t = rnd(3, H, 576), torch.from_numpy(ops.pair_tiles(np.arange(4), H)).cuda(), cache[:, :, :512].transpose(1, 2).contiguous()
-    for n in (1, 4):
-        checked(f"latent attention staged {n}", lambda: ops.latent_window_attn_tiles(q, cache, cache_t, bt, tiles, pos, None, None, 1 << 30, 0.1, num_splits=n))
     # the matrix memory's bf16 products: tiles that end early, a sequence that goes on
     H, d, lens, at = 2, 128, (130, 64, 3), (0, 70, 5)
     T, cu = sum(lens), np.concatenate([[0], np.cumsum(lens)])
@@ -645,6 +628,54 @@ def single_launches():
     return done
 
 
+def prompt_and_latent_launches():
+    """Launches of the delta rule by chunks and of the latent attention with its keys staged."""
+    from mi355_decode import ops
+    g, done = torch.Generator().manual_seed(3), []
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()      # noqa: E731
+    f32 = lambda *s: torch.randn(*s, generator=g).cuda()                 # noqa: E731
+    i32 = lambda v: torch.tensor(np.asarray(v), dtype=torch.int32, device="cuda")      # noqa: E731
+
+    def checked(name, call):
+        empty = torch.empty
+
+        def listed(*a, **k):
+            t = empty(*a, **k)
+            bounds.sync_allocations()
+            return t
+
+        torch.empty = listed
+        try:
+            bounds.sync_allocations()
+            call()
+            torch.cuda.synchronize()
+        finally:
+            torch.empty = empty
+        rep = bounds.report()
+        assert rep is None, (name, rep)
+        bounds.clear()
+        done.append(name)
+
+    # the delta rule by chunks of 64 rows: chunks that end early, columns that are not 16, a sequence that goes on
+    H, G, d, dv, lens = 3, 1, 128, 40, (65, 130, 1, 120)
+    T = sum(lens)
+    x, pos = rnd(T, 2 * G * d + H * dv), torch.cat([torch.arange(a, a + n) for a, n in zip((0, 9, 4, 0), lens)]).cuda()
+    args = (x, 0, G * d, 2 * G * d, rnd(T, H), rnd(T, H), f32(H), f32(H), f32(4, H, d, dv), i32(np.concatenate([[0], np.cumsum(lens)])), pos,
+            i32([2, 0, 3, 1]), H, G, d, dv)
+    checked("gated_delta_rule by chunks", lambda: ops.gated_delta_rule(*args, long_chunks=True))
+    # the latent attention with keys staged: contexts that end inside a step, splits without a key
+    lens, H = (40, 1, 97), 5
+    need = [-(-n // 16) for n in lens]
+    bt = torch.zeros(3, 7, dtype=torch.int32, device="cuda")
+    for s, n in enumerate(need):
+        bt[s, :n] = torch.arange(sum(need[:s]), sum(need[:s]) + n)
+    cache, pos = rnd(sum(need), 16, 576), torch.tensor([n - 1 for n in lens]).cuda()
+    q, tiles, cache_t = rnd(3, H, 576), torch.from_numpy(ops.pair_tiles(np.arange(4), H)).cuda(), cache[:, :, :512].transpose(1, 2).contiguous()
+    for n in (1, 4):
+        checked(f"latent attention staged {n}", lambda: ops.latent_window_attn_tiles(q, cache, cache_t, bt, tiles, pos, None, None, 1 << 30, 0.1, num_splits=n))
+    return done
+
+
 if __name__ == "__main__":
     assert bounds.enabled(), "not the bounds-checking build: set MI355_DECODE_LIB"
     res = {"negative_control": negative_control()}
@@ -659,4 +690,5 @@ if __name__ == "__main__":
     res["post_norms"] = post_norm_generation()
     res["table_mixtures"] = table_mixture_generation()
     res["windows_and_deltas"] = window_and_delta_generation()
+    res["prompt_and_latent_launches"] = prompt_and_latent_launches()
     print(json.dumps(res))

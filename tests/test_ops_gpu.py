@@ -728,6 +728,41 @@ def test_sample_from_counts_of_all_values_and_of_masked_rows(ops, monkeypatch, V
                                       R.sample_topk_topp(lg.float().numpy(), temperature, k, p, seeds, steps))
 
 
+@pytest.mark.parametrize("B,V", [(1, 16391), (8, 20000), (24, 16384), (40, 16391), (7, 40)])
+def test_sample_draws_decided_by_bounds(ops, monkeypatch, B, V):
+    """Draws over whole rows and over nuclei that hold most of a row, which form few scores: flat rows and steep ones, temperatures
+    from where a reciprocal is infinite to where all scores are the draw's, infinities of either sign alone and among others, NaN, the
+    largest finite numbers.  Against the restatement, exactly."""
+    monkeypatch.setattr(ops, "SAMPLE_SPREAD_VOCAB", 0)
+    rng = np.random.default_rng(B + V)
+    for turn in range(2):
+        lg = torch.from_numpy((rng.normal(0, 1, (B, V)) * 10.0 ** rng.integers(-3, 4, (B, 1))).astype(np.float32)).bfloat16()
+        temperature = rng.choice([1.0, 0.7, 1e-3, 1e-30, 1e-40, 1e4, 3e38], B).astype(np.float32)
+        top_p = np.where(rng.random(B) < 0.4, np.float32(0.98), np.float32(1.0)).astype(np.float32)
+        for r in range(B):
+            kind = (r + 3 * turn) % 8
+            if kind == 0:
+                lg[r] = -float("inf")
+            elif kind == 1:
+                lg[r] = -float("inf")
+                lg[r, rng.integers(0, V, 3)] = torch.tensor([-5.0, 2.0, 1.0], dtype=torch.bfloat16)
+            elif kind == 2:
+                lg[r, rng.integers(0, V, 2)] = float("inf")
+            elif kind == 3 and top_p[r] == 1.0:
+                lg[r, rng.integers(0, V, 2)] = float("nan")
+            elif kind == 4:
+                lg[r] = torch.from_numpy(rng.choice([3.38e38, -3.38e38], V).astype(np.float32)).bfloat16()
+            elif kind == 5:
+                lg[r] = 0.25
+        top_k, seeds, steps = np.zeros(B, np.int32), rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B, dtype=np.int64)
+        wide = torch.zeros(B, (V + 7) // 8 * 8, dtype=torch.bfloat16, device="cuda")
+        wide[:, :V] = lg.cuda()
+        args = [torch.from_numpy(a).cuda() for a in (temperature, top_k, top_p, seeds, steps)]
+        with np.errstate(all="ignore"):
+            ref = R.sample_topk_topp(lg.float().numpy(), temperature, top_k, top_p, seeds, steps)
+        np.testing.assert_array_equal(ops.sample(wide[:, :V], *args).cpu().numpy(), ref)
+
+
 @pytest.mark.parametrize("ldt,B", [("bfloat16", 32), ("bfloat16", 33), ("float16", 5), ("float32", 5)])
 def test_sample_of_short_cuts_is_the_same_either_way(ops, ldt, B):
     """The caller's word that every cut is short moves rows to another way through the sampler and no token."""

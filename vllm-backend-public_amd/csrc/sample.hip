@@ -56,6 +56,14 @@ __device__ __forceinline__ unsigned long long lane64(unsigned long long v, int l
 __device__ __forceinline__ unsigned long long wave_max64(unsigned long long v) {
   return lane64(wave_scan64(v, [](unsigned long long a, unsigned long long b) { return umax64(a, b); }), 63);
 }
+__device__ __forceinline__ float wave_maxf(float v) {                  // of numbers, no NaN among them
+  auto step = [&](float o) { v = fmaxf(v, o); };
+#define MI355_DPP_MAX(CTRL, ROWS) step(__int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xF, false)))
+  MI355_DPP_MAX(0x111, 0xF), MI355_DPP_MAX(0x112, 0xF), MI355_DPP_MAX(0x114, 0xF), MI355_DPP_MAX(0x118, 0xF);
+  MI355_DPP_MAX(0x142, 0xA), MI355_DPP_MAX(0x143, 0xC);
+#undef MI355_DPP_MAX
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
 __device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
   return lane64(wave_scan64(v, [](unsigned long long a, unsigned long long b) { return a + b; }), 63);
 }
@@ -1335,29 +1343,30 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
   }
 }
 
-// ---- bf16 logits with a caller's workspace: three launches.  A 16-bit logit has 65536 values, so a row is its counts of
+// ---- bf16 logits with a caller's workspace: two launches.  A 16-bit logit has 65536 values, so a row is its counts of
 // them, and everything a cut needs -- the k-th largest key, the mass of what is left (a value's mass times its count), the
 // key at which the nucleus ends -- follows from the counts without another look at the row:
 //   sample_count   a workgroup per (row, part of its columns) counts its logits by key in LDS (65536 counters of 16 bits)
 //                  and writes the lines of 32 counters that hold any, with a byte a line that says so
-//   sample_pick    a workgroup a row adds up the counts of all parts (a few hundred lines: a trained model's logits have
-//                  some thousand values) and selects by prefix sums
-//   sample_draw    every row spread over many workgroups, those without a cut too (their pass is arithmetic: two logarithms a
-//                  logit); the last one to end turns the row's best key into the token
-// What bounds the launch per eight key bits (exact_hist_kernel) is the launches: seven for bf16, each of 3 to 12 us for a pass of
-// about 1 us.  32 rows of 128256 logits with a mix of cuts: 40 us a call that way, here 27 (alone count 6.5, pick 10, draw 12); top-p
-// alone 43 / 29, top-k of 50 alone 30 / 20; 4 rows 30 / 22, 64 rows 51 / 35, 32 rows of 32000 31 / 21.  From 1 to 64 rows, 16384 to 262144
-// logits like a model's, normal ones of any scale or masked ones it is nowhere slower; rows of some forty orders of magnitude
-// (batches in the pick) 24.8 / 25.4 at worst, and rows of three values, whose cut has a third of the row at its key, up to 83 / 112.
-// fp16 keeps the passes: its rows have some ten thousand values, and the pick then takes them in several batches (16 rows
+//   sample_draw    a workgroup per (row, range of its columns) adds up the counts of all parts (a few hundred lines: a trained
+//                  model's logits have some thousand values), selects by prefix sums, and draws over its range; the row's last one to
+//                  end turns the best key into the token.  A row's workgroups repeat the selection side by side instead of waiting
+//                  for a launch that makes it once
+// What bounds it: two chains of look-ups, scans and atomics.  32 rows of 128256 logits with a mix of cuts, us a call: 27.3 as three
+// launches with two logarithms for every token that stays (count 6.5, pick 10, draw 12), here 21.7 (count 6.2, draw 15.5); top-p alone
+// 25.4 / 21.2, top-k of 50 alone 19.4 / 17.2, no cut 21.4 / 16.4; 64 rows 35.3 / 25.1, 4 rows 21.4 / 20.6 (by then the host's two
+// launches).  Rows of three values (the cut's key holds a third of them) in such a mix are the exception: 48 rows 67 / 73.  The launch
+// per eight key bits (exact_hist_kernel), seven for bf16, takes 40.
+// fp16 keeps the passes: its rows have some ten thousand values, and the selection then takes them in several batches (16 rows
 // with a top-p 38 us by passes, 48 by counts).
 constexpr int kCountRows = 64;                              // rows up to which a row has four parts and more
 constexpr int kCountParts = 16;                             // most parts of a row
+constexpr int kSampleListed = 256;                          // tokens at the cut's key that a workgroup of the draw ranks from a list
+constexpr int kSampleKept = 1024;                           // tokens that stay for sure that it lists ahead of their draw
 constexpr int kCountLines = 2048;                           // lines of 32 counters, 64 bytes each
 // parts of a row: 256 workgroups (a CU holds one: 128 KB of counters)
 __host__ __device__ __forceinline__ int count_parts(int rows) { return rows >= 64 ? 4 : rows <= 16 ? kCountParts : 256 / rows; }
-// workspace, in 64-bit words: [rows] x 32 (the draw's key at 0, the cut's key and how many tokens with it stay at 1 and 2,
-// such tokens ahead of every part (32 bits each) from 3 on, workgroups done at 16) | flags [rows][parts][2048 bytes] |
+// workspace, in 64-bit words: [rows] x 32 (the draw's key at 0, workgroups done at 16) | flags [rows][parts][2048 bytes] |
 // counters [rows][parts][65536] of 16 bits
 __host__ __device__ __forceinline__ int64_t count_ws_words(int64_t rows) {
   return rows * (kSampleWsHead + count_parts(static_cast<int>(rows)) * static_cast<int64_t>(kCountLines / 8 + 16384));
@@ -1373,11 +1382,20 @@ __device__ __forceinline__ float key16_logit(uint32_t key) {
   return BF16::to_f(static_cast<uint16_t>(key & 0x8000u ? key ^ 0x8000u : ~key));
 }
 
+// The workgroups of a row on one XCD (every eighth block), where the rows are dealt evenly so: its L2 then holds the row and its counts
+// (32 rows with a mix of cuts 23.0 -> 21.7 us, rows of nearly all values with a top-k of 50 25.7 -> 18.8).
+__device__ __forceinline__ int2 row_and_piece(int rows, int pieces) {
+  const int id = blockIdx.x;
+  if (rows % 8 != 0) return make_int2(id / pieces, id % pieces);
+  return make_int2((id & 7) + 8 * ((id >> 3) / pieces), (id >> 3) % pieces);
+}
+
 __global__ __launch_bounds__(kSampleThreads) void sample_count_kernel(
     unsigned long long* __restrict__ ws, const uint16_t* __restrict__ logits, int64_t stride, int vocab,
-    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int part_vecs) {
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p, int rows, int parts, int part_vecs) {
   __shared__ __attribute__((aligned(16))) uint32_t counts[32768];      // two keys a word
-  const int row = blockIdx.y, part = blockIdx.x, parts = gridDim.x, tid = threadIdx.x, lane = tid & 63;
+  const int2 at = row_and_piece(rows, parts);
+  const int row = at.x, part = at.y, tid = threadIdx.x, lane = tid & 63;
   if (part == 0 && tid == 0) {
     unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
     MI355_ST(unsigned long long, ws, head, 0ull);
@@ -1409,9 +1427,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_count_kernel(
   if (part == parts - 1)
     for (int i = (vocab & ~7) + tid; i < vocab; i += kSampleThreads) add(key16(MI355_LD(uint16_t, logits, base + i)), 1u);
   __syncthreads();
-  uint8_t* flags = reinterpret_cast<uint8_t*>(ws + static_cast<int64_t>(gridDim.y) * kSampleWsHead) +
+  uint8_t* flags = reinterpret_cast<uint8_t*>(ws + static_cast<int64_t>(rows) * kSampleWsHead) +
                    (static_cast<int64_t>(row) * parts + part) * kCountLines;
-  unsigned long long* lines = ws + static_cast<int64_t>(gridDim.y) * (kSampleWsHead + parts * (kCountLines / 8)) +
+  unsigned long long* lines = ws + static_cast<int64_t>(rows) * (kSampleWsHead + parts * (kCountLines / 8)) +
                               (static_cast<int64_t>(row) * parts + part) * 16384;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {                                        // four lanes a line
@@ -1442,25 +1460,27 @@ __device__ __forceinline__ unsigned long long block_scan64(unsigned long long v,
   return v + before;
 }
 
-__global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(
-    unsigned long long* __restrict__ ws, int parts, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-    const float* __restrict__ top_p) {
-  __shared__ unsigned long long scratch[kSampleThreads / 64], found[2];
-  __shared__ uint16_t used[kCountLines];                               // the row's lines that hold any, from the highest keys down
-  const int row = blockIdx.x, tid = threadIdx.x;
-  unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
-  const uint8_t* flags = reinterpret_cast<const uint8_t*>(ws + static_cast<int64_t>(gridDim.x) * kSampleWsHead) +
-                         static_cast<int64_t>(row) * parts * kCountLines;
-  const uint16_t* counters = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(gridDim.x) * (kSampleWsHead + parts * (kCountLines / 8))) +
-                             static_cast<int64_t>(row) * parts * 65536;
+// What the counts of a row with a cut say: its largest key, the key at which the cut falls, and how many tokens with that key stay
+// (~0: all of them).  All 1024 threads call it, the result is the same in all.
+struct CountedCut {
+  uint32_t top, key;
+  unsigned long long take;
+};
+struct CountedScratch {
+  unsigned long long scratch[kSampleThreads / 64], found[2];
+  uint16_t used[kCountLines];                                          // the row's lines that hold any, from the highest keys down
+};
+__device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, const uint8_t* flags, const uint16_t* counters, int parts, int K1,
+                                                  float temp, float tp, CountedScratch& sh) {
+  unsigned long long(&scratch)[kSampleThreads / 64] = sh.scratch;
+  unsigned long long(&found)[2] = sh.found;
+  uint16_t(&used)[kCountLines] = sh.used;
+  const int tid = threadIdx.x;
   // lines in use, highest first: thread t looks at lines 2047 - 2t and 2046 - 2t
   const int hi = kCountLines - 1 - 2 * tid;
   uint32_t mine = 0u;
 #pragma unroll
   for (int c = 0; c < kCountParts; ++c) mine |= MI355_LD(uint16_t, ws, flags + (c < parts ? c : 0) * kCountLines + hi - 1);
-  const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
-  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
-  if (sample_one_key(temp, K1, tp)) return;                            // (its flags were not written)
   unsigned long long lines, at = block_scan64((mine >> 8 & 1u) + (mine & 1u), scratch, lines);
   if (mine & 1u) used[--at] = static_cast<uint16_t>(hi - 1);
   if (mine >> 8 & 1u) used[--at] = static_cast<uint16_t>(hi);
@@ -1584,67 +1604,181 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(
     const unsigned long long need = found[0], Fp = sample_mass(key16_logit(Tp), l0, temp);
     take = Fp > 0ull ? (need + Fp - 1ull) / Fp : ~0ull;
   }
-  if (tid == 0) {
-    // (a NaN: everything stays, and the draw's first pass is the greedy one)
-    MI355_ST(unsigned long long, ws, head + 1, best_key == 0xFFFFu ? 0xFFFFull : static_cast<unsigned long long>(Tp));
-    MI355_ST(unsigned long long, ws, head + 2, take);
-  }
-  if (take != ~0ull && tid < 64) {                                     // tokens at the cut key in the parts ahead of each
-    unsigned long long c = 0ull;
-    if (tid < parts && MI355_LD(uint8_t, ws, flags + tid * kCountLines + (Tp >> 5)) != 0) c = MI355_LD(uint16_t, ws, counters + tid * 65536 + Tp);
-    const unsigned long long upto = wave_scan64(c, [](unsigned long long x, unsigned long long y) { return x + y; });
-    if (tid < parts) MI355_ST(uint32_t, ws, reinterpret_cast<uint32_t*>(head + 3) + tid, static_cast<uint32_t>(upto - c));
-  }
+  return {best_key, Tp, take};
 }
 
-__global__ __launch_bounds__(kSampleWsThreads) void sample_draw_kernel(
+// Gumbel-max over many tokens without two logarithms (of some forty operations) for each: as -ln u >= 1 - u, a score is at most
+// l / t - ln(1 - u), which the hardware's logarithm gives to a margin, and as -ln u <= (1 - u) / u it is at least that plus ln u.  The
+// scores themselves, bit for bit as everywhere, are formed only for tokens whose bound reaches the best lower bound that the wave
+// has seen, one or two of a row.  (64 rows of 128256 logits without a cut, us a call: all scores 32.6, here 19.6.)
+__device__ __forceinline__ uint32_t raw16_at(const uint4& raw, int j) {
+  const uint32_t x = raw.x, y = raw.y, z = raw.z, w = raw.w, lo = j & 2 ? y + 0u : x + 0u, hi = j & 2 ? w + 0u : z + 0u;      // (values: a choice between members would need an address)
+  return (j & 4 ? hi + 0u : lo + 0u) >> (j & 1 ? 16 : 0) & 0xFFFFu;
+}
+__device__ __forceinline__ unsigned long long gumbel_or_nan(float l, uint32_t i, float temp, uint32_t row_hash) {
+  return l != l ? argmax_key(l, i) : gumbel_key(l, i, temp, row_hash);
+}
+// the best of the tokens `keep` (a bit each) of eight adjacent logits; inv: 1 / temp, low: the wave's lower bound so far.  All lanes of
+// the wave call it.
+__device__ __forceinline__ unsigned long long bounded_gumbel(const uint4 raw, int i0, uint32_t keep, float temp, float inv, uint32_t row_hash, float& low) {
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float top[8], most = -__builtin_inff(), far = 1.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float rest = 1.0f - sample_uniform_at(row_hash, static_cast<uint32_t>(i0 + j));        // (exact)
+    const float l = BF16::to_f(static_cast<uint16_t>(j & 1 ? w[j >> 1] >> 16 : w[j >> 1] & 0xFFFFu));
+    const float b = l * inv - 0.69314718f * __builtin_amdgcn_logf(rest);
+    top[j] = keep >> j & 1u ? b : -__builtin_inff();
+    if (top[j] > most) most = top[j], far = rest;
+  }
+  float at_least = most + 0.69314718f * __builtin_amdgcn_logf(1.0f - far) - (fabsf(most) * 2e-6f + 1e-3f);
+  at_least = at_least != at_least ? -__builtin_inff() : at_least;      // (an infinity less its margin)
+  low = fmaxf(low, wave_maxf(at_least));
+  uint32_t near = 0u;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) near |= top[j] + (fminf(fabsf(top[j]), 1e30f) * 2e-6f + 1e-3f) < low ? 0u : 1u << j;      // (a NaN stays)
+  near &= keep;
+  unsigned long long best = 0ull;
+  if (low == -__builtin_inff()) {                                      // (uniform) logits of -inf have that score whatever their draw
+    uint32_t none = 0u;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) none |= (j & 1 ? w[j >> 1] >> 16 : w[j >> 1] & 0xFFFFu) == 0xFF80u ? 1u << j : 0u;
+    none &= near;
+    if (none != 0u) best = argmax_key(-__builtin_inff(), static_cast<uint32_t>(i0 + __ffs(none) - 1));
+    near &= ~none;
+  }
+  while (near != 0u) {
+    const int j = __ffs(near) - 1;
+    near &= near - 1u;
+    best = umax64(best, gumbel_or_nan(BF16::to_f(static_cast<uint16_t>(raw16_at(raw, j))), static_cast<uint32_t>(i0 + j), temp, row_hash));
+  }
+  return best;
+}
+
+// Every workgroup of a row works the cut out for itself (they share the lines in the caches), draws over its range of the columns and
+// merges its best key; the row's last one turns the key into the token.
+__global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(
     int64_t* __restrict__ out, unsigned long long* __restrict__ ws, const uint16_t* __restrict__ logits, int64_t stride, int vocab,
     const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
-    const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps, int part_vecs, int chunk_vecs) {
+    const int64_t* __restrict__ seeds, const int64_t* __restrict__ steps, int rows, int parts, int part_vecs, int ranges, int chunk_vecs) {
+  __shared__ CountedScratch sh;
   __shared__ unsigned long long part_best[kSampleThreads / 64];
-  __shared__ int eq_base[kSampleThreads / 64 + 1], ties[2], listed[kSampleWsThreads];
-  const int row = blockIdx.y, range = blockIdx.x, ranges = gridDim.x, tid = threadIdx.x;
-  const float temp = MI355_LD(float, temperature, temperature + row);
+  __shared__ int eq_base[kSampleThreads / 64 + 1], ties[3], listed[kSampleListed];
+  __shared__ uint2 kept[kSampleKept];                                  // index, logit
+  const int2 place_of = row_and_piece(rows, ranges);
+  const int row = place_of.x, range = place_of.y, tid = threadIdx.x, lane = tid & 63;
+  const float temp = MI355_LD(float, temperature, temperature + row), tp = MI355_LD(float, top_p, top_p + row);
   const uint64_t seed = static_cast<uint64_t>(MI355_LD(int64_t, seeds, seeds + row)), step = static_cast<uint64_t>(MI355_LD(int64_t, steps, steps + row));
+  const int K1 = active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab);
   const uint16_t* base = logits + row * stride;
   unsigned long long* head = ws + static_cast<int64_t>(row) * kSampleWsHead;
-  const bool one = sample_one_key(temp, active_top_k(MI355_LD(int32_t, top_k, top_k + row), vocab), MI355_LD(float, top_p, top_p + row));
-  const uint32_t Tp = static_cast<uint32_t>(MI355_LD(unsigned long long, ws, head + 1));       // (written for rows with a cut)
+  const bool one = sample_one_key(temp, K1, tp);
+  const int nvec = vocab >> 3, v0 = range * chunk_vecs, v1 = min(v0 + chunk_vecs, nvec);
+  // this thread's first vector travels while the cut is worked out
+  uint4 first = make_uint4(0u, 0u, 0u, 0u);
+  if (nvec > 0) first = MI355_LD(uint4, logits, base + 8 * min(v0 + tid, nvec - 1));
+  CountedCut cut = {0u, 0u, ~0ull};                                    // (a row without a cut: every key is above it)
+  const uint8_t* flags = reinterpret_cast<const uint8_t*>(ws + static_cast<int64_t>(rows) * kSampleWsHead) + static_cast<int64_t>(row) * parts * kCountLines;
+  const uint16_t* counters = reinterpret_cast<const uint16_t*>(ws + static_cast<int64_t>(rows) * (kSampleWsHead + parts * (kCountLines / 8))) +
+                             static_cast<int64_t>(row) * parts * 65536;
+  if (tid < 3) ties[tid] = 0;
+  if (!one) cut = counted_cut(ws, flags, counters, parts, K1, temp, tp, sh);
   unsigned long long best = 0ull;
-  if (one || Tp == 0xFFFFu) {
-    best = sample_one_key_best<MI355_BF16>(base, vocab, !one || !(temp > 0.0f), temp, seed, step, range, ranges, chunk_vecs, part_best);
+  if (!(temp > 0.0f) || cut.top == 0xFFFFu) {                          // greedy (and a NaN in a row with a cut: its first index)
+    best = sample_one_key_best<MI355_BF16>(base, vocab, true, temp, seed, step, range, ranges, chunk_vecs, part_best);
   } else {
-    const unsigned long long take = MI355_LD(unsigned long long, ws, head + 2);
-    const int v0 = range * chunk_vecs, v1 = min(v0 + chunk_vecs, vocab >> 3);
+    const uint32_t Tp = cut.key;
+    const unsigned long long take = cut.take;
     const uint32_t row_hash = sample_hash(seed, step);
-    // one look: what stays for sure is drawn, the cut key's tokens are listed
-    if (tid < 2) ties[tid] = 0;
+    const float inv = 1.0f / temp;
+    float low = -__builtin_inff();
     __syncthreads();
-    auto look = [&](uint32_t raw, int i) {
-      const uint32_t k = key16(raw);
-      if (k > Tp || (k == Tp && take == ~0ull)) {
-        best = umax64(best, gumbel_key(key16_logit(k), static_cast<uint32_t>(i), temp, row_hash));
-      } else if (k == Tp) {
-        const int at = atomicAdd(&ties[0], 1);
-        if (at < kSampleWsThreads) listed[at] = i;
-      }
+    // What stays for sure is listed and drawn behind the look, a token a lane, or, where most lanes have some, drawn as it lies; the cut
+    // key's tokens are listed.  Most vectors hold neither: their largest logits say so (as 16-bit numbers; a cut below zero: the
+    // smallest unsigned ones).
+    auto place = [&](int& count, unsigned long long lanes) {           // of a lane in a list to which these lanes add
+      const int leader = __ffsll(lanes) - 1;
+      int at = 0;
+      if (lane == leader) at = atomicAdd(&count, __popcll(lanes));
+      return __builtin_amdgcn_readlane(at, leader) + __popcll(lanes & ((1ull << lane) - 1ull));
     };
-    for (int v = v0 + tid; v < v1; v += kSampleWsThreads) {
-      const uint4 raw = MI355_LD(uint4, logits, base + 8 * v);
-      const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    auto tie = [&](bool equal, int i) {
+      const unsigned long long same = __ballot(equal);
+      if (same == 0ull) return;
+      const int at = place(ties[0], same);
+      if (equal && at < kSampleListed) listed[at] = i;
+    };
+    typedef short s16x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const bool above_zero = Tp > 0x8000u;
+    const uint32_t Traw = above_zero ? Tp & 0x7FFFu : Tp == 0x8000u ? Tp : ~Tp & 0xFFFFu;
+    auto reaches = [&](const uint4& q) {
+      if (above_zero) {
+        const s16x2 m = __builtin_elementwise_max(
+            __builtin_elementwise_max(__builtin_bit_cast(s16x2, q.x), __builtin_bit_cast(s16x2, q.y)),
+            __builtin_elementwise_max(__builtin_bit_cast(s16x2, q.z), __builtin_bit_cast(s16x2, q.w)));
+        return max(static_cast<int>(m.x), static_cast<int>(m.y)) >= static_cast<int>(Traw);
+      }
+      const u16x2 m = __builtin_elementwise_min(
+          __builtin_elementwise_min(__builtin_bit_cast(u16x2, q.x), __builtin_bit_cast(u16x2, q.y)),
+          __builtin_elementwise_min(__builtin_bit_cast(u16x2, q.z), __builtin_bit_cast(u16x2, q.w)));
+      return min(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y)) <= Traw;
+    };
+    for (int vb = v0; vb < v1; vb += kSampleThreads) {
+      const int v = vb + tid;
+      const uint4 raw = vb == v0 ? first : MI355_LD(uint4, logits, base + 8 * min(v, nvec - 1));
+      uint32_t stay = v < v1 ? 0xFFu : 0u;
+      if (!one) {
+        if (__ballot(stay != 0u && reaches(raw)) == 0ull) continue;
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+        uint32_t equal = 0u, above = 0u;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) look(w[j] & 0xFFFFu, 8 * v + 2 * j), look(w[j] >> 16, 8 * v + 2 * j + 1);
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t k = key16(j & 1 ? w[j >> 1] >> 16 : w[j >> 1] & 0xFFFFu);
+          equal |= k == Tp ? 1u << j : 0u, above |= k > Tp ? 1u << j : 0u;
+        }
+        equal &= stay;
+        if (take == ~0ull) above |= equal, equal = 0u;
+        stay &= above;
+        while (__ballot(equal != 0u) != 0ull) {
+          tie(equal != 0u, 8 * v + __ffs(equal) - 1);
+          equal &= equal - 1u;
+        }
+        if (__popcll(__ballot(stay != 0u)) < 32) {
+          for (unsigned long long some; (some = __ballot(stay != 0u)) != 0ull;) {
+            const int at = place(ties[2], some), j = __ffs(stay) - 1;
+            if (stay != 0u) {
+              const uint32_t x = raw16_at(raw, j);
+              if (at < kSampleKept) kept[at] = make_uint2(8 * v + j, x);
+              else best = umax64(best, gumbel_key(BF16::to_f(static_cast<uint16_t>(x)), 8 * v + j, temp, row_hash));
+              stay &= stay - 1u;
+            }
+          }
+          continue;
+        }
+      }
+      if (__ballot(stay != 0u) != 0ull) best = umax64(best, bounded_gumbel(raw, 8 * v, stay, temp, inv, row_hash, low));
     }
     if (range == ranges - 1)
-      for (int i = (vocab & ~7) + tid; i < vocab; i += kSampleWsThreads) look(MI355_LD(uint16_t, logits, base + i), i);
+      for (int ib = vocab & ~7; ib < vocab; ib += kSampleThreads) {  // (fewer than eight)
+        const int i = ib + tid;
+        const uint32_t raw = i < vocab ? MI355_LD(uint16_t, logits, base + i) : 0u, k = key16(raw);
+        const bool equal = !one && i < vocab && k == Tp;
+        if (i < vocab && (one || k > Tp || (equal && take == ~0ull)))
+          best = umax64(best, gumbel_or_nan(BF16::to_f(static_cast<uint16_t>(raw)), static_cast<uint32_t>(i), temp, row_hash));
+        tie(equal && take != ~0ull, i);
+      }
     __syncthreads();
+    for (int i = tid; i < min(ties[2], kSampleKept); i += kSampleThreads)
+      best = umax64(best, gumbel_key(BF16::to_f(static_cast<uint16_t>(kept[i].y)), kept[i].x, temp, row_hash));
     const int num = ties[0];
     if (num > 0) {                                                     // ranked: behind those of the part ahead of this range
       // (the vectors past the row's last whole one belong to the last part, wherever this range begins)
-      const int part = min(v0 / part_vecs, count_parts(gridDim.y) - 1);
+      const int part = min(v0 / part_vecs, parts - 1);
       int c = 0;
+      if (tid < part && MI355_LD(uint8_t, ws, flags + tid * kCountLines + (Tp >> 5)) != 0) c = MI355_LD(uint16_t, ws, counters + tid * 65536 + Tp);
 #pragma unroll 4
-      for (int v = part * part_vecs + tid; v < v0; v += kSampleWsThreads) {
+      for (int v = part * part_vecs + tid; v < min(v0, nvec); v += kSampleThreads) {
         const uint4 raw = MI355_LD(uint4, logits, base + 8 * v);
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -1652,9 +1786,9 @@ __global__ __launch_bounds__(kSampleWsThreads) void sample_draw_kernel(
       }
       if (c != 0) atomicAdd(&ties[1], c);
       __syncthreads();
-      const unsigned long long before = static_cast<unsigned long long>(ties[1]) + MI355_LD(uint32_t, ws, reinterpret_cast<const uint32_t*>(head + 3) + part);
+      const unsigned long long before = static_cast<unsigned long long>(ties[1]);
       const float l = key16_logit(Tp);
-      if (num <= kSampleWsThreads) {
+      if (num <= kSampleListed) {
         if (tid < num) {
           const int i = listed[tid];
           unsigned long long rank = before;
@@ -1663,7 +1797,7 @@ __global__ __launch_bounds__(kSampleWsThreads) void sample_draw_kernel(
         }
       } else if (before < take) {
         ordered_kept_pass<MI355_BF16>(base, vocab, v0, v0 + chunk_vecs, range == ranges - 1, sample_key(l), take, before, eq_base, [&](float f, int i) {
-          best = umax64(best, gumbel_key(f, static_cast<uint32_t>(i), temp, row_hash));
+          if (f == l) best = umax64(best, gumbel_key(f, static_cast<uint32_t>(i), temp, row_hash));      // (the others are drawn)
         });
       }
       __syncthreads();
@@ -1684,14 +1818,17 @@ __global__ __launch_bounds__(kSampleWsThreads) void sample_draw_kernel(
 
 static int32_t launch_counted(const char* name, int64_t* out, unsigned long long* ws, const void* logits, int64_t stride, int rows, int vocab,
                               const float* temperature, const int32_t* top_k, const float* top_p, const int64_t* seeds, const int64_t* steps,
-                              int chunks, int chunk_vecs, hipStream_t s) {
-  const int parts = count_parts(rows), part_vecs = ((vocab >> 3) + parts - 1) / parts + (vocab < 8);
+                              hipStream_t s) {
+  const int nvec = vocab >> 3, parts = count_parts(rows), part_vecs = (nvec + parts - 1) / parts + (vocab < 8);
+  // ranges of the draw: a workgroup a CU, but whole turns of 256 vectors each
+  int ranges = 256 / rows < 64 ? 256 / rows : 64;
+  const int chunk_vecs = ((nvec + ranges * 256 - 1) / (ranges * 256) + (nvec == 0)) * 256;
+  ranges = nvec > chunk_vecs ? (nvec + chunk_vecs - 1) / chunk_vecs : 1;
   const uint16_t* p = static_cast<const uint16_t*>(logits);
-  hipLaunchKernelGGL(sample_count_kernel, dim3(parts, rows), dim3(kSampleThreads), 0, s, ws, p, stride, vocab, temperature, top_k, top_p,
-                     part_vecs);
-  hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(kSampleThreads), 0, s, ws, parts, vocab, temperature, top_k, top_p);
-  hipLaunchKernelGGL(sample_draw_kernel, dim3(chunks, rows), dim3(kSampleWsThreads), 0, s, out, ws, p, stride, vocab, temperature, top_k,
-                     top_p, seeds, steps, part_vecs, chunk_vecs);
+  hipLaunchKernelGGL(sample_count_kernel, dim3(parts * rows), dim3(kSampleThreads), 0, s, ws, p, stride, vocab, temperature, top_k, top_p,
+                     rows, parts, part_vecs);
+  hipLaunchKernelGGL(sample_draw_kernel, dim3(ranges * rows), dim3(kSampleThreads), 0, s, out, ws, p, stride, vocab, temperature, top_k,
+                     top_p, seeds, steps, rows, parts, part_vecs, ranges, chunk_vecs);
   return check_launch(name);
 }
 
@@ -2121,8 +2258,7 @@ extern "C" int32_t mi355_sample_topk_topp_ws(int64_t* out_ids, const void* logit
   // counts of 16 bits (a part of a row: at most 65535 logits), and room for them
   if (logits_dtype == MI355_BF16 && num_rows <= kCountRows && workspace_bytes >= 8 * count_ws_words(num_rows) &&
       ((vocab >> 3) / count_parts(num_rows) + 2) * 8 <= 65535) {
-    return launch_counted(name, out_ids, ws, logits, logits_stride, num_rows, vocab, temperature, top_k, top_p, seeds, steps, chunks,
-                                      chunk_vecs, s);
+    return launch_counted(name, out_ids, ws, logits, logits_stride, num_rows, vocab, temperature, top_k, top_p, seeds, steps, s);
   }
   const int64_t words = sample_ws_words(num_rows, 2 * (logits_dtype == MI355_F32 ? 4 : logits_dtype == MI355_BF16 ? 2 : 3));
   const int64_t threads = words / 2;                     // (two words each)
