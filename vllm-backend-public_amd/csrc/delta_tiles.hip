@@ -13,10 +13,11 @@
 // <= 0, so a strong decay neither overflows nor costs a later weak one its digits.
 //
 // What bounds it: the walk, one tile after the other; 25 matrix instructions a wave and tile at 32 cycles
-// each, and one barrier.  Measured, 4 x 2048 rows of 128 x 128 heads in bf16: 16 heads with a decay per head 322 us
-// (prep 116, walk 206), 8 heads with a decay per channel 267 us (130, 140), where the recurrence token by token took
-// 1351 and 1140 us; one prompt of 2048 rows 171 and 172 us, before 1114 and 1054.  A state column's d rows are dealt to the 4 waves of a workgroup; the accumulator layout
-// (row 4 (lane / 16) + r, column lane % 16) serves as the right operand as it stands if step r of a product takes
+// each, one barrier, and the tile's 33 KB through the vector caches (80 of 125 us with neither loads nor stores; more sets of them in
+// flight, or each set asked for right behind its last use: the same).  Measured, 4 x 2048 rows of 128 x 128 heads in bf16, 8 heads with a
+// decay per channel: prep 93, walk 125 us; with the rows of all heads side by side in the workspace (every head's
+// 4 KB apart) and 43 KB of LDS, three workgroups a CU, 128 and 144.  A state column's d rows are dealt to the 4 waves of a workgroup; the
+// accumulator layout (row 4 (lane / 16) + r, column lane % 16) serves as the right operand as it stands if step r of a product takes
 // rows {4 g + r}, so the state never leaves its registers.
 #include "common.h"
 #include "delta_tiles.h"
@@ -34,8 +35,9 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __bui
 // padded key channels: a multiple of the 4 waves' 16-row blocks
 __host__ __device__ __forceinline__ int padded(int d) { return (d + 63) & ~63; }
 
-// workspace: W [rows][H][dp] | P [rows][H][16] | q | k | e, of `plane` floats each:
-//   a decay per channel   [rows + 16][H][dp] e^G q | e^(G_end - G) k | e^G_end (a tile's, at its first row)
+// workspace: W [H][rows][dp] | P [H][rows][16] | q | k | e, of `plane` floats each (W, P and a channel's q within a tile of n rows
+// as the walk's lanes hold them: vectors of four channels or rows by (wave, vector, lane / 16, row), see `lane_order`):
+//   a decay per channel   [H][rows + 16][dp] e^G q | e^(G_end - G) k | e^G_end (a tile's, at its first row)
 //   a decay per head      [H][rows + 16] factors of the raw query and key, e^G / (|q| sqrt(d)) and e^(G_end - G) / |k|,
 //                         and e^G_end (a tile's, at its first row)
 struct Layout {
@@ -56,12 +58,56 @@ __device__ __forceinline__ Layout layout(float* ws, int64_t rows, int H, int dp)
   return l;
 }
 
+// log(1 + e^z) for z <= 20: max(z, 0) + log(1 + w), w = e^-|z| as two numbers (2^n and a series in the rest), log(1 + w) = 2 artanh(s) with
+// s = w / (2 + w) <= 1/3, its rounding carried along.  Largest and mean square error against 64 bits over [-80, 20]: 9.4e-8 and
+// 3.0e-8 of it, where log1pf(expf(z)) has 1.35e-7 and 3.6e-8; sixteen of them a thread, so that they were 27 of 102 us of the preparation
+// (8 heads, 4 x 2048 rows) and are 18.
+__device__ __forceinline__ float softplus(float z) {
+  float m = -fabsf(z);                                    // (a NaN stays one)
+  m = m < -120.f ? -120.f : m;
+  const float n = rintf(m * 1.44269504088896340736f);
+  const float h = fmaf(n, -0.693145751953125f, m), g = fmaf(n, -1.428606820309417e-6f, h), gl = fmaf(n, -1.428606820309417e-6f, h - g);
+  float t = 1.0f / 5040.0f;
+  t = fmaf(t, g, 1.0f / 720.0f), t = fmaf(t, g, 1.0f / 120.0f), t = fmaf(t, g, 1.0f / 24.0f), t = fmaf(t, g, 1.0f / 6.0f);
+  t = fmaf(fmaf(t, g, 0.5f), g * g, gl);
+  const int ni = static_cast<int>(n);
+  const float a = 1.0f + g, al = (g - (a - 1.0f)) + t;
+  float w = a + al, wl = al - (w - a);
+  w = ldexpf(w, ni), wl = ldexpf(wl, ni);
+  const float q = 2.0f + w, ql = (w - (q - 2.0f)) + wl, r = __builtin_amdgcn_rcpf(q), s = w * r;
+  const float sl = (fmaf(-s, q, w) + fmaf(-s, ql, wl)) * r, x = s * s;
+  float y = 1.0f / 15.0f;
+  y = fmaf(y, x, 1.0f / 13.0f), y = fmaf(y, x, 1.0f / 11.0f), y = fmaf(y, x, 1.0f / 9.0f), y = fmaf(y, x, 1.0f / 7.0f);
+  y = fmaf(y, x, 0.2f), y = fmaf(y, x, 1.0f / 3.0f);
+  const float low = fmaf(s * x, y, sl);
+  return z > 0.f ? z + fmaf(2.0f, low, 2.0f * s) : fmaf(2.0f, low, 2.0f * s);
+}
+// Where channels 4 c .. 4 c + 3 of a row lie within a tile of n rows, in float4: the walk's wave has 16 DT channels, its lane 4 DT of one
+// row.  (By rows each of a wave's loads touches 16 lines, another with every lane: the walk of 4 x 2048 rows of 16 heads took 255 us where
+// this takes 205; of 8 heads 125 either way.)
+template <int DT>
+__device__ __forceinline__ int lane_order(int c, int row, int n) {
+  const int wave = c / (4 * DT), kg = c % (4 * DT) / DT, j = c % DT;
+  return ((wave * DT + j) * 4 + kg) * n + row;
+}
+// lanes l, l + 16, l + 32, l + 48 hold four numbers each: lane l + 16 m gets the m-th of the four lanes'
+__device__ __forceinline__ void transpose4(float (&y)[4]) {
+  auto swap = [](float& a, float& b, auto f) {
+    const auto r = f(__float_as_uint(a), __float_as_uint(b));
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+  };
+  auto p32 = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+  auto p16 = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+  swap(y[0], y[2], p32), swap(y[1], y[3], p32);
+  swap(y[0], y[1], p16), swap(y[2], y[3], p16);
+}
+
 template <typename T, bool PC, int DT>
-__global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int vec, int dvec) {
+__global__ __launch_bounds__(256, DT <= 2 ? 4 : 1) void delta_tiles_prep_kernel(DeltaTiles a, int vec, int dvec) {
   typedef typename Elem<T>::S E;
   constexpr int dp = 64 * DT, ld = dp + 4, lg = dp + 2, NV = (DT + 1) / 2;
   __shared__ __attribute__((aligned(16))) float Ks[C * ld], Qs[C * ld];        // unit keys, unit queries / sqrt(d)
-  __shared__ __attribute__((aligned(16))) float As[C * C], part[4][2][C * C];
+  __shared__ __attribute__((aligned(16))) float As[C * C], part[4][2][3][64];
   __shared__ __attribute__((aligned(16))) double Gs[PC ? C * lg : C];          // log2 decays, then their sums
   __shared__ __attribute__((aligned(16))) float bs[C], rk[C], rq[C];           // beta, 1 / |key|, 1 / (|query| sqrt(d))
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.y, g = h / (a.H / a.G), d = a.d;
@@ -157,7 +203,7 @@ __global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int
     // log2 of a decay; below 2^-200 a float is zero all the same
     const float na = -expf(alog) * 1.44269504088896340736f;
     auto log_decay = [&](float z) {
-      const float l = na * (z > 20.0f ? z : log1pf(expf(z)));
+      const float l = na * (z > 20.0f ? z : softplus(z));
       return t < n ? static_cast<double>(l < -200.0f ? -200.0f : l) : 0.0;
     };
 #pragma unroll
@@ -228,30 +274,37 @@ __global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int
       for (int x = 0; x < 4; ++x) aa[0] = mfma4(k4[x], k4[x], aa[0]), pp[0] = mfma4(q4[x], k4[x], pp[0]);
     }
   }
+  // wave w sums rows 4 g + w of the waves' parts, its own from its registers (so that four workgroups of 128 channels fit a CU's LDS)
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  float u = 0.f, y = 0.f;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int i = 4 * kg + r, diff = i ^ li;
-    float u = aa[0][r], y = pp[0][r];
+    float ur = aa[0][r], yr = pp[0][r];
     if constexpr (PC) {
-      u = diff & 8 ? aa[3][r] : diff & 4 ? aa[2][r] : diff & 2 ? aa[1][r] : aa[0][r];
-      y = diff & 8 ? pp[3][r] : diff & 4 ? pp[2][r] : diff & 2 ? pp[1][r] : diff ? pp[0][r] : diag[r];
+      const int diff = (4 * kg + r) ^ li;
+      ur = diff & 8 ? aa[3][r] : diff & 4 ? aa[2][r] : diff & 2 ? aa[1][r] : aa[0][r];
+      yr = diff & 8 ? pp[3][r] : diff & 4 ? pp[2][r] : diff & 2 ? pp[1][r] : diff ? pp[0][r] : diag[r];
     }
-    part[wave][0][i * C + li] = u;
-    part[wave][1][i * C + li] = y;
+    if (r == wv) u = ur, y = yr;
+    else part[wv][0][r < wv ? r : r - 1][lane] = ur, part[wv][1][r < wv ? r : r - 1][lane] = yr;
   }
   __syncthreads();
   const Layout l = layout<PC>(a.ws, a.rows, a.H, dp);
   const int64_t at0 = row0 * a.H + h;                     // (row, head) of the tile's first row; a row further: + H
+  const int64_t hw = h * a.rows + row0, hq = h * (a.rows + C) + row0;
   {
-    float u = 0.f, y = 0.f;
+    const int t = 4 * kg + wv, x = li;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) u += part[w][0][tid], y += part[w][1][tid];
+    for (int w = 0; w < 4; ++w) {
+      if (w == wv) continue;
+      u += part[w][0][wv < w ? wv : wv - 1][lane], y += part[w][1][wv < w ? wv : wv - 1][lane];
+    }
     if (!PC) {
       const float e = __builtin_amdgcn_exp2f(fminf(static_cast<float>(Gs[t] - Gs[x]), 0.f));
       u *= e, y *= e;
     }
-    As[tid] = x < t ? bs[t] * u : 0.f;
-    if (t < n) MI355_ST(float, a.ws, l.p + (at0 + static_cast<int64_t>(t) * a.H) * C + x, x <= t ? y : 0.f);
+    As[t * C + x] = x < t ? bs[t] * u : 0.f;
+    if (t < n) MI355_ST(float, a.ws, l.p + hw * C + ((x & 3) * 4 + (x >> 2)) * n + t, x <= t ? y : 0.f);
     if (!PC && x == 0 && t < n) {
       const double end = Gs[C - 1];                       // (rows past the last add 0)
       const int64_t at = static_cast<int64_t>(h) * (a.rows + C) + row0 + t;
@@ -262,25 +315,37 @@ __global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int
   }
   __syncthreads();
   // ---- forward substitution, a column a thread: first the dp columns of b e^G k, then the dv of b V
-  for (int col = tid; col < dp + a.dv; col += 256) {
+  for (int at = tid; at < dp + a.dv; at += 256) {
     float y[C];
-    const bool value = col >= dp;
+    const bool value = at >= dp;
+    // (keys: four adjacent columns in lanes 16 apart, to be transposed below)
+    const int col = value ? at : (at & ~63) + 4 * (lane & 15) + (lane >> 4);
+    auto put = [&](float* to, float (&v)[4], int i) {    // rows i .. i + 3 of the keys' columns
+      transpose4(v);
+      const int r = i + (lane >> 4);
+      if (r < n)
+        MI355_ST(float4, a.ws, reinterpret_cast<float4*>(to) + lane_order<DT>((at & ~63) / 4 + (lane & 15), r, n),
+                 make_float4(v[0], v[1], v[2], v[3]));
+    };
     if (!value) {
       const double end = PC ? Gs[(C - 1) * lg + col] : 0.0;
-      int64_t at = at0 * dp + col;
 #pragma unroll
-      for (int i = 0; i < C; ++i) {
-        const double G = PC ? Gs[i * lg + col] : Gs[i];
-        const float e = __builtin_amdgcn_exp2f(static_cast<float>(G)), k = Ks[i * ld + col];
-        y[i] = bs[i] * (k * e);
-        if (PC && i < n) {
-          MI355_ST(float, a.ws, l.q + at, Qs[i * ld + col] * e);
-          MI355_ST(float, a.ws, l.k + at, k * __builtin_amdgcn_exp2f(static_cast<float>(end - G)));
-          at += static_cast<int64_t>(a.H) * dp;
+      for (int i0 = 0; i0 < C; i0 += 4) {
+        float q[4];
+#pragma unroll
+        for (int i = i0; i < i0 + 4; ++i) {
+          const double G = PC ? Gs[i * lg + col] : Gs[i];
+          const float e = __builtin_amdgcn_exp2f(static_cast<float>(G)), k = Ks[i * ld + col];
+          y[i] = bs[i] * (k * e);
+          if constexpr (PC) {
+            q[i - i0] = Qs[i * ld + col] * e;
+            if (i < n) MI355_ST(float, a.ws, l.k + (hq + i) * dp + col, k * __builtin_amdgcn_exp2f(static_cast<float>(end - G)));
+          }
+          if (i & 1) asm volatile("" ::: "memory");
         }
-        if (i & 1) asm volatile("" ::: "memory");
+        if constexpr (PC) put(l.q + hq * dp, q, i0);
       }
-      if (PC) MI355_ST(float, a.ws, l.e + at0 * dp + col, __builtin_amdgcn_exp2f(static_cast<float>(end)));
+      if (PC) MI355_ST(float, a.ws, l.e + hq * dp + col, __builtin_amdgcn_exp2f(static_cast<float>(end)));
     } else {
 #pragma unroll
       for (int i = 0; i < C; ++i) y[i] = bs[i] * elem_to_f<T>(vraw[i]);
@@ -293,14 +358,22 @@ __global__ __launch_bounds__(256) void delta_tiles_prep_kernel(DeltaTiles a, int
       for (int j = 0; j < i; ++j) sum += As[i * C + j] * y[j];
       y[i] -= sum;
     }
-    float* to = value ? a.o + at0 * a.dv + (col - dp) : l.w + at0 * dp + col;
-    const int64_t step = static_cast<int64_t>(a.H) * (value ? a.dv : dp);
+    if (value) {
+      float* to = a.o + at0 * a.dv + (col - dp);
+      const int64_t step = static_cast<int64_t>(a.H) * a.dv;
 #pragma unroll
-    for (int i = 0; i < C; ++i) {
-      if (i < n) MI355_ST(float, (value ? a.o : a.ws), to, y[i]);
-      to += step;
+      for (int i = 0; i < C; ++i) {
+        if (i < n) MI355_ST(float, a.o, to, y[i]);
+        to += step;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < C; i += 4) {
+        float v[4] = {y[i], y[i + 1], y[i + 2], y[i + 3]};
+        put(l.w + hw * dp, v, i);
+      }
     }
-    load_v(col + 256);
+    load_v(at + 256);
   }
 }
 
@@ -359,12 +432,13 @@ __global__ __launch_bounds__(256, 2) void delta_tiles_walk_kernel(DeltaTiles a, 
   };
   Rows ring[NS];
   const int cl = live ? col : dv - 1;
-  const uint32_t row_w = static_cast<uint32_t>(a.H) * dp * 4u, row_k = PC ? row_w : static_cast<uint32_t>(a.stride * ES);
-  uint32_t vp, vw, vq, vu, vk[4];
+  const uint32_t row_w = dp * 4u, row_k = PC ? row_w : static_cast<uint32_t>(a.stride * ES);
+  uint32_t vp, vw[DT], vq, vu, vk[4];
   auto offsets = [&](int n) {
     const uint32_t rq = li < n ? li : n - 1, ru = 4 * kg + wave < n ? 4 * kg + wave : n - 1;
-    vp = (rq * a.H * C + 4 * kg + wave) * 4u;
-    vw = rq * row_w + cw * 4u;
+    vp = ((4 * wave + kg) * n + rq) * 4u;
+#pragma unroll
+    for (int j = 0; j < DT; ++j) vw[j] = ((4 * (DT * wave + j) + kg) * n + rq) * 16u;
     vq = rq * row_k + (PC || cw < d ? cw : 0) * static_cast<uint32_t>(ES);
     vu = (ru * a.H * dv + cl) * 4u;
 #pragma unroll
@@ -374,41 +448,53 @@ __global__ __launch_bounds__(256, 2) void delta_tiles_walk_kernel(DeltaTiles a, 
     }
   };
 #define AT(base, off) (reinterpret_cast<const char*>(base) + (off))
-  // NS register sets: a tile's loads travel while the tile ahead of it is worked on
-  auto fetch = [&](Rows& f, int i) {
-    const int64_t row0 = cs + i * C, hr = row0 * a.H + h;
-    if (len - i * C < C) offsets(len - i * C);
-    const K *q0, *k0;
-    if constexpr (PC) {
-      q0 = l.q + hr * dp, k0 = l.k + hr * dp;
-      f.e = MI355_LD(RunW, a.ws, AT(l.e + hr * dp, cw * 4u));
-    } else {
-      q0 = static_cast<const E*>(a.qkv) + row0 * a.stride + a.q_off + g * d;
-      k0 = static_cast<const E*>(a.qkv) + row0 * a.stride + a.k_off + g * d;
+  // What a tile adds to the bases of its first (worked out anew from the rows, the addresses of a tile were some 130 scalar instructions
+  // that the one wave of a SIMD has nothing to hide behind).
+  const int64_t hr = cs * a.H + h, hw = h * a.rows + cs, hq = h * (a.rows + C) + cs;
+  const float *w0 = l.w + hw * dp, *p0 = l.p + hw * C, *e0 = l.e + hq * (PC ? dp : 1), *u0 = a.o + hr * dv;
+  const float *q0 = l.q + hq * (PC ? dp : 1), *k0 = l.k + hq * (PC ? dp : 1);
+  const E* rows = static_cast<const E*>(a.qkv) + cs * a.stride + g * d;
+  const int64_t rows_step = C * a.stride, u_step = static_cast<int64_t>(C) * a.H * dv;
+  auto vectors = [&](float (&to)[4 * DT], const float* from) {
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+      const float4 u = MI355_LD(float4, a.ws, AT(from, vw[j]));
+      to[4 * j] = u.x, to[4 * j + 1] = u.y, to[4 * j + 2] = u.z, to[4 * j + 3] = u.w;
     }
-    f.w = MI355_LD(RunW, a.ws, AT(l.w + hr * dp, vw));
-    if constexpr (VEC) {
-      f.q = MI355_LD(RunQ, kv_base, AT(q0, vq));
+  };
+  // NS register sets: a tile's loads travel while the tile ahead of it is worked on
+  auto fetch = [&](Rows& f, int64_t i) {
+    if (len - i * C < C) offsets(static_cast<int>(len - i * C));
+    const int64_t at = i * (C * dp);
+    const E* row = rows + i * rows_step;
+    [[maybe_unused]] const K* kr;
+    if constexpr (PC) kr = k0 + at;
+    else kr = row + a.k_off;
+    if constexpr (PC) f.e = MI355_LD(RunW, a.ws, AT(e0 + at, cw * 4u));
+    vectors(f.w.v, w0 + at);
+    if constexpr (PC) {
+      vectors(f.q.v, q0 + at);
+    } else if constexpr (VEC) {
+      f.q = MI355_LD(RunQ, kv_base, AT(row + a.q_off, vq));
     } else {
 #pragma unroll
-      for (int x = 0; x < 4 * DT; ++x) f.q.v[x] = MI355_LD(K, kv_base, AT(q0 + (cw + x < d ? x : 0), vq));
+      for (int x = 0; x < 4 * DT; ++x) f.q.v[x] = MI355_LD(K, kv_base, AT(row + a.q_off + (cw + x < d ? x : 0), vq));
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if constexpr (VEC) {
-        f.k[r] = MI355_LD(RunK, kv_base, AT(k0, vk[r]));
+        f.k[r] = MI355_LD(RunK, kv_base, AT(kr, vk[r]));
       } else {
 #pragma unroll
-        for (int x = 0; x < DT; ++x) f.k[r].v[x] = MI355_LD(K, kv_base, AT(k0 + (ck + x < d ? x : 0), vk[r]));
+        for (int x = 0; x < DT; ++x) f.k[r].v[x] = MI355_LD(K, kv_base, AT(kr + (ck + x < d ? x : 0), vk[r]));
       }
     }
-    f.u = MI355_LD(float, a.o, AT(a.o + hr * dv, vu));
-    f.p = MI355_LD(float, a.ws, AT(l.p + hr * C, vp));
+    f.u = MI355_LD(float, a.o, AT(u0 + i * u_step, vu));
+    f.p = MI355_LD(float, a.ws, AT(p0 + i * (C * C), vp));
     if constexpr (!PC) {                                  // (the rows of these are padded by a tile)
-      const int64_t fr = static_cast<int64_t>(h) * (a.rows + C) + row0;
-      f.qf = MI355_LD(decltype(f.qf), a.ws, AT(l.q + fr, 16u * kg));
-      f.kf = MI355_LD(decltype(f.kf), a.ws, AT(l.k + fr, 16u * kg));
-      f.end = MI355_LD(float, a.ws, AT(l.e + fr, 0u * kg));
+      f.qf = MI355_LD(decltype(f.qf), a.ws, AT(q0 + i * C, 16u * kg));
+      f.kf = MI355_LD(decltype(f.kf), a.ws, AT(k0 + i * C, 16u * kg));
+      f.end = MI355_LD(float, a.ws, AT(e0 + i * C, 0u * kg));
     }
   };
 #undef AT
@@ -422,7 +508,7 @@ __global__ __launch_bounds__(256, 2) void delta_tiles_walk_kernel(DeltaTiles a, 
 #pragma unroll
     for (int w = 0; w < 4; ++w) y += (&yp[i & 1][w][lane].x)[wave];
     if (i * C + 4 * kg + wave < len && live)
-      MI355_ST(float, a.o, reinterpret_cast<char*>(a.o + ((cs + i * C) * a.H + h) * dv) + vs, y);
+      MI355_ST(float, a.o, reinterpret_cast<char*>(a.o + hr * dv + i * u_step) + vs, y);
   };
   const int num = (len + C - 1) / C;
   auto work = [&](Rows& f, int i) {
