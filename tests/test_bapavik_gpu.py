@@ -1057,3 +1057,41 @@ def test_trace_replay_program(tmp_path):
         got = np.fromfile(out_dir / f"{n}.f32", dtype="<f4").reshape(-1, V)
         assert got.shape[0] == len(rows)
         _close(got, np.stack(rows))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cap,d,dv", [(5.0, 64, 64), (30.0, 192, 128), (31.0, 128, 128), (31.5, 128, 64), (50.0, 128, 128), (0.0, 192, 64)])
+def test_capped_scores_from_one_end_to_the_other(dtype, cap, d, dv):
+    """Prompts of 1, 31, 33 and 150 rows whose first 32 keys have scores near -3 cap where the later ones reach 3 cap, the other way
+    round in every other head, and a sink that weighs as much as a key or nothing.  Against float64.  Bound: a weight is
+    within 2^-8 of its share, the output is rounded once more (2^-9), and a capped score is within 1e-6 of its cap."""
+    from mi355_decode import ops
+    g = torch.Generator().manual_seed(int(cap) + d)
+    H, G, lens = 4, 2, [1, 31, 33, 150]
+    top = cap or 20.0
+    kc, vc = torch.zeros(40, G, 16, d), torch.randn(40, G, dv, 16, generator=g) + 0.5
+    bt, page = torch.zeros(len(lens), 10, dtype=torch.int32), 0
+    q, keys = torch.randn(sum(lens), H, d, generator=g) * 0.3, []
+    q[..., 0] = 3.0 * top * (-1.0) ** torch.arange(H)
+    for s, n in enumerate(lens):
+        k = torch.randn(n, G, d, generator=g) * 0.3
+        k[:, :, 0] = (torch.where(torch.arange(n) < 32, -1.0, 1.0) * torch.rand(n, generator=g))[:, None]
+        keys.append(k.to(dtype))
+        for b in range((n + 15) // 16):
+            bt[s, b] = page
+            kc[page, :, : min(16, n - 16 * b)] = k[16 * b: 16 * b + 16].transpose(0, 1)
+            page += 1
+    q, kc, vc = q.to(dtype), kc.to(dtype), vc.to(dtype)
+    sink = torch.tensor([top if cap else 0.0, -top, 0.0, -1e4])
+    cu, ctx = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0, dtype=torch.int32), torch.tensor(lens, dtype=torch.int32)
+    out = ops.paged_attn_prefill_ext(q.reshape(len(q), -1).cuda(), kc.cuda(), vc.cuda(), bt.cuda(), cu.cuda(), ctx.cuda(), max(lens), H, G, d,
+                                     1.0, sink=sink.cuda(), softcap=cap).cpu().double().view(-1, H, dv)
+    for s, n in enumerate(lens):
+        v = torch.cat([vc[int(bt[s, b])].permute(2, 0, 1) for b in range((n + 15) // 16)])[:n].double()
+        for h in range(H):
+            x = q[int(cu[s]): int(cu[s]) + n, h].double() @ keys[s][:, h // 2].double().t()
+            x = cap * torch.tanh(x / cap) if cap else x
+            x = x.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), -torch.inf)
+            w = torch.softmax(torch.cat([x, sink[h].double().expand(n, 1)], 1), 1)[:, :n]
+            bound = (2.0 ** -8 + 2.0 ** -9 + 1e-6 * top) * (w @ v[:, h // 2].abs()) + 1e-5
+            assert ((out[int(cu[s]): int(cu[s]) + n, h] - w @ v[:, h // 2]).abs() <= bound).all(), (n, h)

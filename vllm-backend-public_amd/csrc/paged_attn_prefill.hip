@@ -48,6 +48,8 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace mi355 {
 
 constexpr int kPrefillThreads = 256;
@@ -265,15 +267,15 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    // soft cap: the scores become tanh(q.k scale / cap) = 1 - 2 / (1 + 2^(cap_x q.k)), cap_x = 2 log2(e) scale / cap;
-    // scale_log2e is then cap log2(e)
+    // soft cap: tanh(q.k scale / cap) = 1 - 2 / (1 + 2^(cap_x q.k)), cap_x = 2 log2(e) scale / cap; the scores become
+    // -1 / (1 + ..), to which weight and shift below give the rest
     if (CAP && cap_x > 0.f) {
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          sa[t][j] = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sa[t][j] * cap_x));
-          sb[t][j] = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sb[t][j] * cap_x));
+          sa[t][j] = __builtin_amdgcn_rcpf(-1.0f - __builtin_amdgcn_exp2f(sa[t][j] * cap_x));
+          sb[t][j] = __builtin_amdgcn_rcpf(-1.0f - __builtin_amdgcn_exp2f(sb[t][j] * cap_x));
         }
       }
     }
@@ -312,6 +314,18 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
   };
 
   // ================= one pass: scores, probabilities against a lazy reference, O =================
+  // A score's exponent is weight s + shift (scale_log2e: of capped scores cap log2 e); references and thresholds leave shift out.
+  // Capped scores lie within 2 cap of one another, so that of bf16 rows the largest of a column's first 32 keys serves as its reference to the
+  // end if weights and sums of 2^90 (caps up to 31) are far inside bf16 and fp32.  The sum of the weights is one more product, with a
+  // column of ones: of the weights as V meets them.  What bounds this mode is the count of vector instructions beside the products (a
+  // series for tanh, without transcendentals but with one or three more instructions, is no faster).  Measured, causal, us before / now: five
+  // prompts of 1050 to 2100, 16 heads, keys of 192 on 16 kv heads 217 / 206, of 128 on four 172 / 160; 8192 rows, 32 heads on eight 695 / 651.
+  // Errors against 64 bits 2.19e-3 / 2.10e-3 (scores of one), 2.18e-3 / 2.00e-3 (2.5) and 2.03e-3 / 1.83e-3 (8).
+  const bool capped = CAP && cap_x > 0.f;
+  const bool fixed = capped && std::is_same<T, BF16>::value && scale_log2e <= 45.f;
+  const float weight = capped ? 2.0f * scale_log2e : scale_log2e, shift = capped ? scale_log2e : 0.f;
+  [[maybe_unused]] f32x4 ls[NQ];                  // CAP: the column's sum, in every row
+  [[maybe_unused]] const uint4 ones = make_uint4(T::pack2(1.f, 1.f), T::pack2(1.f, 1.f), T::pack2(1.f, 1.f), T::pack2(1.f, 1.f));
   float m_ref[NQ], m_thr[NQ], neg_m[NQ];          // in the exponent's units (score * scale * log2 e)
   f32x2 l[NQ];                                    // sum of the lane's probabilities, two partial sums
   f32x4 o[NQ][NT];
@@ -320,6 +334,7 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     m_ref[t] = m_thr[t] = -INFINITY;
     neg_m[t] = 0.f;                               // a column that has seen no key yet: exponent reference 0
     l[t] = f32x2{0.f, 0.f};
+    if (CAP) ls[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int n = 0; n < NT; ++n) o[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -338,40 +353,43 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     } else {
       // does any score of this lane leave the slack above its column's reference?  (scale > 0: the
       // maximum commutes with the scaling; a masked score is -inf and never does)
-      float lm[NQ];
-      bool grow = false;
-#pragma unroll
-      for (int t = 0; t < NQ; ++t) {
-        lm[t] = scale_log2e * max3(max3(max3(sa[t][0], sa[t][1], sa[t][2]), sa[t][3], sb[t][0]),
-                                   max3(sb[t][1], sb[t][2], sb[t][3]), -INFINITY);
-        grow |= lm[t] > m_thr[t];
-      }
-      if (__any(grow)) {                                           // wave-uniform; rare after a tile's first step
+      if (!fixed || s == 0) {                                      // wave-uniform
+        float lm[NQ];
+        bool grow = false;
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
-          float v = lm[t];
-          v = fmaxf(v, __shfl_xor(v, 16, 64));                     // the column's keys of this step sit on 4 lanes
-          v = fmaxf(v, __shfl_xor(v, 32, 64));
-          const float m_new = fmaxf(m_ref[t], v);
-          // -inf -> finite: alpha = 0 (O and l are still zero); no key seen yet: nothing to rescale
-          const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
-          l[t] *= alpha;                                           // both halves
+          lm[t] = weight * max3(max3(max3(sa[t][0], sa[t][1], sa[t][2]), sa[t][3], sb[t][0]),
+                                     max3(sb[t][1], sb[t][2], sb[t][3]), -INFINITY);
+          grow |= lm[t] > m_thr[t];
+        }
+        if (__any(grow)) {                                           // wave-uniform; rare after a tile's first step
 #pragma unroll
-          for (int n = 0; n < NT; ++n) {
-            o[t][n][0] *= alpha;
-            o[t][n][1] *= alpha;
-            o[t][n][2] *= alpha;
-            o[t][n][3] *= alpha;
+          for (int t = 0; t < NQ; ++t) {
+            float v = lm[t];
+            v = fmaxf(v, __shfl_xor(v, 16, 64));                     // the column's keys of this step sit on 4 lanes
+            v = fmaxf(v, __shfl_xor(v, 32, 64));
+            const float m_new = fmaxf(m_ref[t], v);
+            // -inf -> finite: alpha = 0 (O and l are still zero); no key seen yet: nothing to rescale
+            const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref[t] - m_new);
+            if (CAP) ls[t] *= alpha;
+            else l[t] *= alpha;                                      // both halves
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+              o[t][n][0] *= alpha;
+              o[t][n][1] *= alpha;
+              o[t][n][2] *= alpha;
+              o[t][n][3] *= alpha;
+            }
+            m_ref[t] = m_new;
+            m_thr[t] = m_new + kSlack;                               // -inf stays -inf
+            neg_m[t] = (m_new == -INFINITY) ? 0.f : -m_new;
           }
-          m_ref[t] = m_new;
-          m_thr[t] = m_new + kSlack;                               // -inf stays -inf
-          neg_m[t] = (m_new == -INFINITY) ? 0.f : -m_new;
         }
       }
       // p = exp2(s * scale - m_ref): the softmax scale is folded into the exponent, one fma per score
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
-        const f32x2 sc = {scale_log2e, scale_log2e}, nm = {neg_m[t], neg_m[t]};
+        const f32x2 sc = {weight, weight}, nm = {neg_m[t], neg_m[t]};
         const f32x2 e[4] = {__builtin_elementwise_fma(f32x2{sa[t][0], sa[t][1]}, sc, nm),   // v_pk_fma_f32
                             __builtin_elementwise_fma(f32x2{sa[t][2], sa[t][3]}, sc, nm),
                             __builtin_elementwise_fma(f32x2{sb[t][0], sb[t][1]}, sc, nm),
@@ -382,7 +400,7 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
           p[2 * j] = __builtin_amdgcn_exp2f(e[j][0]);
           p[2 * j + 1] = __builtin_amdgcn_exp2f(e[j][1]);
         }
-        l[t] += (f32x2{p[0], p[1]} + f32x2{p[2], p[3]}) + (f32x2{p[4], p[5]} + f32x2{p[6], p[7]});   // v_pk_add_f32
+        if (!CAP) l[t] += (f32x2{p[0], p[1]} + f32x2{p[2], p[3]}) + (f32x2{p[4], p[5]} + f32x2{p[6], p[7]});   // v_pk_add_f32
         pf[t] = pack8<T>(p);
       }
     }
@@ -390,6 +408,10 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
     // the tile's last query were cleared when the image was staged)
     const unsigned char* vbase = &lds[image * BUF + KBYTES + lane * 16];
     __builtin_amdgcn_s_setprio(1);
+    if constexpr (CAP) {
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) ls[t] = T::mfma(ones, pf[t], ls[t]);
+    }
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const uint4 vf = *reinterpret_cast<const uint4*>(vbase + n * 1024);
@@ -428,12 +450,11 @@ __global__ __launch_bounds__(kPrefillThreads, NQ <= 2 ? 2 : 1) void paged_attn_p
 
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
-    float lt = l[t][0] + l[t][1];
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    float lt = CAP ? ls[t][0] : l[t][0] + l[t][1];
+    if (!CAP) lt += __shfl_xor(lt, 16, 64), lt += __shfl_xor(lt, 32, 64);
     if (!col_ok[t]) continue;
     if (EXT && sink != nullptr)          // the value-less term, against the column's reference (a valid column has seen a key)
-      lt += __builtin_amdgcn_exp2f(MI355_LD(float, sink, sink + col_head[t]) * 1.4426950408889634f - m_ref[t]);
+      lt += __builtin_amdgcn_exp2f(MI355_LD(float, sink, sink + col_head[t]) * 1.4426950408889634f - shift - m_ref[t]);
     float inv = SIG ? 1.0f : lt > 0.f ? 1.0f / lt : 0.f;
     if (EXT) inv *= out_scale;
     if (EXT && gate != nullptr)
