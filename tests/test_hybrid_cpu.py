@@ -212,6 +212,27 @@ def test_query_tiles_cover_every_row_once_in_order(rows):
         assert got.dtype == np.int32 and got.flags.c_contiguous and got.shape == (len(want), 3) and got.tolist() == want
 
 
+def test_step_fields_come_with_the_first_that_is_read():
+    """Token ids, sizes and plans are there at once; the first other field brings all of them, once; an unknown one is an error."""
+    calls = []
+
+    def rest():
+        calls.append(1)
+        return {"positions": 1, "slot_mapping": 2, "block_tables": 3, "cu_seqlens": 4, "context_lens": None, "tok_seq": 5, "state_slots": 6,
+                "tiles": 7}
+
+    b = HR.StepBatch.behind(rest, torch.zeros(9, dtype=torch.int64), 3, True, None, 5, None, None, 8)
+    assert (b.num_tokens, b.num_seqs, b.long_chunks, b.max_q_len, b.max_context, b.routes, b.keep_tail, b.tail) == \
+        (9, 3, True, 5, 8, {}, False, None) and b.latent_plan is None and not calls
+    assert b.context_lens is None and b.tiles == 7 and b.positions == 1 and b.tok_seq == 5 and calls == [1]
+    with pytest.raises(AttributeError):
+        b.no_such_field
+    plain = HR.StepBatch(torch.zeros(2), 1, 2, 3, torch.zeros(3), 4, 5)
+    assert plain.num_seqs == 2 and plain.tiles is None
+    with pytest.raises(AttributeError):
+        plain.no_such_field
+
+
 def test_upload_keeps_values_shapes_and_types():
     from mi355_decode import ops
     src = [np.arange(5, dtype=np.int64) - 2, np.zeros((0,), np.int32), np.arange(6, dtype=np.int32).reshape(2, 3)[:, ::2], np.zeros((3, 0), np.int64)]

@@ -83,7 +83,7 @@ class StepBatch:
     """Device-side description of one packed step (see csrc/seqmix.hip)."""
     __slots__ = ("ids", "positions", "slot_mapping", "block_tables", "cu_seqlens", "tok_seq", "state_slots",
                  "num_tokens", "num_seqs", "tiles", "long_chunks", "pair_tiles", "context_lens", "max_q_len", "row_tiles",
-                 "routes", "latent_plan", "max_context", "keep_tail", "tail")
+                 "routes", "latent_plan", "max_context", "keep_tail", "tail", "_rest")
 
     def __init__(self, ids, positions, slot_mapping, block_tables, cu_seqlens, tok_seq, state_slots, tiles=None,
                  long_chunks=False, pair_tiles=None, context_lens=None, max_q_len=0, row_tiles=None,
@@ -101,7 +101,27 @@ class StepBatch:
         self.long_chunks = long_chunks                # some chunk holds several tokens (prompts and portions)
         self.ids, self.positions, self.slot_mapping, self.block_tables = ids, positions, slot_mapping, block_tables
         self.cu_seqlens, self.tok_seq, self.state_slots = cu_seqlens, tok_seq, state_slots
-        self.num_tokens, self.num_seqs = int(ids.numel()), int(cu_seqlens.numel()) - 1
+        self.num_tokens, self.num_seqs, self._rest = int(ids.numel()), int(cu_seqlens.numel()) - 1, None
+
+    @classmethod
+    def behind(cls, rest, ids, num_seqs, long_chunks, pair_tiles, max_q_len, row_tiles, latent_plan, max_context):
+        """A step of which only the token ids are on the device yet: rest() uploads the fields it returns when the first
+        of them is read, by then behind the launches that need none (embedding, norm and first product, some 200 us of a long
+        prompt step for which the host otherwise keeps the device waiting)."""
+        b = cls.__new__(cls)
+        b.routes, b.keep_tail, b.tail = {}, False, None
+        b.ids, b.num_tokens, b.num_seqs, b.long_chunks, b._rest = ids, int(ids.numel()), int(num_seqs), long_chunks, rest
+        b.pair_tiles, b.row_tiles, b.latent_plan = pair_tiles, row_tiles, latent_plan
+        b.max_q_len, b.max_context = int(max_q_len), int(max_context)
+        return b
+
+    def __getattr__(self, name):                      # (of a field that has not been set)
+        if name == "_rest" or self._rest is None:
+            raise AttributeError(name)
+        rest, self._rest = self._rest, None
+        for field, value in rest().items():
+            setattr(self, field, value)
+        return getattr(self, name)
 
 
 def _out_product(r, x: torch.Tensor, w: torch.Tensor):
@@ -1246,8 +1266,6 @@ class HybridRunner(ModelRunner):
         if state_slots is None:
             raise ValueError("hybrid decoders need the state slot of every chunk")
         self._step_state_slots = np.asarray(state_slots, dtype=np.int32)
-        # rows go to the matrix cores in tiles of up to 16 rows of one chunk
-        self._step_tiles = ops.query_tiles(cu_seqlens)
         self._step_cu, self._pair_tiles, self._row_tiles = np.asarray(cu_seqlens, dtype=np.int64), {}, {}
         self._step_ctx, self._step_tables, self._latent_plan = context_lens, block_tables, None
         self._step_long = int(max_q_len) > 1
@@ -1255,11 +1273,10 @@ class HybridRunner(ModelRunner):
             return super().run_prefill(token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens,
                                        max_q_len, sampling=sampling, logprobs=logprobs, prompt_logprobs=prompt_logprobs)
         rows = np.asarray(logit_rows, dtype=np.int64)
-        host = [np.asarray(a, dtype=dt) for a, dt in ((token_ids, np.int64), (positions, np.int64), (slot_mapping, np.int64),
-                                                      (rows, np.int64), (block_tables, np.int32), (cu_seqlens, np.int32),
-                                                      (context_lens, np.int32))]
-        ids, pos, slots, at, tables, cu, ctx = ops.upload(self.device, *host)
-        resid, tail = self._run_chunks(ids, pos, slots, tables, cu, ctx, max_q_len)
+        host = [np.asarray(a, dtype=dt) for a, dt in ((positions, np.int64), (slot_mapping, np.int64), (block_tables, np.int32),
+                                                      (cu_seqlens, np.int32), (context_lens, np.int32))]
+        ids, at = ops.upload(self.device, np.asarray(token_ids, dtype=np.int64), rows)
+        resid, tail = self._run_chunks(ids, *host, max_q_len)
         if rows.size == 0:
             torch.cuda.current_stream().synchronize()
             return np.zeros((0, self.V), dtype=np.float32)
@@ -1268,15 +1285,25 @@ class HybridRunner(ModelRunner):
 
     def _run_chunks(self, token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens=None,
                     max_q_len: int = 0):
-        """The residual of every row, and what its last sub-layer has still to add to it (StepBatch.tail)."""
-        lens = self._step_cu[1:] - self._step_cu[:-1]
-        tok_seq, slots, tiles = ops.upload(self.device, np.repeat(np.arange(len(lens), dtype=np.int32), lens),
-                                           self._step_state_slots, self._step_tiles)
-        b = StepBatch(token_ids, positions, slot_mapping, block_tables.contiguous(), cu_seqlens,
-                      tok_seq, slots, tiles, self._step_long, pair_tiles=self._chunk_pair_tiles,
-                      context_lens=None if context_lens is None else context_lens.to(torch.int32).contiguous(),
-                      max_q_len=max_q_len, row_tiles=self._chunk_row_tiles, latent_plan=self._chunk_latent_plan,
-                      max_context=np.asarray(self._step_ctx).max(initial=0))
+        """The residual of every row, and what its last sub-layer has still to add to it (StepBatch.tail).  The arrays behind the token
+        ids: all on the device or all on the host."""
+        fields = {"positions": positions, "slot_mapping": slot_mapping, "block_tables": block_tables, "cu_seqlens": cu_seqlens,
+                  "context_lens": context_lens}
+        cu, state_slots = self._step_cu, self._step_state_slots
+
+        def rest():
+            # rows go to the matrix cores in tiles of up to 16 rows of one chunk
+            own = [np.repeat(np.arange(len(cu) - 1, dtype=np.int32), cu[1:] - cu[:-1]), state_slots, ops.query_tiles(cu)]
+            given = [k for k, v in fields.items() if isinstance(v, np.ndarray)]
+            up = ops.upload(self.device, *own, *(fields[k] for k in given))
+            full = dict(fields, **dict(zip(("tok_seq", "state_slots", "tiles", *given), up)))
+            full["block_tables"] = full["block_tables"].contiguous()
+            if full["context_lens"] is not None:
+                full["context_lens"] = full["context_lens"].to(torch.int32).contiguous()
+            return full
+
+        b = StepBatch.behind(rest, token_ids, len(cu_seqlens) - 1, self._step_long, self._chunk_pair_tiles, max_q_len,
+                             self._chunk_row_tiles, self._chunk_latent_plan, np.asarray(self._step_ctx).max(initial=0))
         b.keep_tail = b.num_tokens >= self.EXPERT_TAIL_MIN_TOKENS or not (self.ffs and isinstance(self.ffs[-1], TableMoE))
         return self._forward(b), b.tail
 
