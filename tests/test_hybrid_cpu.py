@@ -214,6 +214,7 @@ def test_query_tiles_cover_every_row_once_in_order(rows):
 
 def test_step_fields_come_with_the_first_that_is_read():
     """Token ids, sizes and plans are there at once; the first other field brings all of them, once; an unknown one is an error."""
+    from mi355_decode import hybrid_runner as HR
     calls = []
 
     def rest():
