@@ -878,6 +878,24 @@ int32_t mi355_window_delta_decode(void* attn_out, const void* q, int64_t q_strid
                                   const int32_t* state_slots, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads,
                                   int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream);
 /*
+ * The same for the attention's rows as they are projected: rope_partial_kv_write (16-bit rows, rot_dims a multiple of 16, 16-byte aligned
+ * rows) is part of the launch, but for q, which stays as it is.  A row whose slot is negative writes neither key nor value.
+ */
+int32_t mi355_window_delta_decode_rows(void* attn_out, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                       const void* v, int64_t v_stride, const float* cos_sin, int32_t max_pos,
+                                       int32_t rot_dims, const int64_t* slot_mapping, void* k_cache, void* v_cache,
+                                       const int32_t* block_tables, int32_t max_blocks, const int32_t* tok_seq,
+                                       const float* temp, const float* bias, const void* gate, int64_t gate_stride,
+                                       int32_t attn_heads, int32_t attn_kv_heads, int32_t window, float scale,
+                                       void* out, int64_t out_stride, const void* proj, int64_t proj_stride,
+                                       int32_t qkv_off, int32_t beta_off, int32_t a_off, int32_t g_off,
+                                       const void* conv_w, float* conv_state, int32_t taps, const void* a2,
+                                       const void* g2, int32_t rank, const float* a_log, const float* dt_bias,
+                                       const float* norm_w, int32_t norm_heads, int32_t act, float eps, float* state,
+                                       const int64_t* positions, const int32_t* state_slots, int32_t num_rows,
+                                       int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t v_dim,
+                                       int32_t dtype, void* stream);
+/*
  * An update of the residual and the norm that reads it next, in one launch:
  *   resid_add_norm_f32      resid += other (fp32 rows) + rows + vec (one row), each may be null, in this order; then
  *                           out = resid / rms(resid) * weight (one number or one per column)

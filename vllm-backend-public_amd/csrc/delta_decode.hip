@@ -182,11 +182,15 @@ __global__ __launch_bounds__(512 * R) void delta_decode_kernel(DeltaDecode a) {
 // either leaves half of the chip idle at a few dozen rows.  Workgroups of 16 waves for both: first the attention's, one per
 // (row, kv head), then the recurrence's.  Measured in a step of 32 rows, 16 heads on 4 kv heads behind 1024 keys and 8 heads on 4:
 // 24.4 us, one after the other 21.9 and 13.4.
-template <typename T, bool PC>
-__global__ __launch_bounds__(1024) void window_delta_decode_kernel(WindowDecode w, DeltaDecode a, int rows) {
+// FRESH: the attention's rows as they are projected (WindowFresh), for which a launch of 5 us went ahead: 32 rows 27.3 us with it, 24.2
+// here (the table's and the rows' loads travel with the pages').
+template <typename T, bool PC, bool FRESH>
+__global__ __launch_bounds__(1024) void window_delta_decode_kernel(WindowDecode w, DeltaDecode a, int rows, WindowFresh f) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int b = blockIdx.x, attention = rows * w.G;
-  if (b < attention) sigmoid_window_decode<T, 128, 128, 16, 1>(w, b % rows, b / rows, 0, 1, smem);
+  if (b < attention)
+    sigmoid_window_decode<T, 128, 128, 16, 1, FRESH>(w, b % rows, b / rows, 0, 1, smem, f,
+                                                     reinterpret_cast<uint16_t*>(smem + 16 * (w.H / w.G) * (128 + 4)));
   else delta_decode<T, PC, 2>(a, (b - attention) % rows, (b - attention) / rows, *reinterpret_cast<DeltaLds<2>*>(smem));
 }
 
@@ -241,18 +245,16 @@ extern "C" int32_t mi355_delta_decode(void* out, int64_t out_stride, const void*
   return check_launch("delta_decode");
 }
 
-extern "C" int32_t mi355_window_delta_decode(void* attn_out, const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
-                                             const int32_t* block_tables, int32_t max_blocks, const int32_t* tok_seq, const float* temp,
-                                             const float* bias, const void* gate, int64_t gate_stride, int32_t attn_heads,
-                                             int32_t attn_kv_heads, int32_t window, float scale, void* out, int64_t out_stride,
-                                             const void* proj, int64_t proj_stride, int32_t qkv_off, int32_t beta_off, int32_t a_off,
-                                             int32_t g_off, const void* conv_w, float* conv_state, int32_t taps, const void* a2,
-                                             const void* g2, int32_t rank, const float* a_log, const float* dt_bias, const float* norm_w,
-                                             int32_t norm_heads, int32_t act, float eps, float* state, const int64_t* positions,
-                                             const int32_t* state_slots, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads,
-                                             int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream) {
+static int32_t window_delta_decode(const char* name, const mi355::WindowFresh* fresh, void* attn_out, const void* q, int64_t q_stride,
+                                   const void* k_cache, const void* v_cache, const int32_t* block_tables, int32_t max_blocks,
+                                   const int32_t* tok_seq, const float* temp, const float* bias, const void* gate, int64_t gate_stride,
+                                   int32_t attn_heads, int32_t attn_kv_heads, int32_t window, float scale, void* out, int64_t out_stride,
+                                   const void* proj, int64_t proj_stride, int32_t qkv_off, int32_t beta_off, int32_t a_off, int32_t g_off,
+                                   const void* conv_w, float* conv_state, int32_t taps, const void* a2, const void* g2, int32_t rank,
+                                   const float* a_log, const float* dt_bias, const float* norm_w, int32_t norm_heads, int32_t act, float eps,
+                                   float* state, const int64_t* positions, const int32_t* state_slots, int32_t num_rows, int32_t num_heads,
+                                   int32_t num_kv_heads, int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream) {
   using namespace mi355;
-  const char* name = "window_delta_decode";
   const DeltaDecode a = {static_cast<uint16_t*>(out), out_stride, static_cast<const uint16_t*>(proj), proj_stride, qkv_off, beta_off, a_off,
                          g_off, static_cast<const uint16_t*>(conv_w), static_cast<const uint16_t*>(a2), static_cast<const uint16_t*>(g2),
                          conv_state, taps, rank, a_log, dt_bias, norm_w, norm_heads, act, eps, state, positions, state_slots, num_heads,
@@ -266,17 +268,68 @@ extern "C" int32_t mi355_window_delta_decode(void* attn_out, const void* q, int6
   MI355_REQUIRE(sums <= 65536 && num_heads == 2 * num_kv_heads && q_stride % 8 == 0 && aligned16(q) && aligned16(k_cache) &&
                     aligned16(v_cache) && aligned16(attn_out),
                 MI355_ERR_UNSUPPORTED, "%s: at most 7 query heads a kv head, two heads a key head, 16-byte aligned rows", name);
+  if (fresh != nullptr) {
+    MI355_REQUIRE(fresh->k && fresh->v && fresh->cos_sin && fresh->slot_mapping && fresh->max_pos > 0 && fresh->rot >= 0 && fresh->rot <= 128 &&
+                      fresh->k_stride >= attn_kv_heads * 128 && fresh->v_stride >= attn_kv_heads * 128,
+                  MI355_ERR_INVALID, "%s: keys, values, table and slots", name);
+    MI355_REQUIRE(fresh->rot % 16 == 0 && fresh->k_stride % 8 == 0 && fresh->v_stride % 8 == 0 && aligned16(fresh->k) && aligned16(fresh->v) &&
+                      aligned16(fresh->cos_sin),
+                  MI355_ERR_UNSUPPORTED, "%s: rotated coordinates a multiple of 16, 16-byte aligned rows", name);
+  }
   if (num_rows == 0) return MI355_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const WindowDecode w = {static_cast<uint16_t*>(attn_out), static_cast<const uint16_t*>(q), q_stride, static_cast<const uint16_t*>(k_cache),
                           static_cast<const uint16_t*>(v_cache), block_tables, max_blocks, tok_seq, positions, temp, bias,
                           static_cast<const uint16_t*>(gate), gate_stride, attn_heads, attn_kv_heads, window, scale, nullptr, 0};
-  const size_t lds = sums > sizeof(DeltaLds<2>) ? sums : sizeof(DeltaLds<2>);
+  const size_t mine = sums + (fresh != nullptr ? sizeof(uint16_t) * window_fresh_lds(attn_heads / attn_kv_heads, 128, 128) : 0);
+  const size_t lds = mine > sizeof(DeltaLds<2>) ? mine : sizeof(DeltaLds<2>);
   const dim3 grid(static_cast<unsigned>(num_rows) * static_cast<unsigned>(attn_kv_heads + num_kv_heads));
-#define MI355_WDD(TT, PC) hipLaunchKernelGGL((window_delta_decode_kernel<TT, PC>), grid, dim3(1024), lds, s, w, a, num_rows)
-  if (dtype == MI355_BF16) { if (a2 != nullptr) MI355_WDD(BF16, true); else MI355_WDD(BF16, false); }
+#define MI355_WDD(TT, PC)                                                                                                               \
+  do {                                                                                                                                  \
+    if (fresh != nullptr)                                                                                                               \
+      hipLaunchKernelGGL((window_delta_decode_kernel<TT, PC, true>), grid, dim3(1024), lds, s, w, a, num_rows, *fresh);                 \
+    else hipLaunchKernelGGL((window_delta_decode_kernel<TT, PC, false>), grid, dim3(1024), lds, s, w, a, num_rows, WindowFresh{});      \
+  } while (0)
+  if (dtype == MI355_BF16 && a2 != nullptr) MI355_WDD(BF16, true);
+  else if (dtype == MI355_BF16) MI355_WDD(BF16, false);
   else if (a2 != nullptr) MI355_WDD(F16, true);
   else MI355_WDD(F16, false);
 #undef MI355_WDD
   return check_launch(name);
+}
+
+extern "C" int32_t mi355_window_delta_decode(void* attn_out, const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                                             const int32_t* block_tables, int32_t max_blocks, const int32_t* tok_seq, const float* temp,
+                                             const float* bias, const void* gate, int64_t gate_stride, int32_t attn_heads,
+                                             int32_t attn_kv_heads, int32_t window, float scale, void* out, int64_t out_stride,
+                                             const void* proj, int64_t proj_stride, int32_t qkv_off, int32_t beta_off, int32_t a_off,
+                                             int32_t g_off, const void* conv_w, float* conv_state, int32_t taps, const void* a2,
+                                             const void* g2, int32_t rank, const float* a_log, const float* dt_bias, const float* norm_w,
+                                             int32_t norm_heads, int32_t act, float eps, float* state, const int64_t* positions,
+                                             const int32_t* state_slots, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads,
+                                             int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream) {
+  return window_delta_decode("window_delta_decode", nullptr, attn_out, q, q_stride, k_cache, v_cache, block_tables, max_blocks, tok_seq, temp,
+                             bias, gate, gate_stride, attn_heads, attn_kv_heads, window, scale, out, out_stride, proj, proj_stride, qkv_off,
+                             beta_off, a_off, g_off, conv_w, conv_state, taps, a2, g2, rank, a_log, dt_bias, norm_w, norm_heads, act, eps,
+                             state, positions, state_slots, num_rows, num_heads, num_kv_heads, head_dim, v_dim, dtype, stream);
+}
+
+extern "C" int32_t mi355_window_delta_decode_rows(void* attn_out, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
+                                                  const void* v, int64_t v_stride, const float* cos_sin, int32_t max_pos, int32_t rot_dims,
+                                                  const int64_t* slot_mapping, void* k_cache, void* v_cache, const int32_t* block_tables,
+                                                  int32_t max_blocks, const int32_t* tok_seq, const float* temp, const float* bias,
+                                                  const void* gate, int64_t gate_stride, int32_t attn_heads, int32_t attn_kv_heads,
+                                                  int32_t window, float scale, void* out, int64_t out_stride, const void* proj,
+                                                  int64_t proj_stride, int32_t qkv_off, int32_t beta_off, int32_t a_off, int32_t g_off,
+                                                  const void* conv_w, float* conv_state, int32_t taps, const void* a2, const void* g2,
+                                                  int32_t rank, const float* a_log, const float* dt_bias, const float* norm_w,
+                                                  int32_t norm_heads, int32_t act, float eps, float* state, const int64_t* positions,
+                                                  const int32_t* state_slots, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads,
+                                                  int32_t head_dim, int32_t v_dim, int32_t dtype, void* stream) {
+  const mi355::WindowFresh fresh = {static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_stride, v_stride, cos_sin, max_pos,
+                                    slot_mapping, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), rot_dims};
+  return window_delta_decode("window_delta_decode_rows", &fresh, attn_out, q, q_stride, k_cache, v_cache, block_tables, max_blocks, tok_seq,
+                             temp, bias, gate, gate_stride, attn_heads, attn_kv_heads, window, scale, out, out_stride, proj, proj_stride,
+                             qkv_off, beta_off, a_off, g_off, conv_w, conv_state, taps, a2, g2, rank, a_log, dt_bias, norm_w, norm_heads, act,
+                             eps, state, positions, state_slots, num_rows, num_heads, num_kv_heads, head_dim, v_dim, dtype, stream);
 }

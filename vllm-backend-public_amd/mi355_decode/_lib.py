@@ -181,6 +181,9 @@ def _load() -> ctypes.CDLL:
                                      I32, I32, I32, P]),
         "mi355_window_delta_decode": (I32, [P, P, I64, P, P, P, I32, P, P, P, P, I64, I32, I32, I32, F, P, I64, P, I64, I32, I32, I32, I32, P, P,
                                             I32, P, P, I32, P, P, P, I32, I32, F, P, P, P, I32, I32, I32, I32, I32, I32, P]),
+        "mi355_window_delta_decode_rows": (I32, [P, P, I64, P, I64, P, I64, P, I32, I32, P, P, P, P, I32, P, P, P, P, I64, I32, I32, I32, F,
+                                                 P, I64, P, I64, I32, I32, I32, I32, P, P, I32, P, P, I32, P, P, P, I32, I32, F, P, P, P,
+                                                 I32, I32, I32, I32, I32, I32, P]),
         "mi355_resid_add_norm_f32": (I32, [P, P, I32, P, P, P, I32, P, I64, I32, F, I32, P]),
         "mi355_rms_norm_mix_norm_f32": (I32, [P, P, I32, P, P, I32, P, P, I32, P, I64, I32, F, F, I32, P]),
         "mi355_mingru_scan_workspace": (I64, [I32, I32, I32]),
@@ -233,7 +236,7 @@ EXPORTS = ("mi355_abi_version", "mi355_last_error", "mi355_target_arch",
            "mi355_linear_attn_chunks", "mi355_decay_attn_step", "mi355_mlstm_step",
            "mi355_moe_linear_rows", "mi355_moe_table_sort", "mi355_add_layer_norm_f32", "mi355_expert_gemm",
            "mi355_head_gemm", "mi355_latent_q_rotate", "mi355_paged_attn_decode_ext", "mi355_resid_add_norm_f32",
-           "mi355_rms_norm_mix_norm_f32", "mi355_delta_decode", "mi355_window_delta_decode", "mi355_moe_linear_rows_hinted")
+           "mi355_rms_norm_mix_norm_f32", "mi355_delta_decode", "mi355_window_delta_decode", "mi355_window_delta_decode_rows", "mi355_moe_linear_rows_hinted")
 
 
 def check(status: int) -> None:

@@ -157,6 +157,12 @@ def staged_window_pays(tokens: int, chunks: int, longest: int, context: int, hea
 # and 256 rows (6144) 368 / 359, behind 20 tokens 165 / 177: rounds of workgroups that have little to walk cover nobody's start.
 BESIDE_MAX_WORKGROUPS = 4096
 
+# Attention workgroups (rows x kv heads) up to which that launch also rotates the rows and writes them to their pages.  us, a launch ahead /
+# within, 16 heads on 4 and 8 on 4 behind 1024 keys: 1 row 15.8 / 14.1, 32 rows 27.3 / 24.2, 64 rows 54.4 / 50.8, 128 rows 100.5 / 96.7,
+# 256 rows 192 / 186; behind 20 keys 18.3 / 15.3 (32 rows), 25.1 / 23.8, 46.3 / 46.8, 91.7 / 96.3; 16 on 16 of window 512 1 row 14.6 / 11.1,
+# 32 rows 51.3 / 50.6, 128 rows 159.7 / 161.3: each of many short workgroups then has the rotation's trip to memory of its own.
+FRESH_MAX_WORKGROUPS = 512
+
 
 class WindowAttention:
     """Sliding-window attention with sigmoid weights over the paged K/V of one layer run."""
@@ -184,10 +190,16 @@ class WindowAttention:
                 or lw.seg["lq"][0] % 8 or (s.window > 1024 and self.r.key_splits(b, s)) \
                 or b.num_tokens * (s.kv_heads + d.kv_heads) > BESIDE_MAX_WORKGROUPS:
             return None
-        q, g, kc, vc = self._rows(proj, b)
+        col = {n: proj[:, lw.seg[n][0]: lw.seg[n][0] + lw.seg[n][1]] for n in ("lq", "lk", "lv", "lg")}
+        fresh, table = {}, self.r.rotary(s.rot_dims, s.rot_base)
+        if b.num_tokens * s.kv_heads <= FRESH_MAX_WORKGROUPS and s.rot_dims % 16 == 0 and lw.seg["lk"][0] % 8 == 0 and lw.seg["lv"][0] % 8 == 0 and table.data_ptr() % 16 == 0:
+            q, g, kc, vc = col["lq"], col["lg"], self.r.k_cache[self.ci], self.r.v_cache[self.ci]
+            fresh = dict(k=col["lk"], v=col["lv"], cos_sin=table, slot_mapping=b.slot_mapping)
+        else:
+            q, g, kc, vc = self._rows(proj, b)
         rows, on = delta.step(proj, b, attention=dict(q=q, k_cache=kc, v_cache=vc, block_tables=b.block_tables, tok_seq=b.tok_seq,
                                                       temp=lw.attn_temp, bias=lw.attn_bias, gate=g, num_heads=s.heads,
-                                                      window=s.window, scale=s.scale))
+                                                      window=s.window, scale=s.scale, **fresh))
         return _out_product(self.r, rows, lw.attn_o_w), _out_product(self.r, on, lw.delta_o_w)
 
     def __call__(self, proj: torch.Tensor, b: StepBatch) -> torch.Tensor:

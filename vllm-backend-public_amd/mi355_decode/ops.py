@@ -1557,7 +1557,8 @@ def delta_decode(proj: torch.Tensor, seg: dict, conv_w: torch.Tensor, conv_state
     """causal_conv_silu, the products with a2 and g2 (a decay a channel), gated_delta_rule and gated_head_rms_norm for rows
     that are one token of a sequence each, in one launch.  seg: (offset, width) of the columns q, k, v (adjacent), b and
     a, g or a1, g1 in proj's rows.  attention: sigmoid_window_attn's arguments (q, k_cache, v_cache, block_tables, tok_seq, temp,
-    bias, gate, num_heads, window, scale) of an attention of the same rows that the launch takes along; its rows come first then."""
+    bias, gate, num_heads, window, scale) of an attention of the same rows that the launch takes along; its rows come first then.
+    With k, v, cos_sin and slot_mapping beside them it does what rope_partial_kv_write would have done ahead (q stays as it is)."""
     S, (H, G) = proj.shape[0], (num_heads, num_kv_heads)
     C, taps = conv_w.shape
     low = a2 is not None
@@ -1579,7 +1580,15 @@ def delta_decode(proj: torch.Tensor, seg: dict, conv_w: torch.Tensor, conv_state
             raise ValueError("pages of 128 keys and values, block_tables contiguous int32 [chunks, max_blocks]")
         rows = torch.empty(S, nh * 128, dtype=proj.dtype, device=proj.device)
         launch = lib.mi355_window_delta_decode
-        attn = (rows.data_ptr(), _same(q, proj, "q"), _cols(q, "q", nh * 128), _same(kc, proj, "k_cache"), _same(vc, proj, "v_cache"),
+        fresh = ()
+        if "k" in at:
+            launch, k, v, table = lib.mi355_window_delta_decode_rows, at["k"], at["v"], at["cos_sin"]
+            if kc.shape[0] != vc.shape[0] or not kc.is_contiguous() or not vc.is_contiguous():
+                raise ValueError("K pages must be [blocks, kv_heads, 16, 128] and V pages [blocks, kv_heads, 128, 16]")
+            fresh = (_same(k, proj, "k"), _cols(k, "k", kc.shape[1] * 128), _same(v, proj, "v"), _cols(v, "v", kc.shape[1] * 128),
+                     _f32(table, "cos_sin") or q.data_ptr(), max(table.shape[0], 1), table.shape[1],
+                     _idx(at["slot_mapping"], "slot_mapping", torch.int64, S))
+        attn = (rows.data_ptr(), _same(q, proj, "q"), _cols(q, "q", nh * 128), *fresh, _same(kc, proj, "k_cache"), _same(vc, proj, "v_cache"),
                 bt.data_ptr(), bt.shape[1], _idx(at["tok_seq"], "tok_seq", torch.int32, S), _f32(at["temp"], "temp", nh),
                 _f32(at["bias"], "bias", nh), None if gate is None else _same(gate, proj, "gate"),
                 0 if gate is None else _cols(gate, "gate", nh), nh, kc.shape[1], int(at["window"]), float(at["scale"]))
