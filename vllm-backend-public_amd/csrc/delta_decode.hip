@@ -98,7 +98,7 @@ __device__ __forceinline__ void delta_decode(const DeltaDecode& a, int s, int g,
 #pragma unroll
     for (int j = 0; j < kDeltaTaps; ++j)
       if (j < taps && p - (taps - 1 - j) >= 0) acc += wv[j] * in[j];  // (zeros before the start of the sequence)
-    ys[tid] = round_f<T>(acc / (1.0f + expf(-acc)));
+    ys[tid] = round_f<T>(silu_any(acc));          // (the same bits as the convolution of prompts)
 #pragma unroll
     for (int j = 0; j < kDeltaTaps - 1; ++j)
       if (j < taps - 1) MI355_ST(float, a.conv_state, cst + static_cast<int64_t>(j) * C, in[j + 1]);

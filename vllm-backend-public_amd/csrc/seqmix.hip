@@ -308,10 +308,24 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
   }
 }
 
+// silu_lean of eight values, by one branch where all of them are in its range (a NaN passes: either form gives it back)
+__device__ __forceinline__ void silu8(float (&x)[8]) {
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(x[i]));
+  if (m < kSiluLeanRange) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = silu_lean(x[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = silu_any(x[i]);
+  }
+}
+
 // 16-bit rows, 8 channels per thread, the taps a template constant; RT rows a thread, whose weights (four times the
 // bytes of a row's inputs) and inputs it then loads once for all of them.  Rows too near the start of their
-// chunk, or a group across chunks, go row by row.  Bound by the trips to L2 for prompts: 8192 rows of 4096 channels and 4 taps
-// 65 us with a row a thread, 45 with 4.
+// chunk, or a group across chunks, go row by row.  Bound by the trips to L2 for prompts and, with the library's exp and divide, by
+// vector instructions: 8192 rows of 4096 channels and 4 taps 65 us with a row a thread, 45 with 4, 37 with silu8.
 template <typename T, int TAPS, int RT>
 __global__ __launch_bounds__(256) void causal_conv_silu_vec_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
@@ -329,8 +343,7 @@ __global__ __launch_bounds__(256) void causal_conv_silu_vec_kernel(
       for (int j = 0; j < TAPS; ++j) unpack8<T>(MI355_LD(uint4, w, w + static_cast<int64_t>(c8) * TAPS + 8 * j), wv[j]);
     };
     auto finish = [&](int64_t t, float (&acc)[8]) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] = acc[i] / (1.0f + expf(-acc[i]));
+      silu8(acc);
       MI355_ST(uint4, y, y + t * C + c8, pack8<T>(acc));
     };
     auto row = [&](int64_t t, bool first) {             // any row, by itself
@@ -450,8 +463,7 @@ __global__ __launch_bounds__(64) void conv_silu_step_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] += (&wv[0][0])[i * TAPS + j] * in[j][i];
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = acc[i] / (1.0f + expf(-acc[i]));
+    silu8(acc);
     MI355_ST(uint4, y, y + t * C + c8, pack8<T>(acc));
 #pragma unroll
     for (int j = 0; j < TAPS - 1; ++j) {
