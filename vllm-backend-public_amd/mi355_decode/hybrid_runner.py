@@ -730,6 +730,10 @@ class HybridRunner(ModelRunner):
     # from this many tokens on a prompt step leaves its last experts' rows to the final norm (StepBatch.tail).  They are two selects
     # and an index more: 30 us of the host, which a small step waits for, where the launch saved takes 5 us at 300 rows and 36 at 8211
     EXPERT_TAIL_MIN_TOKENS = 2048
+    # from this many tokens on only a prompt step's ids are uploaded ahead of its first launch (StepBatch.behind), which gives 60 to 90 us
+    # at 8192 tokens.  A smaller step waits for the host, about 1.3 ms whatever its size, so that one upload in place of two is what
+    # counts: 60 to 800 tokens 15 to 50 us faster than with the second one
+    LATE_FIELDS_MIN_TOKENS = 2048
 
     def __init__(self, cfg: ModelConfig, weights: ModelWeights, dtype: torch.dtype, device, num_blocks: int,
                  max_num_seqs: int, max_model_len: int, tp_rank: int = 0, tp_size: int = 1, tp_group=None,
@@ -1287,28 +1291,38 @@ class HybridRunner(ModelRunner):
         rows = np.asarray(logit_rows, dtype=np.int64)
         host = [np.asarray(a, dtype=dt) for a, dt in ((positions, np.int64), (slot_mapping, np.int64), (block_tables, np.int32),
                                                       (cu_seqlens, np.int32), (context_lens, np.int32))]
-        ids, at = ops.upload(self.device, np.asarray(token_ids, dtype=np.int64), rows)
-        resid, tail = self._run_chunks(ids, *host, max_q_len)
+        first = [np.asarray(token_ids, dtype=np.int64), rows]
+        if first[0].size >= self.LATE_FIELDS_MIN_TOKENS:
+            (ids, at), own = ops.upload(self.device, *first), None
+        else:
+            ids, at, *up = ops.upload(self.device, *first, *host, *self._row_arrays())
+            host, own = up[:len(host)], up[len(host):]
+        resid, tail = self._run_chunks(ids, *host, max_q_len, own)
         if rows.size == 0:
             torch.cuda.current_stream().synchronize()
             return np.zeros((0, self.V), dtype=np.float32)
         z = self._logits(resid.index_select(0, at), tail=self._tail_rows(tail, at))
         return z.float().cpu().numpy()
 
+    def _row_arrays(self) -> list:
+        """Every row's chunk, every chunk's state slot, and the tiles of up to 16 rows of one chunk in which rows go to the matrix
+        cores, on the host."""
+        cu = self._step_cu
+        return [np.repeat(np.arange(len(cu) - 1, dtype=np.int32), cu[1:] - cu[:-1]), self._step_state_slots, ops.query_tiles(cu)]
+
     def _run_chunks(self, token_ids, positions, slot_mapping, block_tables, cu_seqlens, context_lens=None,
-                    max_q_len: int = 0):
+                    max_q_len: int = 0, own=None):
         """The residual of every row, and what its last sub-layer has still to add to it (StepBatch.tail).  The arrays behind the token
-        ids: all on the device or all on the host."""
+        ids: all on the device or all on the host.  own: _row_arrays() on the device, if they are there."""
         fields = {"positions": positions, "slot_mapping": slot_mapping, "block_tables": block_tables, "cu_seqlens": cu_seqlens,
                   "context_lens": context_lens}
-        cu, state_slots = self._step_cu, self._step_state_slots
 
         def rest():
-            # rows go to the matrix cores in tiles of up to 16 rows of one chunk
-            own = [np.repeat(np.arange(len(cu) - 1, dtype=np.int32), cu[1:] - cu[:-1]), state_slots, ops.query_tiles(cu)]
-            given = [k for k, v in fields.items() if isinstance(v, np.ndarray)]
-            up = ops.upload(self.device, *own, *(fields[k] for k in given))
-            full = dict(fields, **dict(zip(("tok_seq", "state_slots", "tiles", *given), up)))
+            names = ("tok_seq", "state_slots", "tiles")
+            full = dict(fields, **dict(zip(names, own if own is not None else self._row_arrays())))
+            late = [k for k, v in full.items() if isinstance(v, np.ndarray)]
+            if late:
+                full.update(zip(late, ops.upload(self.device, *(full[k] for k in late))))
             full["block_tables"] = full["block_tables"].contiguous()
             if full["context_lens"] is not None:
                 full["context_lens"] = full["context_lens"].to(torch.int32).contiguous()
