@@ -623,7 +623,10 @@ def single_launches():
     checked("rms_norm_mix_norm", lambda: ops.rms_norm_mix_norm_f32(x, rows, w, rows, w, 1e-6, 0.5, w))
     x, w = rnd(17, 1024), rnd(96, 1024, m=1 / 32)
     tiled, (gate, up) = ops.tile_weights(w), (x.float() @ w.float().t()).split(48, dim=1)
-    checked("gelu in the product", lambda: ops.linear_tiled(x, tiled, 96, tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL),
+    q, scale = ops.tile_weights_fp8(w)                       # (beside it fp8 weights with K split across waves, whole and in blocks)
+    x33 = torch.cat([x, x])[:33]
+    checked("gelu in the product", lambda: (ops.linear_tiled_w8(x, q, scale, 96, tiles_per_wg=507), ops.linear_tiled_w8(x33, q, scale, 96, tiles_per_wg=2504),
+                                            ops.linear_tiled(x, tiled, 96, tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL))[2],
             torch.nn.functional.gelu(gate, approximate="tanh") * up)
     return done
 

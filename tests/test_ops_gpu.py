@@ -1881,6 +1881,32 @@ def test_linear_tiled_w8_swiglu(ops, M, F, K):
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,N,K,tiles,groups,bias", [(1, 16, 512, 504, 1, False), (16, 1000, 1152, 509, 2, True), (17, 144, 640, 507, 1, True),
+                                                     (32, 3584, 2944, 510, 5, False), (64, 1010, 1664, 2506, 3, True), (33, 336, 2048, 2508, 4, False)])
+def test_linear_tiled_w8_slices(ops, dtype, M, N, K, tiles, groups, bias):
+    """K split across the waves of a workgroup: tile counts that leave the last workgroup part empty, units of K that do not deal
+    evenly to the waves or the K groups, row blocks of one row."""
+    rng = rng_for("w8s", dtype, M, N, K)
+    x, w = grid(rng, (M, K), dtype), grid(rng, (N, K), dtype, 0.05)
+    b = grid(rng, (N,), dtype) if bias else None
+    q, scale = ops.tile_weights_fp8(dev(w, dtype))
+    q_ref, s_ref = R.quantize_rows_fp8(w)
+    ref64 = (x.astype(np.float64) @ q_ref.astype(np.float64).T) * s_ref[None, :].astype(np.float64) + (b.astype(np.float64) if bias else 0.0)
+    tol = _linear_tol(ref64, x, q_ref * s_ref[:, None], K, dtype)
+    xd = dev(x, dtype)
+    y = host(ops.linear_tiled_w8(xd, q, scale, N, bias=dev(b, dtype) if bias else None, tiles_per_wg=tiles))
+    assert (np.abs(y - ref64) <= tol).all(), f"max err {np.abs(y - ref64).max()}"
+    part = ops.linear_tiled_w8(xd, q, scale, N, k_groups=groups, epilogue=ops.EPI_PARTIAL, tiles_per_wg=tiles).cpu().numpy()
+    y = _slab_sum(part, b, dtype)
+    assert (np.abs(y - ref64) <= tol).all(), f"max err {np.abs(y - ref64).max()}"
+    if N % 32 == 0 and tiles % 2 == 0:
+        qi, si = ops.tile_weights_fp8(dev(w, dtype), interleave_halves=True)
+        gated = host(ops.linear_tiled_w8(xd, qi, si, N, epilogue=ops.EPI_SILU_MUL, tiles_per_wg=tiles))
+        gu = ops.linear_tiled_w8(xd, q, scale, N, tiles_per_wg=tiles)     # the same sums in the same order
+        np.testing.assert_array_equal(gated, host(ops.silu_and_mul(gu)))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 def test_linear_tiled_w8_decodes_every_fp8_code_exactly(ops, dtype):
     """Weights whose quantised codes run over the whole e4m3fn table (subnormals and both zeros
     included), read back through one-hot inputs: the in-register fp8 -> 16-bit conversion is exact."""

@@ -43,6 +43,7 @@
 //   a fixed order) -- the RMSNorm between two GEMMs costs no launch of its own.
 // HBM bytes: N*K*2 once; x is read from L2 once per workgroup.
 #include "common.h"
+#include "linear_slices.h"
 
 namespace mi355 {
 
@@ -1169,15 +1170,17 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
   // 302 / 304 / 308, 402 / 404: K split across 2 / 4 / 8 waves of an 8-wave workgroup (1024- / 512-wide slices)
   const bool kws = tiles_per_wg == 302 || tiles_per_wg == 304 || tiles_per_wg == 308 || tiles_per_wg == 402 ||
                    tiles_per_wg == 404;
+  // 504, 506 .. 510: so many tiles a workgroup, K split over its four waves (linear_slices.hip), fp8 weights and up to 32 rows (of a row block)
+  const bool slices = tiles_per_wg >= 500 && tiles_per_wg < 600;
   const int nw = two ? (tiles_per_wg - 200) / 2 : tiles_per_wg % 100;
-  MI355_REQUIRE(two || kws || ((nw == 4 || nw == 8) && (tiles_per_wg == nw || tiles_per_wg == nw + 100)),
+  MI355_REQUIRE(two || kws || slices || ((nw == 4 || nw == 8) && (tiles_per_wg == nw || tiles_per_wg == nw + 100)),
                 MI355_ERR_INVALID, "%s: tiles_per_wg must be 4, 8, 104, 108, 208-216 (even), 302, 304, 308, 402 or 404", name);
   // Rows of a row block (gridDim.z): 128, or with tiles_per_wg + 1000 / + 2000 blocks of 64 / 32 rows, each run
   // by the kernel form built for that many rows (a wave's fragments of x from LDS per weight fragment halve with
   // the block; the blocks of a column block read the same weights, once from HBM).
   const int Mb = min(M, rb_rows);
   const int mt = Mb <= 16 ? 1 : Mb <= 32 ? 2 : Mb <= 64 ? 4 : 8;
-  const int ksl = ((kws ? tiles_per_wg >= 400 : two ? tiles_per_wg == 208 : tiles_per_wg >= 100) ? 512 : 1024) /
+  const int ksl = slices ? 128 : ((kws ? tiles_per_wg >= 400 : two ? tiles_per_wg == 208 : tiles_per_wg >= 100) ? 512 : 1024) /
                   (mt <= 2 ? 1 : mt / 2);
   MI355_REQUIRE(!kws || (!norm && !reduce && fa.w_scale == nullptr), MI355_ERR_UNSUPPORTED,
                 "%s: the K split across waves (tiles_per_wg %d) is built for 16-bit weights and epilogues 0-2", name,
@@ -1196,9 +1199,13 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
                 "%s: K %d must be a multiple of the x slice %d (M %d)", name, K, ksl, M);
   MI355_REQUIRE(fa.w_scale == nullptr || (aligned16(fa.w_scale) && epilogue <= EPI_PARTIAL), MI355_ERR_INVALID,
                 "%s: fp8 weights need a 16-byte aligned scale vector and epilogue 0-2", name);
-  const int phases = K / ksl;
-  MI355_REQUIRE(k_groups >= 1 && k_groups <= phases, MI355_ERR_INVALID, "%s: k_groups %d outside [1, %d] (K / %d)",
-                name, k_groups, phases, ksl);
+  MI355_REQUIRE(!slices || (!norm && !reduce && epilogue != EPI_GELU_MUL && Mb <= 32 && fa.w_scale != nullptr), MI355_ERR_UNSUPPORTED,
+                "%s: K split over the waves with x in registers (tiles_per_wg %d) is built for fp8 weights, up to 32 rows (of a row block) and "
+                "epilogues 0-2", name, tiles_per_wg);
+  MI355_REQUIRE(!slices || epilogue != EPI_SILU_MUL || (y_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0),
+                MI355_ERR_UNSUPPORTED, "%s: this SwiGLU epilogue needs rows on 8-byte boundaries", name);
+  const int phases = slices ? K / 512 : K / ksl;          // (slices: a unit of 128 columns for each wave)
+  MI355_REQUIRE(k_groups >= 1 && k_groups <= phases, MI355_ERR_INVALID, "%s: k_groups %d outside [1, %d]", name, k_groups, phases);
   MI355_REQUIRE(k_groups == 1 || epilogue == EPI_PARTIAL || reduce, MI355_ERR_INVALID,
                 "%s: k_groups > 1 needs a partial-sum or reducing epilogue", name);
   MI355_REQUIRE(x_stride >= K && x_stride % 8 == 0 && aligned16(x) && aligned16(w_tiled), MI355_ERR_INVALID,
@@ -1240,7 +1247,10 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
   auto* wp = static_cast<const uint16_t*>(w_tiled);
   auto* bp = static_cast<const uint16_t*>(bias);
   bool ok;
-  if (kws)
+  if (slices)
+    ok = launch_linear_slices({yp, y_stride, partial, xp, x_stride, w_tiled, fa.w_scale, bp, M, N, K, tiles_total, rb_rows},
+                              tiles_per_wg % 100, k_groups, epilogue, dtype == MI355_BF16, s);
+  else if (kws)
     ok = dtype == MI355_BF16 ? launch_geometry_kw<BF16>(mt, tiles_per_wg % 100, ksl, epilogue, grid, s, yp, partial, xp, wp, bp,
                                                         M, N, K, x_stride, y_stride, tiles_total, phases)
                              : launch_geometry_kw<F16>(mt, tiles_per_wg % 100, ksl, epilogue, grid, s, yp, partial, xp, wp, bp,
@@ -1257,7 +1267,7 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
                                                     x_stride, y_stride, tiles_total, phases, fa);
   MI355_REQUIRE(ok, MI355_ERR_UNSUPPORTED,
                 "%s: no kernel for M %d with tiles_per_wg %d, epilogue %d%s (M <= 32: 4/8/104/108/302/304/308/402/404, "
-                "fused and fp8 forms 8/104; M <= 64: 8/104/108/208-216/302/304/402; beyond: 8/210-216/302)", name, M,
+                "fused and fp8 forms 8/104; M <= 64: 8/104/108/208-216/302/304/402; fp8, blocks of up to 32 rows: 504/506-510; beyond: 8/210-216/302)", name, M,
                 tiles_per_wg, epilogue,
                 norm ? " + norm prologue" : "");
   return check_launch(name);

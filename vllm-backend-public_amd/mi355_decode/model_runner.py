@@ -290,7 +290,7 @@ class ModelRunner:
         """(tiles_per_wg, k_groups) forms of projection `kind` worth timing at m rows."""
         n, kk, split = self.tiled_shapes[kind]
         out = []
-        for cand in ops.linear_tiled_candidates(n, kk, split, m, swiglu=(kind == "gu")):
+        for cand in ops.linear_tiled_candidates(n, kk, split, m, swiglu=(kind == "gu"), fp8=self.weight_fp8):
             if kind == "qkv" and cand[1] > self.QKV_MAX_SLABS:
                 continue
             # gate_up pays a kernel of its own for taking slabs: worth timing only where the unsplit

@@ -662,6 +662,7 @@ LINEAR_TILED_MAX_M = 256             # beyond 128 rows: two row blocks of one la
 
 
 KW_CODES = (302, 304, 308, 402, 404)   # K split across 2 / 4 / 8 waves of an 8-wave workgroup (4xx: 512-wide x slices)
+SLICE_CODES = (504, 506, 507, 508, 509, 510)   # fp8 weights: 4 .. 10 tiles a workgroup, K split across its 4 waves, x in registers
 
 
 def row_block_rows(tiles_per_wg: int) -> int:
@@ -673,6 +674,8 @@ def tiled_slice_width(M: int, tiles_per_wg: int) -> int:
     """K slice of x a workgroup of linear_tiled stages at a time."""
     M = min(M, row_block_rows(tiles_per_wg))
     tiles_per_wg %= 1000
+    if tiles_per_wg in SLICE_CODES:
+        return 512                                # (nothing is staged: 128 columns for each of the 4 waves at least)
     mt = 1 if M <= 16 else 2 if M <= 32 else 4 if M <= 64 else 8
     narrow = tiles_per_wg in (104, 108, 208, 402, 404)      # 210 .. 216 (two tiles per wave, 5 .. 8 waves) stage the wide slice
     return (512 if narrow else 1024) // (1 if mt <= 2 else mt // 2)
@@ -680,7 +683,7 @@ def tiled_slice_width(M: int, tiles_per_wg: int) -> int:
 
 def tiles_per_workgroup(tiles_per_wg: int) -> int:
     """Weight tiles one workgroup covers for a tiles_per_wg code (208 .. 216: two tiles per wave;
-    30x / 40x: 8 waves, x waves per tile; + 1000 / + 2000: the same in row blocks of 64 / 32)."""
+    30x / 40x: 8 waves, x waves per tile; 5xx: xx; + 1000 / + 2000: the same in row blocks of 64 / 32)."""
     tiles_per_wg %= 1000
     if tiles_per_wg in KW_CODES:
         return 8 // (tiles_per_wg % 100)
@@ -747,7 +750,7 @@ def gelu_in_product(N: int, K: int, M: int) -> bool:
         and K % tiled_slice_width(M, 304) == 0
 
 
-def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: bool = False):
+def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: bool = False, fp8: bool = False):
     """Every (tiles_per_wg, k_groups) worth timing for linear_tiled on an [N, K] weight and M rows:
     both workgroup shapes that every kernel form (fp8, fused epilogues) is built for, K split into
     1, 2, 4 or 8 groups when the caller can take partial sums, beyond 32 rows also the forms with
@@ -756,8 +759,9 @@ def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: 
     rows and few tiles also the forms that split K across the waves of a workgroup (`swiglu`: the
     gate / up pair must share a workgroup, at most 4 waves per tile); beyond 64 / 32 rows also the forms of
     the 64- / 32-row class run in row blocks of 64 / 32 (tiles_per_wg + 1000 / + 2000).  Not
-    every form exists for every code (fp8 at up to 32 rows: 8 and 104 only): the caller skips a
-    candidate the library refuses.  plan_linear_tiled's choice comes first."""
+    every form exists for every code (fp8 at up to 32 rows: 8, 104 and 5xx only): the caller skips a
+    candidate the library refuses.  plan_linear_tiled's choice comes first.  `fp8`: up to 64 rows also the forms with x in
+    registers (5xx), in blocks of 32 rows, where one to two rounds of workgroups cover the matrix."""
     first = plan_linear_tiled(N, K, split_k, M)
     if first is None:
         return []
@@ -799,6 +803,12 @@ def linear_tiled_candidates(N: int, K: int, split_k: bool, M: int = 32, swiglu: 
             for g in ((1, 2, 4, 8) if split_k else (1,)):
                 if g <= K // ksl and 48 <= wgs * g <= 1024 and (tiles, g) not in out:
                     out.append((tiles, g))
+    if fp8 and M <= 64 and K % 128 == 0:
+        for tiles in SLICE_CODES:
+            wgs = -(-tiles_total // (tiles % 100)) * (1 if M <= 32 else 2)
+            for g in ((1, 2, 3, 4, 6, 7, 8) if split_k else (1,)):
+                if g <= K // 512 and 192 <= wgs * g <= 512 and not (swiglu and tiles % 2):
+                    out.append((tiles + (0 if M <= 32 else 2000), g))
     return out
 
 
