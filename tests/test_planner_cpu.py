@@ -87,3 +87,18 @@ def test_row_blocks_count_as_workgroups():
     assert ops.tiled_slice_width(256, 8) == ops.tiled_slice_width(128, 8) == 256
     # a tensor-parallel rank's gate_up slice at 128 rows may split K (a SwiGLU-from-slabs kernel follows)
     assert any(g > 1 for _, g in ops.linear_tiled_candidates(7168, 4096, True, 128, swiglu=True))
+
+
+def test_act_in_product_takes_what_the_tiles_take():
+    import torch
+    rows = lambda m, k, pad=0, dt=torch.bfloat16: torch.empty(m, k + pad, dtype=dt)[:, :k]      # noqa: E731
+    w = torch.empty(8192, 2048, dtype=torch.bfloat16)
+    yes = lambda x, w=w, act=ops.ACT_GELU_MUL: ops.act_in_product(x, w, act)                     # noqa: E731
+    assert yes(rows(8192, 2048)) and yes(rows(8192, 2048, 8)) and yes(rows(2048, 2048))
+    assert not yes(rows(8192, 2048, 4)) and not yes(rows(8192, 2048, 0, torch.float32)) and not yes(rows(8192, 2048, 0, torch.float16))
+    assert not yes(torch.empty(8192, 2049, dtype=torch.bfloat16)[:, 1:]) and not yes(torch.empty(2048, 8192, dtype=torch.bfloat16).t())
+    assert not yes(rows(8192, 2048), torch.empty(2048, 8192, dtype=torch.bfloat16).t())
+    assert not yes(rows(8192, 2048), torch.empty(8200, 2048, dtype=torch.bfloat16)) and not yes(rows(8192, 1000), torch.empty(8192, 1000, dtype=torch.bfloat16))
+    assert not yes(rows(128, 2048)) and not yes(rows(300, 2048))           # decoded rows; tiles that are mostly empty
+    assert yes(rows(1280, 2048), act=ops.ACT_RELU2) and not yes(rows(1280, 2048))
+    assert not yes(rows(640, 2048), act=ops.ACT_RELU2)

@@ -92,13 +92,14 @@ __device__ __forceinline__ float pin_f32(float v) {
 // Results that bf16 rounds the wrong way, against 64 bits, in 8192 rows of 4096 channels: 150 of 33.5 million, the library's
 // form 254.
 constexpr float kSiluLeanRange = 80.0f;
-__device__ __forceinline__ float silu_lean(float x) {
+__device__ __forceinline__ float over_one_plus_exp_lean(float y, float x) {      // y / (1 + exp(-x))
   const float t = x * -1.44269504088896340736f, lo = fmaf(x, -1.44269504088896340736f, -t);
   const float e0 = __builtin_amdgcn_exp2f(t);
   const float e = fmaf(e0, fmaf(lo, 0.693147180559945f, x * -1.33497e-8f), e0);
-  const float r = __builtin_amdgcn_rcpf(1.0f + e), q = x * r;
-  return fmaf(fmaf(-q, fminf(e, 1.0f), fmaf(-q, fmaxf(e, 1.0f), x)), r, q);
+  const float r = __builtin_amdgcn_rcpf(1.0f + e), q = y * r;
+  return fmaf(fmaf(-q, fminf(e, 1.0f), fmaf(-q, fmaxf(e, 1.0f), y)), r, q);
 }
+__device__ __forceinline__ float silu_lean(float x) { return over_one_plus_exp_lean(x, x); }
 __device__ __forceinline__ float silu_any(float x) {
   return fabsf(x) < kSiluLeanRange ? silu_lean(x) : x / (1.0f + expf(-x));
 }

@@ -33,6 +33,7 @@ struct GroupGemmArgs {
   int groups;
   int64_t rows;                        // rows of every group (heads) or of all together (experts)
   int n, k, copy, relu2;
+  float limit;
 };
 
 // MW: waves along the rows (the other 4 / MW lie along the outputs)
@@ -216,7 +217,10 @@ __global__ __launch_bounds__(256, 2) void group_gemm_kernel(GroupGemmArgs a) {
 // phases a step, three images of 48 KB.
 //
 // Measured in bf16: 32844 rows of 32 experts 2048 -> 1536 195 us (1060 TFLOP/s of the products asked for), 1536 -> 2048
-// 205 us; by tiles of 128 x 128 351 and 326 us on the same card.  One plain product of 8192^3 runs at 1510 TFLOP/s here.
+// 205 us; by tiles of 128 x 128 351 and 326 us on the same card.  One plain product of 8192^3 runs at 1510 TFLOP/s here (the library's at
+// 1590), and one whose activation would be a launch of its own is the faster way with it at the tile's end (mi355_linear_act): 4096 rows
+// 4096 -> 28672 with SwiGLU 667 us (the library and the launch 702), 8192 rows 2048 -> 6144 with relu^2 144 (168), 2048 -> 8192 with GELU 213
+// (231).  The units of a gated tile take some 7 us of a CU, during which its matrix cores are idle but for half a phase.
 constexpr int kWideThreads = 512, kWideMaxGroups = 512;
 
 // Fragments of one read phase.  By instructions of our own, each block with its wait: the compiler cannot tell which loads
@@ -252,8 +256,38 @@ __device__ __forceinline__ int wide_read_int(const int* p) {
   return v;
 }
 
+// Eight units of a gated activation.  silu and the limited unit by the lean quotient while all of a wave's gates are in its range (a
+// NaN passes through it), else as they stand.
+template <typename T, int ACT>
+__device__ __forceinline__ void gated_units(float (&g)[8], const float (&u)[8], float limit, float (&v)[8]) {
+  if constexpr (ACT == MI355_ACT_GELU_MUL) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = gelu_tanh_fast(g[e]) * u[e];
+    return;
+  }
+  constexpr float c = ACT == MI355_ACT_SILU_MUL ? 1.0f : 1.702f;
+  float top = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    if (ACT == MI355_ACT_LIMITED_MUL) g[e] = fminf(g[e], limit);
+    top = fmaxf(top, fabsf(g[e]));
+  }
+  auto finish = [&](int e, float q) {
+    v[e] = ACT == MI355_ACT_SILU_MUL ? round_f<T>(pin_f32(q)) * u[e] : q * (fminf(fmaxf(u[e], -limit), limit) + 1.0f);
+  };
+  if (__all(top < kSiluLeanRange / c)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) finish(e, over_one_plus_exp_lean(g[e], c * g[e]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) finish(e, g[e] / (1.0f + expf(-c * g[e])));
+  }
+}
+
 // per: outputs of a group that lie side by side in y (experts: all n; heads: a head's); a.n: outputs of a row tile
-template <typename T, bool TRANS>
+// GATED (an MI355_ACT_*_MUL, 0: none): the one matrix holds n / 2 gate rows and as many up rows, y = a(gate) * up of n / 2 columns.  A wave's
+// 64 rows of W are 32 gates and their ups then, so that both lie in the same lane.
+template <typename T, bool TRANS, int GATED = 0>
 __global__ __launch_bounds__(kWideThreads, 2) void group_gemm_wide_kernel(GroupGemmArgs a, int per) {
   constexpr int kFull = 512 * kBK, kHalf = 384 * kBK;                  // an image: X rows | 256 W rows
   __shared__ __attribute__((aligned(16))) uint16_t lds[3 * kHalf];
@@ -352,7 +386,11 @@ __global__ __launch_bounds__(kWideThreads, 2) void group_gemm_wide_kernel(GroupG
     return static_cast<uint32_t>(p * a.x_stride) * 2u + sx;
   };
   auto w_at = [&](const Tile& t, int row) {
-    const int n = t.n0 + row < a.n ? t.n0 + row : a.n - 1;
+    int n = t.n0 + row < a.n ? t.n0 + row : a.n - 1;
+    if constexpr (GATED != 0) {
+      const int half = a.n >> 1, col = (t.n0 >> 1) + (row >> 6) * 32 + (row & 31);
+      n = (col < half ? col : half - 1) + (row & 32 ? half : 0);
+    }
     return static_cast<uint32_t>(n) * static_cast<uint32_t>(a.k) * 2u + sw;
   };
   auto w_base = [&](const Tile& t) { return reinterpret_cast<const char*>(a.w + t.g * a.w_group); };
@@ -388,7 +426,17 @@ __global__ __launch_bounds__(kWideThreads, 2) void group_gemm_wide_kernel(GroupG
     uint16_t* y = a.y + (t.g + nb / per) * a.y_group;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (TRANS) {                                                     // rows m .. m + 3 of output n
+      if constexpr (GATED != 0) {                                      // columns n .. n + 7 of row m
+        const int m = m0 + 16 * i + li, n = (nb >> 1) + kk * 8;
+        float g[8], u[8], v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)                                    // (the products as a 16-bit buffer would hold them)
+          g[e] = round_f<T>(c[i][e >> 2][e & 3]), u[e] = round_f<T>(c[i][2 + (e >> 2)][e & 3]);
+        gated_units<T, GATED>(g, u, a.limit, v);
+        uint16_t* p = a.y + static_cast<int64_t>(m) * a.y_stride + n;
+        if (whole) store_one(a.y, p, pack8<T>(v));
+        else if (m < t.hi && 2 * n < a.n) MI355_ST(uint4, a.y, p, pack8<T>(v));
+      } else if (TRANS) {                                                     // rows m .. m + 3 of output n
         const int m = m0 + 16 * i + 4 * kk;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -425,7 +473,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void group_gemm_wide_kernel(GroupG
       }
     }
   };
-  constexpr int S = TRANS ? 16 : 8;                                    // stores of 64 whole rows, an instruction each (store_one)
+  constexpr int S = TRANS ? 16 : GATED ? 4 : 8;                        // stores of 64 whole rows, an instruction each (store_one)
   if (!halves) {
     const int total = full_tiles * ntn, lo = static_cast<int>(static_cast<int64_t>(total) * xcd / nx),
               end = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / nx);
@@ -674,6 +722,41 @@ extern "C" int32_t mi355_expert_gemm(void* y, const void* x, int64_t x_rows, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == MI355_BF16) launch_group_gemm<BF16>(a, false, tiles, 128, s); else launch_group_gemm<F16>(a, false, tiles, 128, s);
   return check_launch("expert_gemm");
+}
+
+extern "C" int32_t mi355_linear_act(void* y, int64_t y_stride, const void* x, int64_t x_stride, const void* w, int64_t num_rows,
+                                    int32_t out_width, int32_t in_width, int32_t activation, float limit, int32_t dtype, void* stream) {
+  MI355_REQUIRE(activation >= MI355_ACT_RELU2 && activation <= MI355_ACT_LIMITED_MUL, MI355_ERR_INVALID, "linear_act: unknown activation %d", activation);
+  const bool gated = activation != MI355_ACT_RELU2;
+  GroupGemmArgs a = {static_cast<uint16_t*>(y), 16 * y_stride, y_stride, 0, static_cast<const uint16_t*>(x), x_stride, 0, num_rows,
+                     nullptr, 1, static_cast<const uint16_t*>(w), static_cast<int64_t>(out_width) * in_width, nullptr, nullptr, 1,
+                     num_rows, out_width, in_width, 0, !gated, limit};
+  MI355_REQUIRE(y && x && w, MI355_ERR_INVALID, "linear_act: null pointer");
+  MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "linear_act: 16-bit storage only");
+  MI355_REQUIRE(num_rows >= 0 && out_width > 0 && in_width > 0, MI355_ERR_INVALID, "linear_act: sizes");
+  MI355_REQUIRE(x_stride >= in_width && y_stride >= (gated ? out_width / 2 : out_width), MI355_ERR_INVALID, "linear_act: rows overlap");
+  if (num_rows == 0) return MI355_OK;
+  MI355_REQUIRE(wide_fits(a, false, false) && x_stride % 8 == 0 && out_width % 64 == 0 && aligned16(x) && aligned16(w) && aligned16(y),
+                MI355_ERR_UNSUPPORTED, "linear_act: %d inputs (a multiple of 64, 128 at least), %d outputs (of 64), 16-byte aligned rows, "
+                "operands below 4 GB", in_width, out_width);
+  const int64_t most = (num_rows / 128 + 1) * ((out_width + 255) / 256);
+  const dim3 grid(static_cast<unsigned>(most < 256 ? most : 256));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define MI355_LA(A)                                                                                                            \
+  case A:                                                                                                                      \
+    if (dtype == MI355_BF16)                                                                                                   \
+      hipLaunchKernelGGL((group_gemm_wide_kernel<BF16, false, A>), grid, dim3(kWideThreads), 0, s, a, out_width);              \
+    else                                                                                                                       \
+      hipLaunchKernelGGL((group_gemm_wide_kernel<F16, false, A>), grid, dim3(kWideThreads), 0, s, a, out_width);               \
+    break
+  switch (activation) {
+    MI355_LA(MI355_ACT_RELU2);                          // (0: the ungated kernel)
+    MI355_LA(MI355_ACT_GELU_MUL);
+    MI355_LA(MI355_ACT_SILU_MUL);
+    MI355_LA(MI355_ACT_LIMITED_MUL);
+  }
+#undef MI355_LA
+  return check_launch("linear_act");
 }
 
 extern "C" int32_t mi355_head_gemm(void* y, int64_t y_block, int64_t y_stride, int64_t y_group, const void* x, int64_t x_stride,

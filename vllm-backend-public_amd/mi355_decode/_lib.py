@@ -153,6 +153,7 @@ def _load() -> ctypes.CDLL:
         "mi355_moe_table_sort": (I32, [P, P, P, P, P, P, I64, I64, I32, I32, I32, I32, P]),
         "mi355_add_layer_norm_f32": (I32, [P, P, P, P, I32, F, P, I64, I32, F, I32, P]),
         "mi355_expert_gemm": (I32, [P, P, I64, P, P, P, P, I32, I64, I32, I32, I32, I32, I32, P]),
+        "mi355_linear_act": (I32, [P, I64, P, I64, P, I64, I32, I32, I32, F, I32, P]),
         "mi355_head_gemm": (I32, [P, I64, I64, I64, P, I64, I64, I64, P, P, I64, I32, I32, I32, I32, I32, I32, P]),
         "mi355_latent_q_rotate": (I32, [P, I64, I32, I32, P, I32, P, I64, I32, I32, I32, I32, P]),
         "mi355_moe_silu_and_mul": (I32, [P, P, I64, I32, I32, F, I32, P]),
@@ -239,7 +240,7 @@ EXPORTS = ("mi355_abi_version", "mi355_last_error", "mi355_target_arch",
            "mi355_moe_linear_rows", "mi355_moe_table_sort", "mi355_add_layer_norm_f32", "mi355_expert_gemm",
            "mi355_head_gemm", "mi355_latent_q_rotate", "mi355_paged_attn_decode_ext", "mi355_resid_add_norm_f32",
            "mi355_rms_norm_mix_norm_f32", "mi355_delta_decode", "mi355_window_delta_decode", "mi355_window_delta_decode_rows", "mi355_moe_linear_rows_hinted",
-           "mi355_latent_window_attn_tiles_hinted")
+           "mi355_latent_window_attn_tiles_hinted", "mi355_linear_act")
 
 
 def check(status: int) -> None:

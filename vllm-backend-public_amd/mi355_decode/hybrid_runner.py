@@ -581,7 +581,7 @@ class ReluSquaredFF:
         self.lw, self.r = lw, runner
 
     def __call__(self, h: torch.Tensor) -> torch.Tensor:
-        return self.r.linear(ops.relu_squared(self.r.linear(h, self.lw.up_w)), self.lw.down_w)
+        return self.r.linear(self.r.relu2_linear(h, self.lw.up_w), self.lw.down_w)
 
 
 class LimitedFF:
@@ -592,7 +592,10 @@ class LimitedFF:
         self.ff, self.limit, self.lw, self.r = spec.ff, spec.ff_limit, lw, runner
 
     def __call__(self, h: torch.Tensor, b: "StepBatch") -> torch.Tensor:
-        gu = self.r.linear(h, self.lw.gate_up_w)
+        w = self.lw.gate_up_w
+        if self.limit is not None and ops.act_in_product(h, w, ops.ACT_LIMITED_MUL):
+            return _out_product(self.r, ops.linear_act(h, w, ops.ACT_LIMITED_MUL, self.limit), self.lw.down_w)
+        gu = self.r.linear(h, w)
         return _out_product(self.r, ops.gated_act_rows(gu[:, : self.ff], gu[:, self.ff:], self.limit), self.lw.down_w)
 
 
@@ -1049,7 +1052,13 @@ class HybridRunner(ModelRunner):
         if tw is not None and tw.dtype == x.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 \
                 and ops.gelu_in_product(w.shape[0], w.shape[1], x.shape[0]):
             return ops.linear_tiled(x, tw, w.shape[0], tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL)
+        if ops.act_in_product(x, w, ops.ACT_GELU_MUL):
+            return ops.linear_act(x, w, ops.ACT_GELU_MUL)
         return ops.gelu_tanh_and_mul(self.linear(x, w, slabs=True))
+
+    def relu2_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """max(x @ w.T, 0)^2; in one launch where that is the faster way."""
+        return ops.linear_act(x, w, ops.ACT_RELU2) if ops.act_in_product(x, w, ops.ACT_RELU2) else ops.relu_squared(self.linear(x, w))
 
     def out_linear(self, x: torch.Tensor, w: torch.Tensor):
         """A sub-layer's last product.  In the pre arrangement its consumers (the norms that it is added ahead of, the mix)
@@ -1226,7 +1235,7 @@ class HybridRunner(ModelRunner):
             row = self.mixers[ri](self.linear(x, lw.in_w, bias=lw.in_b), resid, b)
             ops.norm_resid_f32(resid, self.linear(row, lw.out_w), lw.norm1, eps, act_out=act)
             if L.ff:
-                y = self.linear(ops.relu_squared(self.linear(x, lw.up_w)), lw.down_w)
+                y = self.linear(self.relu2_linear(x, lw.up_w), lw.down_w)
                 ops.norm_resid_f32(resid, y, lw.norm2, eps, act_out=act)
             if n and T <= self.SIDE_FUSED_ROWS and self.H * n <= self.SIDE_FUSED_WEIGHTS and self.H <= 8192 and n <= 4096:
                 ops.token_side_f32(resid, lw.side_gate_w, lw.side_proj_w, lw.side_norm, w.side_embed, li * n, b.ids, eps, act_out=act)

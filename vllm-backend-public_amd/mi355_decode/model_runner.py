@@ -817,8 +817,12 @@ class ModelRunner:
             torch.mm(attn, self._rm(i, "o").t(), out=o)
             self._allreduce(o)
             ops.fused_add_rms_norm(o, resid, lw.post_norm, self.eps, out=x)
-            torch.mm(x, self._rm(i, "gu").t(), out=gu)
-            ops.silu_and_mul(gu, out=act)
+            w_gu = self._rm(i, "gu")
+            if ops.act_in_product(x, w_gu, ops.ACT_SILU_MUL):
+                ops.linear_act(x, w_gu, ops.ACT_SILU_MUL, out=act)
+            else:
+                torch.mm(x, w_gu.t(), out=gu)
+                ops.silu_and_mul(gu, out=act)
             torch.mm(act, self._rm(i, "down").t(), out=dn)
             if self.mlp_sharded:
                 self._allreduce(dn)

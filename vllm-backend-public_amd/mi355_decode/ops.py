@@ -2010,6 +2010,48 @@ def head_gemm(x: torch.Tensor, x_group: int, w: torch.Tensor, out: torch.Tensor,
     return out
 
 
+ACT_RELU2, ACT_GELU_MUL, ACT_SILU_MUL, ACT_LIMITED_MUL = 0, 1, 2, 3
+
+
+def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
+    """Whether linear_act takes x and w and is faster than a library product with the activation's launch behind it.  The launch moves
+    2 (gated 1.5) times the product's bytes; the product itself is 4 to 8 % slower by the tiles here than by the library's, whose rounds
+    of workgroups are also finer: what counts is the share of the tiles' rounds that is work (us, two launches / one, bfloat16).
+    relu^2, 2048 inputs, 8192 outputs: 640 rows (0.54 of a round) 29.8 / 30.4, 1280 (0.62) 47.1 / 44.3, 8192 225 / 190; 6144 outputs 1536 rows
+    (0.56) 44.1 / 44.4, 8192 168 / 144.  4096 inputs, 12288 outputs: 640 rows (0.81) 62.0 / 57.1, 1536 (0.65) 148 / 156, 3000 (0.76) 252 / 269.
+    Gated units have more to work out at a tile's end: silu 4096 -> 28672 4096 rows (1.0) 702 / 667, 7731 (0.94) 1379 / 1265; gelu 2048 -> 8192
+    8192 rows 231 / 213, 2560 (0.72) 0.98 of two launches' speed, 2048 -> 6144 6000 rows (0.76) 0.93, 4096 -> 12288 3000 rows (0.76) 0.92."""
+    M, (N, K) = x.shape[0], w.shape
+    if x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or K % 64 or K < 128 or N % 64 or M <= LINEAR_DECODE_MAX_M \
+            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous() \
+            or M * x.stride(0) >= 1 << 31 or N * K >= 1 << 31:
+        return False
+    # as group_gemm's wide tiles lie: rounds of 256 workgroups, in halves (tiles of 128 rows)
+    col, last = -(-N // 256), M & 255
+    full, rest, half = ((M >> 8) + (last > 128)) * col, col if 0 < last <= 128 else 0, -(-M // 128) * col
+    more = max(rest - 2 * (256 - full % 256), 0) if full % 256 else rest
+    halves = min(2 * -(-full // 256) + -(-more // 256), 29 / 25 * -(-half // 256))
+    busy = M * N / (128 * 256 * 256 * halves)
+    return busy >= (0.6 if activation == ACT_RELU2 and K <= 2048 else 0.8)
+
+
+def linear_act(x: torch.Tensor, w: torch.Tensor, activation: int, limit: float = 0.0, out: torch.Tensor | None = None):
+    """a(x @ w.T) in one launch of wide matrix-core tiles: max(v, 0)^2, or, with gate rows of w ahead of up rows, gelu_tanh(gate) * up,
+    silu(gate) * up, or the limited unit of gated_act_rows."""
+    dt = _dt16(x, "x")
+    N, K = w.shape
+    if x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != K or not w.is_contiguous():
+        raise ValueError("x must be [rows, in], w contiguous [out, in]")
+    width = N if activation == ACT_RELU2 else N // 2
+    if out is None:
+        out = torch.empty(x.shape[0], width, dtype=x.dtype, device=x.device)
+    elif out.dtype != x.dtype or tuple(out.shape) != (x.shape[0], width):
+        raise ValueError(f"out must be [rows, {width}] in the dtype of x")
+    check(lib.mi355_linear_act(out.data_ptr(), _rows(out, "out"), x.data_ptr(), x.stride(0), _same(w, x, "w"), x.shape[0], N, K, int(activation),
+                               float(limit), dt, _stream()))
+    return out
+
+
 def latent_q_rotate(q: torch.Tensor, num_heads: int, q_head_width: int, q_rot_offset: int, cos_sin: torch.Tensor,
                     positions: torch.Tensor, interleaved: bool = False):
     """q [tokens, heads * q_head_width] (a column slice is fine): the columns at q_rot_offset of every head rotated in
