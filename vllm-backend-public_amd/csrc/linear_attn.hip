@@ -40,6 +40,20 @@ struct LaDims {
   int C;                        // rows of a tile
 };
 
+// silu of eight numbers; the lean form (half the instructions) where all of them are in its range, a NaN passes through it
+__device__ __forceinline__ void silu8(float (&f)[8]) {
+  float top = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(f[j]));
+  if (top < kSiluLeanRange) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = silu_lean(f[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = silu_f(f[j]);
+  }
+}
+
 // rows [0, n) x cols [0, d) of a row-strided tensor -> fp32 LDS [rows_p][ld], activation and a factor per
 // row applied, zeros up to rows_p rows and cols_p columns
 template <typename T>
@@ -55,8 +69,14 @@ __device__ __forceinline__ void stage_rows(float* dst, int ld, const typename El
         if (r < n && c < d) {
           unpack8<T>(MI355_LD(uint4, base, src + r * stride + c), f);
           const float w = row_factor != nullptr ? row_factor[r] : 1.0f;
+          if (silu) {
+            silu8(f);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] = (silu ? silu_f(f[j]) : f[j] * scale) * w;
+            for (int j = 0; j < 8; ++j) f[j] *= w;
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = f[j] * scale * w;
+          }
         }
         float4* o = reinterpret_cast<float4*>(dst + r * ld + c);
         o[0] = make_float4(f[0], f[1], f[2], f[3]);
