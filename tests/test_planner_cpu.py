@@ -102,3 +102,11 @@ def test_act_in_product_takes_what_the_tiles_take():
     assert not yes(rows(128, 2048)) and not yes(rows(300, 2048))           # decoded rows; tiles that are mostly empty
     assert yes(rows(1280, 2048), act=ops.ACT_RELU2) and not yes(rows(1280, 2048))
     assert not yes(rows(640, 2048), act=ops.ACT_RELU2)
+
+
+def test_rows_past_rounds():
+    f = ops.rows_past_rounds
+    assert f(8193, 2048) == 8192 and f(8320, 6144) == 8192 and f(4224, 4096) == 4096 and f(2049, 8192) == 2048
+    assert f(8192, 2048) == 0 and f(8321, 2048) == 0                       # none, more than the stream takes at its best
+    assert f(4160, 3072) == 0 and f(2100, 4096) == 0 and f(8211, 3648) == 0   # tiles that leave a round part empty
+    assert f(100, 65536) == 0 and f(1, 8192) == 0

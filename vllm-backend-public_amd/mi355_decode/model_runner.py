@@ -223,7 +223,7 @@ class ModelRunner:
         self.tiled_policy = {True: "on", False: "off", None: "auto"}[want]
         if want is None and os.environ.get("MI355_TILED_LINEARS") in ("0", "1"):
             self.tiled_policy = "on" if os.environ["MI355_TILED_LINEARS"] == "1" else "off"
-        self.tiled = None
+        self.tiled = self.lm_head_tiled = None
         self._rm_attr = {"qkv": "qkv_w", "o": "o_w", "gu": "gate_up_w", "down": "down_w"}
         self._rm_shape = {"qkv": (self.qw, self.H), "o": (self.H, self.nh * self.d), "gu": (2 * self.F, self.H),
                           "down": (self.H, self.F)}
@@ -809,12 +809,9 @@ class ModelRunner:
                 ops.rms_norm(resid, lw.input_norm, self.eps, out=x)
             else:
                 ops.fused_add_rms_norm(dn, resid, lw.input_norm, self.eps, out=x)
-            if lw.qkv_b is None:
-                torch.mm(x, self._rm(i, "qkv").t(), out=qkv)
-            else:
-                torch.addmm(lw.qkv_b, x, self._rm(i, "qkv").t(), out=qkv)
+            self._product(x, i, "qkv", qkv, lw.qkv_b)
             attend(i, qkv, attn)
-            torch.mm(attn, self._rm(i, "o").t(), out=o)
+            self._product(attn, i, "o", o)
             self._allreduce(o)
             ops.fused_add_rms_norm(o, resid, lw.post_norm, self.eps, out=x)
             w_gu = self._rm(i, "gu")
@@ -823,10 +820,32 @@ class ModelRunner:
             else:
                 torch.mm(x, w_gu.t(), out=gu)
                 ops.silu_and_mul(gu, out=act)
-            torch.mm(act, self._rm(i, "down").t(), out=dn)
+            self._product(act, i, "down", dn)
             if self.mlp_sharded:
                 self._allreduce(dn)
         return dn
+
+    def _product(self, x: torch.Tensor, i: int, kind: str, out: torch.Tensor, bias: Optional[torch.Tensor] = None) -> None:
+        """out = x W^T (+ bias) of projection `kind` (qkv / o / down) of layer i for prompts: a library GEMM, and the rows past its whole
+        rounds of tiles by the decode weight stream."""
+        w, tw = self._rm(i, kind), self.tiled[i].get(kind) if self.tiled is not None else None
+        (N, K), head = w.shape, 0
+        if torch.is_tensor(tw):                                     # (not fp8 copies: prompts multiply by what they decode to)
+            head = ops.rows_past_rounds(x.shape[0], N)
+            plan = ops.plan_linear_tiled(N, K, True, x.shape[0] - head) if head else None
+            head = head if plan is not None else 0
+        if head:
+            tiles, groups = plan
+            if groups == 1:
+                ops.linear_tiled(x[head:], tw, N, bias=bias, out=out[head:], tiles_per_wg=tiles)
+            else:
+                part = ops.linear_tiled(x[head:], tw, N, tiles_per_wg=tiles, k_groups=groups, epilogue=ops.EPI_PARTIAL)
+                ops.sum_slabs(part, groups, out[head:], bias=bias)
+            x, out = x[:head], out[:head]
+        if bias is None:
+            torch.mm(x, w.t(), out=out)
+        else:
+            torch.addmm(bias, x, w.t(), out=out)
 
     # ------------------------------------------------------------------ #
     # decode: one token per sequence, static buffers, HIP-graph replay
@@ -1082,7 +1101,10 @@ class ModelRunner:
                 lg = self.full_logits(torch.mm(hs, self.w.lm_head.t()))
                 parts.append(self._logprobs(lg, targets[a:a + 1024], k))
             self.prompt_scores = torch.cat(parts, dim=0)
-        logits = torch.mm(xs, self.w.lm_head.t())
+        # few rows stream the head once, as in decode steps (128256 x 4096, us, library / stream: 2 rows 181 / 157, 32 rows 196 / 166)
+        plan = ops.plan_linear_tiled(self.Vl, self.H, False, xs.shape[0]) if self.lm_head_tiled is not None and 0 < xs.shape[0] <= 64 else None
+        logits = torch.mm(xs, self.w.lm_head.t()) if plan is None else \
+            ops.linear_tiled(xs, self.lm_head_tiled, self.Vl, tiles_per_wg=plan[0])
         nxt = torch.empty(logits.shape[0], dtype=torch.int64, device=self.device)
         self.greedy(logits, nxt)
         return nxt, (self.full_logits(logits) if want_logits else None)

@@ -2010,6 +2010,16 @@ def head_gemm(x: torch.Tensor, x_group: int, w: torch.Tensor, out: torch.Tensor,
     return out
 
 
+def rows_past_rounds(M: int, N: int) -> int:
+    """How many of M rows to give a library product of N outputs where the rest, up to 128, cost less by the decode weight stream; 0: all.
+    256 x 256 tiles that fill whole rounds of the 256 CUs run at the library's best, and a few rows more open another round or make it
+    choose smaller tiles for all of them (us, all by the library / the rest streamed, bfloat16): 8193 rows 2048 -> 2048 71.0 / 56.8, 8211
+    4096 -> 2048 124 / 99, 8320 2048 -> 6144 223 / 160, 4224 14336 -> 4096 707 / 348, 2112 2048 -> 8192 84 / 64, 4190 4096 -> 28672 687 / 682.
+    Where the tiles do not fill rounds the rest mostly costs more: 4160 rows 2048 -> 3072 43 / 54, 2100 4096 -> 4096 68 / 70."""
+    rest = M & 255
+    return M - rest if M > 256 and 0 < rest <= 128 and N % 256 == 0 and (M >> 8) * (N >> 8) % 256 == 0 else 0
+
+
 ACT_RELU2, ACT_GELU_MUL, ACT_SILU_MUL, ACT_LIMITED_MUL = 0, 1, 2, 3
 
 
