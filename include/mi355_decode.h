@@ -1224,12 +1224,12 @@ int32_t mi355_head_gemm(void* y, int64_t y_block, int64_t y_stride, int64_t y_gr
                         int32_t in_width, int32_t copy, int32_t transposed, int32_t dtype, void* stream);
 
 /*
- * y = a(X W^T) for many rows, w [out_width, in_width], one dense product with its activation in the same launch: MI355_ACT_RELU2
- * max(v, 0)^2, or of out_width / 2 columns, gate rows of w ahead of up rows, MI355_ACT_GELU_MUL gelu_tanh(gate) * up,
+ * y = a(X W^T) for many rows, w [out_width, in_width], one dense product with its activation in the same launch: MI355_ACT_NONE the
+ * product, MI355_ACT_RELU2 max(v, 0)^2, or of out_width / 2 columns, gate rows of w ahead of up rows, MI355_ACT_GELU_MUL gelu_tanh(gate) * up,
  * MI355_ACT_SILU_MUL silu(gate) * up (the silu rounded to 16 bits), MI355_ACT_LIMITED_MUL g sigmoid(1.702 g) (u + 1) with
  * g = min(gate, limit), u = clamp(up, -limit, limit).  The activations see the products as 16-bit values.
  */
-enum { MI355_ACT_RELU2 = 0, MI355_ACT_GELU_MUL = 1, MI355_ACT_SILU_MUL = 2, MI355_ACT_LIMITED_MUL = 3 };
+enum { MI355_ACT_RELU2 = 0, MI355_ACT_GELU_MUL = 1, MI355_ACT_SILU_MUL = 2, MI355_ACT_LIMITED_MUL = 3, MI355_ACT_NONE = 4 };
 int32_t mi355_linear_act(void* y, int64_t y_stride, const void* x, int64_t x_stride, const void* w, int64_t num_rows,
                          int32_t out_width, int32_t in_width, int32_t activation, float limit, int32_t dtype, void* stream);
 

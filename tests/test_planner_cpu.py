@@ -110,3 +110,14 @@ def test_rows_past_rounds():
     assert f(8192, 2048) == 0 and f(8321, 2048) == 0                       # none, more than the stream takes at its best
     assert f(4160, 3072) == 0 and f(2100, 4096) == 0 and f(8211, 3648) == 0   # tiles that leave a round part empty
     assert f(100, 65536) == 0 and f(1, 8192) == 0
+
+
+def test_wide_product_rule():
+    import torch
+    x, w = torch.empty(8192, 2048, dtype=torch.bfloat16), torch.empty(6208, 2048, dtype=torch.bfloat16)
+    out = torch.empty(8192, 6216, dtype=torch.bfloat16)
+    f = ops.wide_product
+    assert f(x, w) and f(x, w, out[:, :6208]) and f(x, torch.empty(5208, 2048, dtype=torch.bfloat16))
+    assert not f(x, w, torch.empty(8192, 6209, dtype=torch.bfloat16)[:, :6208]) and not f(x, w, out[:, 4: 6212])
+    assert not f(x, torch.empty(6144, 2048, dtype=torch.bfloat16)) and not f(x, torch.empty(6204, 2048, dtype=torch.bfloat16))
+    assert not f(x[:1000], w[:2112]) and not f(x.float(), w.float()) and not f(x[:, :2040], w[:, :2040])

@@ -636,14 +636,15 @@ __global__ __launch_bounds__(256) void group_copy_kernel(GroupGemmArgs a) {
 }
 
 // What the wide tiles take: whole steps of K, 16-byte stores, byte offsets of 32 bits
-static bool wide_fits(const GroupGemmArgs& a, bool trans, bool experts) {
+// (one: a single matrix, whose last outputs may end inside a wave's 64)
+static bool wide_fits(const GroupGemmArgs& a, bool trans, bool experts, bool one = false) {
   const int64_t w_rows = experts ? a.n : static_cast<int64_t>(a.n) * a.groups;
   if (a.k % kBK != 0 || a.k < 2 * kBK || a.x_rows * a.x_stride * 2 >= (1ll << 32) || w_rows * a.k * 2 >= (1ll << 32) || a.rows >= (1 << 30) ||
       w_rows >= (1 << 30))
     return false;
   if (a.n % 8 != 0 || a.y_stride % 8 != 0 || a.y_block % 8 != 0 || a.y_group % 8 != 0) return false;
   if (experts) return a.groups <= kWideMaxGroups;
-  return a.x_group == 0 && a.n % 64 == 0 && a.w_group == static_cast<int64_t>(a.n) * a.k && (!trans || a.copy == 0);
+  return a.x_group == 0 && (one || a.n % 64 == 0) && a.w_group == static_cast<int64_t>(a.n) * a.k && (!trans || a.copy == 0);
 }
 
 // Where the wide tiles are the faster ones (bf16, us, 128 x 128 tiles / wide; 12 and less are the host's).  They need about
@@ -726,18 +727,18 @@ extern "C" int32_t mi355_expert_gemm(void* y, const void* x, int64_t x_rows, con
 
 extern "C" int32_t mi355_linear_act(void* y, int64_t y_stride, const void* x, int64_t x_stride, const void* w, int64_t num_rows,
                                     int32_t out_width, int32_t in_width, int32_t activation, float limit, int32_t dtype, void* stream) {
-  MI355_REQUIRE(activation >= MI355_ACT_RELU2 && activation <= MI355_ACT_LIMITED_MUL, MI355_ERR_INVALID, "linear_act: unknown activation %d", activation);
-  const bool gated = activation != MI355_ACT_RELU2;
+  MI355_REQUIRE(activation >= MI355_ACT_RELU2 && activation <= MI355_ACT_NONE, MI355_ERR_INVALID, "linear_act: unknown activation %d", activation);
+  const bool gated = activation != MI355_ACT_RELU2 && activation != MI355_ACT_NONE;
   GroupGemmArgs a = {static_cast<uint16_t*>(y), 16 * y_stride, y_stride, 0, static_cast<const uint16_t*>(x), x_stride, 0, num_rows,
                      nullptr, 1, static_cast<const uint16_t*>(w), static_cast<int64_t>(out_width) * in_width, nullptr, nullptr, 1,
-                     num_rows, out_width, in_width, 0, !gated, limit};
+                     num_rows, out_width, in_width, 0, activation == MI355_ACT_RELU2, limit};
   MI355_REQUIRE(y && x && w, MI355_ERR_INVALID, "linear_act: null pointer");
   MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "linear_act: 16-bit storage only");
   MI355_REQUIRE(num_rows >= 0 && out_width > 0 && in_width > 0, MI355_ERR_INVALID, "linear_act: sizes");
   MI355_REQUIRE(x_stride >= in_width && y_stride >= (gated ? out_width / 2 : out_width), MI355_ERR_INVALID, "linear_act: rows overlap");
   if (num_rows == 0) return MI355_OK;
-  MI355_REQUIRE(wide_fits(a, false, false) && x_stride % 8 == 0 && out_width % 64 == 0 && aligned16(x) && aligned16(w) && aligned16(y),
-                MI355_ERR_UNSUPPORTED, "linear_act: %d inputs (a multiple of 64, 128 at least), %d outputs (of 64), 16-byte aligned rows, "
+  MI355_REQUIRE(wide_fits(a, false, false, true) && x_stride % 8 == 0 && (!gated || out_width % 64 == 0) && aligned16(x) && aligned16(w) && aligned16(y),
+                MI355_ERR_UNSUPPORTED, "linear_act: %d inputs (a multiple of 64, 128 at least), %d outputs (of 8, gated 64), 16-byte aligned rows, "
                 "operands below 4 GB", in_width, out_width);
   const int64_t most = (num_rows / 128 + 1) * ((out_width + 255) / 256);
   const dim3 grid(static_cast<unsigned>(most < 256 ? most : 256));
@@ -749,8 +750,8 @@ extern "C" int32_t mi355_linear_act(void* y, int64_t y_stride, const void* x, in
     else                                                                                                                       \
       hipLaunchKernelGGL((group_gemm_wide_kernel<F16, false, A>), grid, dim3(kWideThreads), 0, s, a, out_width);               \
     break
-  switch (activation) {
-    MI355_LA(MI355_ACT_RELU2);                          // (0: the ungated kernel)
+  switch (activation == MI355_ACT_NONE ? MI355_ACT_RELU2 : activation) {
+    MI355_LA(MI355_ACT_RELU2);                          // (0: the ungated kernel, whose arguments say whether)
     MI355_LA(MI355_ACT_GELU_MUL);
     MI355_LA(MI355_ACT_SILU_MUL);
     MI355_LA(MI355_ACT_LIMITED_MUL);

@@ -1018,7 +1018,8 @@ class HybridRunner(ModelRunner):
         """x @ w.T (+ bias, in the accumulator's float32 ahead of the rounding).  Decode-sized row counts stream the weights once: through the fragment-tiled copy
         (K split over workgroups into fp32 slabs where one pass would leave most of the chip idle, a
         second launch adds the slabs) or, for matrices that have none, row-major through
-        mi355_linear_decode.  A library GEMM otherwise (prefill, but for rows past its whole rounds; float32; odd widths).  slabs: the caller takes
+        mi355_linear_decode.  A library GEMM otherwise (prefill, but for rows past its whole
+        rounds, and widths that the tiles of linear_act serve better; float32; odd widths).  slabs: the caller takes
         ops.Slabs where K is split and adds them itself."""
         M, K = x.shape
         N = w.shape[0]
@@ -1040,6 +1041,8 @@ class HybridRunner(ModelRunner):
                 return ops.sum_slabs(part, groups, out, bias=bias)
         if ok16 and M <= ops.LINEAR_DECODE_MAX_M and K % 32 == 0 and N % 4 == 0:
             return ops.linear_decode(x, w, bias, out=out)
+        if bias is None and ops.wide_product(x, w, out):
+            return ops.linear_act(x, w, ops.ACT_NONE, out=out)
         head = ops.rows_past_rounds(M, N) if ok16 and w.data_ptr() in self._tiled_w else 0
         if head and ops.plan_linear_tiled(N, K, True, M - head) is not None:
             if out is None:

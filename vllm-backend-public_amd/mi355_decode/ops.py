@@ -2020,7 +2020,32 @@ def rows_past_rounds(M: int, N: int) -> int:
     return M - rest if M > 256 and 0 < rest <= 128 and N % 256 == 0 and (M >> 8) * (N >> 8) % 256 == 0 else 0
 
 
-ACT_RELU2, ACT_GELU_MUL, ACT_SILU_MUL, ACT_LIMITED_MUL = 0, 1, 2, 3
+ACT_RELU2, ACT_GELU_MUL, ACT_SILU_MUL, ACT_LIMITED_MUL, ACT_NONE = 0, 1, 2, 3, 4
+
+
+def _wide_share(x: torch.Tensor, w: torch.Tensor, multiple: int) -> float:
+    """The share of their rounds in which linear_act's tiles have work for x @ w.T (outputs a multiple of `multiple`); 0: it does not take them."""
+    M, (N, K) = x.shape[0], w.shape
+    if x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or K % 64 or K < 128 or N % multiple or M <= LINEAR_DECODE_MAX_M \
+            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous() \
+            or M * x.stride(0) >= 1 << 31 or N * K >= 1 << 31:
+        return 0.0
+    # as group_gemm's wide tiles lie: rounds of 256 workgroups, in halves (tiles of 128 rows)
+    col, last = -(-N // 256), M & 255
+    full, rest, half = ((M >> 8) + (last > 128)) * col, col if 0 < last <= 128 else 0, -(-M // 128) * col
+    more = max(rest - 2 * (256 - full % 256), 0) if full % 256 else rest
+    halves = min(2 * -(-full // 256) + -(-more // 256), 29 / 25 * -(-half // 256))
+    return M * N / (128 * 256 * 256 * halves)
+
+
+def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> bool:
+    """Whether x @ w.T by linear_act's tiles is faster than by the library: outputs that end inside a tile of 256 columns, which the
+    library's best kernels do not take, where the tiles' rounds are mostly work (us, bfloat16, library / tiles: 2048 -> 3648 8211 rows 135 / 101,
+    4096 61 / 54, 2048 38 / 34; 2048 -> 6208 8192 rows (0.76 of the rounds) 215 / 177; 1024 -> 6720 7731 rows 151 / 105; 4096 -> 9280 3333 rows
+    217 / 196; 2048 -> 3648 6189 rows (0.77) 87 / 89, 5000 (0.62) 79 / 86).  Whole columns of tiles are within 10 % either way."""
+    if w.shape[0] % 256 == 0 or (out is not None and (out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16)):
+        return False
+    return _wide_share(x, w, 8) >= 0.75
 
 
 def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
@@ -2031,28 +2056,17 @@ def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
     (0.56) 44.1 / 44.4, 8192 168 / 144.  4096 inputs, 12288 outputs: 640 rows (0.81) 62.0 / 57.1, 1536 (0.65) 148 / 156, 3000 (0.76) 252 / 269.
     Gated units have more to work out at a tile's end: silu 4096 -> 28672 4096 rows (1.0) 702 / 667, 7731 (0.94) 1379 / 1265; gelu 2048 -> 8192
     8192 rows 231 / 213, 2560 (0.72) 0.98 of two launches' speed, 2048 -> 6144 6000 rows (0.76) 0.93, 4096 -> 12288 3000 rows (0.76) 0.92."""
-    M, (N, K) = x.shape[0], w.shape
-    if x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or K % 64 or K < 128 or N % 64 or M <= LINEAR_DECODE_MAX_M \
-            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous() \
-            or M * x.stride(0) >= 1 << 31 or N * K >= 1 << 31:
-        return False
-    # as group_gemm's wide tiles lie: rounds of 256 workgroups, in halves (tiles of 128 rows)
-    col, last = -(-N // 256), M & 255
-    full, rest, half = ((M >> 8) + (last > 128)) * col, col if 0 < last <= 128 else 0, -(-M // 128) * col
-    more = max(rest - 2 * (256 - full % 256), 0) if full % 256 else rest
-    halves = min(2 * -(-full // 256) + -(-more // 256), 29 / 25 * -(-half // 256))
-    busy = M * N / (128 * 256 * 256 * halves)
-    return busy >= (0.6 if activation == ACT_RELU2 and K <= 2048 else 0.8)
+    return _wide_share(x, w, 64) >= (0.6 if activation == ACT_RELU2 and w.shape[1] <= 2048 else 0.8)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, activation: int, limit: float = 0.0, out: torch.Tensor | None = None):
-    """a(x @ w.T) in one launch of wide matrix-core tiles: max(v, 0)^2, or, with gate rows of w ahead of up rows, gelu_tanh(gate) * up,
+    """a(x @ w.T) in one launch of wide matrix-core tiles: max(v, 0)^2, the product itself (ACT_NONE), or, with gate rows of w ahead of up rows, gelu_tanh(gate) * up,
     silu(gate) * up, or the limited unit of gated_act_rows."""
     dt = _dt16(x, "x")
     N, K = w.shape
     if x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != K or not w.is_contiguous():
         raise ValueError("x must be [rows, in], w contiguous [out, in]")
-    width = N if activation == ACT_RELU2 else N // 2
+    width = N if activation in (ACT_RELU2, ACT_NONE) else N // 2
     if out is None:
         out = torch.empty(x.shape[0], width, dtype=x.dtype, device=x.device)
     elif out.dtype != x.dtype or tuple(out.shape) != (x.shape[0], width):
