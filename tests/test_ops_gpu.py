@@ -728,6 +728,27 @@ def test_sample_from_counts_of_all_values_and_of_masked_rows(ops, monkeypatch, V
                                       R.sample_topk_topp(lg.float().numpy(), temperature, k, p, seeds, steps))
 
 
+@pytest.mark.parametrize("V", [16384, 20003])
+def test_sample_from_counts_of_few_and_many_lines(ops, monkeypatch, V):
+    """Rows whose values lie in as many lines of 32 counters as the selection takes by four keys a thread, one fewer and one more, flat
+    and steep over them.  Against the restatement."""
+    monkeypatch.setattr(ops, "SAMPLE_SPREAD_VOCAB", 0)
+    rng, lines = np.random.default_rng(V), [1, 2, 127, 128, 129, 300, 128, 129]
+    B = len(lines)
+    at = [rng.permutation(np.concatenate([np.arange(n), (n * rng.random(V - n) ** (1 if r < 6 else 6)).astype(np.int64)])) for r, n in enumerate(lines)]
+    raw = np.stack([0x4100 - 32 * a + rng.integers(0, 32, V) for a in at]).astype(np.int16)
+    lg = torch.from_numpy(raw).view(torch.bfloat16)
+    temperature = np.resize(np.array([1.0, 0.7, 3.0], dtype=np.float32), B)
+    seeds, steps = rng.integers(0, 2 ** 62, B).astype(np.int64), np.arange(B, dtype=np.int64)
+    wide = torch.zeros(B, (V + 7) // 8 * 8, dtype=torch.bfloat16, device="cuda")
+    wide[:, :V] = lg.cuda()
+    for top_k, top_p in ((0, 0.9), (0, 0.999999), (3000, 0.97), (50, 1.0), (V - 1, 1.0), (1, 0.5)):
+        k, p = np.full(B, top_k, dtype=np.int32), np.full(B, top_p, dtype=np.float32)
+        args = [torch.from_numpy(a).cuda() for a in (temperature, k, p, seeds, steps)]
+        np.testing.assert_array_equal(ops.sample(wide[:, :V], *args).cpu().numpy(),
+                                      R.sample_topk_topp(lg.float().numpy(), temperature, k, p, seeds, steps))
+
+
 @pytest.mark.parametrize("B,V", [(1, 16391), (8, 20000), (24, 16384), (40, 16391), (7, 40)])
 def test_sample_draws_decided_by_bounds(ops, monkeypatch, B, V):
     """Draws over whole rows and over nuclei that hold most of a row, which form few scores: flat rows and steep ones, temperatures

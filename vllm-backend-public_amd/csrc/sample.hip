@@ -9,6 +9,8 @@
 // exchange.  HBM-bound single pass: vocab * sizeof(logit) bytes per row.
 #include "common.h"
 
+#include <type_traits>
+
 namespace mi355 {
 
 constexpr int kArgmaxThreads = 1024;
@@ -1353,9 +1355,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(
 //                  end turns the best key into the token.  A row's workgroups repeat the selection side by side instead of waiting
 //                  for a launch that makes it once
 // What bounds it: two chains of look-ups, scans and atomics.  32 rows of 128256 logits with a mix of cuts, us a call: 27.1 as three
-// launches with two logarithms for every token that stays (count 6.5, pick 10, draw 12), here 20.8 (count 6.2, draw 14.6); top-p alone
-// 25.4 / 21.2, top-k of 50 alone 19.4 / 17.2, no cut 21.4 / 16.4; 64 rows 35.3 / 25.1, 4 rows 21.4 / 20.6 (by then the host's two
-// launches).  Rows of three values (the cut's key holds a third of them) in such a mix: 48 rows 68 / 55.  The launch
+// launches with two logarithms for every token that stays (count 6.5, pick 10, draw 12), here 19.5 (count 6.2, draw 13.3; 20.8 with eight
+// keys a thread in the selection, of whose masses two threads in five had all); top-p alone 25.4 / 20.2, top-k of 50 alone 19.4 / 17.2, no
+// cut 21.4 / 16.4; 64 rows 35.3 / 24.9, 4 rows 21.4 / 20.0 (by then the host's two launches).  Rows of three values (the cut's key holds a third of them) in such a mix: 48 rows 68 / 55.  The launch
 // per eight key bits (exact_hist_kernel), seven for bf16, takes 40.
 // fp16 keeps the passes: its rows have some ten thousand values, and the selection then takes them in several batches (16 rows
 // with a top-p 38 us by passes, 48 by counts).
@@ -1471,51 +1473,63 @@ struct CountedScratch {
   unsigned long long scratch[kSampleThreads / 64], found[2];
   uint16_t used[kCountLines];                                          // the row's lines that hold any, from the highest keys down
 };
-__device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, const uint8_t* flags, const uint16_t* counters, int parts, int K1,
-                                                  float temp, float tp, CountedScratch& sh) {
+// The smallest number of tokens of mass F > 0 that hold `need` > 0, fewer than 2^22: a quotient to 2^-20 of it, then made exact (the 64-bit
+// division is some 150 instructions one after the other).
+__device__ __forceinline__ unsigned long long tokens_for(unsigned long long need, unsigned long long F) {
+  unsigned long long t = static_cast<uint32_t>(static_cast<double>(need) * __builtin_amdgcn_rcp(static_cast<double>(F)));
+  t = t > 0ull ? t - 1ull : 0ull;
+  while (t * F < need) ++t;
+  return t;
+}
+
+// ... from the lines in use on, an item being W of a line's keys to a thread
+template <int W>
+__device__ __forceinline__ CountedCut counted_cut_of(const unsigned long long* ws, const uint8_t* flags, const uint16_t* counters, int parts, int K1,
+                                                     float temp, float tp, int lines, CountedScratch& sh) {
+  static_assert(W == 4 || W == 8, "8 or 16 bytes of counters");
+  constexpr int IL = 32 / W;                                           // items of a line
+  typedef typename std::conditional<W == 8, uint4, uint2>::type Counts;
   unsigned long long(&scratch)[kSampleThreads / 64] = sh.scratch;
   unsigned long long(&found)[2] = sh.found;
   uint16_t(&used)[kCountLines] = sh.used;
   const int tid = threadIdx.x;
-  // lines in use, highest first: thread t looks at lines 2047 - 2t and 2046 - 2t
-  const int hi = kCountLines - 1 - 2 * tid;
-  uint32_t mine = 0u;
-#pragma unroll
-  for (int c = 0; c < kCountParts; ++c) mine |= MI355_LD(uint16_t, ws, flags + (c < parts ? c : 0) * kCountLines + hi - 1);
-  unsigned long long lines, at = block_scan64((mine >> 8 & 1u) + (mine & 1u), scratch, lines);
-  if (mine & 1u) used[--at] = static_cast<uint16_t>(hi - 1);
-  if (mine >> 8 & 1u) used[--at] = static_cast<uint16_t>(hi);
-  __syncthreads();
-  const int items = static_cast<int>(lines) * 4;                       // an item: 8 keys of a line
+  const int items = lines * IL;
   // The counts of an item by key, highest first; its highest key.  No branch around a load: all of eight parts' are on
   // their way together (a line that a part has not written holds anything: its flag clears it).
-  auto load_item = [&](int item, uint32_t (&n)[8]) -> uint32_t {
+  auto load_item = [&](int item, uint32_t (&n)[W]) -> uint32_t {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) n[e] = 0u;
+    for (int e = 0; e < W; ++e) n[e] = 0u;
     if (item >= items) return 0u;
-    const int line = used[item >> 2], piece = line * 4 + 3 - (item & 3);
+    const int line = used[item / IL], piece = line * IL + IL - 1 - item % IL;
     for (int c0 = 0; c0 < parts; c0 += 8) {
-      uint4 q[8];
+      Counts q[8];
       uint32_t on[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int c = c0 + j < parts ? c0 + j : parts - 1;
         on[j] = MI355_LD(uint8_t, ws, flags + c * kCountLines + line);
-        q[j] = MI355_LD(uint4, ws, counters + c * 65536 + piece * 8);
+        q[j] = MI355_LD(Counts, ws, counters + c * 65536 + piece * W);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const uint32_t keep = on[j] != 0u && c0 + j < parts ? 0xFFFFFFFFu : 0u;
-        const uint32_t w[4] = {q[j].w & keep, q[j].z & keep, q[j].y & keep, q[j].x & keep};
+        uint32_t w[W / 2];
+        if constexpr (W == 8) w[0] = q[j].w, w[1] = q[j].z, w[2] = q[j].y, w[3] = q[j].x;
+        else w[0] = q[j].y, w[1] = q[j].x;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) n[2 * e] += w[e] >> 16, n[2 * e + 1] += w[e] & 0xFFFFu;
+        for (int e = 0; e < W / 2; ++e) n[2 * e] += (w[e] & keep) >> 16, n[2 * e + 1] += w[e] & keep & 0xFFFFu;
       }
     }
-    return static_cast<uint32_t>(piece * 8 + 7);
+    return static_cast<uint32_t>(piece * W + W - 1);
   };
-  uint32_t n[8];
+  uint32_t n[W];
   uint32_t top = load_item(tid, n);
-  auto sum8 = [&]() { return static_cast<unsigned long long>(n[0] + n[1] + n[2] + n[3] + n[4] + n[5] + n[6] + n[7]); };
+  auto sum_n = [&]() {
+    uint32_t v = 0u;
+#pragma unroll
+    for (int e = 0; e < W; ++e) v += n[e];
+    return static_cast<unsigned long long>(v);
+  };
   // batches of 1024 items (one, unless the row has more than 8192 values' worth of lines)
   int here = 0;
   auto batch = [&](int b) {
@@ -1523,10 +1537,10 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
     here = b;
   };
   const int batches = (items + kSampleThreads - 1) / kSampleThreads;
-  if (tid < 64) {                                                      // the row's largest key: of its first line's four items
+  if (tid < 64) {                                                      // the row's largest key: of its first line's items
     uint32_t k = 0u;
 #pragma unroll
-    for (int e = 7; e >= 0; --e) k = n[e] != 0u ? top - e : k;
+    for (int e = W - 1; e >= 0; --e) k = n[e] != 0u ? top - e : k;
     const unsigned long long most = wave_max64(k);
     if (tid == 0) found[0] = most;
   }
@@ -1539,10 +1553,10 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
     unsigned long long carry = 0ull;
     for (int b = 0; b < batches; ++b) {
       batch(b);
-      unsigned long long total, end = block_scan64(sum8(), scratch, total) + carry, run = end - sum8();
+      unsigned long long total, end = block_scan64(sum_n(), scratch, total) + carry, run = end - sum_n();
       if (run < need && need <= end) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < W; ++e) {
           if (run < need && run + n[e] >= need) found[1] = top - e;
           run += n[e];
         }
@@ -1557,11 +1571,11 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
   uint32_t Tp = Tk;
   unsigned long long take = ~0ull;
   if (tp < 1.0f) {
-    unsigned long long m[8], sum, Z = 0ull, end = 0ull;
+    unsigned long long m[W], sum, Z = 0ull, end = 0ull;
     auto masses = [&]() {
       sum = 0ull;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < W; ++e) {
         m[e] = n[e] != 0u && top - e >= Tk ? n[e] * sample_mass(key16_logit(top - e), l0, temp) : 0ull;
         sum += m[e];
       }
@@ -1576,7 +1590,7 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
       ++seen;
       // keys below a batch whose lowest has not half of the smallest mass have none
       if (seen < batches) {
-        const uint32_t low = static_cast<uint32_t>(used[seen * (kSampleThreads / 4) - 1]) * 32u;
+        const uint32_t low = static_cast<uint32_t>(used[seen * (kSampleThreads / IL) - 1]) * 32u;
         if (low < Tk || exp_det((key16_logit(low) - l0) / temp) * 2199023255552.0f < 1.0f) break;      // 2^41
       }
     }
@@ -1592,7 +1606,7 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
       unsigned long long run = carry + end - sum;
       if (run < P && P <= carry + end) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < W; ++e) {
           if (run < P && run + m[e] >= P) found[0] = P - run, found[1] = top - e;
           run += m[e];
         }
@@ -1603,9 +1617,29 @@ __device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, 
     __syncthreads();
     Tp = static_cast<uint32_t>(found[1]);
     const unsigned long long need = found[0], Fp = sample_mass(key16_logit(Tp), l0, temp);
-    take = Fp > 0ull ? (need + Fp - 1ull) / Fp : ~0ull;
+    take = Fp > 0ull ? tokens_for(need, Fp) : ~0ull;
   }
   return {best_key, Tp, take};
+}
+
+__device__ __forceinline__ CountedCut counted_cut(const unsigned long long* ws, const uint8_t* flags, const uint16_t* counters, int parts, int K1,
+                                                  float temp, float tp, CountedScratch& sh) {
+  unsigned long long(&scratch)[kSampleThreads / 64] = sh.scratch;
+  uint16_t(&used)[kCountLines] = sh.used;
+  const int tid = threadIdx.x;
+  // lines in use, highest first: thread t looks at lines 2047 - 2t and 2046 - 2t
+  const int hi = kCountLines - 1 - 2 * tid;
+  uint32_t mine = 0u;
+#pragma unroll
+  for (int c = 0; c < kCountParts; ++c) mine |= MI355_LD(uint16_t, ws, flags + (c < parts ? c : 0) * kCountLines + hi - 1);
+  unsigned long long lines, at = block_scan64((mine >> 8 & 1u) + (mine & 1u), scratch, lines);
+  if (mine & 1u) used[--at] = static_cast<uint16_t>(hi - 1);
+  if (mine >> 8 & 1u) used[--at] = static_cast<uint16_t>(hi);
+  __syncthreads();
+  // (rows of up to 4096 keys' worth of lines, a model's some 3000: every thread has a part of them then, not two in five)
+  const int n_lines = static_cast<int>(lines);
+  return n_lines <= kSampleThreads / 8 ? counted_cut_of<4>(ws, flags, counters, parts, K1, temp, tp, n_lines, sh)
+                                       : counted_cut_of<8>(ws, flags, counters, parts, K1, temp, tp, n_lines, sh);
 }
 
 // Gumbel-max over many tokens without two logarithms (of some forty operations) for each: as -ln u >= 1 - u, a score is at most
