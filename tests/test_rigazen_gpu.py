@@ -450,6 +450,19 @@ def test_constant_decay_in_both_forms(d, dv, decay):
         _near(_decay_in_cuts(q, k, v, decay, cuts, tiled), ref, 5e-6)      # (float32 inside: only the inputs are rounded)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,dv", [(128, 128), (136, 120), (120, 136), (8, 256)])
+def test_constant_decay_of_tiles_loaded_at_once_and_row_by_row(d, dv, dtype):
+    """Four vectors a thread of all of a tile's rows at once, or one after the other: 64 rows of 128, 56 of 144 and 32 of 256 are the largest
+    of the first kind.  The recurrence is float32 on the rounded inputs."""
+    g = torch.Generator().manual_seed(d + dv)
+    T, decay = 64 + 57 + 56 + 33 + 32 + 1, (0.97, 1.0)
+    q, k, v = (torch.randn(T, 2, n, generator=g).to(dtype) for n in (d, d, dv))
+    ref = _decay_ref(q, k, v, decay)
+    _near(_decay_in_cuts(q, k, v, decay, [64, 57, 56, 33, 32, 1], True), ref, 5e-6)
+    _near(_decay_in_cuts(q, k, v, decay, [T], True), ref, 5e-6)
+
+
 def test_a_value_written_early_is_read_far_behind():
     """Decay one: the first token's value comes back 400 tokens later through a key that nothing else uses; with
     a decay of 0.9 it is gone."""

@@ -96,6 +96,41 @@ __device__ __forceinline__ void stage_rows(float* dst, int ld, const typename El
   }
 }
 
+// The same for at most U vectors of 8 a thread of 16-bit rows, in two halves, so that the loads of all tensors of a tile (and the decays'
+// exponentials before their use) are on their way together: stage_rows waits for memory once a vector and tensor.  Tiles with more than U
+// vectors a thread (heads above 128 at 64 rows) stay with stage_rows.  8192 rows of 8 heads of 128 / 128, us: la_out 91 -> 87, la_states
+// 56 -> 54.  Lanes without a row or a column load one that is there and store zeros (n is at least 1).
+template <typename T, int U>
+struct StagedRows {
+  uint4 raw[U];
+  __device__ __forceinline__ void load(const uint16_t* base, const uint16_t* src, int64_t stride, int n, int d, int cols_p) {
+    const int per = cols_p >> 3;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = threadIdx.x + u * blockDim.x, r = i / per, c = (i - r * per) * 8;
+      raw[u] = MI355_LD(uint4, base, src + (r < n ? r : n - 1) * stride + (c < d ? c : 0));
+    }
+  }
+  __device__ __forceinline__ void store(float* dst, int ld, int n, int rows_p, int d, int cols_p, int silu, float scale, const float* row_factor) {
+    const int per = cols_p >> 3;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = threadIdx.x + u * blockDim.x, r = i / per, c = (i - r * per) * 8;
+      if (r >= rows_p) break;
+      float f[8];
+      unpack8<T>(raw[u], f);
+      const bool have = r < n && c < d;
+      const float w = row_factor != nullptr && have ? row_factor[r] : 1.0f;
+      if (silu) silu8(f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = have ? (silu ? f[j] : f[j] * scale) * w : 0.f;
+      float4* o = reinterpret_cast<float4*>(dst + r * ld + c);
+      o[0] = make_float4(f[0], f[1], f[2], f[3]);
+      o[1] = make_float4(f[4], f[5], f[6], f[7]);
+    }
+  }
+};
+
 // ---- 1: a, F, m of every row.  One workgroup per (chunk, head): its 16 waves scan a tile each (lane = row), then
 // m at the tiles' starts follows from the tiles' ends, wave by wave.  ga / gm [H][T] float, gf [H][T] double,
 // mstart [tiles][H].
@@ -173,6 +208,14 @@ __global__ __launch_bounds__(256) void la_states_kernel(
   const int64_t row0 = MI355_LD(int32_t, tiles, tiles + 3 * tile + 1);
   const int n = MI355_LD(int32_t, tiles, tiles + 3 * tile + 2);
   const int np = (n + 3) & ~3;
+  [[maybe_unused]] StagedRows<T, 4> ks, vs;
+  const bool quick = sizeof(typename Elem<T>::S) == 2 && vec && n > 0 && np * (dp >> 3) <= 4 * 256 && np * (dvp >> 3) <= 4 * 256;
+  if constexpr (sizeof(typename Elem<T>::S) == 2) {
+    if (quick) {
+      ks.load(k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, d, dp);
+      vs.load(v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, dv, dvp);
+    }
+  }
   for (int i = tid; i < n; i += blockDim.x) {
     if (MEM) {
       const int64_t at = h * total_rows + row0;
@@ -197,8 +240,15 @@ __global__ __launch_bounds__(256) void la_states_kernel(
     MI355_ST(float, ws, ws + num_tiles * D.H * D.us + static_cast<int64_t>(tile) * D.H + h, f);
   }
   __syncthreads();
-  stage_rows<T>(Ks, kl, k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, np, d, dp, !MEM, 1.0f, wr, vec);
-  stage_rows<T>(Vs, vl, v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, np, dv, dvp, !MEM, 1.0f, nullptr, vec);
+  if (quick) {
+    if constexpr (sizeof(typename Elem<T>::S) == 2) {
+      ks.store(Ks, kl, n, np, d, dp, !MEM, 1.0f, wr);
+      vs.store(Vs, vl, n, np, dv, dvp, !MEM, 1.0f, nullptr);
+    }
+  } else {
+    stage_rows<T>(Ks, kl, k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, np, d, dp, !MEM, 1.0f, wr, vec);
+    stage_rows<T>(Vs, vl, v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, np, dv, dvp, !MEM, 1.0f, nullptr, vec);
+  }
   __syncthreads();
   float* U = ws + (static_cast<int64_t>(tile) * D.H + h) * D.us;
   const int wave = tid >> 6, lane = tid & 63, li = lane & 15, kk = lane >> 4;
@@ -307,6 +357,15 @@ __global__ __launch_bounds__(512) void la_out_kernel(
   const int64_t row0 = MI355_LD(int32_t, tiles, tiles + 3 * tile + 1);
   const int n = MI355_LD(int32_t, tiles, tiles + 3 * tile + 2);
   const int np = (n + 15) & ~15;
+  [[maybe_unused]] StagedRows<T, 2> qs, ks, vs;
+  const bool quick = sizeof(typename Elem<T>::S) == 2 && vec && n > 0 && np * (dp >> 3) <= 2 * 512 && np * (dvp >> 3) <= 2 * 512;
+  if constexpr (sizeof(typename Elem<T>::S) == 2) {
+    if (quick) {
+      qs.load(q, q + row0 * q_stride + static_cast<int64_t>(h) * d, q_stride, n, d, dp);
+      ks.load(k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, d, dp);
+      vs.load(v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, dv, dvp);
+    }
+  }
   for (int i = tid; i < np; i += blockDim.x) {
     double F = 0.0;
     float a = 0.f, m = 0.f, e = 0.f;
@@ -325,9 +384,17 @@ __global__ __launch_bounds__(512) void la_out_kernel(
     }
     Fr[i] = F, ar[i] = a, mr[i] = m, er[i] = e;
   }
-  stage_rows<T>(Qs, ql, q, q + row0 * q_stride + static_cast<int64_t>(h) * d, q_stride, n, np, d, dp, !MEM, q_scale, nullptr, vec);
-  stage_rows<T>(Ks, ql, k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, np, d, dp, !MEM, 1.0f, nullptr, vec);
-  stage_rows<T>(Vs, vl, v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, np, dv, dvp, !MEM, 1.0f, nullptr, vec);
+  if (quick) {
+    if constexpr (sizeof(typename Elem<T>::S) == 2) {
+      qs.store(Qs, ql, n, np, d, dp, !MEM, q_scale, nullptr);
+      ks.store(Ks, ql, n, np, d, dp, !MEM, 1.0f, nullptr);
+      vs.store(Vs, vl, n, np, dv, dvp, !MEM, 1.0f, nullptr);
+    }
+  } else {
+    stage_rows<T>(Qs, ql, q, q + row0 * q_stride + static_cast<int64_t>(h) * d, q_stride, n, np, d, dp, !MEM, q_scale, nullptr, vec);
+    stage_rows<T>(Ks, ql, k, k + row0 * k_stride + static_cast<int64_t>(h) * d, k_stride, n, np, d, dp, !MEM, 1.0f, nullptr, vec);
+    stage_rows<T>(Vs, vl, v, v + row0 * v_stride + static_cast<int64_t>(h) * dv, v_stride, n, np, dv, dvp, !MEM, 1.0f, nullptr, vec);
+  }
   __syncthreads();
   const int wave = tid >> 6, lane = tid & 63, li = lane & 15, kk = lane >> 4, nw = blockDim.x >> 6;
   const int rb = np >> 4;
