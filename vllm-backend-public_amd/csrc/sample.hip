@@ -1473,8 +1473,9 @@ struct CountedScratch {
   unsigned long long scratch[kSampleThreads / 64], found[2];
   uint16_t used[kCountLines];                                          // the row's lines that hold any, from the highest keys down
 };
-// The smallest number of tokens of mass F > 0 that hold `need` > 0, fewer than 2^22: a quotient to 2^-20 of it, then made exact (the 64-bit
-// division is some 150 instructions one after the other).
+// The smallest number of tokens of mass F > 0 that hold `need` > 0, fewer than 2^22 (a row by counts has at most 2^20): the hardware's reciprocal is
+// within 2^-23 of itself, so that the quotient less one is never above the answer, which is counted up to from there.  (The 64-bit
+// division is some 150 instructions one after the other.)
 __device__ __forceinline__ unsigned long long tokens_for(unsigned long long need, unsigned long long F) {
   unsigned long long t = static_cast<uint32_t>(static_cast<double>(need) * __builtin_amdgcn_rcp(static_cast<double>(F)));
   t = t > 0ull ? t - 1ull : 0ull;
