@@ -93,15 +93,15 @@ def test_act_in_product_takes_what_the_tiles_take():
     import torch
     rows = lambda m, k, pad=0, dt=torch.bfloat16: torch.empty(m, k + pad, dtype=dt)[:, :k]      # noqa: E731
     w = torch.empty(8192, 2048, dtype=torch.bfloat16)
-    yes = lambda x, w=w, act=ops.ACT_GELU_MUL: ops.act_in_product(x, w, act)                     # noqa: E731
+    yes = lambda x, w=w, act=ops.LINEAR_GELU_MUL: ops.act_in_product(x, w, act)                     # noqa: E731
     assert yes(rows(8192, 2048)) and yes(rows(8192, 2048, 8)) and yes(rows(2048, 2048))
     assert not yes(rows(8192, 2048, 4)) and not yes(rows(8192, 2048, 0, torch.float32)) and not yes(rows(8192, 2048, 0, torch.float16))
     assert not yes(torch.empty(8192, 2049, dtype=torch.bfloat16)[:, 1:]) and not yes(torch.empty(2048, 8192, dtype=torch.bfloat16).t())
     assert not yes(rows(8192, 2048), torch.empty(2048, 8192, dtype=torch.bfloat16).t())
     assert not yes(rows(8192, 2048), torch.empty(8200, 2048, dtype=torch.bfloat16)) and not yes(rows(8192, 1000), torch.empty(8192, 1000, dtype=torch.bfloat16))
     assert not yes(rows(128, 2048)) and not yes(rows(300, 2048))           # decoded rows; tiles that are mostly empty
-    assert yes(rows(1280, 2048), act=ops.ACT_RELU2) and not yes(rows(1280, 2048))
-    assert not yes(rows(640, 2048), act=ops.ACT_RELU2)
+    assert yes(rows(1280, 2048), act=ops.LINEAR_RELU2) and not yes(rows(1280, 2048))
+    assert not yes(rows(640, 2048), act=ops.LINEAR_RELU2)
 
 
 def test_rows_past_rounds():
@@ -121,3 +121,10 @@ def test_wide_product_rule():
     assert not f(x, w, torch.empty(8192, 6209, dtype=torch.bfloat16)[:, :6208]) and not f(x, w, out[:, 4: 6212])
     assert not f(x, torch.empty(6144, 2048, dtype=torch.bfloat16)) and not f(x, torch.empty(6204, 2048, dtype=torch.bfloat16))
     assert not f(x[:1000], w[:2112]) and not f(x.float(), w.float()) and not f(x[:, :2040], w[:, :2040])
+
+
+def test_gated_activation_codes_are_the_abis():
+    """What the mixtures' and the row kernels' entries read; linear_act counts its activations by names of its own."""
+    assert ops._gate_act(None) == (0, 0.0) and ops._gate_act(7.0) == (1, 7.0)
+    assert (ops.ACT_SILU, ops.ACT_SIGMOID) == (0, 1)
+    assert (ops.LINEAR_RELU2, ops.LINEAR_GELU_MUL, ops.LINEAR_SILU_MUL, ops.LINEAR_LIMITED_MUL, ops.LINEAR_NONE) == (0, 1, 2, 3, 4)

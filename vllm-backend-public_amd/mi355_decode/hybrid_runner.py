@@ -593,8 +593,8 @@ class LimitedFF:
 
     def __call__(self, h: torch.Tensor, b: "StepBatch") -> torch.Tensor:
         w = self.lw.gate_up_w
-        if self.limit is not None and ops.act_in_product(h, w, ops.ACT_LIMITED_MUL):
-            return _out_product(self.r, ops.linear_act(h, w, ops.ACT_LIMITED_MUL, self.limit), self.lw.down_w)
+        if self.limit is not None and ops.act_in_product(h, w, ops.LINEAR_LIMITED_MUL):
+            return _out_product(self.r, ops.linear_act(h, w, ops.LINEAR_LIMITED_MUL, self.limit), self.lw.down_w)
         gu = self.r.linear(h, w)
         return _out_product(self.r, ops.gated_act_rows(gu[:, : self.ff], gu[:, self.ff:], self.limit), self.lw.down_w)
 
@@ -1042,7 +1042,7 @@ class HybridRunner(ModelRunner):
         if ok16 and M <= ops.LINEAR_DECODE_MAX_M and K % 32 == 0 and N % 4 == 0:
             return ops.linear_decode(x, w, bias, out=out)
         if bias is None and ops.wide_product(x, w, out):
-            return ops.linear_act(x, w, ops.ACT_NONE, out=out)
+            return ops.linear_act(x, w, ops.LINEAR_NONE, out=out)
         head = ops.rows_past_rounds(M, N) if ok16 and w.data_ptr() in self._tiled_w else 0
         if head and ops.plan_linear_tiled(N, K, True, M - head) is not None:
             if out is None:
@@ -1062,13 +1062,13 @@ class HybridRunner(ModelRunner):
         if tw is not None and tw.dtype == x.dtype and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 \
                 and ops.gelu_in_product(w.shape[0], w.shape[1], x.shape[0]):
             return ops.linear_tiled(x, tw, w.shape[0], tiles_per_wg=304, epilogue=ops.EPI_GELU_MUL)
-        if ops.act_in_product(x, w, ops.ACT_GELU_MUL):
-            return ops.linear_act(x, w, ops.ACT_GELU_MUL)
+        if ops.act_in_product(x, w, ops.LINEAR_GELU_MUL):
+            return ops.linear_act(x, w, ops.LINEAR_GELU_MUL)
         return ops.gelu_tanh_and_mul(self.linear(x, w, slabs=True))
 
     def relu2_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """max(x @ w.T, 0)^2; in one launch where that is the faster way."""
-        return ops.linear_act(x, w, ops.ACT_RELU2) if ops.act_in_product(x, w, ops.ACT_RELU2) else ops.relu_squared(self.linear(x, w))
+        return ops.linear_act(x, w, ops.LINEAR_RELU2) if ops.act_in_product(x, w, ops.LINEAR_RELU2) else ops.relu_squared(self.linear(x, w))
 
     def out_linear(self, x: torch.Tensor, w: torch.Tensor):
         """A sub-layer's last product.  In the pre arrangement its consumers (the norms that it is added ahead of, the mix)

@@ -815,8 +815,8 @@ class ModelRunner:
             self._allreduce(o)
             ops.fused_add_rms_norm(o, resid, lw.post_norm, self.eps, out=x)
             w_gu = self._rm(i, "gu")
-            if ops.act_in_product(x, w_gu, ops.ACT_SILU_MUL):
-                ops.linear_act(x, w_gu, ops.ACT_SILU_MUL, out=act)
+            if ops.act_in_product(x, w_gu, ops.LINEAR_SILU_MUL):
+                ops.linear_act(x, w_gu, ops.LINEAR_SILU_MUL, out=act)
             else:
                 torch.mm(x, w_gu.t(), out=gu)
                 ops.silu_and_mul(gu, out=act)

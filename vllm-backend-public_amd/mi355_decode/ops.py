@@ -2020,7 +2020,7 @@ def rows_past_rounds(M: int, N: int) -> int:
     return M - rest if M > 256 and 0 < rest <= 128 and N % 256 == 0 and (M >> 8) * (N >> 8) % 256 == 0 else 0
 
 
-ACT_RELU2, ACT_GELU_MUL, ACT_SILU_MUL, ACT_LIMITED_MUL, ACT_NONE = 0, 1, 2, 3, 4
+LINEAR_RELU2, LINEAR_GELU_MUL, LINEAR_SILU_MUL, LINEAR_LIMITED_MUL, LINEAR_NONE = 0, 1, 2, 3, 4
 
 
 def _wide_share(x: torch.Tensor, w: torch.Tensor, multiple: int) -> float:
@@ -2056,17 +2056,17 @@ def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
     (0.56) 44.1 / 44.4, 8192 168 / 144.  4096 inputs, 12288 outputs: 640 rows (0.81) 62.0 / 57.1, 1536 (0.65) 148 / 156, 3000 (0.76) 252 / 269.
     Gated units have more to work out at a tile's end: silu 4096 -> 28672 4096 rows (1.0) 702 / 667, 7731 (0.94) 1379 / 1265; gelu 2048 -> 8192
     8192 rows 231 / 213, 2560 (0.72) 0.98 of two launches' speed, 2048 -> 6144 6000 rows (0.76) 0.93, 4096 -> 12288 3000 rows (0.76) 0.92."""
-    return _wide_share(x, w, 64) >= (0.6 if activation == ACT_RELU2 and w.shape[1] <= 2048 else 0.8)
+    return _wide_share(x, w, 64) >= (0.6 if activation == LINEAR_RELU2 and w.shape[1] <= 2048 else 0.8)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, activation: int, limit: float = 0.0, out: torch.Tensor | None = None):
-    """a(x @ w.T) in one launch of wide matrix-core tiles: max(v, 0)^2, the product itself (ACT_NONE), or, with gate rows of w ahead of up rows, gelu_tanh(gate) * up,
+    """a(x @ w.T) in one launch of wide matrix-core tiles: max(v, 0)^2, the product itself (LINEAR_NONE), or, with gate rows of w ahead of up rows, gelu_tanh(gate) * up,
     silu(gate) * up, or the limited unit of gated_act_rows."""
     dt = _dt16(x, "x")
     N, K = w.shape
     if x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != K or not w.is_contiguous():
         raise ValueError("x must be [rows, in], w contiguous [out, in]")
-    width = N if activation in (ACT_RELU2, ACT_NONE) else N // 2
+    width = N if activation in (LINEAR_RELU2, LINEAR_NONE) else N // 2
     if out is None:
         out = torch.empty(x.shape[0], width, dtype=x.dtype, device=x.device)
     elif out.dtype != x.dtype or tuple(out.shape) != (x.shape[0], width):
