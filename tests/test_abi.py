@@ -4,6 +4,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 from conftest import ROOT
 
 HEADER = os.path.join(ROOT, "include", "mi355_decode.h")
@@ -52,6 +54,22 @@ def test_argument_validation_needs_no_gpu():
     rc = _lib.lib.mi355_paged_attn_decode(p, p, 4096, p, p, 8, p, 4, p, 2, 8, 2, 128, 0.1, 4, None, 0, 0, None)
     assert rc == -1 and b"workspace" in _lib.lib.mi355_last_error()
     assert _lib.lib.mi355_paged_attn_decode_workspace(32, 32, 128, 4) == 32 * 32 * 4 * 130 * 4
+
+
+def _fp8_product(code, rows=32, x_stride=4096, epilogue=0, k_groups=1):
+    """mi355_linear_tiled_w8 of 4096 inputs and outputs on host memory: only for calls that are refused ahead of a launch."""
+    from mi355_decode import _lib
+    buf = (ctypes.c_char * 64)()
+    p = ctypes.addressof(buf) + -ctypes.addressof(buf) % 16
+    rc = _lib.lib.mi355_linear_tiled_w8(p, 4096, p, p, x_stride, p, p, None, rows, 4096, 4096, code, k_groups, epilogue, 0, None)
+    return rc, _lib.lib.mi355_last_error()
+
+
+@pytest.mark.parametrize("code", [500, 501, 502, 503, 505, 511, 512, 550, 599, 1500, 2500, 2505, 2511])
+def test_codes_of_no_kernel_are_refused(code):
+    """Tile counts beside those that are built, none at all among them (a division by it comes behind)."""
+    rc, message = _fp8_product(code)
+    assert rc == -1 and b"504 or 506-510" in message
 
 
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):

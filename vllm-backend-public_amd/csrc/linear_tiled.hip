@@ -1171,10 +1171,10 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
   const bool kws = tiles_per_wg == 302 || tiles_per_wg == 304 || tiles_per_wg == 308 || tiles_per_wg == 402 ||
                    tiles_per_wg == 404;
   // 504, 506 .. 510: so many tiles a workgroup, K split over its four waves (linear_slices.hip), fp8 weights and up to 32 rows (of a row block)
-  const bool slices = tiles_per_wg >= 500 && tiles_per_wg < 600;
+  const bool slices = tiles_per_wg == 504 || (tiles_per_wg >= 506 && tiles_per_wg <= 510);
   const int nw = two ? (tiles_per_wg - 200) / 2 : tiles_per_wg % 100;
   MI355_REQUIRE(two || kws || slices || ((nw == 4 || nw == 8) && (tiles_per_wg == nw || tiles_per_wg == nw + 100)),
-                MI355_ERR_INVALID, "%s: tiles_per_wg must be 4, 8, 104, 108, 208-216 (even), 302, 304, 308, 402 or 404", name);
+                MI355_ERR_INVALID, "%s: tiles_per_wg must be 4, 8, 104, 108, 208-216 (even), 302, 304, 308, 402, 404, 504 or 506-510", name);
   // Rows of a row block (gridDim.z): 128, or with tiles_per_wg + 1000 / + 2000 blocks of 64 / 32 rows, each run
   // by the kernel form built for that many rows (a wave's fragments of x from LDS per weight fragment halve with
   // the block; the blocks of a column block read the same weights, once from HBM).
