@@ -687,7 +687,7 @@ int32_t mi355_tile_weights_fp8(void* dst, float* scale_tiled, const void* src,
  * Epilogues 0-2 and geometries as mi355_linear_tiled_fused (tiles_per_wg 8 or 104
  * up to 64 rows, 8 beyond); also 504, 506 .. 510 up to 32 rows (+ 2000: in blocks of 32): so many tiles
  * a workgroup, K (a multiple of 128, at least 512 a K group) split across its four waves, x straight to
- * registers; with SwiGLU an even number of tiles and rows of y on 8-byte boundaries.
+ * registers; with SwiGLU an even number of tiles and rows of y on 8-byte boundaries; the (up to 32) rows of x of a block within 4 GB.
  */
 int32_t mi355_linear_tiled_w8(void* y, int64_t y_stride, void* partial,
                               const void* x, int64_t x_stride,

@@ -72,6 +72,14 @@ def test_codes_of_no_kernel_are_refused(code):
     assert rc == -1 and b"504 or 506-510" in message
 
 
+@pytest.mark.parametrize("code,rows,stride", [(508, 32, 1 << 27), (508, 32, 69273672), (504, 9, 1 << 28), (504, 2, 1 << 31),
+                                              (2508, 64, 1 << 27), (2506, 33, 69273672), (510, 17, 1 << 62)])
+def test_rows_too_far_apart_for_32_bits_are_refused(code, rows, stride):
+    """Rows of x in registers are found by 32-bit byte offsets from the first of their block."""
+    rc, message = _fp8_product(code, rows=rows, x_stride=stride)
+    assert rc == -2 and b"within 4 GB" in message
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     import importlib
     import sys

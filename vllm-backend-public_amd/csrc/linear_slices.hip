@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256, 1) void linear_slices_kernel(LinearSlices a) {
   const int64_t unit_bytes = static_cast<int64_t>(a.tiles) * 2048;
   const int last = a.tiles - 1 - tile0;                     // tiles past the matrix: the last one again, never stored
   const char* xb = reinterpret_cast<const char*>(a.x + static_cast<int64_t>(m0) * a.x_stride) + static_cast<int64_t>(u0) * 256;
-  uint32_t xo[MT];
+  uint32_t xo[MT];                                          // (the rows of a block lie within 4 GB: linear_tiled_launch)
 #pragma unroll
   for (int m = 0; m < MT; ++m) xo[m] = static_cast<uint32_t>(min(16 * m + c, M - 1)) * static_cast<uint32_t>(a.x_stride) * 2u + 16u * h;
   vec w[2][TP], xf[2][2 * MT];

@@ -1238,6 +1238,9 @@ static int32_t linear_tiled_launch(const char* name, void* y, int64_t y_stride, 
     MI355_REQUIRE(N % 32 == 0 && bias == nullptr, MI355_ERR_UNSUPPORTED,
                   "%s: SwiGLU epilogue needs N %% 32 == 0 and no bias", name);
   if (M == 0) return MI355_OK;
+  MI355_REQUIRE(!slices || Mb == 1 || x_stride <= ((1ll << 31) - 32) / (Mb - 1), MI355_ERR_UNSUPPORTED,
+                "%s: this form's rows of x (tiles_per_wg %d, %d rows of stride %lld) must lie within 4 GB", name, tiles_per_wg, Mb,
+                static_cast<long long>(x_stride));
   const int tiles_total = (N + 15) / 16;
   const int tiles_wg = kws ? 8 / (tiles_per_wg % 100) : two ? 2 * nw : nw;
   dim3 grid((tiles_total + tiles_wg - 1) / tiles_wg, k_groups, (M + rb_rows - 1) / rb_rows);
