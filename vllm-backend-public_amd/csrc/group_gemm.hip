@@ -256,8 +256,9 @@ __device__ __forceinline__ int wide_read_int(const int* p) {
   return v;
 }
 
-// Eight units of a gated activation.  silu and the limited unit by the lean quotient while all of a wave's gates are in its range (a
-// NaN passes through it), else as they stand.
+// Eight units of a gated activation.  silu and the limited unit by the lean quotient where the gate is in its range (a NaN passes through
+// it), else as they stand: by every gate for itself, so that a unit's bits depend on its own gate and up alone.  A wave whose gates
+// are all in range skips the other form.
 template <typename T, int ACT>
 __device__ __forceinline__ void gated_units(float (&g)[8], const float (&u)[8], float limit, float (&v)[8]) {
   if constexpr (ACT == MI355_ACT_GELU_MUL) {
@@ -271,17 +272,16 @@ __device__ __forceinline__ void gated_units(float (&g)[8], const float (&u)[8], 
   for (int e = 0; e < 8; ++e) {
     if (ACT == MI355_ACT_LIMITED_MUL) g[e] = fminf(g[e], limit);
     top = fmaxf(top, fabsf(g[e]));
+    v[e] = over_one_plus_exp_lean(g[e], c * g[e]);
   }
-  auto finish = [&](int e, float q) {
-    v[e] = ACT == MI355_ACT_SILU_MUL ? round_f<T>(pin_f32(q)) * u[e] : q * (fminf(fmaxf(u[e], -limit), limit) + 1.0f);
-  };
-  if (__all(top < kSiluLeanRange / c)) {
+  if (!__all(top < kSiluLeanRange / c)) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) finish(e, over_one_plus_exp_lean(g[e], c * g[e]));
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) finish(e, g[e] / (1.0f + expf(-c * g[e])));
+    for (int e = 0; e < 8; ++e)
+      if (fabsf(g[e]) >= kSiluLeanRange / c) v[e] = g[e] / (1.0f + expf(-c * g[e]));
   }
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = ACT == MI355_ACT_SILU_MUL ? round_f<T>(pin_f32(v[e])) * u[e] : v[e] * (fminf(fmaxf(u[e], -limit), limit) + 1.0f);
 }
 
 // per: outputs of a group that lie side by side in y (experts: all n; heads: a head's); a.n: outputs of a row tile
