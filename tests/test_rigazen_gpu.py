@@ -463,6 +463,30 @@ def test_constant_decay_of_tiles_loaded_at_once_and_row_by_row(d, dv, dtype):
     _near(_decay_in_cuts(q, k, v, decay, [T], True), ref, 5e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,dv", [(128, 128), (136, 120)])
+def test_constant_decay_of_tiles_gives_the_same_bits_however_rows_lie(d, dv, dtype):
+    """Rows by vectors of eight (all at once, or one after the other) and, a column off their boundaries, by elements; numbers past the short
+    silu's range (80) beside others in a vector."""
+    from mi355_decode import ops
+    T, H, n = 200, 2, 2 * (2 * d + dv)
+    x = torch.randn(T, n, generator=torch.Generator().manual_seed(d))
+    x[::7, ::13], x[::5, ::19] = 85.0, -85.0
+    got = []
+    for shift in (0, 1):
+        buf = torch.zeros(T, n + 8, dtype=dtype, device="cuda")
+        rows = buf[:, shift: shift + n]
+        rows.copy_(x)
+        state = torch.zeros(1, H, ops.linear_attn_state_floats(d, dv, False), device="cuda")
+        cu, pos, sl = _chunk(0, T, 0)
+        ld = torch.tensor([-0.1, 0.0], dtype=torch.float64, device="cuda")
+        o = ops.decay_attn(rows[:, : H * d], rows[:, H * d: 2 * H * d], rows[:, 2 * H * d:], ld, state, cu, pos, sl, H, d, dv,
+                           tiles=ops.RowTiles([0, T], ops.linear_attn_tile_rows(d, dv), "cuda"))
+        got.append((o, state))
+    assert torch.isfinite(got[0][1]).all()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_a_value_written_early_is_read_far_behind():
     """Decay one: the first token's value comes back 400 tokens later through a key that nothing else uses; with
     a decay of 0.9 it is gone."""

@@ -40,7 +40,7 @@ struct LaDims {
   int C;                        // rows of a tile
 };
 
-// silu of eight numbers; the lean form (half the instructions) where all of them are in its range, a NaN passes through it
+// silu_any of eight numbers, by one branch where all of them are in the lean form's range (half the instructions; a NaN passes through it)
 __device__ __forceinline__ void silu8(float (&f)[8]) {
   float top = 0.f;
 #pragma unroll
@@ -50,7 +50,7 @@ __device__ __forceinline__ void silu8(float (&f)[8]) {
     for (int j = 0; j < 8; ++j) f[j] = silu_lean(f[j]);
   } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = silu_f(f[j]);
+    for (int j = 0; j < 8; ++j) f[j] = silu_any(f[j]);
   }
 }
 
@@ -90,7 +90,8 @@ __device__ __forceinline__ void stage_rows(float* dst, int ld, const typename El
     float f = 0.f;
     if (r < n && c < d) {
       f = MI355_LDF(T, base, src + r * stride + c);
-      f = (silu ? silu_f(f) : f * scale) * (row_factor != nullptr ? row_factor[r] : 1.0f);
+      // (16-bit rows: the bits of the vectors above, however they lie)
+      f = (silu ? (sizeof(typename Elem<T>::S) == 2 ? silu_any(f) : silu_f(f)) : f * scale) * (row_factor != nullptr ? row_factor[r] : 1.0f);
     }
     dst[r * ld + c] = f;
   }
