@@ -123,6 +123,20 @@ def test_wide_product_rule():
     assert not f(x[:1000], w[:2112]) and not f(x.float(), w.float()) and not f(x[:, :2040], w[:, :2040])
 
 
+def test_product_route_says_what_the_rules_say_and_is_worked_out_once():
+    import torch
+    seen = set()
+    for M in (257, 1000, 4100, 8192, 8211):
+        x = torch.empty(M, 2048, dtype=torch.bfloat16)
+        for N in (2048, 3648, 6176, 6204, 8192):
+            want = -1 if ops.wide_product(x, torch.empty(N, 2048, dtype=torch.bfloat16)) else ops.rows_past_rounds(M, N)
+            assert ops.product_route(M, N, 2048) == want
+            seen.add(min(want, 1))
+    assert seen == {-1, 0, 1}
+    misses = ops.product_route.cache_info().misses
+    assert ops.product_route(8192, 6176, 2048) == -1 and ops.product_route.cache_info().misses == misses
+
+
 def test_gated_activation_codes_are_the_abis():
     """What the mixtures' and the row kernels' entries read; linear_act counts its activations by names of its own."""
     assert ops._gate_act(None) == (0, 0.0) and ops._gate_act(7.0) == (1, 7.0)

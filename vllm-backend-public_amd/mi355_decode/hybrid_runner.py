@@ -1041,10 +1041,10 @@ class HybridRunner(ModelRunner):
                 return ops.sum_slabs(part, groups, out, bias=bias)
         if ok16 and M <= ops.LINEAR_DECODE_MAX_M and K % 32 == 0 and N % 4 == 0:
             return ops.linear_decode(x, w, bias, out=out)
-        if bias is None and ops.wide_product(x, w, out):
+        head = ops.product_route(M, N, K)
+        if head < 0 and bias is None and ops.wide_product(x, w, out):
             return ops.linear_act(x, w, ops.LINEAR_NONE, out=out)
-        head = ops.rows_past_rounds(M, N) if ok16 and w.data_ptr() in self._tiled_w else 0
-        if head and ops.plan_linear_tiled(N, K, True, M - head) is not None:
+        if head > 0 and ok16 and w.data_ptr() in self._tiled_w and ops.plan_linear_tiled(N, K, True, M - head) is not None:
             if out is None:
                 out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             self.linear(x[:head], w, out[:head], bias)

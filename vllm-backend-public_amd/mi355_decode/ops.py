@@ -8,6 +8,7 @@ new tensor (pass ``out=`` to avoid that, e.g. under HIP graph capture).
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -2023,13 +2024,9 @@ def rows_past_rounds(M: int, N: int) -> int:
 LINEAR_RELU2, LINEAR_GELU_MUL, LINEAR_SILU_MUL, LINEAR_LIMITED_MUL, LINEAR_NONE = 0, 1, 2, 3, 4
 
 
-def _wide_share(x: torch.Tensor, w: torch.Tensor, multiple: int) -> float:
-    """The share of their rounds in which linear_act's tiles have work for x @ w.T (outputs a multiple of `multiple`); 0: it does not take them."""
-    M, (N, K) = x.shape[0], w.shape
-    if x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or K % 64 or K < 128 or N % multiple or M <= LINEAR_DECODE_MAX_M \
-            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous() \
-            or M * x.stride(0) >= 1 << 31 or N * K >= 1 << 31:
-        return 0.0
+@functools.lru_cache(maxsize=4096)
+def _wide_share(M: int, N: int) -> float:
+    """The share of their rounds in which linear_act's tiles have work for M rows and N outputs."""
     # as group_gemm's wide tiles lie: rounds of 256 workgroups, in halves (tiles of 128 rows)
     col, last = -(-N // 256), M & 255
     full, rest, half = ((M >> 8) + (last > 128)) * col, col if 0 < last <= 128 else 0, -(-M // 128) * col
@@ -2038,14 +2035,40 @@ def _wide_share(x: torch.Tensor, w: torch.Tensor, multiple: int) -> float:
     return M * N / (128 * 256 * 256 * halves)
 
 
+@functools.lru_cache(maxsize=4096)
+def _wide_pays(M: int, N: int, K: int, activation: int) -> bool:
+    """Whether linear_act takes a product of this size and is the faster way (the lines: wide_product, act_in_product).  Of sizes alone, so that
+    it is worked out once for the many products of a step: asked of every product of a short prompt step, 3.5 us each of host time were
+    3 to 5 % of it (Lozupel, 400 tokens, 1.75 ms; now 0.3)."""
+    if M <= LINEAR_DECODE_MAX_M or K % 64 or K < 128 or N % (8 if activation == LINEAR_NONE else 64) or N * K >= 1 << 31:
+        return False
+    if activation == LINEAR_NONE:
+        return N % 256 != 0 and _wide_share(M, N) >= 0.75
+    return _wide_share(M, N) >= (0.6 if activation == LINEAR_RELU2 and K <= 2048 else 0.8)
+
+
+def _wide_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether linear_act's tiles can read x and w as they lie."""
+    return x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and x.stride(1) == 1 and x.stride(0) >= x.shape[1] \
+        and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous() \
+        and x.shape[0] * x.stride(0) < 1 << 31
+
+
+@functools.lru_cache(maxsize=4096)
+def product_route(M: int, N: int, K: int) -> int:
+    """Of sizes alone, what to look at for a prompt's product: -1 linear_act's tiles (then wide_product says), more than 0 the rows ahead of
+    those past whole rounds (rows_past_rounds), 0 neither."""
+    return -1 if _wide_pays(M, N, K, LINEAR_NONE) else rows_past_rounds(M, N)
+
+
 def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> bool:
     """Whether x @ w.T by linear_act's tiles is faster than by the library: outputs that end inside a tile of 256 columns, which the
     library's best kernels do not take, where the tiles' rounds are mostly work (us, bfloat16, library / tiles: 2048 -> 3648 8211 rows 135 / 101,
     4096 61 / 54, 2048 38 / 34; 2048 -> 6208 8192 rows (0.76 of the rounds) 215 / 177; 1024 -> 6720 7731 rows 151 / 105; 4096 -> 9280 3333 rows
     217 / 196; 2048 -> 3648 6189 rows (0.77) 87 / 89, 5000 (0.62) 79 / 86).  Whole columns of tiles are within 10 % either way."""
-    if w.shape[0] % 256 == 0 or (out is not None and (out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16)):
-        return False
-    return _wide_share(x, w, 8) >= 0.75
+    N, K = w.shape
+    return _wide_pays(x.shape[0], N, K, LINEAR_NONE) and _wide_takes(x, w) and \
+        (out is None or (out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))
 
 
 def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
@@ -2056,7 +2079,8 @@ def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
     (0.56) 44.1 / 44.4, 8192 168 / 144.  4096 inputs, 12288 outputs: 640 rows (0.81) 62.0 / 57.1, 1536 (0.65) 148 / 156, 3000 (0.76) 252 / 269.
     Gated units have more to work out at a tile's end: silu 4096 -> 28672 4096 rows (1.0) 702 / 667, 7731 (0.94) 1379 / 1265; gelu 2048 -> 8192
     8192 rows 231 / 213, 2560 (0.72) 0.98 of two launches' speed, 2048 -> 6144 6000 rows (0.76) 0.93, 4096 -> 12288 3000 rows (0.76) 0.92."""
-    return _wide_share(x, w, 64) >= (0.6 if activation == LINEAR_RELU2 and w.shape[1] <= 2048 else 0.8)
+    N, K = w.shape
+    return _wide_pays(x.shape[0], N, K, activation) and _wide_takes(x, w)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, activation: int, limit: float = 0.0, out: torch.Tensor | None = None):
