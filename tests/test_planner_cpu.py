@@ -123,6 +123,13 @@ def test_wide_product_rule():
     assert not f(x[:1000], w[:2112]) and not f(x.float(), w.float()) and not f(x[:, :2040], w[:, :2040])
 
 
+@pytest.mark.parametrize("M,N,K,takes", [(6189, 3648, 2048, False), (7168, 5184, 2048, False), (8211, 3648, 2048, True), (8192, 6176, 2048, True),
+                                         (4096, 5208, 2048, False), (6189, 10352, 4096, False), (8192, 4544, 3584, False), (6000, 2112, 1024, True)])
+def test_wide_products_where_they_were_the_faster_way(M, N, K, takes):
+    """Sizes on both sides of the line that were measured."""
+    assert (ops.product_route(M, N, K) == -1) == takes
+
+
 def test_product_route_says_what_the_rules_say_and_is_worked_out_once():
     import torch
     seen = set()

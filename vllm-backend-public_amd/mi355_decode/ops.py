@@ -2043,7 +2043,7 @@ def _wide_pays(M: int, N: int, K: int, activation: int) -> bool:
     if M <= LINEAR_DECODE_MAX_M or K % 64 or K < 128 or N % (8 if activation == LINEAR_NONE else 64) or N * K >= 1 << 31:
         return False
     if activation == LINEAR_NONE:
-        return N % 256 != 0 and _wide_share(M, N) >= 0.75
+        return N % 256 != 0 and K <= 2048 and _wide_share(M, N) >= (0.84 if K > 1536 and N % 192 == 0 else 0.75)
     return _wide_share(M, N) >= (0.6 if activation == LINEAR_RELU2 and K <= 2048 else 0.8)
 
 
@@ -2063,9 +2063,14 @@ def product_route(M: int, N: int, K: int) -> int:
 
 def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> bool:
     """Whether x @ w.T by linear_act's tiles is faster than by the library: outputs that end inside a tile of 256 columns, which the
-    library's best kernels do not take, where the tiles' rounds are mostly work (us, bfloat16, library / tiles: 2048 -> 3648 8211 rows 135 / 101,
-    4096 61 / 54, 2048 38 / 34; 2048 -> 6208 8192 rows (0.76 of the rounds) 215 / 177; 1024 -> 6720 7731 rows 151 / 105; 4096 -> 9280 3333 rows
-    217 / 196; 2048 -> 3648 6189 rows (0.77) 87 / 89, 5000 (0.62) 79 / 86).  Whole columns of tiles are within 10 % either way."""
+    library's best kernels do not take, where the tiles' rounds are mostly work; whole columns of tiles are within 10 % either way.  The line
+    is drawn over 35 shapes of 128 to 4096 inputs and some 40 row counts each, odd ones among them (the library's time over the tiles'):
+    up to 1536 inputs, a share of 0.75 and more, 1.02 to 2.4 (2112 outputs, 6000 rows, 1024 inputs 1.28; from 0.70 to 0.75 0.92 to 1.9);
+    2048 inputs 0.98 to 1.6 (6176 outputs, 2048 / 4096 / 8192 rows, 0.75 each, 1.17 / 1.02 / 1.25; 5208, 4202 rows 0.98; 12352, 3054 rows 0.98; below,
+    5208 outputs, 4096 rows, 0.73, 0.95; 6208, 5632 rows, 0.72, 0.92; 8256, 4096 rows, 0.69, 0.87), but widths that tiles of 192 columns divide, which
+    the library has, 0.92 to 1.15 up to a share of 0.84 (5184, 7100 rows, 0.76, 0.93; 3648, 6189 rows, 0.77, 0.98) and 1.00 to 1.4 from there on
+    (3648, 4096 / 8211 rows 1.14 / 1.4); beyond 2048 inputs the library wins here and there at any share (10352 outputs, 4096 inputs, 3531 / 6189
+    rows, 0.75 / 0.95, 0.87 / 0.97; 4544, 3584 inputs, 8192 rows 0.86), though it loses more at others (10352, 4096 rows 1.5): left to it."""
     N, K = w.shape
     return _wide_pays(x.shape[0], N, K, LINEAR_NONE) and _wide_takes(x, w) and \
         (out is None or (out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))
