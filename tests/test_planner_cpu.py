@@ -100,8 +100,13 @@ def test_act_in_product_takes_what_the_tiles_take():
     assert not yes(rows(8192, 2048), torch.empty(2048, 8192, dtype=torch.bfloat16).t())
     assert not yes(rows(8192, 2048), torch.empty(8200, 2048, dtype=torch.bfloat16)) and not yes(rows(8192, 1000), torch.empty(8192, 1000, dtype=torch.bfloat16))
     assert not yes(rows(128, 2048)) and not yes(rows(300, 2048))           # decoded rows; tiles that are mostly empty
-    assert yes(rows(1280, 2048), act=ops.LINEAR_RELU2) and not yes(rows(1280, 2048))
-    assert not yes(rows(640, 2048), act=ops.LINEAR_RELU2)
+    assert yes(rows(1500, 2048), act=ops.LINEAR_RELU2) and not yes(rows(1500, 2048))
+    assert not yes(rows(640, 2048), act=ops.LINEAR_RELU2) and not yes(rows(1280, 2048), act=ops.LINEAR_RELU2)     # (1280: 46.6 us, two launches 45.6)
+    # inputs at which the launch that is saved is a smaller part: sizes on both sides of the lines that were measured
+    sizes = lambda m, n, k, act: ops._wide_pays(m, n, k, act)                                       # noqa: E731
+    assert sizes(4096, 28672, 4096, ops.LINEAR_SILU_MUL) and sizes(512, 28672, 4096, ops.LINEAR_SILU_MUL) and not sizes(1280, 28672, 4096, ops.LINEAR_SILU_MUL)
+    assert not sizes(1500, 16384, 4096, ops.LINEAR_GELU_MUL) and sizes(8192, 16384, 4096, ops.LINEAR_GELU_MUL)
+    assert not sizes(4096, 14336, 8192, ops.LINEAR_SILU_MUL) and not sizes(7168, 14336, 8192, ops.LINEAR_SILU_MUL)
 
 
 def test_rows_past_rounds():

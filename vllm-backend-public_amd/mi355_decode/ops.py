@@ -2044,7 +2044,9 @@ def _wide_pays(M: int, N: int, K: int, activation: int) -> bool:
         return False
     if activation == LINEAR_NONE:
         return N % 256 != 0 and K <= 2048 and _wide_share(M, N) >= (0.84 if K > 1536 and N % 192 == 0 else 0.75)
-    return _wide_share(M, N) >= (0.6 if activation == LINEAR_RELU2 and K <= 2048 else 0.8)
+    if activation == LINEAR_RELU2:
+        return K <= 4096 and _wide_share(M, N) >= (0.6 if K <= 1536 else 0.67 if K <= 2048 else 0.8)
+    return K <= 4096 and _wide_share(M, N) >= (0.8 if K <= 2048 else 0.85)
 
 
 def _wide_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -2079,11 +2081,15 @@ def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = No
 def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
     """Whether linear_act takes x and w and is faster than a library product with the activation's launch behind it.  The launch moves
     2 (gated 1.5) times the product's bytes; the product itself is 4 to 8 % slower by the tiles here than by the library's, whose rounds
-    of workgroups are also finer: what counts is the share of the tiles' rounds that is work (us, two launches / one, bfloat16).
-    relu^2, 2048 inputs, 8192 outputs: 640 rows (0.54 of a round) 29.8 / 30.4, 1280 (0.62) 47.1 / 44.3, 8192 225 / 190; 6144 outputs 1536 rows
-    (0.56) 44.1 / 44.4, 8192 168 / 144.  4096 inputs, 12288 outputs: 640 rows (0.81) 62.0 / 57.1, 1536 (0.65) 148 / 156, 3000 (0.76) 252 / 269.
-    Gated units have more to work out at a tile's end: silu 4096 -> 28672 4096 rows (1.0) 702 / 667, 7731 (0.94) 1379 / 1265; gelu 2048 -> 8192
-    8192 rows 231 / 213, 2560 (0.72) 0.98 of two launches' speed, 2048 -> 6144 6000 rows (0.76) 0.93, 4096 -> 12288 3000 rows (0.76) 0.92."""
+    of workgroups are also finer: what counts is the share of the tiles' rounds that is work, and, as the launch's share of the time falls with
+    the inputs, their number.  The lines are drawn over 30 shapes of 128 to 8192 inputs and some 30 to 60 row counts each, odd ones among
+    them (bfloat16, two launches' time over one's; what is taken 0.975 to 3, 1.13 to 1.19 in the mean of each activation):
+    relu^2, up to 1536 inputs a share of 0.6 and more, 1.06 to 3; 2048 inputs 0.67, 0.99 to 1.6 (8192 outputs, 1443 / 2560 / 8192 rows 1.04 / 1.00 / 1.16;
+    below it 1280 rows, 0.62, 0.97, 2325, 0.65, 0.98; 4096 outputs, 2519 rows, 0.61, 0.96); to 4096 inputs 0.8, 1.00 to 1.5 (12288 outputs, 3000 rows,
+    0.76, 0.92).  Gated units have more to work out at a tile's end: up to 2048 inputs 0.8, 0.99 to 2.5 (gelu, 8192 outputs, 8192 rows 1.07; 4500, 0.76,
+    0.96; 6144 outputs, 6144 rows, 0.78, 0.96); to 4096 inputs 0.85, 0.98 to 1.5 (silu, 28672 outputs, 512 / 1024 / 2048 / 4096 / 7731 rows 1.07 / 1.05 / 1.01
+    / 1.05 / 1.08; 768, 0.75, 0.95, 1280, 0.75, 0.94; gelu, 16384 outputs, 1500 rows, 0.84, 0.97); beyond, the tiles cost what the launch saves (silu, 8192
+    inputs, 14336 outputs, 4096 / 7168 rows, 0.88, 0.95 / 0.94; 57344, 2304 rows, 0.98, 0.99): two launches."""
     N, K = w.shape
     return _wide_pays(x.shape[0], N, K, activation) and _wide_takes(x, w)
 
