@@ -115,6 +115,8 @@ def test_rows_past_rounds():
     assert f(8192, 2048) == 0 and f(8321, 2048) == 0                       # none, more than the stream takes at its best
     assert f(4160, 3072) == 0 and f(2100, 4096) == 0 and f(8211, 3648) == 0   # tiles that leave a round part empty
     assert f(100, 65536) == 0 and f(1, 8192) == 0
+    # few rows of wide outputs, where the stream of all the weights costs more: both sides of the line
+    assert f(1088, 16384) == 0 and f(300, 65536) == 0 and f(2176, 57344) == 0 and f(2112, 57344) == 2048 and f(3200, 16384) == 3072 and f(2176, 8192) == 2048
 
 
 def test_wide_product_rule():

@@ -2014,11 +2014,17 @@ def head_gemm(x: torch.Tensor, x_group: int, w: torch.Tensor, out: torch.Tensor,
 def rows_past_rounds(M: int, N: int) -> int:
     """How many of M rows to give a library product of N outputs where the rest, up to 128, cost less by the decode weight stream; 0: all.
     256 x 256 tiles that fill whole rounds of the 256 CUs run at the library's best, and a few rows more open another round or make it
-    choose smaller tiles for all of them (us, all by the library / the rest streamed, bfloat16): 8193 rows 2048 -> 2048 71.0 / 56.8, 8211
-    4096 -> 2048 124 / 99, 8320 2048 -> 6144 223 / 160, 4224 14336 -> 4096 707 / 348, 2112 2048 -> 8192 84 / 64, 4190 4096 -> 28672 687 / 682.
-    Where the tiles do not fill rounds the rest mostly costs more: 4160 rows 2048 -> 3072 43 / 54, 2100 4096 -> 4096 68 / 70."""
-    rest = M & 255
-    return M - rest if M > 256 and 0 < rest <= 128 and N % 256 == 0 and (M >> 8) * (N >> 8) % 256 == 0 else 0
+    choose smaller tiles for all of them.  Over 856 points of 1024 to 14336 inputs the library's time for all is 0.99 to 2.3 times that of
+    the two (us, bfloat16: 2049 rows 4096 -> 8192 129 / 104, 4224 14336 -> 4096 711 / 326, 8193 2048 -> 2048 71.0 / 56.8, 8320 2048 -> 6144 223 / 160),
+    but where the whole rounds are few rows of wide outputs, so that the stream of all the weights is much of the whole: 1088 rows
+    8192 -> 16384 241 / 326; 2176 rows 1024 -> 16384 68 / 75, 4096 -> 57344 747 / 768, with 64 rows past 2048 81 / 67 and 744 / 736.  And where the tiles
+    do not fill rounds the rest mostly costs more: 4160 rows 2048 -> 3072 43 / 54, 2100 4096 -> 4096 68 / 70.
+    Whole rounds are 256 / gcd(256, N / 256) times 256 rows: of the steps of up to 8192 tokens 1.6 % have such rows at 4096, 12288 and 28672
+    outputs, 4.7 % at 8192, 8.6 % at 16384, 3.9 % at 57344, and none at 1024 to 3072 and 6144, which need a larger token budget (8193 to 8320 rows first)."""
+    whole, rest = M & ~255, M & 255
+    if not 0 < rest <= 128 or N % 256 or whole * (N >> 8) % 65536 or whole < 2048:
+        return 0
+    return whole if rest <= 64 or whole >= 3072 or N <= 8192 else 0
 
 
 LINEAR_RELU2, LINEAR_GELU_MUL, LINEAR_SILU_MUL, LINEAR_LIMITED_MUL, LINEAR_NONE = 0, 1, 2, 3, 4
