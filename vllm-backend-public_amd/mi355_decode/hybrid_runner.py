@@ -1044,7 +1044,8 @@ class HybridRunner(ModelRunner):
         head = ops.product_route(M, N, K)
         if head < 0 and bias is None and ops.wide_product(x, w, out):
             return ops.linear_act(x, w, ops.LINEAR_NONE, out=out)
-        if head > 0 and ok16 and w.data_ptr() in self._tiled_w and ops.plan_linear_tiled(N, K, True, M - head) is not None:
+        if head > 0 and ok16 and w.data_ptr() in self._tiled_w and ops.plan_linear_tiled(N, K, True, M - head) is not None \
+                and (out is None or ops.vector_rows(out)):
             if out is None:
                 out = torch.empty(M, N, dtype=x.dtype, device=x.device)
             self.linear(x[:head], w, out[:head], bias)

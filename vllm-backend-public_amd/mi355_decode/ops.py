@@ -43,6 +43,11 @@ def _rows(t: torch.Tensor, name: str) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1])
 
 
+def vector_rows(t: torch.Tensor) -> bool:
+    """Whether the rows of a 2-D view of 16-bit numbers lie on 16-byte boundaries."""
+    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor | None = None):
     dt = _dt16(x, "x")
     _dev(weight, "weight")
@@ -2057,9 +2062,8 @@ def _wide_pays(M: int, N: int, K: int, activation: int) -> bool:
 
 def _wide_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether linear_act's tiles can read x and w as they lie."""
-    return x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and x.stride(1) == 1 and x.stride(0) >= x.shape[1] \
-        and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous() \
-        and x.shape[0] * x.stride(0) < 1 << 31
+    return x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and vector_rows(x) and x.stride(0) >= x.shape[1] \
+        and w.data_ptr() % 16 == 0 and w.is_contiguous() and x.shape[0] * x.stride(0) < 1 << 31
 
 
 @functools.lru_cache(maxsize=4096)
@@ -2081,7 +2085,7 @@ def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = No
     rows, 0.75 / 0.95, 0.87 / 0.97; 4544, 3584 inputs, 8192 rows 0.86), though it loses more at others (10352, 4096 rows 1.5): left to it."""
     N, K = w.shape
     return _wide_pays(x.shape[0], N, K, LINEAR_NONE) and _wide_takes(x, w) and \
-        (out is None or (out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0))
+        (out is None or vector_rows(out))
 
 
 def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
