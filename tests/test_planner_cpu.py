@@ -156,3 +156,24 @@ def test_gated_activation_codes_are_the_abis():
     assert ops._gate_act(None) == (0, 0.0) and ops._gate_act(7.0) == (1, 7.0)
     assert (ops.ACT_SILU, ops.ACT_SIGMOID) == (0, 1)
     assert (ops.LINEAR_RELU2, ops.LINEAR_GELU_MUL, ops.LINEAR_SILU_MUL, ops.LINEAR_LIMITED_MUL, ops.LINEAR_NONE) == (0, 1, 2, 3, 4)
+
+
+@pytest.mark.parametrize("in_product", [True, False])
+def test_prompt_layers_hold_gate_and_up_rows_only_where_no_product_takes_the_unit(monkeypatch, in_product):
+    """[tokens, 2 ff] is the largest buffer of a prompt step: made once, and only by the two-launch way."""
+    import torch
+    from types import SimpleNamespace
+    from mi355_decode.model_runner import ModelRunner
+    r, made, real = object.__new__(ModelRunner), [], torch.empty
+    r.w = SimpleNamespace(layers=[SimpleNamespace(input_norm=None, post_norm=None, qkv_b=None)] * 3)
+    r.eps, r.F, r.dtype, r.device, r.mlp_sharded = 1e-6, 24, torch.float32, "cpu", False
+    r._product = r._allreduce = lambda *a: None
+    r._rm = lambda i, kind: torch.ones(48, 16)
+    for name in ("rms_norm", "fused_add_rms_norm", "linear_act"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    monkeypatch.setattr(ops, "act_in_product", lambda *a: in_product)
+    monkeypatch.setattr(ops, "silu_and_mul", lambda gu, out: out.copy_(gu[:, :24]))
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: made.append(a) or real(*a, **k))
+    x, act = torch.ones(5, 16), torch.zeros(5, 24)
+    r._layers(5, None, x, None, None, None, act, None, lambda *a: None)
+    assert made == ([] if in_product else [(5, 48)]) and (act == (0 if in_product else 16)).all()

@@ -800,10 +800,10 @@ class ModelRunner:
         ops.sum_slabs(partial, num_slabs, out)
         self._allreduce(out)
 
-    def _layers(self, n: int, resid, x, qkv, attn, o, gu, act, dn, attend) -> torch.Tensor:
+    def _layers(self, n: int, resid, x, qkv, attn, o, act, dn, attend) -> torch.Tensor:
         """Runs all decoder layers over n packed tokens held in `resid`.  Returns the
         buffer holding the last MLP output (to be added to `resid` by the final norm)."""
-        w = self.w
+        w, gu = self.w, None                                # (gu: gate and up rows, where the product does not take the unit along)
         for i, lw in enumerate(w.layers):
             if i == 0:
                 ops.rms_norm(resid, lw.input_norm, self.eps, out=x)
@@ -818,6 +818,8 @@ class ModelRunner:
             if ops.act_in_product(x, w_gu, ops.LINEAR_SILU_MUL):
                 ops.linear_act(x, w_gu, ops.LINEAR_SILU_MUL, out=act)
             else:
+                if gu is None:
+                    gu = torch.empty(n, 2 * self.F, dtype=self.dtype, device=self.device)
                 torch.mm(x, w_gu.t(), out=gu)
                 ops.silu_and_mul(gu, out=act)
             self._product(act, i, "down", dn)
@@ -1072,7 +1074,6 @@ class ModelRunner:
         qkv = torch.empty(T, self.qw, **f)
         attn = torch.empty(T, self.nh * self.d, **f)
         o = torch.empty(T, self.H, **f)
-        gu = torch.empty(T, 2 * self.F, **f)
         act = torch.empty(T, self.F, **f)
         dn = torch.empty(T, self.H, **f)
 
@@ -1083,7 +1084,7 @@ class ModelRunner:
                                    cu_seqlens, context_lens, max_q_len, self.nh, self.nkv, self.d, self.scale,
                                    out=attn_)
 
-        last = self._layers(T, resid, x, qkv, attn, o, gu, act, dn, attend)
+        last = self._layers(T, resid, x, qkv, attn, o, act, dn, attend)
         rows = (cu_seqlens[1:] - 1).to(torch.int64)
         last_sel = last.index_select(0, rows)
         resid_sel = resid.index_select(0, rows)
