@@ -130,6 +130,13 @@ def test_wide_product_rule():
     assert not f(x[:1000], w[:2112]) and not f(x.float(), w.float()) and not f(x[:, :2040], w[:, :2040])
 
 
+def test_heads_that_stream():
+    """Sizes on both sides of the line that were measured, and no rows at all."""
+    f = ops.head_streams
+    assert f(1, 128256, 4096) and f(64, 128256, 4096) and f(64, 152064, 3584) and f(64, 64128, 4096) and f(32, 16032, 8192) and f(32, 50272, 1024)
+    assert not f(0, 128256, 4096) and not f(65, 128256, 4096) and not f(33, 16032, 8192) and not f(64, 38016, 3584) and not f(33, 50272, 1024)
+
+
 @pytest.mark.parametrize("M,N,K,takes", [(6189, 3648, 2048, False), (7168, 5184, 2048, False), (8211, 3648, 2048, True), (8192, 6176, 2048, True),
                                          (4096, 5208, 2048, False), (6189, 10352, 4096, False), (8192, 4544, 3584, False), (6000, 2112, 1024, True)])
 def test_wide_products_where_they_were_the_faster_way(M, N, K, takes):

@@ -1102,8 +1102,8 @@ class ModelRunner:
                 lg = self.full_logits(torch.mm(hs, self.w.lm_head.t()))
                 parts.append(self._logprobs(lg, targets[a:a + 1024], k))
             self.prompt_scores = torch.cat(parts, dim=0)
-        # few rows stream the head once, as in decode steps (128256 x 4096, us, library / stream: 2 rows 181 / 157, 32 rows 196 / 166)
-        plan = ops.plan_linear_tiled(self.Vl, self.H, False, xs.shape[0]) if self.lm_head_tiled is not None and 0 < xs.shape[0] <= 64 else None
+        plan = ops.plan_linear_tiled(self.Vl, self.H, False, xs.shape[0]) if self.lm_head_tiled is not None and \
+            ops.head_streams(xs.shape[0], self.Vl, self.H) else None
         logits = torch.mm(xs, self.w.lm_head.t()) if plan is None else \
             ops.linear_tiled(xs, self.lm_head_tiled, self.Vl, tiles_per_wg=plan[0])
         nxt = torch.empty(logits.shape[0], dtype=torch.int64, device=self.device)

@@ -2016,6 +2016,15 @@ def head_gemm(x: torch.Tensor, x_group: int, w: torch.Tensor, out: torch.Tensor,
     return out
 
 
+def head_streams(M: int, V: int, K: int) -> bool:
+    """Whether a head of V outputs over the M last rows of a prompt step's sequences is faster by the decode weight stream than by the library
+    (us, library / stream, bfloat16, weights out of memory): up to 32 rows all of 13 heads are (4096 -> 128256 1 / 16 / 32 rows 179 / 151, 185 / 154,
+    195 / 162; 3584 -> 152064 32 rows 251 / 171; 2048 -> 32000 30 / 23; least at 1024 -> 50272 21.0 / 20.7).  Up to 64 those of 0.5 GB and more (4096 ->
+    128256 207 / 176, 3584 -> 152064 202 / 186, 4096 -> 64128 94 / 87, 8192 -> 32064 101 / 81), where smaller ones are not always (3584 -> 38016 58.4 / 61.6, 8192 ->
+    16032 51 / 53, 4096 -> 32000 52.8 / 43.1)."""
+    return 0 < M <= (64 if V * K >= 250_000_000 else 32)
+
+
 def rows_past_rounds(M: int, N: int) -> int:
     """How many of M rows to give a library product of N outputs where the rest, up to 128, cost less by the decode weight stream; 0: all.
     256 x 256 tiles that fill whole rounds of the 256 CUs run at the library's best, and a few rows more open another round or make it
