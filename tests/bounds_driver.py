@@ -632,7 +632,7 @@ def single_launches():
 
 
 def prompt_and_latent_launches():
-    """Launches of the delta rule by chunks and of the latent attention with its keys staged."""
+    """Launches of the delta rule by chunks, of the latent attention with its keys staged and of products of many rows with their activation."""
     from mi355_decode import ops
     g, done = torch.Generator().manual_seed(3), []
     rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()      # noqa: E731
@@ -688,6 +688,13 @@ def prompt_and_latent_launches():
     q, tiles, cache_t = rnd(rows, H, 576), torch.from_numpy(ops.pair_tiles(np.array([0, rows]), H)).cuda(), cache[:, :, :512].transpose(1, 2).contiguous()
     assert ops.latent_tiles_share(len(tiles), 1, 1, n)
     checked("latent attention of shared keys", lambda: ops.latent_window_attn_tiles(q, cache, cache_t, bt, tiles, pos, None, None, 1 << 30, 0.1, max_context=n))
+    # the wide tiles: rows and outputs that end inside a tile, tiles of 128 rows alone and behind large ones, rows of x and of y apart
+    for rows, N, K in ((1, 64, 128), (300, 8192, 128), (1500, 5184, 192), (5001, 6208, 128)):
+        x, w = rnd(rows, K + 8)[:, :K], rnd(N, K)
+        for act in range(5):
+            width = N if act in (ops.LINEAR_RELU2, ops.LINEAR_NONE) else N // 2
+            y = rnd(rows, width + 8)[:, :width]
+            checked(f"linear_act {rows}x{N}x{K} {act}", lambda: ops.linear_act(x, w, act, 7.0, out=y))
     return done
 
 

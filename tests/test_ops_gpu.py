@@ -1903,7 +1903,11 @@ def test_linear_tiled_w8_swiglu(ops, M, F, K):
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("M,N,K,tiles,groups,bias", [(1, 16, 512, 504, 1, False), (16, 1000, 1152, 509, 2, True), (17, 144, 640, 507, 1, True),
-                                                     (32, 3584, 2944, 510, 5, False), (64, 1010, 1664, 2506, 3, True), (33, 336, 2048, 2508, 4, False)])
+                                                     (32, 3584, 2944, 510, 5, False), (64, 1010, 1664, 2506, 3, True), (33, 336, 2048, 2508, 4, False),
+                                                     # SwiGLU too: of each even number of tiles, 22 of them, to 16 and 32 rows and in blocks
+                                                     (1, 352, 512, 504, 1, False), (16, 352, 1152, 508, 2, False), (17, 352, 640, 506, 1, False),
+                                                     (32, 352, 1024, 504, 2, False), (33, 352, 2048, 2504, 3, False), (64, 352, 1664, 2508, 3, False),
+                                                     (49, 352, 1152, 2510, 2, False)])
 def test_linear_tiled_w8_slices(ops, dtype, M, N, K, tiles, groups, bias):
     """K split across the waves of a workgroup: tile counts that leave the last workgroup part empty, units of K that do not deal
     evenly to the waves or the K groups, row blocks of one row."""
