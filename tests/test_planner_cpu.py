@@ -106,6 +106,7 @@ def test_act_in_product_takes_what_the_tiles_take():
     sizes = lambda m, n, k, act: ops._wide_pays(m, n, k, act)                                       # noqa: E731
     assert sizes(4096, 28672, 4096, ops.LINEAR_SILU_MUL) and sizes(512, 28672, 4096, ops.LINEAR_SILU_MUL) and not sizes(1280, 28672, 4096, ops.LINEAR_SILU_MUL)
     assert not sizes(1500, 16384, 4096, ops.LINEAR_GELU_MUL) and sizes(8192, 16384, 4096, ops.LINEAR_GELU_MUL)
+    assert sizes(1789, 37888, 3584, ops.LINEAR_SILU_MUL) and not sizes(760, 32768, 4096, ops.LINEAR_SILU_MUL) and not sizes(2250, 16384, 3072, ops.LINEAR_SILU_MUL)
     assert not sizes(4096, 14336, 8192, ops.LINEAR_SILU_MUL) and not sizes(7168, 14336, 8192, ops.LINEAR_SILU_MUL)
 
 

@@ -2066,7 +2066,7 @@ def _wide_pays(M: int, N: int, K: int, activation: int) -> bool:
         return N % 256 != 0 and K <= 2048 and _wide_share(M, N) >= (0.84 if K > 1536 and N % 192 == 0 else 0.75)
     if activation == LINEAR_RELU2:
         return K <= 4096 and _wide_share(M, N) >= (0.6 if K <= 1536 else 0.67 if K <= 2048 else 0.8)
-    return K <= 4096 and _wide_share(M, N) >= (0.8 if K <= 2048 else 0.85)
+    return K <= 4096 and _wide_share(M, N) >= (0.8 if K <= 3584 else 0.87)
 
 
 def _wide_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -2091,7 +2091,8 @@ def wide_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = No
     5208 outputs, 4096 rows, 0.73, 0.95; 6208, 5632 rows, 0.72, 0.92; 8256, 4096 rows, 0.69, 0.87), but widths that tiles of 192 columns divide, which
     the library has, 0.92 to 1.15 up to a share of 0.84 (5184, 7100 rows, 0.76, 0.93; 3648, 6189 rows, 0.77, 0.98) and 1.00 to 1.4 from there on
     (3648, 4096 / 8211 rows 1.14 / 1.4); beyond 2048 inputs the library wins here and there at any share (10352 outputs, 4096 inputs, 3531 / 6189
-    rows, 0.75 / 0.95, 0.87 / 0.97; 4544, 3584 inputs, 8192 rows 0.86), though it loses more at others (10352, 4096 rows 1.5): left to it."""
+    rows, 0.75 / 0.95, 0.87 / 0.97; 4544, 3584 inputs, 8192 rows 0.86), though it loses more at others (10352, 4096 rows 1.5): left to it.  Of 81
+    sizes drawn at random inside the lines one is slower than 0.98 (768 -> 26016, 7495 rows, 0.93; the mean 1.25)."""
     N, K = w.shape
     return _wide_pays(x.shape[0], N, K, LINEAR_NONE) and _wide_takes(x, w) and \
         (out is None or vector_rows(out))
@@ -2101,14 +2102,15 @@ def act_in_product(x: torch.Tensor, w: torch.Tensor, activation: int) -> bool:
     """Whether linear_act takes x and w and is faster than a library product with the activation's launch behind it.  The launch moves
     2 (gated 1.5) times the product's bytes; the product itself is 4 to 8 % slower by the tiles here than by the library's, whose rounds
     of workgroups are also finer: what counts is the share of the tiles' rounds that is work, and, as the launch's share of the time falls with
-    the inputs, their number.  The lines are drawn over 30 shapes of 128 to 8192 inputs and some 30 to 60 row counts each, odd ones among
-    them (bfloat16, two launches' time over one's; what is taken 0.975 to 3, 1.13 to 1.19 in the mean of each activation):
-    relu^2, up to 1536 inputs a share of 0.6 and more, 1.06 to 3; 2048 inputs 0.67, 0.99 to 1.6 (8192 outputs, 1443 / 2560 / 8192 rows 1.04 / 1.00 / 1.16;
-    below it 1280 rows, 0.62, 0.97, 2325, 0.65, 0.98; 4096 outputs, 2519 rows, 0.61, 0.96); to 4096 inputs 0.8, 1.00 to 1.5 (12288 outputs, 3000 rows,
-    0.76, 0.92).  Gated units have more to work out at a tile's end: up to 2048 inputs 0.8, 0.99 to 2.5 (gelu, 8192 outputs, 8192 rows 1.07; 4500, 0.76,
-    0.96; 6144 outputs, 6144 rows, 0.78, 0.96); to 4096 inputs 0.85, 0.98 to 1.5 (silu, 28672 outputs, 512 / 1024 / 2048 / 4096 / 7731 rows 1.07 / 1.05 / 1.01
-    / 1.05 / 1.08; 768, 0.75, 0.95, 1280, 0.75, 0.94; gelu, 16384 outputs, 1500 rows, 0.84, 0.97); beyond, the tiles cost what the launch saves (silu, 8192
-    inputs, 14336 outputs, 4096 / 7168 rows, 0.88, 0.95 / 0.94; 57344, 2304 rows, 0.98, 0.99): two launches."""
+    the inputs, their number.  The lines are drawn over 41 shapes of 128 to 8192 inputs and some 30 to 60 row counts each, odd ones among
+    them, and 339 sizes drawn at random inside them (bfloat16, two launches' time over one's; what is taken 0.96 to 3, 1.16 to 1.23 in the mean
+    of each activation): relu^2, up to 1536 inputs a share of 0.6 and more, 1.06 to 3; 2048 inputs 0.67, 0.99 to 1.6 (8192 outputs, 1443 / 2560 / 8192 rows
+    1.04 / 1.00 / 1.16; below it 1280 rows, 0.62, 0.97, 2325, 0.65, 0.98; 4096 outputs, 2519 rows, 0.61, 0.96); to 4096 inputs 0.8, 1.00 to 1.5 (12288
+    outputs, 3000 rows, 0.76, 0.92).  Gated units have more to work out at a tile's end: up to 3584 inputs 0.8, 0.99 to 2.5 but for one reading of 0.96 (gelu,
+    2048 -> 8192, 8192 rows 1.07; 4500, 0.76, 0.96; 6144 outputs, 6144 rows, 0.78, 0.96; silu, 3584 -> 37888, 1021 / 1789 / 8192 rows 1.23 / 1.13 / 1.17; 3072 ->
+    16384, 2250 rows, 0.76, 0.95); to 4096 inputs 0.87, which tiles of 128 rows alone do not reach, 0.985 to 1.6 (silu, 28672 outputs, 512 / 2048 / 4096 /
+    7731 rows 1.07 / 1.01 / 1.05 / 1.08; 1384, 0.82, 0.96; 32768 outputs, 760 rows, 0.85, 0.92; gelu, 16384 outputs, 1500 rows, 0.84, 0.97); beyond, the tiles cost
+    what the launch saves (silu, 8192 inputs, 14336 outputs, 4096 / 7168 rows, 0.88, 0.95 / 0.94; 57344, 2304 rows, 0.98, 0.99): two launches."""
     N, K = w.shape
     return _wide_pays(x.shape[0], N, K, activation) and _wide_takes(x, w)
 
